@@ -101,6 +101,40 @@ def test_sgs_unsorted_rows(ctx, nb):
     assert np.array_equal(z, O.block_sgs_apply(rp, ci, v, nb, r))
 
 
+@pytest.mark.parametrize("e,width,n,dtype", [
+    (4, 1, 300, np.float64),        # a chain: one row a level
+    (5, 64, 1000, np.float64),      # a full wave, eight entries' slots
+    (8, 65, 977, np.float32),
+    (9, 130, 2000, np.float64),
+    (16, 512, 3000, np.float64),    # the widest level and the longest row
+    (17, 40, 900, np.float64),      # one entry more: the CSR walk
+    (3, 513, 3000, np.float64),     # one row more a level: the CSR walk
+    (2, 100, 18432, np.float64),    # z just fits LDS
+    (2, 100, 18433, np.float64),    # and no longer does
+    (4, 100, 36865, np.float32),
+])
+def test_sgs_level_widths_and_row_lengths(ctx, e, width, n, dtype):
+    """Row i is coupled to rows i -+ k width, k = 1..e: levels of `width`
+    rows and up to e entries on either side, with one row in seven cut short,
+    so that the level-ordered sweep meets its limits and its tails."""
+    rng = np.random.default_rng(e * 1000 + width)
+    rows = []
+    for i in range(n):
+        k = 1 if i % 7 == 3 else e
+        c = [i + d * width for d in range(-k, k + 1)]
+        rows.append([q for q in c if 0 <= q < n])
+    rp = np.concatenate([[0], np.cumsum([len(q) for q in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    v = rng.uniform(-1, 1, len(ci)).astype(dtype)
+    diag = np.repeat(np.arange(n), np.diff(rp)) == ci
+    v[diag] = 40.0 + rng.uniform(0, 1, n).astype(dtype)
+    r = rng.uniform(-1, 1, n).astype(dtype)
+    z, _ = _apply(ctx, rp, ci, v, r)
+    assert np.array_equal(z, O.sgs_apply(rp, ci, v, r))
+    z, _ = _apply(ctx, rp, ci, v, r, inplace=True)
+    assert np.array_equal(z, O.sgs_apply(rp, ci, v, r))
+
+
 def test_sgs_refuses_missing_diagonal(ctx):
     rp, ci, v = hflmp.fe_system(1, 2, 4)
     ci = ci.copy()
