@@ -79,3 +79,31 @@ def test_isolated_nodes_and_refusals(ctx):
         hflmp.FeMesh(ctx, 4, np.array([[0, 4]], np.int32))       # dof outside the mesh
     with pytest.raises(hflmp.HflmpError):
         hflmp.FeMesh(ctx, 40, np.arange(33, dtype=np.int32).reshape(1, 33))   # nloc > 32
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nnode,ncell,nloc,repeat", [
+    (300, 120, 3, False), (300, 100, 4, False),     # the narrowest groups
+    (300, 90, 5, False), (300, 60, 8, False), (500, 60, 9, False), (900, 60, 16, False),
+    (900, 60, 17, False), (1500, 60, 32, False),    # group widths and their edges
+    (33, 60, 8, False), (32, 60, 8, False),         # rows of 32 entries and more
+    (64, 200, 4, False),                            # more than 64 candidates a row
+    (200, 150, 6, True),                            # a dof twice in a cell
+])
+def test_group_widths_and_row_lengths(ctx, dtype, nnode, ncell, nloc, repeat):
+    rng = np.random.default_rng(nnode * 100 + nloc)
+    dofs = np.stack([rng.choice(nnode, nloc, replace=False) for _ in range(ncell)]).astype(np.int32)
+    if repeat:
+        dofs[::3, nloc - 1] = dofs[::3, 0]
+    mats = rng.uniform(-1, 1, (ncell, nloc, nloc)).astype(dtype)
+    E = rng.uniform(-1, 1, (nloc, nloc)).astype(dtype)
+    f = rng.uniform(0.5, 2, ncell).astype(dtype)
+    mesh = hflmp.FeMesh(ctx, nnode, dofs)
+    try:
+        for kw in (dict(cell_mats=mats), dict(E=E, factor=f), dict(E=E)):
+            rp, ci, v = _device_csr(ctx, mesh, dtype=dtype, **kw)
+            ref = kw if "E" not in kw else dict(E=E, factor=kw.get("factor", np.ones(ncell, dtype)))
+            ro, co, vo = O.fe_assemble_cells(nnode, dofs, dtype=dtype, **ref)
+            assert np.array_equal(rp, ro) and np.array_equal(ci, co) and np.array_equal(v, vo)
+    finally:
+        mesh.free()
