@@ -89,11 +89,52 @@ inline int red_blocks(hflmp_ctx *ctx, long long n) {
 }
 
 // ---- device helpers --------------------------------------------------------
+// v of lane (lane ^ OFF) for OFF 8, 4, 2, 1, where lanes that differ in the
+// bits above OFF of a row of 16 already hold the same value (as in wave_sum):
+// a rotation by 4 then reaches lane ^ 4.
+template <int OFF>
+__device__ __forceinline__ int dpp_xor(int v) {
+  constexpr int ctrl = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4E : 0xB1;
+  return __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, true);
+}
+
+// One step of wave_sum: v + v of lane ^ OFF, on every lane.
+template <int OFF, typename T>
+__device__ __forceinline__ T wave_sum_step(T v) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4 or 8 bytes");
+  constexpr int W = sizeof(T) / 4;
+  struct Words {
+    int w[W];
+  };
+  Words a = __builtin_bit_cast(Words, v), b = a;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    if constexpr (OFF >= 16) {
+      // both halves (of the wave, or of each pair of rows) hold the lower
+      // half's value in a and the upper half's in b
+      const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(a.w[i], a.w[i], false, false)
+                               : __builtin_amdgcn_permlane16_swap(a.w[i], a.w[i], false, false);
+      a.w[i] = r[0];
+      b.w[i] = r[1];
+    } else {
+      b.w[i] = dpp_xor<OFF>(a.w[i]);
+    }
+  }
+  return __builtin_bit_cast(T, a) + __builtin_bit_cast(T, b);
+}
+
+// Sum over the wave on every lane: pairs 32 apart first, then 16, ... 1.
+// The exchanges are lane swaps and DPP moves in the vector unit: through LDS
+// (__shfl_xor) each of the six dependent steps waited for two LDS round
+// trips in FP64.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
-#pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
-  return v;
+  v = wave_sum_step<32>(v);
+  v = wave_sum_step<16>(v);
+  v = wave_sum_step<8>(v);
+  v = wave_sum_step<4>(v);
+  v = wave_sum_step<2>(v);
+  return wave_sum_step<1>(v);
 }
 
 // Sum over the workgroup; the result is valid in thread 0.  `lds` must hold
