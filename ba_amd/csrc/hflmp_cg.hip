@@ -18,7 +18,8 @@
 // and F2 at the start of every workgroup of K3.
 // Every kernel returns at once when the state is no longer "iterate", so
 // the host queues iterations ahead and reads the state every `poll`
-// iterations only.
+// iterations only.  Systems of a few thousand rows run their iterations in
+// one workgroup instead (hflmp_cg_small.hpp), with the same results.
 //
 // The SpMV kernels take the operator as a value (CsrTileOp over the CSR
 // arrays or SellOp over the SELL-64 layout, hflmp_sell.hpp, or the
@@ -28,6 +29,7 @@
 #include <mutex>
 
 #include "hflmp_cg3.hpp"
+#include "hflmp_cg_small.hpp"
 #include "hflmp_sell.hpp"
 #include "hflmp_solver_common.hpp"
 #include "hflmp_stencil.hpp"
@@ -124,17 +126,50 @@ __global__ void __launch_bounds__(kBlock)
     p[i] = beta * p[i] + z[i];
 }
 
+template <typename T>
+int read_state(hflmp_ctx *ctx, const CgState<T> *st, CgState<T> *h) {
+  void *pin = static_cast<char *>(ctx->host_pinned) + 1280;
+  static_assert(sizeof(CgState<T>) <= 512, "the pinned slot ends at 1792");
+  HFLMP_HIP_CHECK(ctx, hipMemcpyAsync(pin, st, sizeof(*h), hipMemcpyDeviceToHost, ctx->stream));
+  HFLMP_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+  std::memcpy(h, pin, sizeof(*h));
+  return HFLMP_OK;
+}
+
+// The iterations of a system that fits one workgroup (hflmp_cg_small.hpp):
+// 1 and the final state in *h, 0 if it does not fit, or an error.
+template <typename Op, typename T>
+int run_small(hflmp_ctx *, const Op &, long long, int, const Cg3Grids &, const T *, T *, T *, T *,
+              CgState<T> *, int, CgState<T> *) {
+  return 0;
+}
+template <typename T, typename IT>
+int run_small(hflmp_ctx *ctx, const SellOp<T, IT> &op, long long entries, int vgrid,
+              const Cg3Grids &G, const T *invd, T *x, T *r, T *p, CgState<T> *st, int maxit,
+              CgState<T> *h) {
+  if (entries <= 0 || !small_fits(op, entries, vgrid, G)) return 0;
+  for (long long done = 0; done < maxit; done += kSmallIters) {
+    small_launch(ctx->stream, op, entries, vgrid, G, invd, x, r, p, st);
+    HFLMP_LAUNCH_CHECK(ctx);
+    const int rc = read_state(ctx, st, h);
+    if (rc) return rc;
+    if (h->status != kIterate) break;
+  }
+  return 1;
+}
+
 // The partial-sum area of the workspace is sized for the CSR tile grid,
 // which is never smaller than the SELL grid (R <= 256 rows per tile vs 256
 // rows per SELL workgroup), so one workspace size serves both operators.
 // `layout` (optional) places the state, partials and vectors differently
 // in `work` (the grids and so the results are the same); `events` false
-// polls without creating events (run_polled_sync).
+// polls without creating events (run_polled_sync).  `entries`: the stored
+// entries of a SELL-64 operator.
 template <typename Op, typename T = typename Op::value_type>
 int pcg_jacobi(hflmp_ctx *ctx, const Op &op, int nnz, const T *invd, const T *b, T *x,
                int maxit, double atol, double rtol, double dtol, void *work,
-               size_t work_bytes, hflmp_solve_info *info, const SolverLayout *layout = nullptr,
-               bool events = true) {
+               size_t work_bytes, hflmp_solve_info *info, long long entries = 0,
+               const SolverLayout *layout = nullptr, bool events = true) {
   const int nrow = op.nrow;
   HFLMP_REQUIRE(ctx, nrow > 0 && nnz > 0, "pcg: empty system");
   HFLMP_REQUIRE(ctx, invd && b && x && work && info, "pcg: null pointer");
@@ -185,12 +220,16 @@ int pcg_jacobi(hflmp_ctx *ctx, const Op &op, int nnz, const T *invd, const T *b,
     cg_beta_final<T><<<1, kFinalBlock, 0, s>>>(st, partials, g2);
     cg_p_kernel<T><<<g3, kBlock, 0, s>>>(nrow, z, p, st);
   };
-  int rc = events ? run_polled(ctx, maxit, &st->status, iteration)
-                  : run_polled_sync(ctx, maxit, &st->status, iteration);
-  if (rc) return rc;
   CgState<T> h;
-  HFLMP_HIP_CHECK(ctx, hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-  HFLMP_HIP_CHECK(ctx, hipStreamSynchronize(s));
+  const int small = run_small(ctx, op, entries, grid1, G, invd, x, r, p, st, maxit, &h);
+  if (small < 0) return small;
+  if (!small) {
+    int rc = events ? run_polled(ctx, maxit, &st->status, iteration)
+                    : run_polled_sync(ctx, maxit, &st->status, iteration);
+    if (rc) return rc;
+    rc = read_state(ctx, st, &h);
+    if (rc) return rc;
+  }
   const auto t1 = std::chrono::steady_clock::now();
   info->iters = h.iter;
   info->status = h.status == kIterate ? kMaxIts : h.status;
@@ -351,7 +390,8 @@ template <typename Op64, typename Op32>
 int mpcg_run(hflmp_ctx *ctx, const Op64 &op64, const Op32 &op32, const MpLayout &L,
              const float *invd32, const double *b, double *x, int max_outer, double atol,
              double rtol, int inner_maxit, double inner_rtol, bool reliable, void *work,
-             hflmp_mp_info *info, std::chrono::steady_clock::time_point t0) {
+             hflmp_mp_info *info, std::chrono::steady_clock::time_point t0,
+             long long entries32 = 0) {
   const int nrow = op64.nrow;
   const int grid64 = op_grid(op64), grid32 = op_grid(op32);
   char *w = static_cast<char *>(work);
@@ -403,13 +443,20 @@ int mpcg_run(hflmp_ctx *ctx, const Op64 &op64, const Op32 &op32, const MpLayout 
       cg_beta_final<float><<<1, kFinalBlock, 0, s>>>(st, part32, L.grid2);
       cg_p_kernel<float><<<g3, kBlock, 0, s>>>(nrow, z, p, st);
     };
-    rc = run_polled(ctx, inner_maxit, &st->status, iteration);
-    if (rc) return rc;
+    CgState<float> h;
+    const int small =
+        run_small(ctx, op32, entries32, grid32, G, invd32, c, r, p, st, inner_maxit, &h);
+    if (small < 0) return small;
+    if (!small) {
+      rc = run_polled(ctx, inner_maxit, &st->status, iteration);
+      if (rc) return rc;
+    }
     mp_correct_kernel<<<grid_for(nrow, 4), kBlock, 0, s>>>(nrow, c, x);
     HFLMP_LAUNCH_CHECK(ctx);
-    CgState<float> h;
-    HFLMP_HIP_CHECK(ctx, hipMemcpyAsync(&h, st, sizeof(h), hipMemcpyDeviceToHost, s));
-    HFLMP_HIP_CHECK(ctx, hipStreamSynchronize(s));
+    if (!small) {
+      rc = read_state(ctx, st, &h);
+      if (rc) return rc;
+    }
     inner_total += h.iter;
     last_breakdown = h.status == kBreakdown;
   }
@@ -504,16 +551,16 @@ int mpcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A64, const hflmp_sell *A3
     const auto o64 = sell_view<double, short>(A64);
     if (A32->col_bytes == 2)
       return mpcg_run(ctx, o64, sell_view<float, short>(A32), L, invd32, b, x, max_outer,
-                        atol, rtol, inner_maxit, inner_rtol, rel, work, info, t0);
+                        atol, rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
     return mpcg_run(ctx, o64, sell_view<float, int>(A32), L, invd32, b, x, max_outer, atol,
-                      rtol, inner_maxit, inner_rtol, rel, work, info, t0);
+                      rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
   }
   const auto o64 = sell_view<double, int>(A64);
   if (A32->col_bytes == 2)
     return mpcg_run(ctx, o64, sell_view<float, short>(A32), L, invd32, b, x, max_outer, atol,
-                      rtol, inner_maxit, inner_rtol, rel, work, info, t0);
+                      rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
   return mpcg_run(ctx, o64, sell_view<float, int>(A32), L, invd32, b, x, max_outer, atol,
-                    rtol, inner_maxit, inner_rtol, rel, work, info, t0);
+                    rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
 }
 
 template <typename T>
@@ -526,9 +573,9 @@ int pcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A, const T *invd, const T 
   HFLMP_REQUIRE(ctx, A->device == ctx->device, "pcg: matrix on another device");
   if (A->col_bytes == 2)
     return pcg_jacobi(ctx, sell_view<T, short>(A), A->nnz, invd, b, x, maxit, atol, rtol, dtol,
-                      work, work_bytes, info);
+                      work, work_bytes, info, A->entries);
   return pcg_jacobi(ctx, sell_view<T, int>(A), A->nnz, invd, b, x, maxit, atol, rtol, dtol,
-                    work, work_bytes, info);
+                    work, work_bytes, info, A->entries);
 }
 
 // ---- the allocation-free Jacobi-PCG -----------------------------------------
@@ -615,9 +662,9 @@ int pcg_jacobi_sell_noalloc(hflmp_ctx *ctx, const hflmp_sell *A, const double *i
   if (rc) return rc;
   if (A->col_bytes == 2)
     return pcg_jacobi(ctx, sell_view<double, short>(A), A->nnz, invd, b, x, maxit, atol, rtol,
-                      dtol, work, kNoAllocBytes, info, &L, false);
+                      dtol, work, kNoAllocBytes, info, A->entries, &L, false);
   return pcg_jacobi(ctx, sell_view<double, int>(A), A->nnz, invd, b, x, maxit, atol, rtol,
-                    dtol, work, kNoAllocBytes, info, &L, false);
+                    dtol, work, kNoAllocBytes, info, A->entries, &L, false);
 }
 
 // One-entry rows give 256-row tiles in solver_layout, the stencil grid.

@@ -1,0 +1,239 @@
+// Jacobi-PCG of a small SELL-64 system in one workgroup.
+//
+// A system of a few thousand rows spends its iteration in launches: the
+// three kernels of hflmp_cg3.hpp take 3.3 + 3.4 + 3.0 us and the gaps between
+// them 3 us on 1,089 rows, whatever the rows cost (12.9 us an iteration).  Here one workgroup runs the iterations with p in LDS, x, r
+// and D^-1 in registers and the matrix read from LDS where it fits, else
+// from L2; the grid-wide sums become three barriers.  2D Q1 32^2 with
+// log-normal diffusivity to 1e-8: 1.78 -> 0.36 ms, 3.4 us an iteration.
+//
+// The iterates are the three-launch form's, bit for bit, so that a system
+// gives the same result whichever form runs it: every sum is formed from
+// the same terms in the same order (per 256-row unit as its workgroups do,
+// the unit's partials in the launch's workgroup order, the update's
+// partials by its workgroups of 256 threads and four elements each), and
+// every product and sum is rounded as there.
+#pragma once
+
+#include "hflmp_cg3.hpp"
+
+namespace {
+
+constexpr int kSmallRows = 8192;           // two sets of 4 elements for 1024 threads
+constexpr size_t kSmallLds = 152 * 1024;
+// Entries' bytes beyond which the L2 of one CU is slower than three launches
+// (64 B a clock: about 150 GB/s).
+constexpr size_t kSmallBytes = 768 * 1024;
+constexpr int kSmallIters = 512;           // iterations of one launch, at most
+
+struct CgSmallArgs {
+  int vgrid, g2;  // units and update workgroups of the three-launch form
+  int entries;    // stored entries of the operator
+};
+
+// LDS: p, Ap | wave sums of p.Ap (one a slice) | wave sums of r.r and r.z
+// (four an update workgroup) | MLDS: values | slices' first entries and
+// lengths | MLDS: columns | row lengths.
+constexpr int kSmallSlices = kSmallRows / kSellRows;
+constexpr int kSmallSums = kSmallSlices + 2 * 4 * (kSmallRows / (4 * kBlock));
+template <typename T, typename IT>
+inline size_t small_lds_bytes(int nrow, long long entries, bool mlds) {
+  const size_t nr = ((size_t)nrow + kSellRows - 1) / kSellRows * kSellRows;
+  return (2 * nr + kSmallSums) * sizeof(T) + 8 * (size_t)kSmallSlices + nr +
+         (mlds ? (size_t)entries * (sizeof(T) + sizeof(IT)) : 0);
+}
+
+// The update's elements are its workgroups': vthread v (workgroup v / 256,
+// thread v % 256, v = j 1024 + thread of this workgroup) has elements v + q
+// g2 256, q < 4, in registers.  The product walks the slices by wave and
+// passes Ap through LDS.
+template <typename T, typename IT, int J, bool MLDS>
+__global__ void __launch_bounds__(kFinalBlock)
+    cg_small_kernel(SellOp<T, IT> op, CgSmallArgs a, const T *__restrict__ invd,
+                    T *__restrict__ xg, T *__restrict__ rg, T *__restrict__ pg,
+                    CgState<T> *st) {
+#pragma clang fp contract(off)
+  constexpr int U = sizeof(T) == 8 ? 4 : 3;  // fits the 128 registers of 1024 threads
+  extern __shared__ __align__(16) unsigned char small_lds[];
+  if (st->status != kIterate) return;
+  const unsigned n = op.nrow, nr = op.nslice * kSellRows;
+  T *ps = reinterpret_cast<T *>(small_lds);
+  T *aps = ps + nr;
+  T *sumA = aps + nr;
+  T *sumB = sumA + kSmallSlices;
+  T *vals = sumA + kSmallSums;
+  int *soff = reinterpret_cast<int *>(vals + (MLDS ? a.entries : 0));
+  int *slen = soff + kSmallSlices;
+  IT *cols = reinterpret_cast<IT *>(slen + kSmallSlices);
+  unsigned char *rlen = reinterpret_cast<unsigned char *>(cols + (MLDS ? a.entries : 0));
+  const int t = threadIdx.x, lane = t & (kWave - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(t / kWave);
+  const unsigned stride = a.g2 * kBlock;
+  if (MLDS) {
+    for (int e = t; e < a.entries; e += kFinalBlock) {
+      vals[e] = op.val[e];
+      cols[e] = op.col[e];
+    }
+  }
+  for (unsigned i = t; i < nr; i += kFinalBlock) rlen[i] = i < n ? op.rlen[i] : 0;
+  if (t < op.nslice) {
+    soff[t] = (int)op.soff[t];
+    slen[t] = op.slen[t];
+  }
+  T x[J][4], r[J][4], d[J][4];
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const unsigned v = j * kFinalBlock + t, i = v + q * stride;
+      const bool ok = v < stride && i < n;
+      x[j][q] = ok ? xg[i] : T(0);
+      r[j][q] = ok ? rg[i] : T(0);
+      d[j][q] = ok ? invd[i] : T(0);
+      if (ok) ps[i] = pg[i];
+    }
+  T rz = st->rz;
+  const double res0 = (double)st->res0, atol = st->atol, rtol = st->rtol, dtol = st->dtol;
+  const int maxit = st->maxit;
+  int iter = st->iter, status = kIterate;
+  T pAp = 0, alpha = 0, rr = 0, res = st->res, beta = st->beta;
+  __syncthreads();
+  for (int k = 0; k < kSmallIters; ++k) {
+    // Ap = A p and the waves' sums of p.Ap
+#pragma unroll 1
+    for (int sl = wid; sl < op.nslice; sl += kFinalBlock / kWave) {
+      const unsigned row = sl * kSellRows + lane;
+      const int len = rlen[row];
+      const int base = __builtin_amdgcn_readfirstlane(soff[sl]);
+      const int smax = __builtin_amdgcn_readfirstlane(slen[sl]);
+      const T *xx = std::is_same<IT, int>::value ? ps : ps + sl * kSellRows;
+      const T s = MLDS ? sell_slice_sum<T, IT, false, false, true, false, U, true>(
+                             cols + base, vals + base, smax, len, lane, xx, 0, T(0))
+                       : sell_slice_sum<T, IT, false, false, true, false, U, true>(
+                             op.col + base, op.val + base, smax, len, lane, xx, 0, T(0));
+      T acc = T(0);
+      if (row < n) {
+        aps[row] = s;
+        acc = __builtin_elementwise_fma(s, ps[row], T(0));
+      }
+      acc = wave_sum(acc);
+      if (lane == 0) sumA[sl] = acc;
+    }
+    __syncthreads();
+    {
+      // partial of workgroup b: unit xcd_tile(b)'s four waves in order
+      const int unit = (int)xcd_tile(lane, a.vgrid);
+      T part = T(0);
+      if (lane < a.vgrid) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          part += unit * 4 + w < op.nslice ? sumA[unit * 4 + w] : T(0);
+      }
+      pAp = T(0) + wave_sum(part);
+    }
+    if (pAp == T(0) || !(pAp == pAp)) {
+      status = kBreakdown;
+      break;
+    }
+    alpha = rz / pAp;
+    const T malpha = -alpha;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const unsigned v = j * kFinalBlock + t;
+      if (__builtin_amdgcn_readfirstlane(v) >= stride) continue;
+      T arr = 0, arz = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const unsigned i = v + q * stride;
+        if (i < n) {
+          x[j][q] = __builtin_elementwise_fma(alpha, ps[i], x[j][q]);
+          r[j][q] = __builtin_elementwise_fma(malpha, aps[i], r[j][q]);
+          const T z = r[j][q] * d[j][q];
+          arr = __builtin_elementwise_fma(r[j][q], r[j][q], arr);
+          arz = __builtin_elementwise_fma(r[j][q], z, arz);
+        }
+      }
+      arr = wave_sum(arr);
+      arz = wave_sum(arz);
+      if (lane == 0) {
+        sumB[2 * (v / kWave)] = arr;
+        sumB[2 * (v / kWave) + 1] = arz;
+      }
+    }
+    __syncthreads();
+    T prr = T(0), prz = T(0);
+    if (lane < a.g2) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        prr += sumB[2 * (4 * lane + w)];
+        prz += sumB[2 * (4 * lane + w) + 1];
+      }
+    }
+    rr = T(0) + wave_sum(prr);
+    const T rzn = T(0) + wave_sum(prz);
+    ++iter;
+    res = sqrt(rr);
+    status = check_state(iter, (double)res, res0, maxit, atol, rtol, dtol);
+    if (status != kIterate) break;
+    beta = rzn / rz;
+    rz = rzn;
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const unsigned v = j * kFinalBlock + t, i = v + q * stride;
+        if (v < stride && i < n) {
+          const T z = r[j][q] * d[j][q];
+          ps[i] = __builtin_elementwise_fma(beta, ps[i], z);
+        }
+      }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const unsigned v = j * kFinalBlock + t, i = v + q * stride;
+      if (v < stride && i < n) {
+        xg[i] = x[j][q];
+        rg[i] = r[j][q];
+        pg[i] = ps[i];
+      }
+    }
+  if (t == 0) {
+    st->rz = rz;
+    st->pAp = pAp;
+    st->alpha = alpha;
+    st->beta = beta;
+    st->rr = rr;
+    st->res = res;
+    st->iter = iter;
+    st->status = status;
+  }
+}
+
+// Whether the one-workgroup form runs this system in place of launches with
+// the grids G over vgrid units, and how.  The unit partials are summed by
+// one wave (vgrid <= 64) in the order of launches of one unit a workgroup
+// (G.g1 == vgrid).
+template <typename T, typename IT>
+bool small_fits(const SellOp<T, IT> &op, long long entries, int vgrid, const Cg3Grids &G) {
+  return op.nrow <= kSmallRows && vgrid <= kWave && G.g1 == vgrid && G.g2 * 4 * kBlock >= op.nrow &&
+         G.g2 <= kSmallRows / (4 * kBlock) &&
+         (size_t)entries * (sizeof(T) + sizeof(IT)) <= kSmallBytes;
+}
+
+template <typename T, typename IT>
+void small_launch(hipStream_t s, const SellOp<T, IT> &op, long long entries, int vgrid,
+                  const Cg3Grids &G, const T *invd, T *x, T *r, T *p, CgState<T> *st) {
+  const CgSmallArgs a{vgrid, G.g2, (int)entries};
+  const bool mlds = small_lds_bytes<T, IT>(op.nrow, entries, true) <= kSmallLds;
+  const size_t lds = small_lds_bytes<T, IT>(op.nrow, entries, mlds);
+  auto go = [&](auto kern) { kern<<<1, kFinalBlock, lds, s>>>(op, a, invd, x, r, p, st); };
+  if (G.g2 <= 4)
+    mlds ? go(cg_small_kernel<T, IT, 1, true>) : go(cg_small_kernel<T, IT, 1, false>);
+  else
+    mlds ? go(cg_small_kernel<T, IT, 2, true>) : go(cg_small_kernel<T, IT, 2, false>);
+}
+
+}  // namespace

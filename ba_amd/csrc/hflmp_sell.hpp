@@ -103,14 +103,21 @@ struct CsrTileOp {
 // column is dcol skipped).  smax: the slice's entries per lane.  The loads
 // cover the row's own entries, or with LOAD_ALL every entry position of the
 // slice (all allocated: 64 x smax entries), so that they need not wait for
-// len; the sum is the same either way.
-template <typename T, typename IT, bool SUB, bool NODIAG, bool LOAD_ALL>
+// len; the sum is the same either way.  NT: entries are loaded past the
+// caches (they are read once a launch).  U: chunk loads in flight per step.
+// GATHER_ALL: x is read for every entry loaded, padding included (its
+// column is 0; for an x that is cheap to read and has no limit to guard).
+template <typename V, bool NT>
+__device__ __forceinline__ V sell_ld(const V *p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
+}
+template <typename T, typename IT, bool SUB, bool NODIAG, bool LOAD_ALL, bool NT = true,
+          int U = SellChunk<T>::U, bool GATHER_ALL = false>
 __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T *__restrict__ val,
                                             int smax, int len, int lane,
                                             const T *__restrict__ x, int dcol, T s) {
 #pragma clang fp contract(off)
   constexpr int P = SellChunk<T>::P;
-  constexpr int U = SellChunk<T>::U;
   typedef typename VecOf<T, P>::type TV;
   typedef typename VecOf<IT, P>::type IV;
   const int full = smax / P * P;  // entries in P-chunks; the rest one per block
@@ -127,8 +134,8 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
   for (int t = 0; t < TM; ++t) {
     if (t < nload) {
       const long long q = (long long)kSellRows * (full + t) + lane;
-      ct[t] = __builtin_nontemporal_load(col + q);
-      vt[t] = __builtin_nontemporal_load(val + q);
+      ct[t] = sell_ld<IT, NT>(col + q);
+      vt[t] = sell_ld<T, NT>(val + q);
     }
   }
   for (int j = 0; j < full; j += P * U) {
@@ -137,8 +144,8 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if ((LOAD_ALL || j + u * P < len) && j + u * P < full) {
-        cc[u] = __builtin_nontemporal_load(c + (j / P + u) * kWave);
-        vv[u] = __builtin_nontemporal_load(v + (j / P + u) * kWave);
+        cc[u] = sell_ld<IV, NT>(c + (j / P + u) * kWave);
+        vv[u] = sell_ld<TV, NT>(v + (j / P + u) * kWave);
       }
     }
     T xx[U][P];
@@ -146,23 +153,31 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int q = 0; q < P; ++q)
-        if (j + u * P + q < len && j + u * P < full) xx[u][q] = x[(int)cc[u][q]];
+        if ((GATHER_ALL || j + u * P + q < len) && j + u * P < full) xx[u][q] = x[(int)cc[u][q]];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int q = 0; q < P; ++q)
+      for (int q = 0; q < P; ++q) {
+        if (GATHER_ALL && !SUB && !NODIAG) {
+          if (j + u * P < full) {
+            const T sn = s + vv[u][q] * xx[u][q];
+            s = j + u * P + q < len ? sn : s;
+          }
+          continue;
+        }
         if (j + u * P + q < len && j + u * P < full && (!NODIAG || (int)cc[u][q] != dcol)) {
           if (SUB)
             s -= vv[u][q] * xx[u][q];
           else
             s += vv[u][q] * xx[u][q];
         }
+      }
   }
   // the tail, in ascending order after the chunks
   T xt[TM];
 #pragma unroll
   for (int t = 0; t < TM; ++t)
-    if (t < ntail) xt[t] = x[(int)ct[t]];
+    if (t < (GATHER_ALL ? nload : ntail)) xt[t] = x[(int)ct[t]];
 #pragma unroll
   for (int t = 0; t < TM; ++t)
     if (t < ntail && (!NODIAG || (int)ct[t] != dcol)) {
