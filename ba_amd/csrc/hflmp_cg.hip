@@ -138,24 +138,28 @@ int read_state(hflmp_ctx *ctx, const CgState<T> *st, CgState<T> *h) {
 
 // The iterations of a system that fits one workgroup (hflmp_cg_small.hpp):
 // 1 and the final state in *h, 0 if it does not fit, or an error.
-template <typename Op, typename T>
-int run_small(hflmp_ctx *, const Op &, long long, int, const Cg3Grids &, const T *, T *, T *, T *,
-              CgState<T> *, int, CgState<T> *) {
-  return 0;
-}
+template <typename Op>
+struct IsSell : std::false_type {};
 template <typename T, typename IT>
-int run_small(hflmp_ctx *ctx, const SellOp<T, IT> &op, long long entries, int vgrid,
-              const Cg3Grids &G, const T *invd, T *x, T *r, T *p, CgState<T> *st, int maxit,
-              CgState<T> *h) {
-  if (entries <= 0 || !small_fits(op, entries, vgrid, G)) return 0;
-  for (long long done = 0; done < maxit; done += kSmallIters) {
-    small_launch(ctx->stream, op, entries, vgrid, G, invd, x, r, p, st);
-    HFLMP_LAUNCH_CHECK(ctx);
-    const int rc = read_state(ctx, st, h);
-    if (rc) return rc;
-    if (h->status != kIterate) break;
+struct IsSell<SellOp<T, IT>> : std::true_type {};
+template <typename T>
+struct IsSell<SellOffOp<T>> : std::true_type {};
+
+template <typename Op, typename T>
+int run_small(hflmp_ctx *ctx, const Op &op, long long entries, int vgrid, const Cg3Grids &G,
+              const T *invd, T *x, T *r, T *p, CgState<T> *st, int maxit, CgState<T> *h) {
+  if constexpr (IsSell<Op>::value) {
+    if (entries <= 0 || !small_fits(op, entries, vgrid, G)) return 0;
+    for (long long done = 0; done < maxit; done += kSmallIters) {
+      small_launch(ctx->stream, op, entries, vgrid, G, invd, x, r, p, st);
+      HFLMP_LAUNCH_CHECK(ctx);
+      const int rc = read_state(ctx, st, h);
+      if (rc) return rc;
+      if (h->status != kIterate) break;
+    }
+    return 1;
   }
-  return 1;
+  return 0;
 }
 
 // The partial-sum area of the workspace is sized for the CSR tile grid,
@@ -546,21 +550,13 @@ int mpcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A64, const hflmp_sell *A3
   HFLMP_REQUIRE(ctx, (flags & ~HFLMP_MP_RELIABLE) == 0, "mpcg: unknown flags %d", flags);
   const bool rel = (flags & HFLMP_MP_RELIABLE) != 0;
   const auto t0 = std::chrono::steady_clock::now();
-  // four instantiations: int32 or int16 columns in each precision
-  if (A64->col_bytes == 2) {
-    const auto o64 = sell_view<double, short>(A64);
-    if (A32->col_bytes == 2)
-      return mpcg_run(ctx, o64, sell_view<float, short>(A32), L, invd32, b, x, max_outer,
-                        atol, rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
-    return mpcg_run(ctx, o64, sell_view<float, int>(A32), L, invd32, b, x, max_outer, atol,
-                      rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
-  }
-  const auto o64 = sell_view<double, int>(A64);
-  if (A32->col_bytes == 2)
-    return mpcg_run(ctx, o64, sell_view<float, short>(A32), L, invd32, b, x, max_outer, atol,
-                      rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
-  return mpcg_run(ctx, o64, sell_view<float, int>(A32), L, invd32, b, x, max_outer, atol,
-                    rtol, inner_maxit, inner_rtol, rel, work, info, t0, A32->entries);
+  // any form (offsets, int16 or int32 columns) in each precision
+  return sell_dispatch<double>(A64, [&](auto o64) {
+    return sell_dispatch<float>(A32, [&](auto o32) {
+      return mpcg_run(ctx, o64, o32, L, invd32, b, x, max_outer, atol, rtol, inner_maxit,
+                      inner_rtol, rel, work, info, t0, A32->entries);
+    });
+  });
 }
 
 template <typename T>
@@ -571,11 +567,10 @@ int pcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A, const T *invd, const T 
   HFLMP_REQUIRE(ctx, A != nullptr, "pcg: null matrix");
   HFLMP_REQUIRE(ctx, A->value_bytes == (int)sizeof(T), "pcg: value type mismatch");
   HFLMP_REQUIRE(ctx, A->device == ctx->device, "pcg: matrix on another device");
-  if (A->col_bytes == 2)
-    return pcg_jacobi(ctx, sell_view<T, short>(A), A->nnz, invd, b, x, maxit, atol, rtol, dtol,
-                      work, work_bytes, info, A->entries);
-  return pcg_jacobi(ctx, sell_view<T, int>(A), A->nnz, invd, b, x, maxit, atol, rtol, dtol,
-                    work, work_bytes, info, A->entries);
+  return sell_dispatch<T>(A, [&](auto op) {
+    return pcg_jacobi(ctx, op, A->nnz, invd, b, x, maxit, atol, rtol, dtol, work, work_bytes, info,
+                      A->entries);
+  });
 }
 
 // ---- the allocation-free Jacobi-PCG -----------------------------------------
@@ -660,11 +655,10 @@ int pcg_jacobi_sell_noalloc(hflmp_ctx *ctx, const hflmp_sell *A, const double *i
   void *work = nullptr;
   int rc = scratch_on_device(ctx, &work);
   if (rc) return rc;
-  if (A->col_bytes == 2)
-    return pcg_jacobi(ctx, sell_view<double, short>(A), A->nnz, invd, b, x, maxit, atol, rtol,
-                      dtol, work, kNoAllocBytes, info, A->entries, &L, false);
-  return pcg_jacobi(ctx, sell_view<double, int>(A), A->nnz, invd, b, x, maxit, atol, rtol,
-                    dtol, work, kNoAllocBytes, info, A->entries, &L, false);
+  return sell_dispatch<double>(A, [&](auto op) {
+    return pcg_jacobi(ctx, op, A->nnz, invd, b, x, maxit, atol, rtol, dtol, work, kNoAllocBytes,
+                      info, A->entries, &L, false);
+  });
 }
 
 // One-entry rows give 256-row tiles in solver_layout, the stencil grid.

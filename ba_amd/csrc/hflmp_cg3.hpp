@@ -81,7 +81,8 @@ struct UnitWalk<StencilOp<T, DIM, ORDER, MULTI>> : std::false_type {};
 // K1: Ap = A p over all units; one partial of p.Ap per workgroup.  At least
 // five waves per SIMD, so that every SELL-64 FP64 form (int16 or int32
 // columns) runs the same grid and the sums, and so the iterates, do not
-// depend on the column width.
+// depend on the column width.  (The offset form takes the grid of int16
+// columns: GridOp.)
 template <typename Op, typename T = typename Op::value_type>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
     cg3_spmv_kernel(Op op, int vgrid, const T *__restrict__ p, T *__restrict__ Ap,
@@ -216,13 +217,24 @@ struct Cg3Grids {
   int g1, g2;
 };
 
+// The operator whose K1 decides the grid.
+template <typename Op>
+struct GridOp {
+  using type = Op;
+};
+template <typename T>
+struct GridOp<SellOffOp<T>> {
+  using type = SellOp<T, short>;
+};
+
 template <typename Op>
 Cg3Grids cg3_grids(hflmp_ctx *ctx, int vgrid, int grid2, int gmax) {
   long long g1 = vgrid;
   if constexpr (UnitWalk<Op>::value) {
     int occ = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &occ, reinterpret_cast<const void *>(&cg3_spmv_kernel<Op>), kBlock, 0) !=
+            &occ, reinterpret_cast<const void *>(&cg3_spmv_kernel<typename GridOp<Op>::type>),
+            kBlock, 0) !=
             hipSuccess ||
         occ < 1)
       occ = 1;

@@ -26,6 +26,18 @@ constexpr size_t kSmallLds = 152 * 1024;
 constexpr size_t kSmallBytes = 768 * 1024;
 constexpr int kSmallIters = 512;           // iterations of one launch, at most
 
+// Bytes of a stored column of an operator over SELL-64.
+template <typename Op>
+struct ColBytes;
+template <typename T, typename IT>
+struct ColBytes<SellOp<T, IT>> {
+  static constexpr size_t value = sizeof(IT);
+};
+template <typename T>
+struct ColBytes<SellOffOp<T>> {
+  static constexpr size_t value = 0;
+};
+
 struct CgSmallArgs {
   int vgrid, g2;  // units and update workgroups of the three-launch form
   int entries;    // stored entries of the operator
@@ -36,24 +48,63 @@ struct CgSmallArgs {
 // lengths | MLDS: columns | row lengths.
 constexpr int kSmallSlices = kSmallRows / kSellRows;
 constexpr int kSmallSums = kSmallSlices + 2 * 4 * (kSmallRows / (4 * kBlock));
-template <typename T, typename IT>
+template <typename Op>
 inline size_t small_lds_bytes(int nrow, long long entries, bool mlds) {
+  const size_t vb = sizeof(typename Op::value_type);
   const size_t nr = ((size_t)nrow + kSellRows - 1) / kSellRows * kSellRows;
-  return (2 * nr + kSmallSums) * sizeof(T) + 8 * (size_t)kSmallSlices + nr +
-         (mlds ? (size_t)entries * (sizeof(T) + sizeof(IT)) : 0);
+  return (2 * nr + kSmallSums) * vb + 8 * (size_t)kSmallSlices + nr +
+         (mlds ? (size_t)entries * (vb + ColBytes<Op>::value) : 0);
+}
+
+// The product of one slice (one wave, its row's sum) from the small kernel's
+// LDS: the slice's entries start at base of val / col (LDS copies or the
+// operator's arrays), m the longest row or the offsets.
+template <typename T, typename IT>
+__device__ __forceinline__ T small_slice(const SellOp<T, IT> &, const T *val, const IT *col,
+                                         int base, int m, int len, int sl, int, int lane,
+                                         const T *ps, unsigned) {
+  constexpr int U = sizeof(T) == 8 ? 4 : 3;  // fits the 128 registers of 1024 threads
+  const T *x = std::is_same<IT, int>::value ? ps : ps + sl * kSellRows;
+  return sell_slice_sum<T, IT, false, false, true, false, U, true>(col + base, val + base, m, len,
+                                                                   lane, x, 0, T(0));
+}
+template <typename T>
+__device__ __forceinline__ T small_slice(const SellOffOp<T> &op, const T *val, const char *,
+                                         int base, int m, int, int, int row, int lane,
+                                         const T *ps, unsigned n) {
+  return sell_offset_sum<T, false, false, false>(
+      val + base, scalar_ptr(op.off) + base / kSellRows, scalar_ptr(op.mask) + base / kSellRows,
+      m, row, lane, [&](int c) { return ps[(unsigned)c < n ? c : 0]; }, T(0));
+}
+template <typename T, typename IT>
+__device__ __forceinline__ const IT *small_cols(const SellOp<T, IT> &op) {
+  return op.col;
+}
+template <typename T>
+__device__ __forceinline__ const char *small_cols(const SellOffOp<T> &) {
+  return nullptr;
+}
+template <typename T, typename IT>
+__device__ __forceinline__ int small_len(const SellOp<T, IT> &op, unsigned i) {
+  return op.rlen[i];
+}
+template <typename T>
+__device__ __forceinline__ int small_len(const SellOffOp<T> &, unsigned) {
+  return 0;
 }
 
 // The update's elements are its workgroups': vthread v (workgroup v / 256,
 // thread v % 256, v = j 1024 + thread of this workgroup) has elements v + q
 // g2 256, q < 4, in registers.  The product walks the slices by wave and
 // passes Ap through LDS.
-template <typename T, typename IT, int J, bool MLDS>
+template <typename Op, int J, bool MLDS, typename T = typename Op::value_type>
 __global__ void __launch_bounds__(kFinalBlock)
-    cg_small_kernel(SellOp<T, IT> op, CgSmallArgs a, const T *__restrict__ invd,
+    cg_small_kernel(Op op, CgSmallArgs a, const T *__restrict__ invd,
                     T *__restrict__ xg, T *__restrict__ rg, T *__restrict__ pg,
                     CgState<T> *st) {
 #pragma clang fp contract(off)
-  constexpr int U = sizeof(T) == 8 ? 4 : 3;  // fits the 128 registers of 1024 threads
+  constexpr bool COLS = ColBytes<Op>::value > 0;
+  using IT = std::remove_cv_t<std::remove_pointer_t<decltype(small_cols(op))>>;
   extern __shared__ __align__(16) unsigned char small_lds[];
   if (st->status != kIterate) return;
   const unsigned n = op.nrow, nr = op.nslice * kSellRows;
@@ -65,17 +116,18 @@ __global__ void __launch_bounds__(kFinalBlock)
   int *soff = reinterpret_cast<int *>(vals + (MLDS ? a.entries : 0));
   int *slen = soff + kSmallSlices;
   IT *cols = reinterpret_cast<IT *>(slen + kSmallSlices);
-  unsigned char *rlen = reinterpret_cast<unsigned char *>(cols + (MLDS ? a.entries : 0));
+  unsigned char *rlen =
+      reinterpret_cast<unsigned char *>(cols + (MLDS && COLS ? a.entries : 0));
   const int t = threadIdx.x, lane = t & (kWave - 1);
   const int wid = __builtin_amdgcn_readfirstlane(t / kWave);
   const unsigned stride = a.g2 * kBlock;
   if (MLDS) {
     for (int e = t; e < a.entries; e += kFinalBlock) {
       vals[e] = op.val[e];
-      cols[e] = op.col[e];
+      if constexpr (COLS) cols[e] = op.col[e];
     }
   }
-  for (unsigned i = t; i < nr; i += kFinalBlock) rlen[i] = i < n ? op.rlen[i] : 0;
+  for (unsigned i = t; i < nr; i += kFinalBlock) rlen[i] = i < n ? small_len(op, i) : 0;
   if (t < op.nslice) {
     soff[t] = (int)op.soff[t];
     slen[t] = op.slen[t];
@@ -106,11 +158,9 @@ __global__ void __launch_bounds__(kFinalBlock)
       const int len = rlen[row];
       const int base = __builtin_amdgcn_readfirstlane(soff[sl]);
       const int smax = __builtin_amdgcn_readfirstlane(slen[sl]);
-      const T *xx = std::is_same<IT, int>::value ? ps : ps + sl * kSellRows;
-      const T s = MLDS ? sell_slice_sum<T, IT, false, false, true, false, U, true>(
-                             cols + base, vals + base, smax, len, lane, xx, 0, T(0))
-                       : sell_slice_sum<T, IT, false, false, true, false, U, true>(
-                             op.col + base, op.val + base, smax, len, lane, xx, 0, T(0));
+      const T s = MLDS ? small_slice(op, vals, cols, base, smax, len, sl, row, lane, ps, n)
+                       : small_slice(op, op.val, small_cols(op), base, smax, len, sl, row, lane,
+                                     ps, n);
       T acc = T(0);
       if (row < n) {
         aps[row] = s;
@@ -216,24 +266,24 @@ __global__ void __launch_bounds__(kFinalBlock)
 // the grids G over vgrid units, and how.  The unit partials are summed by
 // one wave (vgrid <= 64) in the order of launches of one unit a workgroup
 // (G.g1 == vgrid).
-template <typename T, typename IT>
-bool small_fits(const SellOp<T, IT> &op, long long entries, int vgrid, const Cg3Grids &G) {
+template <typename Op>
+bool small_fits(const Op &op, long long entries, int vgrid, const Cg3Grids &G) {
   return op.nrow <= kSmallRows && vgrid <= kWave && G.g1 == vgrid && G.g2 * 4 * kBlock >= op.nrow &&
          G.g2 <= kSmallRows / (4 * kBlock) &&
-         (size_t)entries * (sizeof(T) + sizeof(IT)) <= kSmallBytes;
+         (size_t)entries * (sizeof(typename Op::value_type) + ColBytes<Op>::value) <= kSmallBytes;
 }
 
-template <typename T, typename IT>
-void small_launch(hipStream_t s, const SellOp<T, IT> &op, long long entries, int vgrid,
-                  const Cg3Grids &G, const T *invd, T *x, T *r, T *p, CgState<T> *st) {
+template <typename Op, typename T = typename Op::value_type>
+void small_launch(hipStream_t s, const Op &op, long long entries, int vgrid, const Cg3Grids &G,
+                  const T *invd, T *x, T *r, T *p, CgState<T> *st) {
   const CgSmallArgs a{vgrid, G.g2, (int)entries};
-  const bool mlds = small_lds_bytes<T, IT>(op.nrow, entries, true) <= kSmallLds;
-  const size_t lds = small_lds_bytes<T, IT>(op.nrow, entries, mlds);
+  const bool mlds = small_lds_bytes<Op>(op.nrow, entries, true) <= kSmallLds;
+  const size_t lds = small_lds_bytes<Op>(op.nrow, entries, mlds);
   auto go = [&](auto kern) { kern<<<1, kFinalBlock, lds, s>>>(op, a, invd, x, r, p, st); };
   if (G.g2 <= 4)
-    mlds ? go(cg_small_kernel<T, IT, 1, true>) : go(cg_small_kernel<T, IT, 1, false>);
+    mlds ? go(cg_small_kernel<Op, 1, true>) : go(cg_small_kernel<Op, 1, false>);
   else
-    mlds ? go(cg_small_kernel<T, IT, 2, true>) : go(cg_small_kernel<T, IT, 2, false>);
+    mlds ? go(cg_small_kernel<Op, 2, true>) : go(cg_small_kernel<Op, 2, false>);
 }
 
 }  // namespace

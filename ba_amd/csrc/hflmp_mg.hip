@@ -10,7 +10,8 @@
 // kernel_async_inner_damped_iter_no_offdiag (cuda_async_iter_kernels.h:
 // 116-144), run synchronously (every sweep reads the previous iterate).
 //
-// Every operator is a SELL-64 copy; each row is processed in ascending
+// Every operator is a SELL-64 copy (in its offset form where the level's
+// pattern allows it); each row is processed in ascending
 // storage order, so every kernel is bit-identical to a sequential loop over
 // the CSR rows.  One cycle from level l (right-hand side b_l):
 //   x = (w invd) b, then pre-1 sweeps x' = (w invd (b - (A-D) x)) + ((1-w) x)
@@ -49,8 +50,9 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // xo = (w invd (b - (A - D) xi)) + ((1 - w) xi)
+template <class AOp>
 __global__ void __launch_bounds__(kBlock)
-    mg_sweep_kernel(Op A, double w, double one_minus_w, const double *__restrict__ invd,
+    mg_sweep_kernel(AOp A, double w, double one_minus_w, const double *__restrict__ invd,
                     const double *__restrict__ b, const double *__restrict__ xi,
                     double *__restrict__ xo, const int *status) {
 #pragma clang fp contract(off)
@@ -59,7 +61,7 @@ __global__ void __launch_bounds__(kBlock)
   const long long r = A.thread_row(unit);
   const double b0 = r < A.nrow ? b[r] : 0.0;
   TileRow tr;
-  const double t = A.row_sum<true, true>(unit, xi, b0, tr, nullptr);
+  const double t = A.template row_sum<true, true>(unit, xi, b0, tr, nullptr);
   if (tr.has_row) {
     const int i = tr.row;
     xo[i] = (w * invd[i] * t) + (one_minus_w * xi[i]);
@@ -67,8 +69,9 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // r = b - A x, term by term
+template <class AOp>
 __global__ void __launch_bounds__(kBlock)
-    mg_residual_kernel(Op A, const double *__restrict__ b, const double *__restrict__ x,
+    mg_residual_kernel(AOp A, const double *__restrict__ b, const double *__restrict__ x,
                        double *__restrict__ r, const int *status) {
 #pragma clang fp contract(off)
   if (stopped(status)) return;
@@ -76,7 +79,7 @@ __global__ void __launch_bounds__(kBlock)
   const long long row = A.thread_row(unit);
   const double b0 = row < A.nrow ? b[row] : 0.0;
   TileRow tr;
-  const double s = A.row_sum<true>(unit, x, b0, tr, nullptr);
+  const double s = A.template row_sum<true>(unit, x, b0, tr, nullptr);
   if (tr.has_row) r[tr.row] = s;
 }
 
@@ -302,8 +305,9 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- the multigrid solver: r = b - A x, check ||r||, x += cycle(r) ---------
+template <class AOp>
 __global__ void __launch_bounds__(kBlock)
-    mgs_residual_kernel(Op A, const double *__restrict__ b, const double *__restrict__ x,
+    mgs_residual_kernel(AOp A, const double *__restrict__ b, const double *__restrict__ x,
                         double *__restrict__ r, double *__restrict__ partials, const int *status) {
 #pragma clang fp contract(off)
   if (stopped(status)) return;
@@ -311,7 +315,7 @@ __global__ void __launch_bounds__(kBlock)
   const long long row = A.thread_row(unit);
   const double b0 = row < A.nrow ? b[row] : 0.0;
   TileRow tr;
-  const double ri = A.row_sum<true>(unit, x, b0, tr, nullptr);
+  const double ri = A.template row_sum<true>(unit, x, b0, tr, nullptr);
   double rr = 0;
   if (tr.has_row) {
     r[tr.row] = ri;
@@ -650,7 +654,7 @@ void with_fine_op(const hflmp_mg *m, Fn &&fn) {
   if (m->st)
     (void)stencil_dispatch<double>(m->st, fn);
   else
-    fn(sell_view<double, int>(m->lv[0].A));
+    sell_dispatch<double>(m->lv[0].A, fn);
 }
 
 // The level's smoothing steps and residual.
@@ -673,8 +677,9 @@ void smooth_sweep(hipStream_t s, const hflmp_mg *m, int l, double w, const doubl
       mg_st_sweep_kernel<<<ga, kBlock, 0, s>>>(op, w, L.invd, b, xi, xo, status);
     });
   } else {
-    mg_sweep_kernel<<<ga, kBlock, 0, s>>>(sell_view<double, int>(L.A), w, 1.0 - w, L.invd, b,
-                                          xi, xo, status);
+    sell_dispatch<double>(L.A, [&](auto op) {
+      mg_sweep_kernel<<<ga, kBlock, 0, s>>>(op, w, 1.0 - w, L.invd, b, xi, xo, status);
+    });
   }
 }
 
@@ -688,7 +693,9 @@ void residual(hipStream_t s, const hflmp_mg *m, int l, const double *b, const do
           <<<ga, kBlock, 0, s>>>(op, b, x, r, nullptr, status);
     });
   } else {
-    mg_residual_kernel<<<ga, kBlock, 0, s>>>(sell_view<double, int>(L.A), b, x, r, status);
+    sell_dispatch<double>(L.A, [&](auto op) {
+      mg_residual_kernel<<<ga, kBlock, 0, s>>>(op, b, x, r, status);
+    });
   }
 }
 
@@ -794,16 +801,19 @@ int mg_build(hflmp_ctx *ctx, const hflmp_stencil *S, int nlevels, const hflmp_cs
   m->prm = *prm;
   m->st = S;
   int rc = HFLMP_OK;
-  auto sell_of = [&](const hflmp_csr_f64 &c, hflmp_sell **o) {
-    return hflmp_sell_create_f64(ctx, c.nrow, c.ncol, c.nnz, c.row_ptr, c.col, c.val,
-                                 HFLMP_SELL_ANY_PADDING, o);
+  // the levels' operators in the offset form where it fits, except those the
+  // one-workgroup tail may take (it reads int32 columns)
+  auto sell_of = [&](const hflmp_csr_f64 &c, hflmp_sell **o, int flags = 0) {
+    return sell_create_f64_internal(ctx, c.nrow, c.ncol, c.nnz, c.row_ptr, c.col, c.val,
+                                    HFLMP_SELL_ANY_PADDING | flags, o);
   };
   for (int l = 0; l < nlevels && rc == HFLMP_OK; ++l) {
     auto &L = m->lv[l];
     const bool mf = l == 0 && S;
     L.n = (int)rows(l);
     const size_t bytes = sizeof(double) * (size_t)L.n;
-    if (!mf && (rc = sell_of(A[l], &L.A)) != HFLMP_OK) break;
+    if (!mf && (rc = sell_of(A[l], &L.A, L.n > kTailMaxRows ? kSellOffsets : 0)) != HFLMP_OK)
+      break;
     if (l + 1 < nlevels && ((rc = sell_of(R[l], &L.R)) != HFLMP_OK ||
                             (rc = sell_of(P[l], &L.P)) != HFLMP_OK))
       break;
@@ -1050,8 +1060,9 @@ int hflmp_mg_solve_f64(hflmp_ctx *ctx, const hflmp_mg *m, const double *b, doubl
             <<<ga, kBlock, 0, s>>>(op, b, x, r, partials, stat);
       });
     } else {
-      mgs_residual_kernel<<<ga, kBlock, 0, s>>>(sell_view<double, int>(m->lv[0].A), b, x, r,
-                                                partials, stat);
+      sell_dispatch<double>(m->lv[0].A, [&](auto op) {
+        mgs_residual_kernel<<<ga, kBlock, 0, s>>>(op, b, x, r, partials, stat);
+      });
     }
   };
   const auto t0 = std::chrono::steady_clock::now();

@@ -6,7 +6,9 @@
 // products y = A x and y += A x are those of CPU_CSR_lMatrix::VectorMult /
 // VectorMultAdd (CPUsimple_csr_lmatrix.cc:76-111, lmatrix_csr_cpu.cc:
 // 1424-1450), bit for bit.
+#include <climits>
 #include <cstdio>
+#include <utility>
 
 #include "hflmp_sell.hpp"
 
@@ -17,6 +19,7 @@ enum SellMode { kSellAssign = 0, kSellAdd = 1 };
 struct SellStats {
   unsigned int long_rows;  // rows longer than 255 entries
   unsigned int bad16;      // entries whose offset from the slice start needs more than 16 bits
+  unsigned int bad_off;    // slices that the offset form cannot hold
 };
 
 // Row lengths (a byte each) and, per slice, the longest row (m; where its
@@ -119,6 +122,107 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// ---- offset form ------------------------------------------------------------
+// Walks slice s (one wave, lane = row) over the distinct column offsets of
+// its rows in ascending order: f(position, offset, whether this lane's row
+// has the entry, its CSR index).  Returns the number of offsets, or -1 where
+// a row's columns do not ascend strictly or the slice has more than 255.
+template <typename F>
+__device__ __forceinline__ int for_slice_offsets(int s, int nrow, const int *__restrict__ rp,
+                                                 const int *__restrict__ ci, F &&f) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int row = s * kSellRows + lane;
+  int k = 0, end = 0;
+  if (row < nrow) {
+    k = rp[row];
+    end = rp[row + 1];
+  }
+  int off = k < end ? ci[k] - row : INT_MAX;
+  for (int j = 0;; ++j) {
+    int m = off;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+      const int w = __shfl_xor(m, o);
+      m = w < m ? w : m;
+    }
+    if (m == INT_MAX) return j;
+    if (j == 255) return -1;
+    const bool has = off == m;
+    f(j, m, has, k);
+    bool bad = false;
+    if (has) {
+      ++k;
+      off = k < end ? ci[k] - row : INT_MAX;
+      bad = off <= m;
+    }
+    if (__any(bad)) return -1;
+  }
+}
+
+// klen[s] = the slice's distinct offsets; counts slices the form cannot hold.
+__global__ void __launch_bounds__(kBlock)
+    sell_offsets_count_kernel(int nrow, int nslice, const int *__restrict__ rp,
+                              const int *__restrict__ ci, int *__restrict__ klen,
+                              SellStats *stats) {
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  for (int s = blockIdx.x * kSellSlicesPerBlock + wid; s < nslice;
+       s += gridDim.x * kSellSlicesPerBlock) {
+    const int K = for_slice_offsets(s, nrow, rp, ci, [](int, int, bool, int) {});
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+      klen[s] = K < 0 ? 0 : K;
+      if (K < 0) atomicAdd(&stats->bad_off, 1u);
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    sell_offsets_fill_kernel(int nrow, int nslice, int P, const int *__restrict__ rp,
+                             const int *__restrict__ ci, const T *__restrict__ val,
+                             const long long *__restrict__ koff, const int *__restrict__ klen,
+                             int *__restrict__ off, unsigned long long *__restrict__ mask,
+                             T *__restrict__ sval) {
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int s = blockIdx.x * kSellSlicesPerBlock + wid; s < nslice;
+       s += gridDim.x * kSellSlicesPerBlock) {
+    const long long base = koff[s];
+    const int K = klen[s];
+    for_slice_offsets(s, nrow, rp, ci, [&](int j, int o, bool has, int k) {
+      const unsigned long long m = __ballot(has);
+      if (lane == 0) {
+        off[base / kSellRows + j] = o;
+        mask[base / kSellRows + j] = m;
+      }
+      sval[sell_pos(base, K, P, lane, j)] = has ? val[k] : T(0);
+    });
+  }
+}
+
+// New values for the same pattern (thread per row); rows whose length
+// changed are skipped and counted.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    sell_offsets_values_kernel(int nrow, int P, const int *__restrict__ rp,
+                               const T *__restrict__ val, const long long *__restrict__ koff,
+                               const int *__restrict__ klen,
+                               const unsigned long long *__restrict__ mask,
+                               T *__restrict__ sval, const unsigned char *__restrict__ rlen,
+                               unsigned int *changed) {
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nrow; i += gridDim.x * kBlock) {
+    const int s = i / kSellRows, lane = i % kSellRows;
+    const long long base = koff[s];
+    const int K = klen[s];
+    int k = rp[i];
+    if (rp[i + 1] - k != (int)rlen[i]) {
+      atomicAdd(changed, 1u);
+      continue;
+    }
+    for (int j = 0; j < K; ++j)
+      if ((mask[base / kSellRows + j] >> lane) & 1) sval[sell_pos(base, K, P, lane, j)] = val[k++];
+  }
+}
+
 template <typename Op, int MODE>
 __device__ __forceinline__ void sell_spmv_rows(const Op &op,
                                                const typename Op::value_type *__restrict__ x,
@@ -162,6 +266,8 @@ void sell_free(hflmp_sell *m) {
   (void)hipFree(m->slen);
   (void)hipFree(m->rlen);
   (void)hipFree(m->col);
+  (void)hipFree(m->off);
+  (void)hipFree(m->mask);
   (void)hipFree(m->val);
   (void)hipFree(m->check);
   if (cur >= 0 && cur != m->device) (void)hipSetDevice(cur);
@@ -176,7 +282,7 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   *out = nullptr;
   HFLMP_REQUIRE(ctx, nrow > 0 && ncol > 0 && nnz >= 0, "sell_create: bad sizes");
   HFLMP_REQUIRE(ctx, rp && (nnz == 0 || (ci && val)), "sell_create: null pointer");
-  HFLMP_REQUIRE(ctx, (flags & ~(HFLMP_SELL_COL16 | HFLMP_SELL_ANY_PADDING)) == 0,
+  HFLMP_REQUIRE(ctx, (flags & ~(HFLMP_SELL_COL16 | HFLMP_SELL_ANY_PADDING | kSellOffsets)) == 0,
                 "sell_create: unknown flags %d", flags);
   hipStream_t s = ctx->stream;
   auto *m = new hflmp_sell();
@@ -189,9 +295,13 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   m->value_bytes = sizeof(T);
   m->col_bytes = 4;
   SellStats *stats = nullptr;
+  long long *koff = nullptr;  // the offset form's slices
+  int *klen = nullptr;
   int rc = HFLMP_OK;
   auto fail = [&](int code, const char *msg) {
     (void)hipFree(stats);
+    (void)hipFree(koff);
+    (void)hipFree(klen);
     sell_free(m);
     return set_error(ctx, code, "sell_create: %s", msg);
   };
@@ -210,12 +320,26 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, m->slen, m->soff);
   if ((flags & HFLMP_SELL_COL16) && nnz > 0)
     sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
+  // x is read through 32-bit byte offsets in the offset form
+  const bool try_off = (flags & (HFLMP_SELL_COL16 | kSellOffsets)) && nnz > 0 &&
+                       (size_t)ncol * sizeof(T) < (1ull << 31) &&
+                       (size_t)nrow * sizeof(T) < (1ull << 31);
+  if (try_off) {
+    if (hipMalloc(&koff, sizeof(long long) * ((size_t)m->nslice + 1)) != hipSuccess ||
+        hipMalloc(&klen, sizeof(int) * (size_t)m->nslice) != hipSuccess)
+      return fail(HFLMP_ENOMEM, "out of device memory");
+    sell_offsets_count_kernel<<<grid_for(lanes, 1), kBlock, 0, s>>>(nrow, m->nslice, rp, ci, klen,
+                                                                    stats);
+    sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, klen, koff);
+  }
   if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
   SellStats hs;
-  long long entries = 0;
+  long long entries = 0, kentries = 0;
   if (hipMemcpyAsync(&hs, stats, sizeof(hs), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipMemcpyAsync(&entries, m->soff + m->nslice, sizeof(entries), hipMemcpyDeviceToHost,
                      s) != hipSuccess ||
+      (try_off && hipMemcpyAsync(&kentries, koff + m->nslice, sizeof(kentries),
+                                 hipMemcpyDeviceToHost, s) != hipSuccess) ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail(HFLMP_EHIP, "HIP error while sizing");
   if (hs.long_rows)
@@ -227,6 +351,34 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
     return fail(HFLMP_EFORMAT, "row lengths vary too much within slices (use the CSR kernels)");
   m->entries = entries;
   if ((flags & HFLMP_SELL_COL16) && hs.bad16 == 0) m->col_bytes = 2;
+  // The offset form where it is at least 5% smaller than the columns' (the
+  // product's time follows its bytes): value padding up to a quarter of the
+  // nonzeros in FP64, about half in FP32.  Structured Q1 meshes pad by 1 to
+  // 2%; a Q2 mesh, whose rows alternate between three patterns, by 56%, and
+  // keeps its columns.
+  const double off_bytes = (double)kentries * (sizeof(T) + 12.0 / kSellRows);
+  const double col_bytes = (double)entries * (sizeof(T) + m->col_bytes) + nrow;
+  if (try_off && hs.bad_off == 0 && off_bytes < 0.95 * col_bytes) {
+    m->off_form = 1;
+    m->entries = kentries;
+    std::swap(m->soff, koff);
+    std::swap(m->slen, klen);
+    const size_t np = (size_t)kentries / kSellRows;
+    if (hipMalloc(&m->off, np * sizeof(int)) != hipSuccess ||
+        hipMalloc(&m->mask, np * sizeof(unsigned long long)) != hipSuccess ||
+        hipMalloc(&m->val, (size_t)kentries * sizeof(T)) != hipSuccess)
+      return fail(HFLMP_ENOMEM, "out of device memory");
+    sell_offsets_fill_kernel<T><<<grid_for(lanes, 1), kBlock, 0, s>>>(
+        nrow, m->nslice, m->chunk, rp, ci, val, m->soff, m->slen, m->off, m->mask,
+        static_cast<T *>(m->val));
+    if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
+    if (hipStreamSynchronize(s) != hipSuccess) return fail(HFLMP_EHIP, "HIP error in build");
+    (void)hipFree(stats);
+    (void)hipFree(koff);
+    (void)hipFree(klen);
+    *out = m;
+    return HFLMP_OK;
+  }
   const size_t ne = entries > 0 ? (size_t)entries : 1;
   if (hipMalloc(&m->col, ne * m->col_bytes) != hipSuccess ||
       hipMalloc(&m->val, ne * sizeof(T)) != hipSuccess)
@@ -247,6 +399,8 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   // the stats buffer is freed only after the stream has used it
   if (hipStreamSynchronize(s) != hipSuccess) return fail(HFLMP_EHIP, "HIP error in build");
   (void)hipFree(stats);
+  (void)hipFree(koff);
+  (void)hipFree(klen);
   *out = m;
   return HFLMP_OK;
 }
@@ -261,7 +415,12 @@ int sell_set_values(hflmp_ctx *ctx, hflmp_sell *m, const int *rp, const T *val) 
   hipStream_t s = ctx->stream;
   int rc = hflmp_fill_zero(ctx, m->check, sizeof(unsigned int));
   if (rc) return rc;
-  sell_fill_kernel<T, int, false><<<grid_for(m->nrow, 1), kBlock, 0, s>>>(
+  if (m->off_form)
+    sell_offsets_values_kernel<T><<<grid_for(m->nrow, 1), kBlock, 0, s>>>(
+        m->nrow, m->chunk, rp, val, m->soff, m->slen, m->mask, static_cast<T *>(m->val), m->rlen,
+        m->check);
+  else
+    sell_fill_kernel<T, int, false><<<grid_for(m->nrow, 1), kBlock, 0, s>>>(
       m->nrow, m->chunk, rp, nullptr, val, m->soff, m->slen, nullptr, static_cast<T *>(m->val),
       m->rlen, m->check);
   HFLMP_LAUNCH_CHECK(ctx);
@@ -285,7 +444,9 @@ int sell_spmv(hflmp_ctx *ctx, const hflmp_sell *m, const T *x, T *y) {
   HFLMP_REQUIRE(ctx, m->device == ctx->device, "sell_spmv: matrix on another device");
   const unsigned grid = sell_grid(m->nrow);
   hipStream_t s = ctx->stream;
-  if (m->col_bytes == 2)
+  if (m->off_form)
+    sell_spmv16_kernel<SellOffOp<T>, MODE><<<grid, kBlock, 0, s>>>(sell_off_view<T>(m), x, y);
+  else if (m->col_bytes == 2)
     sell_spmv16_kernel<SellOp<T, short>, MODE><<<grid, kBlock, 0, s>>>(sell_view<T, short>(m),
                                                                         x, y);
   else
@@ -296,14 +457,23 @@ int sell_spmv(hflmp_ctx *ctx, const hflmp_sell *m, const T *x, T *y) {
 
 }  // namespace
 
+int sell_create_f64_internal(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp,
+                             const int *ci, const double *val, int flags, hflmp_sell **out) {
+  return sell_create<double>(ctx, nrow, ncol, nnz, rp, ci, val, flags, out);
+}
+
 extern "C" {
 
 int hflmp_sell_create_f64(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *row_ptr,
                           const int *col, const double *val, int flags, hflmp_sell **out) {
+  if (ctx && (flags & kSellOffsets))
+    return set_error(ctx, HFLMP_EINVAL, "sell_create: unknown flags %d", flags);
   return sell_create<double>(ctx, nrow, ncol, nnz, row_ptr, col, val, flags, out);
 }
 int hflmp_sell_create_f32(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *row_ptr,
                           const int *col, const float *val, int flags, hflmp_sell **out) {
+  if (ctx && (flags & kSellOffsets))
+    return set_error(ctx, HFLMP_EINVAL, "sell_create: unknown flags %d", flags);
   return sell_create<float>(ctx, nrow, ncol, nnz, row_ptr, col, val, flags, out);
 }
 int hflmp_sell_set_values_f64(hflmp_ctx *ctx, hflmp_sell *m, const int *row_ptr,
@@ -323,7 +493,9 @@ int hflmp_sell_get_info(const hflmp_sell *m, hflmp_sell_info *info) {
   info->col_bytes = m->col_bytes;
   info->value_bytes = m->value_bytes;
   info->entries = m->entries;
-  info->device_bytes = (size_t)m->entries * (m->col_bytes + m->value_bytes) +
+  info->device_bytes = (m->off_form ? (size_t)m->entries * m->value_bytes +
+                                          (size_t)m->entries / kSellRows * 12
+                                    : (size_t)m->entries * (m->col_bytes + m->value_bytes)) +
                        sizeof(long long) * ((size_t)m->nslice + 1) +
                        sizeof(int) * (size_t)m->nslice + (size_t)m->nrow;
   return HFLMP_OK;

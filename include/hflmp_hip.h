@@ -205,19 +205,22 @@ int hflmp_cast_csr_f64_to_f32(hflmp_ctx *ctx, int nnz, const double *val,
  * ascending storage order from zero; VectorMult, CPUsimple_csr_lmatrix.cc:
  * 76-111, and VectorMultAdd, lmatrix_csr_cpu.cc:1424-1450).
  * create() builds on the device from the DEVICE CSR arrays (which it does
- * not keep).  flags HFLMP_SELL_COL16 stores columns as int16 offsets from
- * the slice's first row when every offset fits (else int32).  Returns
+ * not keep).  flags HFLMP_SELL_COL16 allows compressed columns: int16
+ * offsets from the slice's first row when every offset fits (else int32),
+ * or none at all where the rows of each slice share their column offsets
+ * (column - row; structured numberings), if that is smaller.  Returns
  * HFLMP_EFORMAT if a row has more than 255 entries or the stored entries
  * (nonzeros plus padding) would exceed 3 nnz + 64 P (unless flags has
- * HFLMP_SELL_ANY_PADDING); use the CSR kernels then.  Each lane stops at
- * its row's length: padding past a row's last chunk of P is never read. */
+ * HFLMP_SELL_ANY_PADDING); use the CSR kernels then.  Padding never takes
+ * part in a sum. */
 #define HFLMP_SELL_COL16 1
 #define HFLMP_SELL_ANY_PADDING 2
 typedef struct hflmp_sell hflmp_sell;
 typedef struct {
   int nrow, ncol, nnz;
   int chunk;          /* P: entries per lane load                         */
-  int col_bytes;      /* 4 (int32) or 2 (int16 slice offsets)             */
+  int col_bytes;      /* 4 (int32) or 2 (int16 slice offsets): the width  */
+                      /* of the columns, stored or not                    */
   int value_bytes;    /* 8 or 4                                           */
   long long entries;  /* stored entries including padding                 */
   size_t device_bytes;
