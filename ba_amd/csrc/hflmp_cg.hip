@@ -15,7 +15,8 @@
 //  (F2  one workgroup: res, stopping test, beta)
 //   K3  p = beta p + z
 // In the three-launch form F1 runs at the start of every workgroup of K2
-// and F2 at the start of every workgroup of K3.
+// and F2 at the start of every workgroup of K3; over the offset form of
+// SELL-64 K3 runs inside the next K1 (two launches, hflmp_cg3.hpp).
 // Every kernel returns at once when the state is no longer "iterate", so
 // the host queues iterations ahead and reads the state every `poll`
 // iterations only.  Systems of a few thousand rows run their iterations in
@@ -27,6 +28,7 @@
 // workgroup one row.  The CSR and SELL-64 products are identical.
 #include <chrono>
 #include <mutex>
+#include <utility>
 
 #include "hflmp_cg3.hpp"
 #include "hflmp_cg_small.hpp"
@@ -133,6 +135,8 @@ int read_state(hflmp_ctx *ctx, const CgState<T> *st, CgState<T> *h) {
   HFLMP_HIP_CHECK(ctx, hipMemcpyAsync(pin, st, sizeof(*h), hipMemcpyDeviceToHost, ctx->stream));
   HFLMP_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   std::memcpy(h, pin, sizeof(*h));
+  // the two-launch form's last verdict, when no update kernel followed it
+  if (h->status == kIterate) h->status = h->go;
   return HFLMP_OK;
 }
 
@@ -158,6 +162,34 @@ int run_small(hflmp_ctx *ctx, const Op &op, long long entries, int vgrid, const 
       if (h->status != kIterate) break;
     }
     return 1;
+  }
+  return 0;
+}
+
+// The iterations of the two-launch form (hflmp_cg3.hpp) from p in p0, with
+// p0 and p1 holding p in turn (iteration j's in p0 for odd j): 1 when they
+// ran, 0 if the operator or the workspace (p1 null) has no such form or the
+// matrix is too large for it, or an error.
+template <typename Op, typename T>
+int run_two_launch(hflmp_ctx *ctx, const Op &op, long long entries, int vgrid, const Cg3Grids &G,
+                   int nrow, const T *invd, T *x, T *r, T *p0, T *p1, T *z, T *Ap, CgState<T> *st,
+                   T *partials, int maxit, bool events) {
+  if constexpr (std::is_same_v<Op, SellOffOp<T>>) {
+    if (!p1 || !G.g1 || (size_t)entries * sizeof(T) > kTwoLaunchBytes) return 0;
+    hipStream_t s = ctx->stream;
+    T *part2 = partials + G.g1;
+    T *pc = p0, *pn = p1;
+    cg3_spmv_kernel<Op><<<G.g1, kBlock, 0, s>>>(op, vgrid, pc, Ap, st, partials);
+    auto iteration = [&]() {
+      cg2_update_kernel<T><<<G.g2, kBlock, 0, s>>>(nrow, G.g1, invd, Ap, r, z, st, partials,
+                                                   part2);
+      cg2_spmv_kernel<T><<<G.g1, kBlock, 0, s>>>(op, vgrid, G.g2, z, pc, pn, Ap, x, st, part2,
+                                                 partials);
+      std::swap(pc, pn);
+    };
+    int rc = events ? run_polled(ctx, maxit, &st->status, iteration)
+                    : run_polled_sync(ctx, maxit, &st->status, iteration);
+    return rc ? rc : 1;
   }
   return 0;
 }
@@ -192,6 +224,8 @@ int pcg_jacobi(hflmp_ctx *ctx, const Op &op, int nnz, const T *invd, const T *b,
   T *p = reinterpret_cast<T *>(w + L.vec + L.vstride);
   T *z = reinterpret_cast<T *>(w + L.vec + 2 * L.vstride);
   T *Ap = reinterpret_cast<T *>(w + L.vec + 3 * L.vstride);
+  // the two-launch form's second p, where the workspace holds it
+  T *p2 = work_bytes >= L.total + L.vstride ? reinterpret_cast<T *>(w + L.total) : nullptr;
   hipStream_t s = ctx->stream;
   const int g2 = L.grid2;
   const unsigned g3 = grid_for(nrow, 4);
@@ -228,9 +262,14 @@ int pcg_jacobi(hflmp_ctx *ctx, const Op &op, int nnz, const T *invd, const T *b,
   const int small = run_small(ctx, op, entries, grid1, G, invd, x, r, p, st, maxit, &h);
   if (small < 0) return small;
   if (!small) {
-    int rc = events ? run_polled(ctx, maxit, &st->status, iteration)
-                    : run_polled_sync(ctx, maxit, &st->status, iteration);
-    if (rc) return rc;
+    int rc = run_two_launch(ctx, op, entries, grid1, G, nrow, invd, x, r, p, p2, z, Ap, st, partials, maxit,
+                            events);
+    if (rc < 0) return rc;
+    if (!rc) {
+      rc = events ? run_polled(ctx, maxit, &st->status, iteration)
+                  : run_polled_sync(ctx, maxit, &st->status, iteration);
+      if (rc) return rc;
+    }
     rc = read_state(ctx, st, &h);
     if (rc) return rc;
   }
@@ -341,9 +380,9 @@ __global__ void __launch_bounds__(kFinalBlock)
     st->res0 = r0;
     st->res = r0;
     st->iter = 0;
-    st->status = status == kIterate ? check_state(0, (double)r0, (double)r0, st->maxit,
-                                                  st->atol, st->rtol, st->dtol)
-                                    : kConverged;
+    st->status = st->go = status == kIterate ? check_state(0, (double)r0, (double)r0, st->maxit,
+                                                           st->atol, st->rtol, st->dtol)
+                                             : kConverged;
   }
 }
 
@@ -395,7 +434,7 @@ int mpcg_run(hflmp_ctx *ctx, const Op64 &op64, const Op32 &op32, const MpLayout 
              const float *invd32, const double *b, double *x, int max_outer, double atol,
              double rtol, int inner_maxit, double inner_rtol, bool reliable, void *work,
              hflmp_mp_info *info, std::chrono::steady_clock::time_point t0,
-             long long entries32 = 0) {
+             long long entries32 = 0, float *p2 = nullptr) {
   const int nrow = op64.nrow;
   const int grid64 = op_grid(op64), grid32 = op_grid(op32);
   char *w = static_cast<char *>(work);
@@ -451,9 +490,15 @@ int mpcg_run(hflmp_ctx *ctx, const Op64 &op64, const Op32 &op32, const MpLayout 
     const int small =
         run_small(ctx, op32, entries32, grid32, G, invd32, c, r, p, st, inner_maxit, &h);
     if (small < 0) return small;
+    int two = 0;
     if (!small) {
-      rc = run_polled(ctx, inner_maxit, &st->status, iteration);
-      if (rc) return rc;
+      two = run_two_launch(ctx, op32, entries32, grid32, G, nrow, invd32, c, r, p, p2, z, Ap, st,
+                           part32, inner_maxit, true);
+      if (two < 0) return two;
+      if (!two) {
+        rc = run_polled(ctx, inner_maxit, &st->status, iteration);
+        if (rc) return rc;
+      }
     }
     mp_correct_kernel<<<grid_for(nrow, 4), kBlock, 0, s>>>(nrow, c, x);
     HFLMP_LAUNCH_CHECK(ctx);
@@ -461,6 +506,8 @@ int mpcg_run(hflmp_ctx *ctx, const Op64 &op64, const Op32 &op32, const MpLayout 
       rc = read_state(ctx, st, &h);
       if (rc) return rc;
     }
+    // the last iteration's p (two launches: the even ones' is in the other buffer)
+    if (two && h.iter > 0 && h.iter % 2 == 0) std::swap(p, p2);
     inner_total += h.iter;
     last_breakdown = h.status == kBreakdown;
   }
@@ -549,12 +596,16 @@ int mpcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A64, const hflmp_sell *A3
                 L.total);
   HFLMP_REQUIRE(ctx, (flags & ~HFLMP_MP_RELIABLE) == 0, "mpcg: unknown flags %d", flags);
   const bool rel = (flags & HFLMP_MP_RELIABLE) != 0;
+  // the two-launch form's second p, where the workspace holds it
+  float *p2 = work_bytes >= L.total + L.vstride
+                  ? reinterpret_cast<float *>(static_cast<char *>(work) + L.total)
+                  : nullptr;
   const auto t0 = std::chrono::steady_clock::now();
   // any form (offsets, int16 or int32 columns) in each precision
   return sell_dispatch<double>(A64, [&](auto o64) {
     return sell_dispatch<float>(A32, [&](auto o32) {
       return mpcg_run(ctx, o64, o32, L, invd32, b, x, max_outer, atol, rtol, inner_maxit,
-                      inner_rtol, rel, work, info, t0, A32->entries);
+                      inner_rtol, rel, work, info, t0, A32->entries, p2);
     });
   });
 }
@@ -698,7 +749,9 @@ extern "C" {
 
 size_t hflmp_pcg_workspace_bytes(int nrow, int nnz, int value_bytes) {
   if (nrow <= 0 || (value_bytes != 4 && value_bytes != 8)) return 0;
-  return solver_layout(nrow, nnz, value_bytes, 4).total;
+  // with the two-launch form's second p, where the matrix can take that form
+  const SolverLayout L = solver_layout(nrow, nnz, value_bytes, 4);
+  return L.total + ((size_t)(nnz > 0 ? nnz : 0) * value_bytes <= kTwoLaunchBytes ? L.vstride : 0);
 }
 
 int hflmp_pcg_jacobi_f64(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
@@ -759,7 +812,9 @@ size_t hflmp_mpcg_workspace_bytes(int nrow, int nnz) {
 
 size_t hflmp_mpcg_sell_workspace_bytes(int nrow) {
   if (nrow <= 0) return 0;
-  return mp_layout(nrow, 0, false).total;
+  // with the two-launch form's second p, where the matrix can take that form
+  const MpLayout L = mp_layout(nrow, 0, false);
+  return L.total + ((size_t)nrow * sizeof(float) <= kTwoLaunchBytes ? L.vstride : 0);
 }
 
 int hflmp_mpcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A64, const hflmp_sell *A32,

@@ -52,8 +52,8 @@ __global__ void __launch_bounds__(kFinalBlock)
     st->res0 = res0;
     st->res = res0;
     st->iter = 0;
-    st->status = check_state(0, (double)res0, (double)res0, st->maxit, st->atol, st->rtol,
-                             st->dtol);
+    st->status = st->go = check_state(0, (double)res0, (double)res0, st->maxit, st->atol,
+                                      st->rtol, st->dtol);
   }
 }
 
@@ -206,6 +206,147 @@ __global__ void __launch_bounds__(kBlock)
       if (i < n) p[i] = beta * pv[q] + zv[q];
     }
   }
+}
+
+// ---- two launches per iteration -----------------------------------------------------
+// For the offset form of SELL-64, whose x loads are 64 consecutive values,
+// K3 goes into the next iteration's K1: the SpMV reads p and z at every
+// position and forms p' = beta p + z there (the p kernel's rounding), stores
+// its own rows' p' to a second buffer, and takes K3's stopping test and
+// K2's x += alpha p with it; K2 keeps r and z.  The sums, their order and the
+// roundings are the three-launch form's.
+// The second gather is cheap where the entries come from L2 and the launch
+// counts, and dear where they stream from memory, so the form is taken
+// for at most kTwoLaunchBytes of entries, what the eight L2s hold.  Solves
+// in ms, three launches against two: 2D Q1 256^2 10.62 / 8.71, 512^2 24.2 /
+// 22.5, 1024^2 109.8 / 113.6; 3D Q1 48^3 2.09 / 2.00, 64^3 4.35 / 4.60, 128^3
+// 43.4 / 46.6; mixed precision, whose entries are half as large, 3D 64^3
+// 4.15 / 3.78, 128^3 28.7 / 29.1.  (With stored columns the second gather
+// costs more than the p kernel at any size.)
+//
+// The verdict of the stopping test is written to `go` while other
+// workgroups of the same launch still read `status`; the update kernel
+// passes it on.
+
+constexpr size_t kTwoLaunchBytes = 32u << 20;
+
+// K1': r.r, r.z, stopping test and beta from K2's partials; x += alpha p;
+// p' = beta p + z; Ap = A p'; partials of p'.Ap
+template <typename T>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5)))
+    cg2_spmv_kernel(SellOffOp<T> op, int vgrid, int g2, const T *__restrict__ z,
+                    const T *__restrict__ p, T *__restrict__ pn, T *__restrict__ Ap,
+                    T *__restrict__ x, CgState<T> *st, const T *__restrict__ part2,
+                    T *__restrict__ part1) {
+  __shared__ T lds[kBlock / kWave];
+  if (st->status != kIterate) return;
+  const T rr = block_total(part2, g2, 2, 0, lds);
+  const T rz = block_total(part2, g2, 2, 1, lds);
+  const int iter = st->iter_prev + 1;
+  const T res = sqrt(rr);
+  const int sv = check_state(iter, (double)res, (double)st->res0, st->maxit, st->atol, st->rtol,
+                             st->dtol);
+  const T beta = rz / st->rz_prev;
+  const T alpha = st->alpha;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->iter = iter;
+    st->rr = rr;
+    st->res = res;
+    if (sv == kIterate) {
+      st->beta = beta;
+      st->rz = rz;
+    }
+    st->go = sv;
+  }
+  T acc = 0;
+  for (int vb = blockIdx.x; vb < vgrid; vb += gridDim.x) {
+    const long long unit = xcd_tile(vb, vgrid);
+    const long long row = op.thread_row(unit);
+    const bool has = row < op.nrow;
+    T pi = 0, xi = 0, zi = 0;
+    if (has) {
+      pi = p[row];
+      xi = x[row];
+      if (sv == kIterate) zi = z[row];
+    }
+    if (sv == kIterate) {
+      const T s = op.direction_sum(unit, p, z, beta);
+      if (has) {
+        const T pv = __builtin_elementwise_fma(beta, pi, zi);
+        pn[row] = pv;
+        __builtin_nontemporal_store(s, Ap + row);
+        acc = __builtin_elementwise_fma(s, pv, acc);
+      }
+    }
+    if (has) x[row] = __builtin_elementwise_fma(alpha, pi, xi);
+  }
+  if (sv != kIterate) return;
+  block_partial1(acc, part1);
+}
+
+// K2': alpha from K1's partials; r -= alpha Ap; z = D^-1 r; partials of r.r
+// and r.z.  The first step's loads are issued before the partials are summed.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    cg2_update_kernel(int n, int g1, const T *__restrict__ invd, const T *__restrict__ Ap,
+                      T *__restrict__ r, T *__restrict__ z, CgState<T> *st,
+                      const T *__restrict__ part1, T *__restrict__ part2) {
+#pragma clang fp contract(off)
+  __shared__ T lds[kBlock / kWave];
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  const int go = st->go;
+  if (go != kIterate) {
+    if (lead && st->status == kIterate) st->status = go;
+    return;
+  }
+  if (st->status != kIterate) return;
+  const long long stride = (long long)gridDim.x * kBlock;
+  long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x;
+  T av[4], rv[4], dv[4];
+  auto load = [&]() {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long i = i0 + q * stride;
+      if (i < n) {
+        av[q] = Ap[i];
+        rv[q] = r[i];
+        dv[q] = invd[i];
+      }
+    }
+  };
+  load();
+  const T pAp = block_total(part1, g1, 1, 0, lds);
+  const T rzc = st->rz;
+  if (lead) {
+    st->pAp = pAp;
+    st->rz_prev = rzc;
+    st->iter_prev = st->iter;
+  }
+  if (pAp == T(0) || !(pAp == pAp)) {
+    if (lead) st->status = kBreakdown;
+    return;
+  }
+  const T alpha = rzc / pAp;
+  if (lead) st->alpha = alpha;
+  const T malpha = -alpha;
+  T rr = 0, rz = 0;
+  while (i0 < n) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long long i = i0 + q * stride;
+      if (i < n) {
+        const T ri = __builtin_elementwise_fma(malpha, av[q], rv[q]);
+        const T zi = ri * dv[q];
+        r[i] = ri;
+        z[i] = zi;
+        rr = __builtin_elementwise_fma(ri, ri, rr);
+        rz = __builtin_elementwise_fma(ri, zi, rz);
+      }
+    }
+    i0 += 4 * stride;
+    if (i0 < n) load();
+  }
+  block_partial2(rr, rz, part2);
 }
 
 // Grids of the three-launch iteration for an operator over `vgrid` units

@@ -469,6 +469,29 @@ struct SellOffOp {
         row, lane, [&](int c) { return buffer_load<T>(xr, (unsigned)c * (unsigned)sizeof(T)); },
         s);
   }
+  // The row's sum over beta p + z in place of x (each rounded as one fused
+  // multiply-add).
+  __device__ __forceinline__ T direction_sum(long long unit, const T *p, const T *z,
+                                             T beta) const {
+    const long long sl = unit * kSellSlicesPerBlock + (threadIdx.x >> 6);
+    if (sl >= nslice) return T(0);
+    const int sid = __builtin_amdgcn_readfirstlane((int)sl);
+    const int lane = threadIdx.x & (kWave - 1);
+    const long long base = scalar_ptr(soff)[sid];
+    const int K = scalar_ptr(slen)[sid];
+    const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T *>(p), 0, ncol * (int)sizeof(T), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<T *>(z), 0, ncol * (int)sizeof(T), kRsrcWord3);
+    return sell_offset_sum<T, false, false, true>(
+        val + base, scalar_ptr(off) + base / kSellRows, scalar_ptr(mask) + base / kSellRows, K,
+        sid * kSellRows + lane, lane,
+        [&](int c) {
+          const unsigned o = (unsigned)c * (unsigned)sizeof(T);
+          return __builtin_elementwise_fma(beta, buffer_load<T>(pr, o), buffer_load<T>(zr, o));
+        },
+        T(0));
+  }
 };
 
 template <typename T>

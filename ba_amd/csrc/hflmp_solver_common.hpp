@@ -31,6 +31,9 @@ struct CgState {
   // rz and iter
   T rz_prev;
   int iter_prev;
+  // the two-launch iteration: the stopping test's verdict, which its SpMV
+  // kernel writes and its update kernel passes on to `status`
+  int go;
 };
 
 // IterateControl::Check (common/iterate_control.cc:80-107); a NaN residual
@@ -114,7 +117,7 @@ __global__ void init_state_kernel(CgState<T> *st, int maxit, double atol, double
     s.rz = s.pAp = s.alpha = s.beta = s.rr = s.res = s.res0 = s.rz_prev = T(0);
     s.iter_prev = 0;
     s.iter = 0;
-    s.status = kIterate;
+    s.status = s.go = kIterate;
     s.maxit = maxit;
     s.atol = atol;
     s.rtol = rtol;
