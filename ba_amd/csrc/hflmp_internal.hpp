@@ -98,9 +98,9 @@ __device__ __forceinline__ int dpp_xor(int v) {
   return __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, true);
 }
 
-// One step of wave_sum: v + v of lane ^ OFF, on every lane.
-template <int OFF, typename T>
-__device__ __forceinline__ T wave_sum_step(T v) {
+// One step of a wave reduction: op(v, v of lane ^ OFF), on every lane.
+template <int OFF, typename T, typename Op>
+__device__ __forceinline__ T wave_step(T v, Op op) {
   static_assert(sizeof(T) == 4 || sizeof(T) == 8, "4 or 8 bytes");
   constexpr int W = sizeof(T) / 4;
   struct Words {
@@ -120,7 +120,17 @@ __device__ __forceinline__ T wave_sum_step(T v) {
       b.w[i] = dpp_xor<OFF>(a.w[i]);
     }
   }
-  return __builtin_bit_cast(T, a) + __builtin_bit_cast(T, b);
+  return op(__builtin_bit_cast(T, a), __builtin_bit_cast(T, b));
+}
+
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  v = wave_step<32>(v, op);
+  v = wave_step<16>(v, op);
+  v = wave_step<8>(v, op);
+  v = wave_step<4>(v, op);
+  v = wave_step<2>(v, op);
+  return wave_step<1>(v, op);
 }
 
 // Sum over the wave on every lane: pairs 32 apart first, then 16, ... 1.
@@ -129,12 +139,11 @@ __device__ __forceinline__ T wave_sum_step(T v) {
 // trips in FP64.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
-  v = wave_sum_step<32>(v);
-  v = wave_sum_step<16>(v);
-  v = wave_sum_step<8>(v);
-  v = wave_sum_step<4>(v);
-  v = wave_sum_step<2>(v);
-  return wave_sum_step<1>(v);
+  return wave_reduce(v, [](T a, T b) { return a + b; });
+}
+
+__device__ __forceinline__ int wave_min(int v) {
+  return wave_reduce(v, [](int a, int b) { return a < b ? a : b; });
 }
 
 // Sum over the workgroup; the result is valid in thread 0.  `lds` must hold

@@ -20,6 +20,7 @@ struct SellStats {
   unsigned int long_rows;  // rows longer than 255 entries
   unsigned int bad16;      // entries whose offset from the slice start needs more than 16 bits
   unsigned int bad_off;    // slices that the offset form cannot hold
+  unsigned int bad16_off;  // bad16 as the offset count saw it (all of it if bad_off is 0)
 };
 
 // Row lengths (a byte each) and, per slice, the longest row (m; where its
@@ -137,14 +138,11 @@ __device__ __forceinline__ int for_slice_offsets(int s, int nrow, const int *__r
     k = rp[row];
     end = rp[row + 1];
   }
+  // the row's current offset and the next one, loaded a step ahead
   int off = k < end ? ci[k] - row : INT_MAX;
+  int next = k + 1 < end ? ci[k + 1] - row : INT_MAX;
   for (int j = 0;; ++j) {
-    int m = off;
-#pragma unroll
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      const int w = __shfl_xor(m, o);
-      m = w < m ? w : m;
-    }
+    const int m = wave_min(off);
     if (m == INT_MAX) return j;
     if (j == 255) return -1;
     const bool has = off == m;
@@ -152,7 +150,8 @@ __device__ __forceinline__ int for_slice_offsets(int s, int nrow, const int *__r
     bool bad = false;
     if (has) {
       ++k;
-      off = k < end ? ci[k] - row : INT_MAX;
+      off = next;
+      next = k + 1 < end ? ci[k + 1] - row : INT_MAX;
       bad = off <= m;
     }
     if (__any(bad)) return -1;
@@ -167,8 +166,13 @@ __global__ void __launch_bounds__(kBlock)
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   for (int s = blockIdx.x * kSellSlicesPerBlock + wid; s < nslice;
        s += gridDim.x * kSellSlicesPerBlock) {
-    const int K = for_slice_offsets(s, nrow, rp, ci, [](int, int, bool, int) {});
-    if ((threadIdx.x & (kWave - 1)) == 0) {
+    const int lane = threadIdx.x & (kWave - 1);
+    bool far = false;  // a column beyond int16 of the slice's first row
+    const int K = for_slice_offsets(s, nrow, rp, ci, [&](int, int o, bool has, int) {
+      far = far || (has && (o + lane < -32768 || o + lane > 32767));
+    });
+    if (__any(far) && lane == 0) atomicAdd(&stats->bad16_off, 1u);
+    if (lane == 0) {
       klen[s] = K < 0 ? 0 : K;
       if (K < 0) atomicAdd(&stats->bad_off, 1u);
     }
@@ -318,8 +322,6 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   sell_lengths_kernel<<<(unsigned)g, kBlock, 0, s>>>(nrow, m->nslice, rp, m->rlen, m->slen,
                                                      stats);
   sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, m->slen, m->soff);
-  if ((flags & HFLMP_SELL_COL16) && nnz > 0)
-    sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
   // x is read through 32-bit byte offsets in the offset form
   const bool try_off = (flags & (HFLMP_SELL_COL16 | kSellOffsets)) && nnz > 0 &&
                        (size_t)ncol * sizeof(T) < (1ull << 31) &&
@@ -332,6 +334,9 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
                                                                     stats);
     sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, klen, koff);
   }
+  const bool try16 = (flags & HFLMP_SELL_COL16) && nnz > 0;
+  if (try16 && !try_off)
+    sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
   if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
   SellStats hs;
   long long entries = 0, kentries = 0;
@@ -342,6 +347,16 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
                                  hipMemcpyDeviceToHost, s) != hipSuccess) ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail(HFLMP_EHIP, "HIP error while sizing");
+  if (try16 && try_off) {
+    hs.bad16 = hs.bad16_off;
+    if (hs.bad_off) {  // the count left slices early: look at every column
+      sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
+      if (hipGetLastError() != hipSuccess ||
+          hipMemcpyAsync(&hs, stats, sizeof(hs), hipMemcpyDeviceToHost, s) != hipSuccess ||
+          hipStreamSynchronize(s) != hipSuccess)
+        return fail(HFLMP_EHIP, "HIP error while sizing");
+    }
+  }
   if (hs.long_rows)
     return fail(HFLMP_EFORMAT, "a row has more than 255 entries (use the CSR kernels)");
   // Padding is never loaded (a lane stops at its row's length), but it
@@ -350,7 +365,7 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   if (!(flags & HFLMP_SELL_ANY_PADDING) && entries > 3LL * nnz + (long long)kSellRows * m->chunk)
     return fail(HFLMP_EFORMAT, "row lengths vary too much within slices (use the CSR kernels)");
   m->entries = entries;
-  if ((flags & HFLMP_SELL_COL16) && hs.bad16 == 0) m->col_bytes = 2;
+  if (try16 && hs.bad16 == 0) m->col_bytes = 2;
   // The offset form where it is at least 5% smaller than the columns' (the
   // product's time follows its bytes): value padding up to a quarter of the
   // nonzeros in FP64, about half in FP32.  Structured Q1 meshes pad by 1 to
