@@ -69,6 +69,10 @@ int hflmp_ctx_create(int device, hflmp_ctx **out) {
     return fail(HFLMP_ENOMEM);
   if (hipHostMalloc(&ctx->host_pinned, 4096, hipHostMallocDefault) != hipSuccess)
     return fail(HFLMP_ENOMEM);
+  if (hipHostMalloc(&ctx->host_partials, 8 * (size_t)kMaxRedBlocks, hipHostMallocDefault) !=
+          hipSuccess ||
+      hipHostGetDevicePointer(&ctx->host_partials_dev, ctx->host_partials, 0) != hipSuccess)
+    return fail(HFLMP_ENOMEM);
   // Counters start at zero; the reductions leave them at zero.
   fill_zero_kernel<<<1, kBlock, 0, ctx->stream>>>(
       reinterpret_cast<unsigned char *>(ctx->red_counter), 64 * sizeof(unsigned int));
@@ -87,6 +91,7 @@ int hflmp_ctx_destroy(hflmp_ctx *ctx) {
   if (ctx->red_counter) (void)hipFree(ctx->red_counter);
   if (ctx->red_result) (void)hipFree(ctx->red_result);
   if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
+  if (ctx->host_partials) (void)hipHostFree(ctx->host_partials);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
   delete ctx;
   return HFLMP_OK;

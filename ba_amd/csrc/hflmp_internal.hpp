@@ -17,7 +17,7 @@ constexpr int kWave = 64;
 // gfx950: 256 CUs in 8 XCDs, workgroups dispatched round-robin over XCDs.
 constexpr int kXcds = 8;
 // Upper bound on reduction partials (one per workgroup of a reduction).
-constexpr int kMaxRedBlocks = 2048;
+constexpr int kMaxRedBlocks = 2048;  // at most twice kFinalBlock (host_sum_partials)
 
 struct hflmp_ctx {
   int device = 0;
@@ -30,6 +30,10 @@ struct hflmp_ctx {
   unsigned int *red_counter = nullptr;
   double *red_result = nullptr;   // 64 device result slots
   void *host_pinned = nullptr;    // 4 KiB pinned host staging
+  // pinned host memory for a reduction's partials (kMaxRedBlocks of 8 B),
+  // and its address on the device
+  void *host_partials = nullptr;
+  void *host_partials_dev = nullptr;
   char last_error[512] = {0};
 };
 
