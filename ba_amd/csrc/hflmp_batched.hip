@@ -227,6 +227,7 @@ template <typename T>
 struct BState {
   T rz[kMaxRhs], alpha[kMaxRhs], beta[kMaxRhs], res[kMaxRhs], res0[kMaxRhs];
   int iter[kMaxRhs], status[kMaxRhs];
+  int moved[kMaxRhs];  // 1 while this iteration's x += alpha p is due
   int any_iterate;  // polled by the host: 1 while some column iterates, else 0
   int n_live;       // columns still iterating; the one that stops the last clears any_iterate
   int maxit;
@@ -234,9 +235,11 @@ struct BState {
 };
 
 // per-column partial sums of one or two quantities, stored [q][column][block]
-// so that each column's partials are contiguous for its finalize workgroup
+// so that each column's partials are contiguous for its finalize workgroup.
+// Lane l holds column l, or with `sub` rows side by side column l mod k.
 template <typename T, int NQ>
-__device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *__restrict__ part) {
+__device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *__restrict__ part,
+                                                   int sub = 1) {
   __shared__ T lds[NQ][kWavesPerBlock][kWave];
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
 #pragma unroll
@@ -247,7 +250,8 @@ __device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *_
     for (int q = 0; q < NQ; ++q) {
       T s = 0;
 #pragma unroll
-      for (int w = 0; w < kWavesPerBlock; ++w) s += lds[q][w][lane];
+      for (int w = 0; w < kWavesPerBlock; ++w)
+        for (int j = 0; j < sub; ++j) s += lds[q][w][lane + j * k];
       part[((size_t)q * k + lane) * gridDim.x + blockIdx.x] = s;
     }
   }
@@ -290,7 +294,7 @@ __global__ void binit_state_kernel(BState<T> *st, int k, int maxit, double atol,
   const int c = threadIdx.x;
   if (c < kMaxRhs) {
     st->rz[c] = st->alpha[c] = st->beta[c] = st->res[c] = st->res0[c] = T(0);
-    st->iter[c] = 0;
+    st->iter[c] = st->moved[c] = 0;
     st->status[c] = c < k ? kIterate : kConverged;
   }
   if (c == 0) {
@@ -303,13 +307,13 @@ __global__ void binit_state_kernel(BState<T> *st, int k, int maxit, double atol,
   }
 }
 
-// R = B - A X, Z = D^-1 R, P = Z; partials r.r, r.z per column
+// R = B - A X, P = Z = D^-1 R; partials r.r, r.z per column
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     bcg_init_kernel(int nrow, int k, const int *__restrict__ rp, const int *__restrict__ ci,
                     const T *__restrict__ val, const T *__restrict__ invd,
                     const T *__restrict__ B, const T *__restrict__ X, T *__restrict__ R,
-                    T *__restrict__ Z, T *__restrict__ P, T *__restrict__ part) {
+                    T *__restrict__ P, T *__restrict__ part) {
   const int lane = threadIdx.x & (kWave - 1);
   T acc[2] = {T(0), T(0)};
   const RowWalk w = row_walk(nrow);
@@ -323,7 +327,6 @@ __global__ void __launch_bounds__(kBlock)
       const T ri = T(-1) * s + B[e];
       const T zi = ri * invd[i];
       R[e] = ri;
-      Z[e] = zi;
       P[e] = zi;
       acc[0] += ri * ri;
       acc[1] += ri * zi;
@@ -402,50 +405,65 @@ template <typename T>
 __global__ void __launch_bounds__(kBlock)
     bcg_alpha_final(BState<T> *st, const T *__restrict__ part, int count, int k) {
   const int c = blockIdx.x;
-  if (!st->any_iterate || st->status[c] != kIterate) return;  // uniform per workgroup
+  if (st->status[c] != kIterate) {  // uniform per workgroup
+    if (threadIdx.x == 0) st->moved[c] = 0;
+    return;
+  }
   const T pap = col_total(part, count, k, 0);
   if (threadIdx.x == 0) {
-    st->alpha[c] = st->rz[c] / pap;
-    if (pap == T(0) || !(pap == pap)) {
+    const bool bad = pap == T(0) || !(pap == pap);
+    st->alpha[c] = bad ? T(0) : st->rz[c] / pap;
+    st->moved[c] = !bad;
+    if (bad) {
       st->status[c] = kBreakdown;
-      st->alpha[c] = T(0);
       column_stops(st);
     }
   }
 }
 
-// x += alpha p, r -= alpha Ap, z = D^-1 r for iterating columns; partials
-// of r.r and r.z
+// The vector updates run over the block's values in order, 64 / k rows side
+// by side in a wave (lane l: column l mod k), so that few columns do not
+// leave lanes idle.  z is formed where it is used (D^-1 is one value a row)
+// and x is updated with p, which the p kernel reads anyway: 3 + 5 block
+// streams an iteration instead of the 8 + 3 of x, r, z together and p after
+// them (2D Q2 128^2, 64 columns: 44.6 + 15.8 us before, 22.6 + 24.8 now).
+struct BlockWalk {
+  long long first, end, step;  // row groups of this wave
+  int sub, span;               // rows side by side, values a group
+};
+
+__device__ __forceinline__ BlockWalk block_walk(int nrow, int k) {
+  const int sub = kWave / k;
+  const RowWalk w = row_walk((nrow + sub - 1) / sub);
+  return {w.first, w.end, w.step, sub, sub * k};
+}
+
+// r -= alpha Ap for iterating columns; partials of r.r and r.z, z = D^-1 r
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    bcg_update_kernel(int nrow, int k, const T *__restrict__ invd, const T *__restrict__ P,
-                      const T *__restrict__ AP, T *__restrict__ X, T *__restrict__ R,
-                      T *__restrict__ Z, const BState<T> *st, T *__restrict__ part) {
-  __shared__ T s_alpha[kMaxRhs];
-  __shared__ int s_live[kMaxRhs];
+    bcg_update_kernel(int nrow, int k, const T *__restrict__ invd, const T *__restrict__ AP,
+                      T *__restrict__ R, const BState<T> *st, T *__restrict__ part) {
+#pragma clang fp contract(off)
   if (!st->any_iterate) return;
-  if (threadIdx.x < kMaxRhs) {
-    s_alpha[threadIdx.x] = st->alpha[threadIdx.x];
-    s_live[threadIdx.x] = threadIdx.x < k && st->status[threadIdx.x] == kIterate;
-  }
-  __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
+  const BlockWalk w = block_walk(nrow, k);
+  const int j = lane / k, c = lane - j * k;
   T acc[2] = {T(0), T(0)};
-  if (lane < k && s_live[lane]) {
-    const T a = s_alpha[lane], ma = -a;
-    const RowWalk w = row_walk(nrow);
-    for (long long i = w.first; i < w.end; i += w.step) {
-      const size_t e = (size_t)i * k + lane;
-      X[e] += a * P[e];
-      const T ri = R[e] + ma * AP[e];
-      const T zi = ri * invd[i];
-      R[e] = ri;
-      Z[e] = zi;
-      acc[0] += ri * ri;
-      acc[1] += ri * zi;
+  if (lane < w.span && st->status[c] == kIterate) {
+    const T ma = -st->alpha[c];
+    for (long long g = w.first; g < w.end; g += w.step) {
+      const long long i = g * w.sub + j;
+      if (i < nrow) {
+        const size_t e = (size_t)g * w.span + lane;
+        const T ri = __builtin_elementwise_fma(ma, AP[e], R[e]);
+        const T zi = ri * invd[i];
+        R[e] = ri;
+        acc[0] = __builtin_elementwise_fma(ri, ri, acc[0]);
+        acc[1] = __builtin_elementwise_fma(ri, zi, acc[1]);
+      }
     }
   }
-  block_col_partials<T, 2>(acc, k, part);
+  block_col_partials<T, 2>(acc, k, part, w.sub);
 }
 
 template <typename T>
@@ -471,26 +489,30 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// p = beta p + z for iterating columns
+// x += alpha p for the columns that took the step, p = beta p + z for those
+// that go on (a column that has just stopped still gets its x)
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    bcg_p_kernel(int nrow, int k, const T *__restrict__ Z, T *__restrict__ P,
-                 const BState<T> *st) {
-  __shared__ T s_beta[kMaxRhs];
-  __shared__ int s_live[kMaxRhs];
-  if (!st->any_iterate) return;
-  if (threadIdx.x < kMaxRhs) {
-    s_beta[threadIdx.x] = st->beta[threadIdx.x];
-    s_live[threadIdx.x] = threadIdx.x < k && st->status[threadIdx.x] == kIterate;
-  }
-  __syncthreads();
+    bcg_xp_kernel(int nrow, int k, const T *__restrict__ invd, const T *__restrict__ R,
+                  T *__restrict__ X, T *__restrict__ P, const BState<T> *st) {
+#pragma clang fp contract(off)
   const int lane = threadIdx.x & (kWave - 1);
-  if (lane >= k || !s_live[lane]) return;
-  const T bt = s_beta[lane];
-  const RowWalk w = row_walk(nrow);
-  for (long long i = w.first; i < w.end; i += w.step) {
-    const size_t e = (size_t)i * k + lane;
-    P[e] = bt * P[e] + Z[e];
+  const BlockWalk w = block_walk(nrow, k);
+  const int j = lane / k, c = lane - j * k;
+  if (lane >= w.span || !st->moved[c]) return;
+  const bool on = st->status[c] == kIterate;
+  const T a = st->alpha[c], bt = st->beta[c];
+  for (long long g = w.first; g < w.end; g += w.step) {
+    const long long i = g * w.sub + j;
+    if (i < nrow) {
+      const size_t e = (size_t)g * w.span + lane;
+      const T p = P[e];
+      X[e] = __builtin_elementwise_fma(a, p, X[e]);
+      if (on) {
+        const T z = R[e] * invd[i];
+        P[e] = __builtin_elementwise_fma(bt, p, z);
+      }
+    }
   }
 }
 
@@ -515,10 +537,11 @@ inline BLayout b_layout(hflmp_ctx *ctx, int nrow, int k, int vb) {
   BLayout L;
   L.grid = spmm_grid(ctx, vb);
   L.state = 0;
-  L.part = 4096;  // BState < 4 KiB
+  L.part = 4096;
+  static_assert(sizeof(BState<double>) <= 4096, "the state ends before the partials");
   L.vec = align256(L.part + 2 * (size_t)L.grid * k * vb);
   L.vstride = align256((size_t)nrow * k * vb);
-  L.total = L.vec + 4 * L.vstride;  // R, P, Z, AP
+  L.total = L.vec + 3 * L.vstride;  // R, P, AP
   return L;
 }
 
@@ -544,8 +567,7 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
   T *part = reinterpret_cast<T *>(w + L.part);
   T *R = reinterpret_cast<T *>(w + L.vec);
   T *P = reinterpret_cast<T *>(w + L.vec + L.vstride);
-  T *Z = reinterpret_cast<T *>(w + L.vec + 2 * L.vstride);
-  T *AP = reinterpret_cast<T *>(w + L.vec + 3 * L.vstride);
+  T *AP = reinterpret_cast<T *>(w + L.vec + 2 * L.vstride);
   hipStream_t s = ctx->stream;
   const int g = L.grid;
   // the block layout's walk: its grid (at most the partial area's) and LDS
@@ -571,7 +593,7 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
   }
   const auto t0 = std::chrono::steady_clock::now();
   binit_state_kernel<T><<<1, kMaxRhs, 0, s>>>(st, k, maxit, atol, rtol, dtol);
-  bcg_init_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, invd, B, X, R, Z, P, part);
+  bcg_init_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, invd, B, X, R, P, part);
   bcg_init_final<T><<<k, kBlock, 0, s>>>(st, part, g, k);
   HFLMP_LAUNCH_CHECK(ctx);
   auto iteration = [&]() {
@@ -582,9 +604,9 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
       bcg_spmm_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, P, AP, st, part);
       bcg_alpha_final<T><<<k, kBlock, 0, s>>>(st, part, g, k);
     }
-    bcg_update_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, invd, P, AP, X, R, Z, st, part);
+    bcg_update_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, invd, AP, R, st, part);
     bcg_beta_final<T><<<k, kBlock, 0, s>>>(st, part, g, k);
-    bcg_p_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, Z, P, st);
+    bcg_xp_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, invd, R, X, P, st);
   };
   // the poll reads any_iterate: stop when it drops to 0 (kConverged)
   int rc = run_polled(ctx, maxit, &st->any_iterate, iteration, 16, 1);
