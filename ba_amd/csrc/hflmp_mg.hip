@@ -49,12 +49,13 @@ __global__ void __launch_bounds__(kBlock)
     x[i] = w * invd[i] * b[i];
 }
 
-// xo = (w invd (b - (A - D) xi)) + ((1 - w) xi)
-template <class AOp>
+// xo = (w invd (b - (A - D) xi)) + ((1 - w) xi) (DOT: and the partials of
+// b.xo, the r.z of CG where the sweep is the cycle's last)
+template <bool DOT, class AOp>
 __global__ void __launch_bounds__(kBlock)
     mg_sweep_kernel(AOp A, double w, double one_minus_w, const double *__restrict__ invd,
                     const double *__restrict__ b, const double *__restrict__ xi,
-                    double *__restrict__ xo, const int *status) {
+                    double *__restrict__ xo, double *__restrict__ partials, const int *status) {
 #pragma clang fp contract(off)
   if (stopped(status)) return;
   const long long unit = xcd_tile(blockIdx.x, gridDim.x);
@@ -62,10 +63,14 @@ __global__ void __launch_bounds__(kBlock)
   const double b0 = r < A.nrow ? b[r] : 0.0;
   TileRow tr;
   const double t = A.template row_sum<true, true>(unit, xi, b0, tr, nullptr);
+  double dot = 0;
   if (tr.has_row) {
     const int i = tr.row;
-    xo[i] = (w * invd[i] * t) + (one_minus_w * xi[i]);
+    const double z = (w * invd[i] * t) + (one_minus_w * xi[i]);
+    xo[i] = z;
+    dot = b0 * z;
   }
+  if (DOT) block_partial1(dot, partials);
 }
 
 // r = b - A x, term by term
@@ -130,19 +135,26 @@ __device__ __forceinline__ double st_residual(const SOp &A, long long unit,
   return A.template row_sum_scaled<true>(unit, x, s, -1.0, tr, lds);
 }
 
-// xo = xi + w ((b - A xi) .* invd)
-template <class SOp>
+// xo = xi + w ((b - A xi) .* invd) (DOT: and the partials of b.xo)
+template <bool DOT, class SOp>
 __global__ void __launch_bounds__(kBlock)
     mg_st_sweep_kernel(SOp A, double w, const double *__restrict__ invd,
                        const double *__restrict__ b, const double *__restrict__ xi,
-                       double *__restrict__ xo, const int *status) {
+                       double *__restrict__ xo, double *__restrict__ partials,
+                       const int *status) {
 #pragma clang fp contract(off)
   __shared__ double lds[SOp::kLds];
   if (stopped(status)) return;
   const long long unit = xcd_tile(blockIdx.x, gridDim.x);
   TileRow tr;
   const double r = st_residual(A, unit, b, xi, tr, lds);
-  if (tr.has_row) xo[tr.row] = xi[tr.row] + w * (r * invd[tr.row]);
+  double dot = 0;
+  if (tr.has_row) {
+    const double z = xi[tr.row] + w * (r * invd[tr.row]);
+    xo[tr.row] = z;
+    dot = b[tr.row] * z;
+  }
+  if (DOT) block_partial1(dot, partials);
 }
 
 // r = b - A x (PART: and the partials of r.r)
@@ -238,11 +250,15 @@ __global__ void __launch_bounds__(kFinalBlock)
   }
 }
 
-// x += alpha p; r -= alpha Ap; partials of r.r
+// x += alpha p; r -= alpha Ap; partials of r.r; and the first step of the
+// next cycle from r where it has one (FIRST 1: as mg_first_kernel, 2: as
+// mg_st_first_kernel), which then reads no r and needs no launch
+template <int FIRST>
 __global__ void __launch_bounds__(kBlock)
     mgcg_update_kernel(int n, const double *__restrict__ p, const double *__restrict__ Ap,
                        double *__restrict__ x, double *__restrict__ r, const CgState<double> *st,
-                       double *__restrict__ partials) {
+                       double *__restrict__ partials, double w, const double *__restrict__ invd,
+                       double *__restrict__ x0) {
   if (st->status != kIterate) return;
   const double alpha = st->alpha, malpha = -alpha;
   double rr = 0;
@@ -251,6 +267,8 @@ __global__ void __launch_bounds__(kBlock)
     const double ri = r[i] + malpha * Ap[i];
     r[i] = ri;
     rr += ri * ri;
+    if (FIRST == 1) x0[i] = w * invd[i] * ri;
+    if (FIRST == 2) x0[i] = w * (ri * invd[i]);
   }
   block_partial1(rr, partials);
 }
@@ -359,13 +377,15 @@ __global__ void __launch_bounds__(kBlock)
 // column index: z, then y, then x) gives results bit-identical to the
 // SELL-64 products over R and P, while reading only the vectors.
 
-// bc = R r: coarse node (I,J,K) interior sums its 3^dim fine neighbours.
+// bc = R r: coarse node (I,J,K) interior sums its 3^dim fine neighbours
+// (FIRST: and the coarse level's first step xc = (w invd) bc with it).
 // Node counts stay below 2^31 (checked when the hierarchy is set), so the
 // index arithmetic is 32-bit with multiply-shift division by pf and pc.
-template <int DIM>
+template <int DIM, bool FIRST>
 __global__ void __launch_bounds__(kBlock)
     mg_restrict_q1_kernel(int pf, int pc, DivMagic dpc, const double *__restrict__ r,
-                          double *__restrict__ bc, const int *status) {
+                          double *__restrict__ bc, double w, const double *__restrict__ invd,
+                          double *__restrict__ xc, const int *status) {
 #pragma clang fp contract(off)
   if (stopped(status)) return;
   const int nc = DIM == 3 ? pc * pc * pc : pc * pc;
@@ -385,11 +405,12 @@ __global__ void __launch_bounds__(kBlock)
         for (int dy = -1; dy <= 1; ++dy)
 #pragma unroll
           for (int dx = -1; dx <= 1; ++dx) {
-            const double w = (dz ? 0.5 : 1.0) * ((dy ? 0.5 : 1.0) * (dx ? 0.5 : 1.0));
-            s += w * r[f0 + dx + pf * (dy + pf * dz)];
+            const double q = (dz ? 0.5 : 1.0) * ((dy ? 0.5 : 1.0) * (dx ? 0.5 : 1.0));
+            s += q * r[f0 + dx + pf * (dy + pf * dz)];
           }
     }
     bc[c] = s;
+    if (FIRST) xc[c] = w * invd[c] * s;
   }
 }
 
@@ -409,55 +430,94 @@ __global__ void __launch_bounds__(kBlock)
     if (i == 0 || i == pf - 1 || j == 0 || j == pf - 1 || (DIM == 3 && (k == 0 || k == pf - 1)))
       continue;
     // parents per direction: g even -> g/2 (weight 1), odd -> (g-1)/2 and
-    // (g+1)/2 (1/2 each); parents on the coarse boundary have no column
-    const int nzp = DIM == 3 ? 1 + (k & 1) : 1, nyp = 1 + (j & 1), nxp = 1 + (i & 1);
+    // (g+1)/2 (1/2 each); parents on the coarse boundary have no column.
+    // All parents' loads go out before the first is added.
+    constexpr int NZ = DIM == 3 ? 2 : 1;
     const int kz0 = DIM == 3 ? k >> 1 : 0, jy0 = j >> 1, ix0 = i >> 1;
     const double wz = DIM == 3 && (k & 1) ? 0.5 : 1.0, wy = (j & 1) ? 0.5 : 1.0,
                  wx = (i & 1) ? 0.5 : 1.0;
-    double s = x[f];
-    for (int a = 0; a < nzp; ++a) {
-      const int K = kz0 + a;
-      if (DIM == 3 && (K == 0 || K == pc - 1)) continue;
-      for (int bq = 0; bq < nyp; ++bq) {
-        const int J = jy0 + bq;
-        if (J == 0 || J == pc - 1) continue;
-        for (int cq = 0; cq < nxp; ++cq) {
-          const int I = ix0 + cq;
-          if (I == 0 || I == pc - 1) continue;
-          const double w = (DIM == 3 ? wz : 1.0) * (wy * wx);
-          s += w * xc[I + pc * (J + pc * K)];
+    const double w = (DIM == 3 ? wz : 1.0) * (wy * wx);
+    double v[NZ][2][2];
+    bool has[NZ][2][2];
+#pragma unroll
+    for (int a = 0; a < NZ; ++a)
+#pragma unroll
+      for (int bq = 0; bq < 2; ++bq)
+#pragma unroll
+        for (int cq = 0; cq < 2; ++cq) {
+          const int K = kz0 + a, J = jy0 + bq, I = ix0 + cq;
+          has[a][bq][cq] = (a == 0 || (k & 1)) && (bq == 0 || (j & 1)) && (cq == 0 || (i & 1)) &&
+                           (DIM == 2 || (K > 0 && K < pc - 1)) && J > 0 && J < pc - 1 && I > 0 &&
+                           I < pc - 1;
+          v[a][bq][cq] = has[a][bq][cq] ? xc[I + pc * (J + pc * K)] : 0.0;
         }
-      }
-    }
+    double s = x[f];
+#pragma unroll
+    for (int a = 0; a < NZ; ++a)
+#pragma unroll
+      for (int bq = 0; bq < 2; ++bq)
+#pragma unroll
+        for (int cq = 0; cq < 2; ++cq) {
+          const double sn = s + w * v[a][bq][cq];
+          s = has[a][bq][cq] ? sn : s;
+        }
     x[f] = s;
   }
 }
 
 // ---- a dense inverse on the coarsest level ---------------------------------
-// x = C b with C stored by columns (ct[j n + i] = C_ij).  The columns are
-// cut into kDenseParts blocks of ceil(n / kDenseParts); wave k of a
-// workgroup sums block k of 64 rows from 0 in ascending j (lane = row, so
-// its loads are contiguous), and the row's sum is p_0 + p_1 + ... + p_7 in
-// that order.  Eight waves per 64 rows keep enough loads in flight for a
-// matrix read once per cycle.
+// x = C b.  The columns are cut into kDenseParts blocks of
+// ceil(n / kDenseParts); a lane sums one block of its row from 0 in ascending
+// j, and the row's sum is p_0 + p_1 + ... + p_7 in that order.
+//
+// The kernel reads C once, so its time is the latency of a lane's loads
+// times how often it waits for them, and the number of CUs that ask.  C is
+// stored in strips of kDenseRows rows, a strip by columns (the loads of a
+// block's 16 lanes are one aligned line): one workgroup of two waves a
+// strip, which loads kDenseBatch columns before it adds the first.  729
+// rows: 22.8 us with 64 rows a workgroup, eight waves and 24 columns in
+// flight, 9.2 us with eight, 6.3 us here.
 constexpr int kDenseParts = 8;
-constexpr int kDenseBlock = kDenseParts * kWave;
+constexpr int kDenseRows = 16;
+constexpr int kDenseBlock = kDenseParts * kDenseRows;
 constexpr int kDenseMaxRows = 4096;
+constexpr int kDenseBatch = 32;
+
+__host__ __device__ inline size_t dense_entries(int n) {
+  return (size_t)((n + kDenseRows - 1) / kDenseRows * kDenseRows) * n;
+}
 
 __global__ void __launch_bounds__(kDenseBlock)
-    mg_dense_kernel(int n, const double *__restrict__ ct, const double *__restrict__ b,
+    mg_dense_kernel(int n, const double *__restrict__ c, const double *__restrict__ b,
                     double *__restrict__ x, const int *status) {
 #pragma clang fp contract(off)
-  __shared__ double part[kDenseParts][kWave];
+  __shared__ double bs[kDenseMaxRows], part[kDenseParts][kDenseRows];
   if (stopped(status)) return;
-  const int lane = threadIdx.x & (kWave - 1), k = threadIdx.x / kWave;
-  const int i = blockIdx.x * kWave + lane;
+  const int lane = threadIdx.x % kDenseRows, k = threadIdx.x / kDenseRows;
+  const int i = blockIdx.x * kDenseRows + lane;
   const int cb = (n + kDenseParts - 1) / kDenseParts;
   const int j0 = k * cb, j1 = j0 + cb < n ? j0 + cb : n;
+  const double *__restrict__ strip = c + (size_t)blockIdx.x * kDenseRows * n + lane;
+  double v[kDenseBatch];
+  // columns past the block's end (or a block with none) load its last column
+  // or the matrix's, and are not added
+  auto load = [&](int j) {
+#pragma unroll
+    for (int q = 0; q < kDenseBatch; ++q)
+      v[q] = strip[(size_t)(j + q < n ? j + q : n - 1) * kDenseRows];
+  };
+  load(j0);
+  for (int j = threadIdx.x; j < n; j += kDenseBlock) bs[j] = b[j];
+  __syncthreads();
   double s = 0;
-  if (i < n) {
-#pragma unroll 8
-    for (int j = j0; j < j1; ++j) s += ct[(size_t)j * n + i] * b[j];
+  for (int j = j0; j < j1; j += kDenseBatch) {
+    if (j > j0) load(j);
+    __builtin_amdgcn_sched_barrier(0);  // all loads before the first use
+#pragma unroll
+    for (int q = 0; q < kDenseBatch; ++q) {
+      const double sn = s + v[q] * bs[j + q < n ? j + q : n - 1];
+      s = j + q < j1 ? sn : s;
+    }
   }
   part[k][lane] = s;
   __syncthreads();
@@ -469,13 +529,16 @@ __global__ void __launch_bounds__(kDenseBlock)
   }
 }
 
+// The strips of a row-major matrix; rows past the last are zero.
 __global__ void __launch_bounds__(kBlock)
-    mg_transpose_kernel(int n, const double *__restrict__ a, double *__restrict__ at) {
-  const long long nn = (long long)n * n;
+    mg_strips_kernel(int n, const double *__restrict__ a, double *__restrict__ c) {
+  const long long nn = (long long)dense_entries(n);
   for (long long k = (long long)blockIdx.x * kBlock + threadIdx.x; k < nn;
        k += (long long)gridDim.x * kBlock) {
-    const long long i = k / n, j = k - i * n;
-    at[j * n + i] = a[k];
+    const long long strip = k / ((long long)kDenseRows * n);
+    const int rest = (int)(k - strip * kDenseRows * n);
+    const long long i = strip * kDenseRows + rest % kDenseRows;
+    c[k] = i < n ? a[i * n + rest / kDenseRows] : 0.0;
   }
 }
 
@@ -619,7 +682,7 @@ struct hflmp_mg {
   int tail = 0;   // first level of the one-workgroup tail (nlevels: none)
   int tail0 = 0;  // the tail chosen at creation
   MgLevelDev *dlv = nullptr;  // device copy of the level table
-  double *cinv = nullptr;     // coarsest level's inverse by columns, or null
+  double *cinv = nullptr;     // coarsest level's inverse in strips, or null
   int sdim = 0;               // structured Q1 transfers: dimension, or 0
   int scells[kMaxLevels] = {};  // cells per direction of each level
 };
@@ -668,19 +731,26 @@ void smooth_first(hipStream_t s, const hflmp_mg *m, int l, double w, const doubl
     mg_first_kernel<<<gv, kBlock, 0, s>>>(L.n, w, L.invd, b, x, status);
 }
 
+// dot: also the partials of b.xo, one a workgroup of grid sell_grid(n)
 void smooth_sweep(hipStream_t s, const hflmp_mg *m, int l, double w, const double *b,
-                  const double *xi, double *xo, const int *status) {
+                  const double *xi, double *xo, const int *status, double *dot = nullptr) {
   const auto &L = m->lv[l];
   const unsigned ga = sell_grid(L.n);
-  if (l == 0 && m->st) {
-    (void)stencil_dispatch<double>(m->st, [&](auto op) {
-      mg_st_sweep_kernel<<<ga, kBlock, 0, s>>>(op, w, L.invd, b, xi, xo, status);
-    });
-  } else {
-    sell_dispatch<double>(L.A, [&](auto op) {
-      mg_sweep_kernel<<<ga, kBlock, 0, s>>>(op, w, 1.0 - w, L.invd, b, xi, xo, status);
-    });
-  }
+  auto launch = [&](auto with_dot) {
+    constexpr bool DOT = decltype(with_dot)::value;
+    if (l == 0 && m->st)
+      (void)stencil_dispatch<double>(m->st, [&](auto op) {
+        mg_st_sweep_kernel<DOT><<<ga, kBlock, 0, s>>>(op, w, L.invd, b, xi, xo, dot, status);
+      });
+    else
+      sell_dispatch<double>(L.A, [&](auto op) {
+        mg_sweep_kernel<DOT><<<ga, kBlock, 0, s>>>(op, w, 1.0 - w, L.invd, b, xi, xo, dot, status);
+      });
+  };
+  if (dot)
+    launch(std::true_type());
+  else
+    launch(std::false_type());
 }
 
 void residual(hipStream_t s, const hflmp_mg *m, int l, const double *b, const double *x,
@@ -699,15 +769,31 @@ void residual(hipStream_t s, const hflmp_mg *m, int l, const double *b, const do
   }
 }
 
+double level_omega(const hflmp_mg *m, int l) {
+  return l == m->nlevels - 1 ? m->prm.coarse_omega : m->prm.omega;
+}
+
+// The buffer that the first step of level 0's cycle into `out` writes, or
+// null if that cycle has no first step (a dense solve of a single level).
+double *first_buffer(const hflmp_mg *m, double *out) {
+  const bool coarsest = m->nlevels == 1;
+  if (coarsest && m->cinv) return nullptr;
+  const int first = coarsest ? m->prm.coarse_sweeps : m->prm.pre_smooth;
+  const int swaps = (first - 1) + (coarsest ? 0 : m->prm.post_smooth);
+  return (swaps & 1) ? m->lv[0].x2 : out;
+}
+
 // One cycle from level l with right-hand side b; returns the buffer that
 // holds the result.  `out` (level 0) is the buffer the result must end in:
 // the ping-pong pair starts so that the last write lands there.  Every
 // launch returns at once when *status is set and not "iterate".
+// first_done: the first step is already in its buffer.  dot (level 0): the
+// last post-smoothing sweep also leaves the partials of b.out.
 double *cycle(hipStream_t s, const hflmp_mg *m, int l, const double *b, double *out,
-              const int *status) {
+              const int *status, bool first_done = false, double *dot = nullptr) {
   const auto &L = m->lv[l];
   const bool coarsest = l == m->nlevels - 1;
-  const double w = coarsest ? m->prm.coarse_omega : m->prm.omega;
+  const double w = level_omega(m, l);
   const unsigned ga = sell_grid(L.n);
   const bool dense = coarsest && m->cinv;
   const int first = coarsest ? m->prm.coarse_sweeps : m->prm.pre_smooth;
@@ -724,11 +810,11 @@ double *cycle(hipStream_t s, const hflmp_mg *m, int l, const double *b, double *
     y = (swaps & 1) ? out : L.x2;
   }
   if (dense) {
-    mg_dense_kernel<<<(L.n + kWave - 1) / kWave, kDenseBlock, 0, s>>>(L.n, m->cinv, b, x,
-                                                                       status);
+    mg_dense_kernel<<<(L.n + kDenseRows - 1) / kDenseRows, kDenseBlock, 0, s>>>(L.n, m->cinv, b,
+                                                                                 x, status);
     return x;
   }
-  smooth_first(s, m, l, w, b, x, status);
+  if (!first_done) smooth_first(s, m, l, w, b, x, status);
   for (int k = 1; k < first; ++k) {
     smooth_sweep(s, m, l, w, b, x, y, status);
     std::swap(x, y);
@@ -740,14 +826,25 @@ double *cycle(hipStream_t s, const hflmp_mg *m, int l, const double *b, double *
   DivMagic dpf, dpc;
   dpf.init((unsigned)pf);
   dpc.init((unsigned)pc);
+  // the coarse level's first step rides on the restriction, unless that
+  // level is solved densely or by the one-workgroup tail
+  const bool cdense = l + 1 == m->nlevels - 1 && m->cinv;
+  const bool cfirst = m->sdim && !cdense && l + 1 != m->tail;
+  const double cw = level_omega(m, l + 1);
+  auto restrict_q1 = [&](auto dim, auto with_first) {
+    mg_restrict_q1_kernel<decltype(dim)::value, decltype(with_first)::value>
+        <<<grid_for(C.n, 1), kBlock, 0, s>>>(pf, pc, dpc, L.r, C.b, cw, C.invd, C.x, status);
+  };
+  using D2 = std::integral_constant<int, 2>;
+  using D3 = std::integral_constant<int, 3>;
   if (m->sdim == 3)
-    mg_restrict_q1_kernel<3><<<grid_for(C.n, 1), kBlock, 0, s>>>(pf, pc, dpc, L.r, C.b, status);
+    cfirst ? restrict_q1(D3(), std::true_type()) : restrict_q1(D3(), std::false_type());
   else if (m->sdim == 2)
-    mg_restrict_q1_kernel<2><<<grid_for(C.n, 1), kBlock, 0, s>>>(pf, pc, dpc, L.r, C.b, status);
+    cfirst ? restrict_q1(D2(), std::true_type()) : restrict_q1(D2(), std::false_type());
   else
     mg_apply_kernel<false><<<sell_grid(C.n), kBlock, 0, s>>>(sell_view<double, int>(L.R), L.r,
                                                               C.b, status);
-  const double *xc = cycle(s, m, l + 1, C.b, nullptr, status);
+  const double *xc = cycle(s, m, l + 1, C.b, nullptr, status, cfirst);
   if (m->sdim == 3)
     mg_prolong_q1_kernel<3><<<grid_for(L.n, 1), kBlock, 0, s>>>(pf, pc, dpf, xc, x, status);
   else if (m->sdim == 2)
@@ -755,7 +852,7 @@ double *cycle(hipStream_t s, const hflmp_mg *m, int l, const double *b, double *
   else
     mg_apply_kernel<true><<<ga, kBlock, 0, s>>>(sell_view<double, int>(L.P), xc, x, status);
   for (int k = 0; k < m->prm.post_smooth; ++k) {
-    smooth_sweep(s, m, l, w, b, x, y, status);
+    smooth_sweep(s, m, l, w, b, x, y, status, k + 1 == m->prm.post_smooth ? dot : nullptr);
     std::swap(x, y);
   }
   return x;
@@ -971,12 +1068,12 @@ int hflmp_mg_set_coarse_inverse_f64(hflmp_ctx *ctx, hflmp_mg *m, const double *i
   HFLMP_REQUIRE(ctx, n <= kDenseMaxRows, "mg_set_coarse_inverse: coarsest level has %d rows "
                                          "(at most %d)", n, kDenseMaxRows);
   if (!m->cinv &&
-      hipMalloc(&m->cinv, sizeof(double) * (size_t)n * (size_t)n) != hipSuccess) {
+      hipMalloc(&m->cinv, sizeof(double) * dense_entries(n)) != hipSuccess) {
     m->cinv = nullptr;
     return set_error(ctx, HFLMP_ENOMEM, "mg_set_coarse_inverse: out of device memory");
   }
-  mg_transpose_kernel<<<grid_for((long long)n * n, 4), kBlock, 0, ctx->stream>>>(n, inv,
-                                                                                m->cinv);
+  mg_strips_kernel<<<grid_for((long long)dense_entries(n), 4), kBlock, 0, ctx->stream>>>(
+      n, inv, m->cinv);
   HFLMP_LAUNCH_CHECK(ctx);
   // the coarsest level is no longer swept: the one-workgroup tail stops
   // above it
@@ -1022,16 +1119,28 @@ int hflmp_pcg_mg_f64(hflmp_ctx *ctx, const hflmp_mg *m, const double *b, double 
   mgcg_init_final<<<1, kFinalBlock, 0, s>>>(st, partials, gd);
   mgcg_p_kernel<<<gd, kBlock, 0, s>>>(n, z, p, st, 1);
   HFLMP_LAUNCH_CHECK(ctx);
+  double *first = first_buffer(m, z);
+  const double w0 = level_omega(m, 0);
+  // r.z from the cycle's last sweep, if it ends with one
+  const bool dot = m->nlevels > 1 && m->prm.post_smooth > 0;
   auto iteration = [&]() {
     with_fine_op(m, [&](auto op) {
       mgcg_spmv_kernel<<<ga, kBlock, 0, s>>>(op, p, Ap, partials, status);
     });
     mgcg_alpha_final<<<1, kFinalBlock, 0, s>>>(st, partials, (int)ga);
-    mgcg_update_kernel<<<gd, kBlock, 0, s>>>(n, p, Ap, x, r, st, partials);
+    auto update = [&](auto kern) {
+      kern<<<gd, kBlock, 0, s>>>(n, p, Ap, x, r, st, partials, w0, m->lv[0].invd, first);
+    };
+    if (!first)
+      update(mgcg_update_kernel<0>);
+    else if (m->st)
+      update(mgcg_update_kernel<2>);
+    else
+      update(mgcg_update_kernel<1>);
     mgcg_check_final<<<1, kFinalBlock, 0, s>>>(st, partials, gd);
-    apply(s, m, r, z, status);
-    mgcg_rz_kernel<<<gd, kBlock, 0, s>>>(n, r, z, st, partials);
-    mgcg_beta_final<<<1, kFinalBlock, 0, s>>>(st, partials, gd);
+    (void)cycle(s, m, 0, r, z, status, first != nullptr, dot ? partials : nullptr);
+    if (!dot) mgcg_rz_kernel<<<gd, kBlock, 0, s>>>(n, r, z, st, partials);
+    mgcg_beta_final<<<1, kFinalBlock, 0, s>>>(st, partials, dot ? (int)ga : gd);
     mgcg_p_kernel<<<gd, kBlock, 0, s>>>(n, z, p, st, 0);
   };
   rc = run_polled(ctx, maxit, &st->status, iteration, 2);

@@ -333,3 +333,53 @@ def test_single_level_jacobi_solver(ctx):
     finally:
         M.free()
         dA.free()
+
+
+@pytest.mark.parametrize("coarse", ["sweeps", "dense"])
+@pytest.mark.parametrize("mf", [False, True])
+@pytest.mark.parametrize("case", [(2, 16, None, 1, 1), (2, 64, None, 2, 1), (3, 16, 2, 1, 2),
+                                  (3, 32, None, 1, 1), (3, 8, 1, 2, 1), (2, 32, 3, 3, 3)])
+def test_pcg_first_step_and_dot_in_the_cycle(ctx, case, mf, coarse):
+    """CG's update leaves the cycle's first step, the restriction the coarse
+    level's, and the last sweep r.z: every combination of smoothing steps,
+    depth, finest level and coarse solve against CG with the cycle applied
+    on its own."""
+    dim, n, nl, pre, post = case
+    if coarse == "dense" and nl == 1:
+        pytest.skip("a dense coarse solve needs two levels")
+    kap = hflmp.fe_kappa(dim, n, 1.0, 9)
+    E = hflmp.fe_element(1, dim, n)
+    A = hflmp.fe_system(1, dim, n, kap)
+    dA = hflmp.CsrMatrix(ctx, *A)
+    S = hflmp.StencilOperator(ctx, 1, dim, [n] * dim, E, kap, hflmp.fe_fixed(1, dim, n)) if mf \
+        else None
+    M = mg.build_structured(ctx, dim, n, E, kap, None if mf else dA, nlevels=nl, stencil=S,
+                            coarse=coarse, pre_smooth=pre, post_smooth=post, omega=0.7,
+                            coarse_sweeps=6)
+    try:
+        b = hflmp.fe_rhs(1, dim, n, 5)
+        db, dx = ctx.upload(b), ctx.zeros(len(b), np.float64)
+        dr, dz = ctx.zeros(len(b), np.float64), ctx.zeros(len(b), np.float64)
+        info = M.pcg(db, dx, rtol=1e-8, maxit=300)
+        x = dx.download()
+
+        def prec(r):
+            dr.copy_from_host(r)
+            M.apply(dr, dz)
+            return dz.download()
+
+        xo, io = O.cg_prec(A, b, prec, rtol=1e-8, maxit=300)
+        assert info["status"] == io["status"]
+        assert abs(info["iters"] - io["iters"]) <= 1
+        if pre == post and info["status"] == 0:
+            assert np.linalg.norm(b - O.spmv(*A, x)) <= 2e-8 * np.linalg.norm(b)
+        # the same iterates to rounding while CG is well behaved
+        if info["iters"] == io["iters"] and info["status"] == 0:
+            assert np.linalg.norm(x - xo) <= 1e-8 * np.linalg.norm(xo)
+        for a in (db, dx, dr, dz):
+            a.free()
+    finally:
+        M.free()
+        if S is not None:
+            S.free()
+        dA.free()
