@@ -146,6 +146,35 @@ __device__ __forceinline__ T wave_sum(T v) {
   return wave_reduce(v, [](T a, T b) { return a + b; });
 }
 
+// lane 0's value, uniform across the wave
+template <typename T>
+__device__ __forceinline__ T bcast0(T v) {
+  constexpr int W = sizeof(T) / 4;
+  struct Words {
+    int w[W];
+  };
+  Words a = __builtin_bit_cast(Words, v);
+#pragma unroll
+  for (int i = 0; i < W; ++i) a.w[i] = __builtin_amdgcn_readfirstlane(a.w[i]);
+  return __builtin_bit_cast(T, a);
+}
+
+// wave_sum of a v that is +0 on lanes `count` and above (count > 0, uniform):
+// the steps that would only add those zeros are left out.
+template <typename T>
+__device__ __forceinline__ T wave_sum_first(T v, int count) {
+  auto add = [](T a, T b) { return a + b; };
+  if (count > 32) v = wave_step<32>(v, add);
+  if (count > 16) v = wave_step<16>(v, add);
+  if (count > 4) {  // wave_step<4> relies on <8> (dpp_xor)
+    v = wave_step<8>(v, add);
+    v = wave_step<4>(v, add);
+  }
+  if (count > 2) v = wave_step<2>(v, add);
+  if (count > 1) v = wave_step<1>(v, add);
+  return bcast0(v);
+}
+
 __device__ __forceinline__ int wave_min(int v) {
   return wave_reduce(v, [](int a, int b) { return a < b ? a : b; });
 }

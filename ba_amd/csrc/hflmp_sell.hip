@@ -21,6 +21,7 @@ struct SellStats {
   unsigned int bad16;      // entries whose offset from the slice start needs more than 16 bits
   unsigned int bad_off;    // slices that the offset form cannot hold
   unsigned int bad16_off;  // bad16 as the offset count saw it (all of it if bad_off is 0)
+  int max_off;             // the largest |offset|
 };
 
 // Row lengths (a byte each) and, per slice, the longest row (m; where its
@@ -168,9 +169,13 @@ __global__ void __launch_bounds__(kBlock)
        s += gridDim.x * kSellSlicesPerBlock) {
     const int lane = threadIdx.x & (kWave - 1);
     bool far = false;  // a column beyond int16 of the slice's first row
+    int most = 0;
     const int K = for_slice_offsets(s, nrow, rp, ci, [&](int, int o, bool has, int) {
       far = far || (has && (o + lane < -32768 || o + lane > 32767));
+      const int a = o < 0 ? -o : o;
+      most = a > most ? a : most;
     });
+    if (lane == 0 && most > stats->max_off) atomicMax(&stats->max_off, most);
     if (__any(far) && lane == 0) atomicAdd(&stats->bad16_off, 1u);
     if (lane == 0) {
       klen[s] = K < 0 ? 0 : K;
@@ -375,6 +380,7 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   const double col_bytes = (double)entries * (sizeof(T) + m->col_bytes) + nrow;
   if (try_off && hs.bad_off == 0 && off_bytes < 0.95 * col_bytes) {
     m->off_form = 1;
+    m->max_off = hs.max_off;
     m->entries = kentries;
     std::swap(m->soff, koff);
     std::swap(m->slen, klen);

@@ -54,6 +54,7 @@ struct hflmp_sell {
   int off_form;         // offset form: no col; slen is the slices' offsets
   int *off;             // offset of position j of slice s at soff[s] / 64 + j
   unsigned long long *mask;  // its rows
+  int max_off;               // the largest |offset|
   unsigned int *check;  // device counter of rows whose length changed (set_values)
   unsigned char *rlen;  // row lengths
   void *col;
@@ -355,7 +356,7 @@ __device__ __forceinline__ ScalarPtr<V> scalar_ptr(const V *p) {
 // a_ij x_j; NODIAG: offset 0 skipped) over the K positions in order, those
 // of the lane's row only.  xf(c) reads x at column c; it is called for every
 // position, present or not, and must accept any c.
-// Blocks of UB chunks have all their loads in flight at once, with no
+// Blocks of UB (or kSmall) chunks have all their loads in flight at once, with no
 // branch between them (a branch would wait for the loads before it): chunks
 // past the last one read the last one again and add nothing.  Two block
 // sizes, so that rows of 27 entries are 7 + 7 chunks of 2 (6 of 4 in FP32)
@@ -366,7 +367,7 @@ struct OffBlock {
   static constexpr int kSmall = sizeof(T) == 8 ? 4 : 3;
 };
 
-template <typename T, bool SUB, bool NODIAG, bool NT, typename XF>
+template <typename T, bool SUB, bool NODIAG, bool NT, int UB = OffBlock<T>::kBig, typename XF>
 __device__ __forceinline__ T sell_offset_sum(const T *__restrict__ val, ScalarPtr<int> off,
                                              ScalarPtr<unsigned long long> mask, int K, int row,
                                              int lane, XF &&xf, T s) {
@@ -396,14 +397,14 @@ __device__ __forceinline__ T sell_offset_sum(const T *__restrict__ val, ScalarPt
     const T sn = SUB ? s - a * x : s + a * x;
     s = __builtin_amdgcn_inverse_ballot_w64(m) ? sn : s;
   };
-  auto block = [&](auto ub, int c0) {
-    constexpr int UB = decltype(ub)::value;
-    TV vv[UB];
-    T xx[UB][P];
-    int oo[UB][P];
-    unsigned long long mm[UB][P];
+  auto block = [&](auto chunks, int c0) {
+    constexpr int NB = decltype(chunks)::value;
+    TV vv[NB];
+    T xx[NB][P];
+    int oo[NB][P];
+    unsigned long long mm[NB][P];
 #pragma unroll
-    for (int u = 0; u < UB; ++u) {
+    for (int u = 0; u < NB; ++u) {
       const int c = c0 + u < nch ? c0 + u : nch - 1;
       vv[u] = sell_ld<TV, NT>(v + c * kWave);
 #pragma unroll
@@ -414,15 +415,15 @@ __device__ __forceinline__ T sell_offset_sum(const T *__restrict__ val, ScalarPt
       }
     }
 #pragma unroll
-    for (int u = 0; u < UB; ++u)
+    for (int u = 0; u < NB; ++u)
 #pragma unroll
       for (int q = 0; q < P; ++q) xx[u][q] = xf(row + oo[u][q]);
 #pragma unroll
-    for (int u = 0; u < UB; ++u)
+    for (int u = 0; u < NB; ++u)
 #pragma unroll
       for (int q = 0; q < P; ++q) add(vv[u][q], xx[u][q], mm[u][q], oo[u][q]);
   };
-  constexpr int UB = OffBlock<T>::kBig, US = OffBlock<T>::kSmall;
+  constexpr int US = OffBlock<T>::kSmall;
   int c = 0;
   for (; nch - c > US; c += UB) block(std::integral_constant<int, UB>(), c);
   if (c < nch) block(std::integral_constant<int, US>(), c);
@@ -436,7 +437,7 @@ template <typename T>
 struct SellOffOp {
   using value_type = T;
   static constexpr int kLds = 1;
-  int nrow, ncol, nslice;
+  int nrow, ncol, nslice, max_off;
   const long long *soff;
   const int *slen;
   const int *off;
@@ -500,6 +501,7 @@ inline SellOffOp<T> sell_off_view(const hflmp_sell *m) {
   op.nrow = m->nrow;
   op.ncol = m->ncol;
   op.nslice = m->nslice;
+  op.max_off = m->max_off;
   op.soff = m->soff;
   op.slen = m->slen;
   op.off = m->off;
