@@ -236,14 +236,16 @@ struct BState {
 
 // per-column partial sums of one or two quantities, stored [q][column][block]
 // so that each column's partials are contiguous for its finalize workgroup.
-// Lane l holds column l, or with `sub` rows side by side column l mod k.
+// Lane l holds column l, or with `sub` rows side by side column l mod k; waves
+// beyond kWavesPerBlock hold nothing.
 template <typename T, int NQ>
 __device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *__restrict__ part,
                                                    int sub = 1) {
   __shared__ T lds[NQ][kWavesPerBlock][kWave];
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) lds[q][wid][lane] = a[q];
+  for (int q = 0; q < NQ; ++q)
+    if (wid < kWavesPerBlock) lds[q][wid][lane] = a[q];
   __syncthreads();
   if (wid == 0 && lane < k) {
 #pragma unroll
@@ -381,7 +383,7 @@ __global__ void __launch_bounds__(kBlock)
 // The same through a block layout (hflmp_spmm_plan.hpp): AP = A P with
 // per-column partials of p.Ap, one set per workgroup of the walk.
 template <typename T, int KC>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kPlanThreads, 4)
     bcg_plan_spmm_kernel(PlanView pv, int k, const int *__restrict__ rp,
                          const T *__restrict__ val, const T *__restrict__ P,
                          T *__restrict__ AP, const BState<T> *st, T *__restrict__ part) {
@@ -598,7 +600,7 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
   HFLMP_LAUNCH_CHECK(ctx);
   auto iteration = [&]() {
     if (plan) {
-      plan_kern<<<gp, kBlock, lds, s>>>(plan_view(plan), k, rp, val, P, AP, st, part);
+      plan_kern<<<gp, kPlanThreads, lds, s>>>(plan_view(plan), k, rp, val, P, AP, st, part);
       bcg_alpha_final<T><<<k, kBlock, 0, s>>>(st, part, gp, k);
     } else {
       bcg_spmm_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, P, AP, st, part);

@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 template <typename T, int KC>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kPlanThreads, 4)
     plan_spmm_kernel(PlanView pv, int k, const int *__restrict__ rp, const T *__restrict__ val,
                      const T *__restrict__ X, T *__restrict__ Y) {
   extern __shared__ __align__(16) unsigned char plan_lds[];
@@ -427,7 +427,7 @@ int plan_spmm(hflmp_ctx *ctx, const hflmp_spmm_plan *p, const int *rp, const T *
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              (int)lds));
   const int g = plan_grid(ctx, reinterpret_cast<const void *>(kern), p->nblk, lds);
-  kern<<<g, kBlock, lds, ctx->stream>>>(plan_view(p), k, rp, val, X, Y);
+  kern<<<g, kPlanThreads, lds, ctx->stream>>>(plan_view(p), k, rp, val, X, Y);
   HFLMP_LAUNCH_CHECK(ctx);
   return HFLMP_OK;
 }

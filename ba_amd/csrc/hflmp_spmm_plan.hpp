@@ -30,7 +30,9 @@
 // A wave holds the next block's X rows in registers: 20 of them in FP64,
 // 32 in FP32.
 __host__ __device__ constexpr int plan_max_cols(int vb) { return vb == 8 ? 80 : 128; }
-constexpr int kPlanMaxEntries = 1024;  // 4 per thread
+constexpr int kPlanMaxEntries = 1024;  // 4 per thread that loads
+// Threads of the walk: kBlock that compute and kBlock that load.
+constexpr int kPlanThreads = 2 * kBlock;
 
 // Block geometry: lines of L rows, blocks of nl runs (one per line) of at
 // most a rows; nseg blocks per line group.
@@ -110,7 +112,7 @@ __host__ __device__ inline size_t plan_lds_bytes(int R, int umax, int emax, int 
 inline int plan_grid(hflmp_ctx *ctx, const void *kern, int nblk, size_t lds) {
   const int cus = ctx->num_cus > 0 ? ctx->num_cus : 256;
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kBlock, lds) != hipSuccess)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kPlanThreads, lds) != hipSuccess)
     per_cu = lds > 0 ? (int)(160 * 1024 / lds) : 8;
   if (per_cu > 8) per_cu = 8;
   if (per_cu < 1) per_cu = 1;
@@ -128,7 +130,7 @@ struct PlanMeta {
   T *v;     // entries' values
   int *uc;  // distinct columns
   int *rp;  // local row pointers of the block's rows (R + 1), from 0
-  int *gr;  // global row of each of the block's rows (R)
+  int *gr;  // global row of each of the block's rows (R), -1 past its last
 };
 
 template <typename T>
@@ -197,7 +199,7 @@ template <typename T>
 __device__ __forceinline__ void plan_meta_load(PlanMetaRegs<T> &m, const PlanHdr &h,
                                                const PlanView &pv, const int *__restrict__ rp,
                                                const T *__restrict__ val) {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x & (kBlock - 1);
   // Local entry e lies in the last run that starts at or before it, and
   // has CSR index e + base for that run's base; local row t likewise has
   // global row t + rbase and its first entry at local index rp[row] + ebase.
@@ -238,13 +240,13 @@ __device__ __forceinline__ void plan_meta_load(PlanMetaRegs<T> &m, const PlanHdr
 
 template <typename T>
 __device__ __forceinline__ void plan_meta_store(const PlanMetaRegs<T> &m, const PlanHdr &h,
-                                                const PlanMeta<T> &d) {
-  const int t = threadIdx.x;
-  if (t < h.nr) {
-    d.rp[t] = m.rp;
-    d.gr[t] = m.gr;
+                                                const PlanView &pv, const PlanMeta<T> &d) {
+  const int t = threadIdx.x & (kBlock - 1);
+  if (t < pv.R) {
+    d.rp[t] = t < h.nr ? m.rp : h.ne;
+    d.gr[t] = t < h.nr ? m.gr : -1;
   }
-  if (t == h.nr) d.rp[t] = h.ne;
+  if (t == pv.R) d.rp[t] = h.ne;
   if (t < h.U) d.uc[t] = m.uc;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -256,22 +258,74 @@ __device__ __forceinline__ void plan_meta_store(const PlanMetaRegs<T> &m, const 
   }
 }
 
+// v of lane Q of the lane's row of 16.
+template <int Q, typename T>
+__device__ __forceinline__ T row_bcast(T v) {
+  constexpr int W = sizeof(T) / 4;
+  struct Words {
+    int w[W];
+  };
+  Words a = __builtin_bit_cast(Words, v);
+#pragma unroll
+  for (int i = 0; i < W; ++i)
+    a.w[i] = __builtin_amdgcn_update_dpp(0, a.w[i], 0x150 + Q, 0xf, 0xf, true);
+  return __builtin_bit_cast(T, a);
+}
+
+// s + the first n (at most 4 NG, more than 4 NG - 4) of 16 entries, in
+// order: lane l holds the value v and the byte offset pos in LDS of the X
+// row of entry l % 16, xl is the lane's value of X row 0.  All X values are
+// read before the first is added.
+constexpr int kPlanStrip = 16;
+
+template <typename T, int NG, int Q = 0>
+__device__ __forceinline__ void plan_strip_load(const unsigned char *xl, int pos, T *x) {
+  if constexpr (Q < 4 * NG) {
+    x[Q] = *reinterpret_cast<const T *>(xl + row_bcast<Q>(pos));
+    plan_strip_load<T, NG, Q + 1>(xl, pos, x);
+  }
+}
+template <typename T, int NG, int Q = 0>
+__device__ __forceinline__ T plan_strip_add(T s, T v, const T *x, int n) {
+#pragma clang fp contract(off)
+  if constexpr (Q < 4 * NG) {
+    const T sn = s + row_bcast<Q>(v) * x[Q];
+    s = Q <= 4 * NG - 4 || Q < n ? sn : s;
+    return plan_strip_add<T, NG, Q + 1>(s, v, x, n);
+  }
+  return s;
+}
+template <typename T, int NG>
+__device__ __forceinline__ T plan_strip(T s, const unsigned char *xl, int pos, T v, int n) {
+  T x[4 * NG];
+  plan_strip_load<T, NG>(xl, pos, x);
+  return plan_strip_add<T, NG>(s, v, x, n);
+}
+
 // The walk.  XCD x (workgroups b with b % 8 == x) takes the contiguous band
 // of blocks [x band, (x+1) band) and its workgroups stride over it, so the
-// workgroups of one XCD are on neighbouring blocks at any time.  Per
-// workgroup a four-stage pipeline: while block m is computed from LDS, the
-// X rows of block m+1 (wave w: rows w, w+4, ...; lane c: value c), the
-// description of block m+2 and the header of block m+3 are in flight into
-// registers; the next step stores them to LDS after waiting for loads
-// issued a whole step before.  Per row, the entries' positions and values
-// are read from LDS (the same address across the wave) and their X values
-// from the staged rows, eight in flight, added in storage order.
-// pre(i) is called for row i before its sum (a value the epilogue needs,
-// loaded early so that its latency hides behind the row's entries); epi(i,
-// c, s, u) gets row i's sum s for column c = lane (c >= k: a copy of
-// column k - 1, not to be stored) and u = pre(i).
-// KC > 0: k is KC, known at compile time (the X-row offsets in LDS are
-// then shifts); KC = 0: k from the argument.
+// workgroups of one XCD are on neighbouring blocks at any time.
+//
+// The first four waves of a workgroup compute block m from LDS while the
+// last four have the next blocks on their way: the X rows of block m+1 (wave
+// w: rows w, w+4, ...; lane c: value c), the description of block m+2 and
+// the header of block m+3 in registers, stored to LDS between two barriers
+// after waiting for loads issued a whole step before.  A wave that loads
+// and stores Y as well waits, with its loads, for the stores of the step
+// (one counter), and spends its issue slots on both.
+//
+// Per row, lane l of each 16 holds the value and the position of entry l and
+// the others receive them as DPP row broadcasts (plan_strip): read by all
+// lanes from LDS they took more of its bandwidth than the X values.  The
+// rows' first 32 entries are read one row ahead.
+// 2D Q2 512^2 (1,050,625 rows, 16.8 M entries), 64 vectors, FP64: 520 us with
+// the entries read from LDS by all lanes, 463 with broadcasts, 412 with the
+// roles apart.
+//
+// pre(i) is called for row i a row ahead of its sum (a value the epilogue
+// needs); epi(i, c, s, u) gets row i's sum s for column c = lane (c >= k: a
+// copy of column k - 1, not to be stored) and u = pre(i).
+// KC > 0: k is KC, known at compile time; KC = 0: k from the argument.
 template <typename T, int KC, typename Pre, typename Epi>
 __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
                                           const int *__restrict__ rp, const T *__restrict__ val,
@@ -282,7 +336,9 @@ __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
   constexpr int nw = kBlock / kWave;
   constexpr int PFX = plan_max_cols((int)sizeof(T)) / nw;  // X rows per wave
   const int lane = threadIdx.x & (kWave - 1);
-  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int wid = wave % nw;
+  const bool loads = wave >= nw;  // the wave's role
   const int lk = lane < k ? lane : k - 1;
   const int per = gridDim.x / kXcds;
   const int xcd = blockIdx.x % kXcds, bx = blockIdx.x / kXcds;
@@ -296,80 +352,124 @@ __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
   auto blk = [&](int m) { return b_beg + (m < nb ? m : nb - 1) * per; };
 
   T *xs = reinterpret_cast<T *>(lds);
+  const unsigned char *xl = lds + lk * sizeof(T);
   unsigned char *mb = lds + (((size_t)pv.umax * k * sizeof(T) + 15) & ~size_t(15));
   const size_t msz = plan_meta_bytes(pv.R, pv.umax, pv.emax, (int)sizeof(T));
   // buffer `i` of the descriptions, recomputed from the LDS base each time
   // (an array of the two pointers would hide that they point into LDS)
   auto meta = [&](int i) { return plan_meta_at<T>(mb + (size_t)i * msz, pv); };
 
+  // The X rows of a block with U columns; past the last column the last one
+  // again, so that no branch lies between the loads.  Lane q holds the
+  // column of the wave's X row q (a read of the list per row would wait for
+  // LDS before each load).
   PlanMetaRegs<T> mr;
   T xr[PFX];
   auto load_x = [&](const PlanMeta<T> &m, int U) {
+    const int ul = wid + lane * nw;
+    const int uc = U > 0 ? m.uc[ul < U ? ul : U - 1] : 0;
 #pragma unroll
-    for (int q = 0; q < PFX; ++q) {
-      const int u = wid + q * nw;
-      if (u < U) xr[q] = X[(size_t)m.uc[u] * k + lk];
-    }
+    for (int q = 0; q < PFX; ++q) xr[q] = X[(size_t)__builtin_amdgcn_readlane(uc, q) * k + lk];
   };
   auto store_x = [&](int U) {
-    if (lane < k) {
+    if (lane < k && U > 0) {
 #pragma unroll
       for (int q = 0; q < PFX; ++q) {
         const int u = wid + q * nw;
-        if (u < U) xs[u * k + lane] = xr[q];
+        xs[(u < U ? u : U - 1) * k + lane] = xr[q];
       }
     }
   };
 
-  // prologue: block 0's description in buffer 0, block 1's in registers,
-  // block 0's X rows and block 2's header in flight
-  const int h0 = plan_hdr_load(blk(0), pv, rp);
-  const int h1 = plan_hdr_load(blk(1), pv, rp);
-  PlanHdr H0 = plan_hdr(h0, blk(0), pv);
-  plan_meta_load(mr, H0, pv, rp, val);
-  plan_meta_store(mr, H0, meta(0));
-  PlanHdr H1 = plan_hdr(h1, blk(1), pv);
-  plan_meta_load(mr, H1, pv, rp, val);
-  __syncthreads();
-  load_x(meta(0), H0.U);
-  int hn = plan_hdr_load(blk(2), pv, rp);  // header of block m+2
-  for (int m = 0; m < nb; ++m) {
-    const int buf = m & 1;
-    // loads of the previous step: X rows of m, description of m+1, header of m+2
-    store_x(H0.U);
-    plan_meta_store(mr, H1, meta(buf ^ 1));
-    const PlanHdr H2 = plan_hdr(hn, blk(m + 2), pv);
-    __syncthreads();
-    // this step's loads
-    hn = plan_hdr_load(blk(m + 3), pv, rp);
-    plan_meta_load(mr, H2, pv, rp, val);
-    load_x(meta(buf ^ 1), H1.U);
-    // block m from LDS
-    const PlanMeta<T> md = meta(buf);
-    for (int r = wid; r < H0.nr; r += nw) {
-      const int a = md.rp[r], e = md.rp[r + 1];
-      const int gi = md.gr[r];
-      const T u = pre(gi);
-      T s = 0;
-      int j = a;
-      for (; j + 8 <= e; j += 8) {
-        int li[8];
-        T vv[8], xv[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          li[q] = md.li[j + q];
-          vv[q] = md.v[j + q];
+  // A row on its way through a wave that computes: its entries, its first
+  // two strips and pre's value.
+  struct Row {
+    int a, e, gi, pos[2];
+    T v[2], u;
+  };
+  auto strip = [&](const PlanMeta<T> &md, int j, int e, int &pos, T &v) {
+    const int je = j + (lane & (kPlanStrip - 1)) < e ? j + (lane & (kPlanStrip - 1)) : e - 1;
+    const int jl = je > 0 ? je : 0;
+    pos = md.li[jl] * (k * (int)sizeof(T));
+    v = md.v[jl];
+  };
+  auto add = [&](T s, int pos, T v, int n) {
+    if (n > 12) return plan_strip<T, 4>(s, xl, pos, v, n);
+    if (n > 8) return plan_strip<T, 3>(s, xl, pos, v, n);
+    if (n > 4) return plan_strip<T, 2>(s, xl, pos, v, n);
+    return n > 0 ? plan_strip<T, 1>(s, xl, pos, v, n) : s;
+  };
+  auto compute = [&](const PlanMeta<T> &md) {
+    // lane q: row wid + nw q of the block
+    const int rq = wid + nw * lane;
+    const int rl = rq < pv.R ? rq : pv.R - 1;
+    const int ra = md.rp[rl], re = md.rp[rl + 1], rg = md.gr[rl];
+    const int rows = __popcll(__ballot(rq < pv.R && rg >= 0));
+    auto row = [&](int q) {
+      Row w;
+      w.a = __builtin_amdgcn_readlane(ra, q);
+      w.e = __builtin_amdgcn_readlane(re, q);
+      w.gi = __builtin_amdgcn_readlane(rg, q);
+      w.u = pre(w.gi);
+      strip(md, w.a, w.e, w.pos[0], w.v[0]);
+      strip(md, w.a + kPlanStrip, w.e, w.pos[1], w.v[1]);
+      return w;
+    };
+    if (rows == 0) return;
+    Row w = row(0);
+    for (int q = 0; q < rows; ++q) {
+      const Row next = row(q + 1 < rows ? q + 1 : q);
+      T s = add(T(0), w.pos[0], w.v[0], w.e - w.a);
+      if (w.e - w.a > kPlanStrip) {
+        s = add(s, w.pos[1], w.v[1], w.e - w.a - kPlanStrip);
+        for (int j = w.a + 2 * kPlanStrip; j < w.e; j += kPlanStrip) {
+          int pos;
+          T v;
+          strip(md, j, w.e, pos, v);
+          s = add(s, pos, v, w.e - j);
         }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) xv[q] = xs[li[q] * k + lk];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) s += vv[q] * xv[q];
       }
-      for (; j < e; ++j) s += md.v[j] * xs[md.li[j] * k + lk];
-      epi(gi, lane, s, u);
+      epi(w.gi, lane, s, w.u);
+      w = next;
     }
+  };
+
+  // Both roles pass the same barriers: one, and two a block.  (The role is
+  // uniform across a wave; two loops keep one's registers out of the other's.)
+  if (loads) {
+    // prologue: block 0's description in buffer 0, block 1's in registers,
+    // block 0's X rows and block 2's header in flight
+    const int h0 = plan_hdr_load(blk(0), pv, rp);
+    const int h1 = plan_hdr_load(blk(1), pv, rp);
+    PlanHdr H0 = plan_hdr(h0, blk(0), pv);
+    plan_meta_load(mr, H0, pv, rp, val);
+    plan_meta_store(mr, H0, pv, meta(0));
+    PlanHdr H1 = plan_hdr(h1, blk(1), pv);
+    plan_meta_load(mr, H1, pv, rp, val);
     __syncthreads();
-    H0 = H1;
-    H1 = H2;
+    load_x(meta(0), H0.U);
+    int hn = plan_hdr_load(blk(2), pv, rp);  // header of block m+2
+    for (int m = 0; m < nb; ++m) {
+      const int buf = m & 1;
+      // loads of the previous step: X rows of m, description of m+1, header of m+2
+      store_x(H0.U);
+      plan_meta_store(mr, H1, pv, meta(buf ^ 1));
+      const PlanHdr H2 = plan_hdr(hn, blk(m + 2), pv);
+      __syncthreads();
+      // this step's loads
+      hn = plan_hdr_load(blk(m + 3), pv, rp);
+      plan_meta_load(mr, H2, pv, rp, val);
+      load_x(meta(buf ^ 1), H1.U);
+      __syncthreads();
+      H0 = H1;
+      H1 = H2;
+    }
+  } else {
+    __syncthreads();
+    for (int m = 0; m < nb; ++m) {
+      __syncthreads();
+      compute(meta(m & 1));
+      __syncthreads();
+    }
   }
 }

@@ -178,3 +178,33 @@ def test_plan_refuses_bad_column(ctx):
     assert not h.value
     bad.free()
     A.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("k", [1, 4, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64])
+def test_plan_row_lengths(ctx, k, dtype):
+    """Rows of 0 to 50 entries (whole strips of 16 and groups of 4, and every
+    remainder) in blocks that mix them, bit for bit; and infinities and NaN
+    in X reach the rows that have an entry there and no others."""
+    rng = np.random.default_rng(k)
+    n = 203
+    cols = [np.sort(rng.choice(np.arange(max(0, min(i - 26, n - 53)), max(0, min(i - 26, n - 53)) + 53),
+                               int(rng.integers(0, 51)), replace=False)) for i in range(n)]
+    cols[7] = cols[7][:0]
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32)
+    ci = np.concatenate(cols).astype(np.int32)
+    v = rng.uniform(-1, 1, len(ci))
+    _check(ctx, rp, ci, v, n, k, dtype)
+    v = v.astype(dtype)
+    X = rng.uniform(-1, 1, (n, k)).astype(dtype)
+    X[[60, 61, 140]] = np.array([np.inf, np.nan, -np.inf], dtype)[:, None]
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    P = hflmp.SpmmPlan(ctx, A, k)
+    dX, dY = ctx.upload(X.ravel()), ctx.empty(n * k, dtype)
+    P.spmm(A, dX, dY, k)
+    Y = dY.download().reshape(n, k)
+    for c in (0, k - 1):
+        assert np.array_equal(Y[:, c], O.spmv(rp, ci, v, np.ascontiguousarray(X[:, c])),
+                              equal_nan=True)
+    for a in (P, dX, dY, A):
+        a.free()
