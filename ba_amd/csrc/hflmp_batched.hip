@@ -236,16 +236,14 @@ struct BState {
 
 // per-column partial sums of one or two quantities, stored [q][column][block]
 // so that each column's partials are contiguous for its finalize workgroup.
-// Lane l holds column l, or with `sub` rows side by side column l mod k; waves
-// beyond kWavesPerBlock hold nothing.
+// Lane l holds column l, or with `sub` rows side by side column l mod k.
 template <typename T, int NQ>
 __device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *__restrict__ part,
                                                    int sub = 1) {
   __shared__ T lds[NQ][kWavesPerBlock][kWave];
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q)
-    if (wid < kWavesPerBlock) lds[q][wid][lane] = a[q];
+  for (int q = 0; q < NQ; ++q) lds[q][wid][lane] = a[q];
   __syncthreads();
   if (wid == 0 && lane < k) {
 #pragma unroll
@@ -382,25 +380,43 @@ __global__ void __launch_bounds__(kBlock)
 
 // The same through a block layout (hflmp_spmm_plan.hpp): AP = A P with
 // per-column partials of p.Ap, one set per workgroup of the walk.
-template <typename T, int KC>
+template <typename T, int CV, bool FULL>
 __global__ void __launch_bounds__(kPlanThreads, 4)
     bcg_plan_spmm_kernel(PlanView pv, int k, const int *__restrict__ rp,
                          const T *__restrict__ val, const T *__restrict__ P,
                          T *__restrict__ AP, const BState<T> *st, T *__restrict__ part) {
+  using Cols = PlanCols<T, CV, FULL>;
   extern __shared__ __align__(16) unsigned char plan_lds[];
+  __shared__ T lds[kWavesPerBlock][kWave];
   if (!st->any_iterate) return;
-  T acc[1] = {T(0)};
-  const int lane = threadIdx.x & (kWave - 1);
-  const int lk = lane < k ? lane : k - 1;
-  plan_walk<T, KC>(
-      pv, k, rp, val, P, plan_lds, [&](int i) { return P[(size_t)i * k + lk]; },
-      [&](int i, int c, T s, T p) {
-        if (c < k) {
-          __builtin_nontemporal_store(s, AP + (size_t)i * k + c);
-          acc[0] += s * p;
-        }
+  T acc[CV] = {};
+  const int li = threadIdx.x & 15;
+  // (four entries ahead leave no registers for p and the partials where a
+  // lane has 32 bytes of columns: 66.9 against 59.7 ms on 2D Q2 128^2, k 64)
+  plan_walk<T, CV, FULL, CV * sizeof(T) < 32 ? 4 : 2>(
+      pv, k, rp, val, P, plan_lds,
+      [&](int i, T *u) { Cols::load(u, P + (size_t)i * k, li, k); },
+      [&](int i, const T *s, const T *p) {
+        Cols::store(AP + (size_t)i * k, s, li, k);
+#pragma unroll
+        for (int c = 0; c < CV; ++c) acc[c] += s[c] * p[c];
       });
-  block_col_partials<T, 1>(acc, k, part);
+  // over the wave's four rows, then over the waves that compute
+  const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  auto add = [](T a, T b) { return a + b; };
+#pragma unroll
+  for (int c = 0; c < CV; ++c) {
+    acc[c] = wave_step<16>(wave_step<32>(acc[c], add), add);
+    const int col = Cols::first(li, c / Cols::kRun) + c % Cols::kRun;
+    if (wid < kWavesPerBlock && lane < 16 && col < k) lds[wid][col] = acc[c];
+  }
+  __syncthreads();
+  if (wid == 0 && lane < k) {
+    T s = 0;
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) s += lds[w][lane];
+    part[(size_t)lane * gridDim.x + blockIdx.x] = s;
+  }
 }
 
 template <typename T>
@@ -575,7 +591,9 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
   // the block layout's walk: its grid (at most the partial area's) and LDS
   int gp = g;
   size_t lds = 0;
-  auto plan_kern = k == 64 ? &bcg_plan_spmm_kernel<T, 64> : &bcg_plan_spmm_kernel<T, 0>;
+  auto plan_kern = plan_dispatch(k, [](auto cv, auto full) {
+    return &bcg_plan_spmm_kernel<T, decltype(cv)::value, decltype(full)::value>;
+  });
   if (plan) {
     HFLMP_REQUIRE(ctx, plan->nrow == nrow && plan->nnz == nnz && plan->device == ctx->device,
                   "batched_pcg: the plan was built for another matrix or device");

@@ -199,16 +199,45 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-template <typename T, int KC>
+template <typename T, int CV, bool FULL>
 __global__ void __launch_bounds__(kPlanThreads, 4)
     plan_spmm_kernel(PlanView pv, int k, const int *__restrict__ rp, const T *__restrict__ val,
                      const T *__restrict__ X, T *__restrict__ Y) {
   extern __shared__ __align__(16) unsigned char plan_lds[];
-  plan_walk<T, KC>(
-      pv, k, rp, val, X, plan_lds, [](int) { return T(0); },
-      [&](int i, int c, T s, T) {
-        if (c < k) __builtin_nontemporal_store(s, Y + (size_t)i * k + c);
+  const int li = threadIdx.x & 15;
+  plan_walk<T, CV, FULL, 4>(
+      pv, k, rp, val, X, plan_lds, [](int, T *) {},
+      [&](int i, const T *s, const T *) {
+        PlanCols<T, CV, FULL>::store(Y + (size_t)i * k, s, li, k);
       });
+}
+
+// The rows of each block, longest first and of equal ones the first first
+// (a wave a block, lane t its row t; R <= 64).
+__global__ void __launch_bounds__(kBlock)
+    plan_rows_kernel(PlanGeom g, int R, int nblk, const int *__restrict__ rp,
+                     int2 *__restrict__ rows) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int b = blockIdx.x * (kBlock / kWave) + (int)threadIdx.x / kWave;
+  if (b >= nblk) return;
+  int gi = -1, first = 0, racc = 0, eacc = 0;
+  for (int t = 0; t < g.nl; ++t) {
+    const PlanRun run = plan_run(g, b, t);
+    const int j0 = rp[run.r0];
+    if (lane >= racc && lane < racc + run.n) {
+      gi = run.r0 + lane - racc;
+      first = rp[gi] - j0 + eacc;
+    }
+    eacc += rp[run.r0 + run.n] - j0;
+    racc += run.n;
+  }
+  const int len = gi >= 0 ? rp[gi + 1] - rp[gi] : -1;
+  int rank = 0;
+  for (int r = 0; r < R; ++r) {
+    const int other = __shfl(len, r, kWave);
+    rank += other > len || (other == len && r < lane);
+  }
+  if (lane < R) rows[(size_t)b * R + rank] = int2{gi, plan_row_pack(first, len > 0 ? len : 0)};
 }
 
 void free_plan(hflmp_spmm_plan *p) {
@@ -219,6 +248,7 @@ void free_plan(hflmp_spmm_plan *p) {
   if (p->uoff) (void)hipFree(p->uoff);
   if (p->ucol) (void)hipFree(p->ucol);
   if (p->lidx) (void)hipFree(p->lidx);
+  if (p->rows) (void)hipFree(p->rows);
   if (sw) (void)hipSetDevice(cur);
   delete p;
 }
@@ -383,7 +413,8 @@ int create_plan(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   if (hipMalloc(&p->uoff, sizeof(int) * ((size_t)nblk + 1)) != hipSuccess ||
       // one entry past the lists: an empty last block still loads ucol[uoff[nblk]]
       hipMalloc(&p->ucol, sizeof(int) * (size_t)(acc + 1)) != hipSuccess ||
-      hipMalloc(&p->lidx, sizeof(int) * (size_t)nnz) != hipSuccess) {
+      hipMalloc(&p->lidx, sizeof(int) * (size_t)nnz) != hipSuccess ||
+      hipMalloc(&p->rows, sizeof(int2) * (size_t)nblk * p->R) != hipSuccess) {
     free_plan(p);
     release();
     return set_error(ctx, HFLMP_ENOMEM, "spmm_plan: allocation failed");
@@ -396,6 +427,8 @@ int create_plan(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
     return set_error(ctx, HFLMP_EHIP, "spmm_plan: upload failed");
   }
   plan_fill_kernel<<<grid, kBlock, 0, s>>>(best.g, nblk, rp, ci, p->uoff, p->ucol, p->lidx);
+  plan_rows_kernel<<<(nblk + kBlock / kWave - 1) / (kBlock / kWave), kBlock, 0, s>>>(
+      best.g, p->R, nblk, rp, p->rows);
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) {
     free_plan(p);
     release();
@@ -420,8 +453,10 @@ int plan_spmm(hflmp_ctx *ctx, const hflmp_spmm_plan *p, const int *rp, const T *
   HFLMP_REQUIRE(ctx, lds <= 160 * 1024,
                 "plan_spmm: %zu bytes of LDS for %d x %zu-byte rows; build the plan for "
                 "these rows", lds, k, sizeof(T));
-  // 64 vectors, the common block width, with the row stride known to the compiler
-  auto kern = k == 64 ? &plan_spmm_kernel<T, 64> : &plan_spmm_kernel<T, 0>;
+  // (64 vectors, the common block width: the row stride known to the compiler)
+  auto kern = plan_dispatch(k, [](auto cv, auto full) {
+    return &plan_spmm_kernel<T, decltype(cv)::value, decltype(full)::value>;
+  });
   if (lds > 64 * 1024)
     HFLMP_HIP_CHECK(ctx, hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -452,7 +487,8 @@ int hflmp_spmm_plan_info(const hflmp_spmm_plan *plan, int *rows_per_block,
   if (max_cols_per_block) *max_cols_per_block = plan->umax;
   if (list_entries) *list_entries = plan->nuniq;
   if (device_bytes)
-    *device_bytes = 4LL * (plan->nblk + 1) + 4LL * plan->nuniq + 4LL * plan->nnz;
+    *device_bytes = 4LL * (plan->nblk + 1) + 4LL * plan->nuniq + 4LL * plan->nnz +
+                    8LL * plan->nblk * plan->R;
   return HFLMP_OK;
 }
 

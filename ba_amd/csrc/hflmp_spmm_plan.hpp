@@ -24,6 +24,8 @@
 // values with the CSR matrix; lidx replaces the column array.
 #pragma once
 
+#include <type_traits>
+
 #include "hflmp_internal.hpp"
 
 // Limits of the pipelined walk: distinct columns and entries of one block.
@@ -76,7 +78,11 @@ struct hflmp_spmm_plan {
   int *uoff;        // nblk + 1 offsets into ucol
   int *ucol;        // each block's distinct columns, ascending
   int *lidx;        // per entry: position of its column in its block's list
+  int2 *rows;       // R per block, longest first: global row (-1: none), plan_row_pack
 };
+
+// A row within its block's entries: first entry and length.
+__host__ __device__ constexpr int plan_row_pack(int first, int len) { return first << 16 | len; }
 
 struct PlanView {
   PlanGeom g;
@@ -84,11 +90,12 @@ struct PlanView {
   const int *__restrict__ uoff;
   const int *__restrict__ ucol;
   const int *__restrict__ lidx;
+  const int2 *__restrict__ rows;
 };
 
 inline PlanView plan_view(const hflmp_spmm_plan *p) {
   return PlanView{plan_geom(p->nrow, p->L, p->a, p->nl), p->nnz, p->R, p->nblk, p->umax,
-                  p->emax, p->uoff, p->ucol, p->lidx};
+                  p->emax, p->uoff, p->ucol, p->lidx, p->rows};
 }
 
 // LDS of the walk: the X rows of one block, then two buffers of the
@@ -129,8 +136,8 @@ struct PlanMeta {
   int *li;  // entries' column positions
   T *v;     // entries' values
   int *uc;  // distinct columns
-  int *rp;  // local row pointers of the block's rows (R + 1), from 0
   int *gr;  // global row of each of the block's rows (R), -1 past its last
+  int *se;  // their plan_row_pack
 };
 
 template <typename T>
@@ -139,8 +146,8 @@ __device__ __forceinline__ PlanMeta<T> plan_meta_at(unsigned char *base, const P
   m.v = reinterpret_cast<T *>(base);
   m.li = reinterpret_cast<int *>(base + (size_t)pv.emax * sizeof(T));
   m.uc = m.li + pv.emax;
-  m.rp = m.uc + pv.umax;
-  m.gr = m.rp + pv.R + 1;
+  m.gr = m.uc + pv.umax;
+  m.se = m.gr + pv.R;
   return m;
 }
 
@@ -162,22 +169,19 @@ __device__ __forceinline__ int plan_hdr_load(int b, const PlanView &pv,
   return *p;
 }
 
-// The uniform values of a block: its number, entries, column list and rows.
+// The uniform values of a block: its number, entries and column list.
 struct PlanHdr {
-  int b, hreg, ne, u0, U, nr;
+  int b, hreg, ne, u0, U;
 };
 
 __device__ __forceinline__ PlanHdr plan_hdr(int hreg, int b, const PlanView &pv) {
   PlanHdr h;
   h.b = b;
   h.hreg = hreg;
-  int ne = 0, nr = 0;
-  for (int t = 0; t < pv.g.nl; ++t) {
+  int ne = 0;
+  for (int t = 0; t < pv.g.nl; ++t)
     ne += __builtin_amdgcn_readlane(hreg, 8 + t) - __builtin_amdgcn_readlane(hreg, t);
-    nr += plan_run(pv.g, b, t).n;
-  }
   h.ne = ne;
-  h.nr = nr;
   h.u0 = __builtin_amdgcn_readlane(hreg, 16);
   h.U = __builtin_amdgcn_readlane(hreg, 17) - h.u0;
   return h;
@@ -185,46 +189,34 @@ __device__ __forceinline__ PlanHdr plan_hdr(int hreg, int b, const PlanView &pv)
 
 // A block's description on its way from memory to LDS: thread t holds
 // entries t, t+256, ... (at most 4) of the block's runs laid end to end,
-// column t of the list, and the local row pointer and global row of row t.
-// Every load is issued (addresses past the block's end are clamped into
-// it), so the number of loads in flight does not depend on the block.
+// column t of the list and row t.  Every load is issued (addresses past the
+// block's end are clamped into it), so the number of loads in flight does
+// not depend on the block.
 template <typename T>
 struct PlanMetaRegs {
   int li[4];
   T v[4];
-  int uc, rp, gr;
+  int uc;
+  int2 row;
 };
 
 template <typename T>
 __device__ __forceinline__ void plan_meta_load(PlanMetaRegs<T> &m, const PlanHdr &h,
-                                               const PlanView &pv, const int *__restrict__ rp,
-                                               const T *__restrict__ val) {
+                                               const PlanView &pv, const T *__restrict__ val) {
   const int t = threadIdx.x & (kBlock - 1);
-  // Local entry e lies in the last run that starts at or before it, and
-  // has CSR index e + base for that run's base; local row t likewise has
-  // global row t + rbase and its first entry at local index rp[row] + ebase.
-  // (Runs are in row order, and an empty run starts where the next one does.)
+  // Local entry e lies in the last run that starts at or before it, and has
+  // CSR index e + base for that run's base.  (Runs are in row order, and an
+  // empty run starts where the next one does.)
   int base[4] = {0, 0, 0, 0};
-  int rbase = 0, ebase = 0;
-  int eacc = 0, racc = 0;
+  int eacc = 0;
   for (int r = 0; r < pv.g.nl; ++r) {
     const int j = __builtin_amdgcn_readlane(h.hreg, r);
-    const int c = __builtin_amdgcn_readlane(h.hreg, 8 + r) - j;
-    const PlanRun run = plan_run(pv.g, h.b, r);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       if (t + q * kBlock >= eacc) base[q] = j - eacc;
-    if (t >= racc) {
-      rbase = run.r0 - racc;
-      ebase = eacc - j;
-    }
-    eacc += c;
-    racc += run.n;
+    eacc += __builtin_amdgcn_readlane(h.hreg, 8 + r) - j;
   }
-  // rows past the block's last take its last row (loaded, never stored)
-  const int tr = t < h.nr ? t : (h.nr > 0 ? h.nr - 1 : 0);
-  m.gr = h.nr > 0 ? tr + rbase : 0;
-  m.rp = h.nr > 0 ? rp[m.gr] + ebase : 0;
+  m.row = pv.rows[(size_t)h.b * pv.R + (t < pv.R ? t : pv.R - 1)];
   m.uc = pv.ucol[h.u0 + (t < h.U ? t : (h.U > 0 ? h.U - 1 : 0))];
   // entries past the block's last read its first run's first entry
   const int j0 = __builtin_amdgcn_readlane(h.hreg, 0);
@@ -243,10 +235,9 @@ __device__ __forceinline__ void plan_meta_store(const PlanMetaRegs<T> &m, const 
                                                 const PlanView &pv, const PlanMeta<T> &d) {
   const int t = threadIdx.x & (kBlock - 1);
   if (t < pv.R) {
-    d.rp[t] = t < h.nr ? m.rp : h.ne;
-    d.gr[t] = t < h.nr ? m.gr : -1;
+    d.gr[t] = m.row.x;
+    d.se[t] = m.row.y;
   }
-  if (t == pv.R) d.rp[t] = h.ne;
   if (t < h.U) d.uc[t] = m.uc;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -272,34 +263,99 @@ __device__ __forceinline__ T row_bcast(T v) {
   return __builtin_bit_cast(T, a);
 }
 
-// s + the first n (at most 4 NG, more than 4 NG - 4) of 16 entries, in
-// order: lane l holds the value v and the byte offset pos in LDS of the X
-// row of entry l % 16, xl is the lane's value of X row 0.  All X values are
-// read before the first is added.
+// The columns of a lane.  Four rows are computed side by side, 16 lanes
+// each; lane i of 16 holds CV of the k columns: i, i + 16, ... or, of 64
+// (FULL), runs of 16 bytes, 16 lanes apart, so that LDS and memory are read
+// and written 16 bytes a lane.  Columns past k - 1 are read (from what lies
+// behind the X row in LDS: the next one, or the descriptions, which are
+// longer than the 15 values) and dropped.
+template <typename T, int CV, bool FULL>
+struct PlanCols {
+  static constexpr int kRun = FULL ? 16 / (int)sizeof(T) : 1;  // columns a piece
+  static constexpr int kPieces = CV / kRun;
+  typedef T Piece __attribute__((ext_vector_type(kRun), aligned(sizeof(T))));
+  // first column of piece p of lane i of 16
+  __device__ __forceinline__ static int first(int i, int p) { return (p * 16 + i) * kRun; }
+  template <typename F>
+  __device__ __forceinline__ static void each(F &&f) {
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) f(p);
+  }
+  __device__ __forceinline__ static void load(T *x, const T *src, int i, int k) {
+    each([&](int p) {
+      const int c = first(i, p);
+      const Piece v = *reinterpret_cast<const Piece *>(src + (FULL || c < k ? c : 0));
+      __builtin_memcpy(x + p * kRun, &v, sizeof(v));
+    });
+  }
+  __device__ __forceinline__ static void store(T *dst, const T *x, int i, int k) {
+    each([&](int p) {
+      const int c = first(i, p);
+      Piece v;
+      __builtin_memcpy(&v, x + p * kRun, sizeof(v));
+      if (FULL || c < k) __builtin_nontemporal_store(v, reinterpret_cast<Piece *>(dst + c));
+    });
+  }
+};
+
+// s += the first n of 16 entries, in order: lane i of 16 holds the value v
+// and the byte offset pos in LDS of the X row of entry i, xl is the lane's
+// place in X row 0.  nmin <= n <= nmax <= 4 NG over the wave's rows.  The
+// X values of the next E entries (2 or 4) are read while E are added.
 constexpr int kPlanStrip = 16;
 
-template <typename T, int NG, int Q = 0>
-__device__ __forceinline__ void plan_strip_load(const unsigned char *xl, int pos, T *x) {
-  if constexpr (Q < 4 * NG) {
-    x[Q] = *reinterpret_cast<const T *>(xl + row_bcast<Q>(pos));
-    plan_strip_load<T, NG, Q + 1>(xl, pos, x);
+template <typename T, int CV, bool FULL, int E, int NG>
+struct PlanStripSum {
+  using Cols = PlanCols<T, CV, FULL>;
+  template <int Q>
+  __device__ __forceinline__ static void read(T (*x)[CV], const unsigned char *xl, int pos) {
+    const unsigned char *at = xl + row_bcast<Q>(pos);
+    Cols::each([&](int p) {
+      typedef T Piece __attribute__((ext_vector_type(Cols::kRun)));
+      const Piece v = *reinterpret_cast<const Piece *>(at + p * 16 * Cols::kRun * sizeof(T));
+      __builtin_memcpy(&x[Q % E][p * Cols::kRun], &v, sizeof(v));
+    });
+    if constexpr (Q % E < E - 1) read<Q + 1>(x, xl, pos);
   }
-}
-template <typename T, int NG, int Q = 0>
-__device__ __forceinline__ T plan_strip_add(T s, T v, const T *x, int n) {
+  template <int Q>
+  __device__ __forceinline__ static void add(T *s, const T (*x)[CV], T v, int n, bool all) {
 #pragma clang fp contract(off)
-  if constexpr (Q < 4 * NG) {
-    const T sn = s + row_bcast<Q>(v) * x[Q];
-    s = Q <= 4 * NG - 4 || Q < n ? sn : s;
-    return plan_strip_add<T, NG, Q + 1>(s, v, x, n);
+    const T vq = row_bcast<Q>(v);
+    if (all || Q < n)
+#pragma unroll
+      for (int j = 0; j < CV; ++j) s[j] += vq * x[Q % E][j];
+    if constexpr (Q % E < E - 1) add<Q + 1>(s, x, v, n, all);
   }
-  return s;
-}
-template <typename T, int NG>
-__device__ __forceinline__ T plan_strip(T s, const unsigned char *xl, int pos, T v, int n) {
-  T x[4 * NG];
-  plan_strip_load<T, NG>(xl, pos, x);
-  return plan_strip_add<T, NG>(s, v, x, n);
+  // entries Q on, Q's group being in x[Q / E % 2]
+  template <int Q>
+  __device__ __forceinline__ static void group(T *s, T (*x)[E][CV], const unsigned char *xl,
+                                               int pos, T v, int n, int nmin) {
+    if constexpr (Q + E < 4 * NG) read<Q + E>(x[(Q / E + 1) % 2], xl, pos);
+    if (nmin >= Q + E)
+      add<Q>(s, x[Q / E % 2], v, n, true);
+    else
+      add<Q>(s, x[Q / E % 2], v, n, false);
+    if constexpr (Q + E < 4 * NG) group<Q + E>(s, x, xl, pos, v, n, nmin);
+  }
+  __device__ __forceinline__ static void run(T *s, const unsigned char *xl, int pos, T v, int n,
+                                             int nmin) {
+    T x[2][E][CV];
+    read<0>(x[0], xl, pos);
+    group<0>(s, x, xl, pos, v, n, nmin);
+  }
+};
+
+template <typename T, int CV, bool FULL, int E>
+__device__ __forceinline__ void plan_strip(T *s, const unsigned char *xl, int pos, T v, int n,
+                                           int nmin, int nmax) {
+  if (nmax > 12)
+    PlanStripSum<T, CV, FULL, E, 4>::run(s, xl, pos, v, n, nmin);
+  else if (nmax > 8)
+    PlanStripSum<T, CV, FULL, E, 3>::run(s, xl, pos, v, n, nmin);
+  else if (nmax > 4)
+    PlanStripSum<T, CV, FULL, E, 2>::run(s, xl, pos, v, n, nmin);
+  else if (nmax > 0)
+    PlanStripSum<T, CV, FULL, E, 1>::run(s, xl, pos, v, n, nmin);
 }
 
 // The walk.  XCD x (workgroups b with b % 8 == x) takes the contiguous band
@@ -307,39 +363,42 @@ __device__ __forceinline__ T plan_strip(T s, const unsigned char *xl, int pos, T
 // workgroups of one XCD are on neighbouring blocks at any time.
 //
 // The first four waves of a workgroup compute block m from LDS while the
-// last four have the next blocks on their way: the X rows of block m+1 (wave
-// w: rows w, w+4, ...; lane c: value c), the description of block m+2 and
-// the header of block m+3 in registers, stored to LDS between two barriers
-// after waiting for loads issued a whole step before.  A wave that loads
-// and stores Y as well waits, with its loads, for the stores of the step
-// (one counter), and spends its issue slots on both.
+// last four have the next blocks on their way: the X rows of block m+1, the
+// description of block m+2 and the header of block m+3 in registers, stored
+// to LDS between two barriers after waiting for loads issued a whole step
+// before.  A wave that loads and stores Y as well waits, with its loads, for
+// the stores of the step (one counter), and spends its issue slots on both.
 //
-// Per row, lane l of each 16 holds the value and the position of entry l and
-// the others receive them as DPP row broadcasts (plan_strip): read by all
-// lanes from LDS they took more of its bandwidth than the X values.  The
-// rows' first 32 entries are read one row ahead.
-// 2D Q2 512^2 (1,050,625 rows, 16.8 M entries), 64 vectors, FP64: 520 us with
-// the entries read from LDS by all lanes, 463 with broadcasts, 412 with the
-// roles apart.
+// The computing waves are bound by their instructions: a product and a sum
+// per entry and column (the CSR loop's rounding, so not fused), and the
+// entry's value and position for every lane.  So a wave computes four rows
+// side by side, 16 lanes each with up to four columns a lane; lane i of a
+// row's 16 holds entry i and the others take it as a DPP row broadcast, once
+// for all the lane's columns.  The rows of a block are in order of length,
+// so that the four are about as long (2D Q2 has rows of 25, 15 and 9), and
+// a wave's turns alternate between the longer and the shorter.  The first 32
+// entries of rows are read a turn ahead.
+// 2D Q2 512^2 (1,050,625 rows, 16.8 M entries), FP64, 64 vectors: 520 us
+// with a row a wave and its entries read from LDS by all lanes, 463 with
+// broadcasts, 412 with the roles apart, 303 with four rows (16 vectors: 449
+// with broadcasts, 390, 155; FP32, 64 vectors: 345, 298, 200).
 //
-// pre(i) is called for row i a row ahead of its sum (a value the epilogue
-// needs); epi(i, c, s, u) gets row i's sum s for column c = lane (c >= k: a
-// copy of column k - 1, not to be stored) and u = pre(i).
-// KC > 0: k is KC, known at compile time; KC = 0: k from the argument.
-template <typename T, int KC, typename Pre, typename Epi>
+// pre(i, u) leaves CV values for row i before its sums (what the epilogue
+// needs, loaded early); epi(i, s, u) gets row i's sums of the lane's columns
+// (PlanCols) on the lanes that have a row.  E: the entries read ahead.
+template <typename T, int CV, bool FULL, int E, typename Pre, typename Epi>
 __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
                                           const int *__restrict__ rp, const T *__restrict__ val,
                                           const T *__restrict__ X, unsigned char *lds,
                                           Pre &&pre, Epi &&epi) {
-#pragma clang fp contract(off)
-  const int k = KC > 0 ? KC : k_arg;
+  const int k = FULL ? 64 : k_arg;
   constexpr int nw = kBlock / kWave;
-  constexpr int PFX = plan_max_cols((int)sizeof(T)) / nw;  // X rows per wave
+  // X rows a load of one wave brings, and its loads
+  constexpr int SUB = CV == 1 ? 4 : CV == 2 ? 2 : 1;
+  constexpr int PFX = plan_max_cols((int)sizeof(T)) / (nw * SUB);
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   const int wid = wave % nw;
-  const bool loads = wave >= nw;  // the wave's role
-  const int lk = lane < k ? lane : k - 1;
   const int per = gridDim.x / kXcds;
   const int xcd = blockIdx.x % kXcds, bx = blockIdx.x / kXcds;
   const int band = (pv.nblk + kXcds - 1) / kXcds;
@@ -352,100 +411,56 @@ __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
   auto blk = [&](int m) { return b_beg + (m < nb ? m : nb - 1) * per; };
 
   T *xs = reinterpret_cast<T *>(lds);
-  const unsigned char *xl = lds + lk * sizeof(T);
   unsigned char *mb = lds + (((size_t)pv.umax * k * sizeof(T) + 15) & ~size_t(15));
   const size_t msz = plan_meta_bytes(pv.R, pv.umax, pv.emax, (int)sizeof(T));
   // buffer `i` of the descriptions, recomputed from the LDS base each time
   // (an array of the two pointers would hide that they point into LDS)
   auto meta = [&](int i) { return plan_meta_at<T>(mb + (size_t)i * msz, pv); };
 
-  // The X rows of a block with U columns; past the last column the last one
-  // again, so that no branch lies between the loads.  Lane q holds the
-  // column of the wave's X row q (a read of the list per row would wait for
-  // LDS before each load).
-  PlanMetaRegs<T> mr;
-  T xr[PFX];
-  auto load_x = [&](const PlanMeta<T> &m, int U) {
-    const int ul = wid + lane * nw;
-    const int uc = U > 0 ? m.uc[ul < U ? ul : U - 1] : 0;
-#pragma unroll
-    for (int q = 0; q < PFX; ++q) xr[q] = X[(size_t)__builtin_amdgcn_readlane(uc, q) * k + lk];
-  };
-  auto store_x = [&](int U) {
-    if (lane < k && U > 0) {
-#pragma unroll
-      for (int q = 0; q < PFX; ++q) {
-        const int u = wid + q * nw;
-        xs[(u < U ? u : U - 1) * k + lane] = xr[q];
-      }
-    }
-  };
-
-  // A row on its way through a wave that computes: its entries, its first
-  // two strips and pre's value.
-  struct Row {
-    int a, e, gi, pos[2];
-    T v[2], u;
-  };
-  auto strip = [&](const PlanMeta<T> &md, int j, int e, int &pos, T &v) {
-    const int je = j + (lane & (kPlanStrip - 1)) < e ? j + (lane & (kPlanStrip - 1)) : e - 1;
-    const int jl = je > 0 ? je : 0;
-    pos = md.li[jl] * (k * (int)sizeof(T));
-    v = md.v[jl];
-  };
-  auto add = [&](T s, int pos, T v, int n) {
-    if (n > 12) return plan_strip<T, 4>(s, xl, pos, v, n);
-    if (n > 8) return plan_strip<T, 3>(s, xl, pos, v, n);
-    if (n > 4) return plan_strip<T, 2>(s, xl, pos, v, n);
-    return n > 0 ? plan_strip<T, 1>(s, xl, pos, v, n) : s;
-  };
-  auto compute = [&](const PlanMeta<T> &md) {
-    // lane q: row wid + nw q of the block
-    const int rq = wid + nw * lane;
-    const int rl = rq < pv.R ? rq : pv.R - 1;
-    const int ra = md.rp[rl], re = md.rp[rl + 1], rg = md.gr[rl];
-    const int rows = __popcll(__ballot(rq < pv.R && rg >= 0));
-    auto row = [&](int q) {
-      Row w;
-      w.a = __builtin_amdgcn_readlane(ra, q);
-      w.e = __builtin_amdgcn_readlane(re, q);
-      w.gi = __builtin_amdgcn_readlane(rg, q);
-      w.u = pre(w.gi);
-      strip(md, w.a, w.e, w.pos[0], w.v[0]);
-      strip(md, w.a + kPlanStrip, w.e, w.pos[1], w.v[1]);
-      return w;
-    };
-    if (rows == 0) return;
-    Row w = row(0);
-    for (int q = 0; q < rows; ++q) {
-      const Row next = row(q + 1 < rows ? q + 1 : q);
-      T s = add(T(0), w.pos[0], w.v[0], w.e - w.a);
-      if (w.e - w.a > kPlanStrip) {
-        s = add(s, w.pos[1], w.v[1], w.e - w.a - kPlanStrip);
-        for (int j = w.a + 2 * kPlanStrip; j < w.e; j += kPlanStrip) {
-          int pos;
-          T v;
-          strip(md, j, w.e, pos, v);
-          s = add(s, pos, v, w.e - j);
-        }
-      }
-      epi(w.gi, lane, s, w.u);
-      w = next;
-    }
-  };
-
   // Both roles pass the same barriers: one, and two a block.  (The role is
   // uniform across a wave; two loops keep one's registers out of the other's.)
-  if (loads) {
+  if (wave >= nw) {
+    PlanMetaRegs<T> mr;
+    T xr[PFX];
+    // Load q brings X rows (wid + nw q) SUB + sub of the block's list, lane l
+    // value l % k of row sub = l / k.  Past the last row the last one again,
+    // so that no branch lies between the loads.
+    const int sub = SUB == 1 ? 0 : lane / k < SUB ? lane / k : SUB - 1;
+    const int col = SUB == 1 ? (lane < k ? lane : k - 1) : lane % k;
+    const bool mine = lane < SUB * k;
+    auto load_x = [&](const PlanMeta<T> &m, int U) {
+      // SUB == 1: lane q holds the column of load q (a read of the list per
+      // load would wait for LDS before it)
+      const int ul = wid + lane * nw;
+      const int uc = SUB == 1 && U > 0 ? m.uc[ul < U ? ul : U - 1] : 0;
+      int c[PFX];
+#pragma unroll
+      for (int q = 0; q < PFX; ++q) {
+        const int u = (wid + q * nw) * SUB + sub;
+        c[q] = SUB == 1 ? __builtin_amdgcn_readlane(uc, q)
+                        : U > 0 ? m.uc[u < U ? u : U - 1] : 0;
+      }
+#pragma unroll
+      for (int q = 0; q < PFX; ++q) xr[q] = X[(size_t)c[q] * k + col];
+    };
+    auto store_x = [&](int U) {
+      if (mine && U > 0) {
+#pragma unroll
+        for (int q = 0; q < PFX; ++q) {
+          const int u = (wid + q * nw) * SUB + sub;
+          xs[(u < U ? u : U - 1) * k + col] = xr[q];
+        }
+      }
+    };
     // prologue: block 0's description in buffer 0, block 1's in registers,
     // block 0's X rows and block 2's header in flight
     const int h0 = plan_hdr_load(blk(0), pv, rp);
     const int h1 = plan_hdr_load(blk(1), pv, rp);
     PlanHdr H0 = plan_hdr(h0, blk(0), pv);
-    plan_meta_load(mr, H0, pv, rp, val);
+    plan_meta_load(mr, H0, pv, val);
     plan_meta_store(mr, H0, pv, meta(0));
     PlanHdr H1 = plan_hdr(h1, blk(1), pv);
-    plan_meta_load(mr, H1, pv, rp, val);
+    plan_meta_load(mr, H1, pv, val);
     __syncthreads();
     load_x(meta(0), H0.U);
     int hn = plan_hdr_load(blk(2), pv, rp);  // header of block m+2
@@ -458,18 +473,84 @@ __device__ __forceinline__ void plan_walk(const PlanView &pv, int k_arg,
       __syncthreads();
       // this step's loads
       hn = plan_hdr_load(blk(m + 3), pv, rp);
-      plan_meta_load(mr, H2, pv, rp, val);
+      plan_meta_load(mr, H2, pv, val);
       load_x(meta(buf ^ 1), H1.U);
       __syncthreads();
       H0 = H1;
       H1 = H2;
     }
-  } else {
-    __syncthreads();
-    for (int m = 0; m < nb; ++m) {
-      __syncthreads();
-      compute(meta(m & 1));
-      __syncthreads();
-    }
+    return;
   }
+
+  // Four rows on their way through a wave: the lane's row, its length and
+  // first two strips, and the wave's longest and shortest.
+  struct Rows {
+    int gi, a, n, nmin, nmax, pos[2];
+    T v[2];
+  };
+  const int li = lane & 15;
+  const unsigned char *xl =
+      lds + (size_t)PlanCols<T, CV, FULL>::first(li, 0) * sizeof(T);
+  auto strip = [&](const PlanMeta<T> &md, int j, int e, int &pos, T &v) {
+    const int je = j + li < e ? j + li : e - 1;
+    const int jl = je > 0 ? je : 0;
+    pos = md.li[jl] * (k * (int)sizeof(T));
+    v = md.v[jl];
+  };
+  const int turns = pv.R / 4;  // R is a multiple of 4
+  auto compute = [&](const PlanMeta<T> &md) {
+    auto rows = [&](int j) {
+      const int t = j * nw + (j & 1 ? nw - 1 - wid : wid);
+      const int r = 4 * (t < turns ? t : turns - 1) + lane / 16;
+      Rows w;
+      const int se = md.se[r];
+      w.gi = t < turns ? md.gr[r] : -1;
+      w.a = se >> 16;
+      w.n = w.gi >= 0 ? se & 0xffff : 0;
+      w.nmax = __builtin_amdgcn_readlane(w.n, 0);
+      w.nmin = __builtin_amdgcn_readlane(w.n, 48);
+      strip(md, w.a, w.a + w.n, w.pos[0], w.v[0]);
+      strip(md, w.a + kPlanStrip, w.a + w.n, w.pos[1], w.v[1]);
+      return w;
+    };
+    Rows w = rows(0);
+    for (int j = 0; j * nw < turns; ++j) {
+      const Rows next = rows(j + 1);
+      T s[CV], u[CV];
+      pre(w.gi >= 0 ? w.gi : 0, u);
+#pragma unroll
+      for (int c = 0; c < CV; ++c) s[c] = 0;
+      plan_strip<T, CV, FULL, E>(s, xl, w.pos[0], w.v[0], w.n, w.nmin, w.nmax);
+      if (w.nmax > kPlanStrip) {
+        plan_strip<T, CV, FULL, E>(s, xl, w.pos[1], w.v[1], w.n - kPlanStrip, w.nmin - kPlanStrip,
+                                w.nmax - kPlanStrip);
+        for (int d = 2 * kPlanStrip; d < w.nmax; d += kPlanStrip) {
+          int pos;
+          T v;
+          strip(md, w.a + d, w.a + w.n, pos, v);
+          plan_strip<T, CV, FULL, E>(s, xl, pos, v, w.n - d, w.nmin - d, w.nmax - d);
+        }
+      }
+      if (w.gi >= 0) epi(w.gi, s, u);
+      w = next;
+    }
+  };
+  __syncthreads();
+  for (int m = 0; m < nb; ++m) {
+    __syncthreads();
+    compute(meta(m & 1));
+    __syncthreads();
+  }
+}
+
+// f with the kernel's column template for k vectors: f(CV, FULL) as
+// integral constants.
+template <typename F>
+inline auto plan_dispatch(int k, F &&f) {
+  using std::integral_constant;
+  if (k == 64) return f(integral_constant<int, 4>(), std::true_type());
+  if (k > 48) return f(integral_constant<int, 4>(), std::false_type());
+  if (k > 32) return f(integral_constant<int, 3>(), std::false_type());
+  if (k > 16) return f(integral_constant<int, 2>(), std::false_type());
+  return f(integral_constant<int, 1>(), std::false_type());
 }
