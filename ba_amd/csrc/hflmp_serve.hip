@@ -18,8 +18,9 @@
 // consecutive rows (one workgroup, four SELL-64 slices).  One launch of each
 // iteration kernel covers the units of all active systems (unit -> system
 // through a device table); each workgroup branches on its system's precision.
-// The two scalar steps run one workgroup per system.  So an iteration of S
-// systems is five launches, as for one.  A system's partial sums are
+// The two scalar steps run in the kernels that use them, or one workgroup
+// per system.  So an iteration of S systems is three launches (or five), as
+// for one.  A system's partial sums are
 // indexed by its own units and added in a fixed order, so its iterates do
 // not depend on which other systems share the launches: a result is
 // bit-identical alone and in any mix.
@@ -159,6 +160,50 @@ __device__ __forceinline__ T units_sum(const T *__restrict__ src, int count, int
   return block_sum(t, lds);
 }
 
+// The same sums (and bits) on every thread: of NQ quantities, quantity q of
+// unit u at src[q][stride[q] u], with one wait for the loads and one barrier.
+// F: 8, or 4 for at most 4 kBlock units (fewer registers).
+template <int F, typename T, int NQ>
+__device__ __forceinline__ void units_all(const T *const (&src)[NQ], const int (&stride)[NQ],
+                                          int count, T (&sum)[NQ]) {
+  __shared__ T lds[NQ][kBlock / kWave];
+  T a[NQ][F];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q)
+#pragma unroll
+    for (int f = 0; f < F; ++f) a[q][f] = 0;
+  for (int u0 = threadIdx.x; u0 < count; u0 += F * kBlock) {
+    T v[NQ][F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+      const int u = u0 + f * kBlock;
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) v[q][f] = u < count ? src[q][(size_t)u * stride[q]] : T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int f = 0; f < F; ++f) a[q][f] += v[q][f];
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    T t = (a[q][0] + a[q][1]) + (a[q][2] + a[q][3]);
+    if constexpr (F == 8)
+      t = t + ((a[q][4] + a[q][5]) + (a[q][6] + a[q][7]));
+    else
+      t = t + T(0);  // as of four zeros
+    t = wave_sum(t);
+    if ((threadIdx.x & (kWave - 1)) == 0) lds[q][threadIdx.x / kWave] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    sum[q] = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / kWave; ++w) sum[q] += lds[q][w];
+  }
+}
+
 // workgroup sums of a and b stored at part[2j], part[2j+1]
 template <typename T>
 __device__ __forceinline__ void unit_partial2(T a, T b, T *part, int j) {
@@ -233,13 +278,52 @@ __device__ __forceinline__ bool quad_of(const SysDesc *__restrict__ sys,
   return true;
 }
 
-// Per-unit sums of a[q] and b[q] over the workgroup, stored at
-// part[2 (j0 + q)], part[2 (j0 + q) + 1] for the units j0 + q < jend: the
-// same wave sums and the same order over the waves as unit_partial2 forms
-// for one unit, so the partials do not depend on the grouping.
+// Where K2 leaves a unit's partials of r.r and r.z (element stride * unit).
+// K2 may still read K1's partials of p.Ap elsewhere in the system, so they
+// lie beside those: of the four floats a unit of a mixed system K1 takes one
+// and K2 the last two; of the two doubles of an FP64 system K1 takes one and
+// r.r the other, and r.z goes into Ap, at the unit's first row, which K2
+// itself has read for the last time.
+template <typename T>
+struct UpdatePartials {
+  T *rr;
+  int rr_stride;
+  T *rz;
+  int rz_stride;
+};
+__device__ __forceinline__ UpdatePartials<double> update_partials64(const SysDesc &d) {
+  return {d.part + d.nunits, 1, d.Ap, kBlock};
+}
+__device__ __forceinline__ UpdatePartials<float> update_partials32(const SysDesc &d) {
+  float *base = part32(d) + 2 * (size_t)d.nunits;
+  return {base, 2, base + 1, 2};
+}
+template <int F, typename T>
+__device__ __forceinline__ void update_totals(const UpdatePartials<T> &u, int nunits, T &rr,
+                                              T &rz) {
+  const T *const src[2] = {u.rr, u.rz};
+  const int stride[2] = {u.rr_stride, u.rz_stride};
+  T sum[2];
+  units_all<F>(src, stride, nunits, sum);
+  rr = sum[0];
+  rz = sum[1];
+}
+template <typename T>
+__device__ __forceinline__ T product_total(const T *part, int nunits) {
+  const T *const src[1] = {part};
+  const int stride[1] = {1};
+  T sum[1];
+  units_all<4>(src, stride, nunits, sum);
+  return sum[0];
+}
+
+// Per-unit sums of a[q] and b[q] over the workgroup, stored for the units
+// j0 + q < jend: the same wave sums and the same order over the waves as
+// unit_partial2 forms for one unit, so the partials do not depend on the
+// grouping.
 template <typename T>
 __device__ __forceinline__ void quad_partial2(const T (&a)[kQuad], const T (&b)[kQuad],
-                                              T *part, int j0, int jend) {
+                                              const UpdatePartials<T> &out, int j0, int jend) {
   __shared__ T lds[kQuad][2][kBlock / kWave];
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
   // only the group's own units (cross-lane sums are not free)
@@ -263,8 +347,8 @@ __device__ __forceinline__ void quad_partial2(const T (&a)[kQuad], const T (&b)[
       sa += lds[q][0][w];
       sb += lds[q][1][w];
     }
-    part[2 * (j0 + q)] = sa;
-    part[2 * (j0 + q) + 1] = sb;
+    out.rr[(size_t)out.rr_stride * (j0 + q)] = sa;
+    out.rz[(size_t)out.rz_stride * (j0 + q)] = sb;
   }
 }
 
@@ -585,6 +669,77 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
+// alpha and the stopping test are formed from partials of every unit of the
+// system.  FOLD: by every workgroup of the kernel that needs them, K2 and
+// K3, from the same terms in the same order; the system's first workgroup
+// stores them.  K2 reads and leaves alone what K1 and K3 read (status, phase,
+// r.z, iter), and leaves what K3 reads (`go`: kGo.., rz_prev, iter_prev),
+// which K3 leaves alone, so that every workgroup decides alike.  Else by one
+// workgroup a system in launches of their own (F1 and F2), with the same
+// bits.  32 mixed systems of up to 90,000 rows: F1 and F2 were 8.1 of an
+// iteration's 27.4 us, the fold adds 1.2 us to K2 and K3.
+//
+// The fold's cost is that every workgroup of a system reads all its
+// partials, the square of its units.  Mixed systems gain at all measured
+// sizes (us an iteration with F1 and F2 and without, units a system x
+// systems: 257 x 8 24.7 19.4, 257 x 128 201.5 196.1, 905 x 16 94.8 92.3);
+// the bound of 1024 is where units_all takes more registers.  FP64 ones,
+// whose r.z partials lie apart, gain up to squares that sum to about 4 M (257 x 8
+// 31.1 28.5, 257 x 64 159.9 159.2, but 257 x 128 334.8 348.2, 905 x 8 78.1
+// 82.2).
+constexpr int kFoldUnits = 4 * kBlock;
+constexpr long long kFoldSquare64 = 4LL << 20;
+constexpr int kGoStopped = 0, kGoOn = 1, kGoBreakdown = 2;
+
+// K2's part: alpha on every thread; false if the system is not to be updated
+template <typename T>
+__device__ __forceinline__ bool fold_alpha(CgState<T> *st, bool live, const T *part, int nunits,
+                                           bool first, T &alpha) {
+  if (!live) {
+    if (first) st->go = kGoStopped;
+    return false;
+  }
+  const T rz = st->rz;
+  const T pAp = product_total(part, nunits);
+  const bool ok = !(pAp == T(0) || !(pAp == pAp));
+  alpha = rz / pAp;
+  if (first) {
+    st->pAp = pAp;
+    st->alpha = alpha;
+    st->rz_prev = rz;
+    st->iter_prev = st->iter;
+    st->go = ok ? kGoOn : kGoBreakdown;
+  }
+  return ok;
+}
+
+// K3's part: beta on every thread, and the status on; the first workgroup
+// stores both.  K2 found the system live.
+template <typename T>
+__device__ __forceinline__ int fold_beta(CgState<T> *st, const UpdatePartials<T> &u, int nunits,
+                                         bool first, T &beta) {
+  int s = kBreakdown;
+  if (st->go == kGoOn) {
+    T rr, rz;
+    update_totals<4>(u, nunits, rr, rz);
+    const int iter = st->iter_prev + 1;
+    const T res = sqrt(rr);
+    s = check_state(iter, (double)res, (double)st->res0, st->maxit, st->atol, st->rtol, st->dtol);
+    beta = rz / st->rz_prev;
+    if (first) {
+      st->iter = iter;
+      st->rr = rr;
+      st->res = res;
+      if (s == kIterate) {
+        st->beta = beta;
+        st->rz = rz;
+      }
+    }
+  }
+  if (first) st->status = s;
+  return s;
+}
+
 // F1: alpha = r.z / p.Ap, one workgroup per system
 __global__ void __launch_bounds__(kBlock) grp_alpha_final(const SysDesc *__restrict__ sys) {
   const SysDesc d = sys[blockIdx.x];
@@ -662,6 +817,7 @@ __device__ __forceinline__ void quad_load5(long long i0, int n, const T *__restr
   }
 }
 
+template <bool FOLD>
 __global__ void __launch_bounds__(kBlock)
     grp_update_kernel(const SysDesc *__restrict__ sys, const int *__restrict__ grp_sys, int G) {
   SysDesc d;
@@ -672,20 +828,27 @@ __global__ void __launch_bounds__(kBlock)
   const long long i0 = (long long)k * g * kBlock + threadIdx.x;
   const int iend = (int)std::min((long long)d.nrow, (long long)(k + 1) * g * kBlock);
   const int jend = std::min(d.nunits, g * (k + 1));
+  const bool first = k == 0 && threadIdx.x == 0;
   if (d.mode == kModeFp64) {
     double pv[kQuad], av[kQuad], xv[kQuad], rv[kQuad], dv[kQuad], rr[kQuad], rz[kQuad];
     quad_load5(i0, iend, d.p, d.Ap, d.x, d.r, d.invd, pv, av, xv, rv, dv);
-    if (d.st->s64.status != kIterate) return;
-    quad_update(i0, iend, d.st->s64.alpha, d.p, d.Ap, d.x, d.r, d.z, pv, av, xv, rv, dv, rr,
-                rz);
-    quad_partial2(rr, rz, d.part, g * k, jend);
+    CgState<double> *st = &d.st->s64;
+    const bool live = st->status == kIterate;
+    double alpha;
+    if (FOLD ? !fold_alpha(st, live, d.part, d.nunits, first, alpha) : !live) return;
+    if (!FOLD) alpha = st->alpha;
+    quad_update(i0, iend, alpha, d.p, d.Ap, d.x, d.r, d.z, pv, av, xv, rv, dv, rr, rz);
+    quad_partial2(rr, rz, update_partials64(d), g * k, jend);
   } else {
     float pv[kQuad], av[kQuad], xv[kQuad], rv[kQuad], dv[kQuad], rr[kQuad], rz[kQuad];
     quad_load5(i0, iend, d.p32, d.Ap32, d.c32, d.r32, d.invd32, pv, av, xv, rv, dv);
-    if (!mixed_inner_live(d.st)) return;
-    quad_update(i0, iend, d.st->s32.alpha, d.p32, d.Ap32, d.c32, d.r32, d.z32, pv, av, xv,
-                rv, dv, rr, rz);
-    quad_partial2(rr, rz, part32(d), g * k, jend);
+    CgState<float> *st = &d.st->s32;
+    const bool live = mixed_inner_live(d.st);
+    float alpha;
+    if (FOLD ? !fold_alpha(st, live, part32(d), d.nunits, first, alpha) : !live) return;
+    if (!FOLD) alpha = st->alpha;
+    quad_update(i0, iend, alpha, d.p32, d.Ap32, d.c32, d.r32, d.z32, pv, av, xv, rv, dv, rr, rz);
+    quad_partial2(rr, rz, update_partials32(d), g * k, jend);
   }
 }
 
@@ -696,8 +859,8 @@ __global__ void __launch_bounds__(kBlock) grp_beta_final(const SysDesc *__restri
   if (d.mode == kModeFp64) {
     CgState<double> *st = &d.st->s64;
     if (st->status != kIterate) return;
-    const double rr = units_sum(d.part, d.nunits, 2, 0);
-    const double rz = units_sum(d.part, d.nunits, 2, 1);
+    double rr, rz;
+    update_totals<8>(update_partials64(d), d.nunits, rr, rz);
     if (threadIdx.x == 0) {
       const int iter = st->iter + 1;
       const double res = sqrt(rr);
@@ -714,8 +877,8 @@ __global__ void __launch_bounds__(kBlock) grp_beta_final(const SysDesc *__restri
   } else {
     if (!mixed_inner_live(d.st)) return;
     CgState<float> *st = &d.st->s32;
-    const float rr = units_sum(part32(d), d.nunits, 2, 0);
-    const float rz = units_sum(part32(d), d.nunits, 2, 1);
+    float rr, rz;
+    update_totals<8>(update_partials32(d), d.nunits, rr, rz);
     if (threadIdx.x == 0) {
       const int iter = st->iter + 1;
       const float res = sqrtf(rr);
@@ -761,6 +924,7 @@ __device__ __forceinline__ void quad_p(long long i0, int n, T beta, T *__restric
   }
 }
 
+template <bool FOLD>
 __global__ void __launch_bounds__(kBlock)
     grp_p_kernel(const SysDesc *__restrict__ sys, const int *__restrict__ quad_sys, int Q) {
   SysDesc d;
@@ -768,16 +932,39 @@ __global__ void __launch_bounds__(kBlock)
   if (!quad_of(sys, quad_sys, Q, d, k, true)) return;
   const long long i0 = (long long)k * kQuad * kBlock + threadIdx.x;
   const int iend = (int)std::min((long long)d.nrow, (long long)(k + 1) * kQuad * kBlock);
+  const bool first = k == 0 && threadIdx.x == 0;
   if (d.mode == kModeFp64) {
-    double pv[kQuad], zv[kQuad];
+    double pv[kQuad], zv[kQuad], beta;
     quad_load2(i0, iend, d.p, d.z, pv, zv);
-    if (d.st->s64.status != kIterate) return;
-    quad_p(i0, iend, d.st->s64.beta, d.p, pv, zv);
+    CgState<double> *st = &d.st->s64;
+    if (FOLD) {
+      if (st->go == kGoStopped ||
+          fold_beta(st, update_partials64(d), d.nunits, first, beta) != kIterate)
+        return;
+    } else {
+      if (st->status != kIterate) return;
+      beta = st->beta;
+    }
+    quad_p(i0, iend, beta, d.p, pv, zv);
   } else {
-    float pv[kQuad], zv[kQuad];
+    float pv[kQuad], zv[kQuad], beta;
     quad_load2(i0, iend, d.p32, d.z32, pv, zv);
-    if (!mixed_inner_live(d.st)) return;
-    quad_p(i0, iend, d.st->s32.beta, d.p32, pv, zv);
+    CgState<float> *st = &d.st->s32;
+    if (FOLD) {
+      if (st->go == kGoStopped) return;
+      const int s = fold_beta(st, update_partials32(d), d.nunits, first, beta);
+      if (first) {
+        // going on, the refreshed p has been used
+        d.st->phase = s == kIterate ? 1 : 0;
+        if (s != kIterate)
+          d.st->inner_total += st->go == kGoOn ? st->iter_prev + 1 : st->iter_prev;
+      }
+      if (s != kIterate) return;
+    } else {
+      if (!mixed_inner_live(d.st)) return;
+      beta = st->beta;
+    }
+    quad_p(i0, iend, beta, d.p32, pv, zv);
   }
 }
 
@@ -1076,6 +1263,7 @@ void plan_job(Job &jb) {
 struct TableSet {
   long long version = -1;  // the version of the active set these tables hold
   int S = 0, U = 0;
+  bool fold = false;  // K2 and K3 form the scalars (kFoldUnits)
   SysDesc *d_sys = nullptr, *h_sys = nullptr;  // [max_active]
   int *d_unit = nullptr, *h_unit = nullptr;    // [unit_cap]: FP64 systems' units first
   size_t unit_cap = 0;
@@ -1202,10 +1390,15 @@ void enqueue_chunk(const hflmp_server *sv, const TableSet &t, hipStream_t s) {
     if (ub[4] > ub[3])
       grp_spmv_pair_kernel<float, int><<<grid((ub[4] - ub[3] + 1) / 2), kBlock, 0, s>>>(
           t.d_rec, ub[3], ub[4] - ub[3]);
-    grp_alpha_final<<<gS, kBlock, 0, s>>>(t.d_sys);
-    grp_update_kernel<<<gG, kBlock, 0, s>>>(t.d_sys, t.d_grp, t.G);
-    grp_beta_final<<<gS, kBlock, 0, s>>>(t.d_sys);
-    grp_p_kernel<<<gQ, kBlock, 0, s>>>(t.d_sys, t.d_quad, t.Q);
+    if (t.fold) {
+      grp_update_kernel<true><<<gG, kBlock, 0, s>>>(t.d_sys, t.d_grp, t.G);
+      grp_p_kernel<true><<<gQ, kBlock, 0, s>>>(t.d_sys, t.d_quad, t.Q);
+    } else {
+      grp_alpha_final<<<gS, kBlock, 0, s>>>(t.d_sys);
+      grp_update_kernel<false><<<gG, kBlock, 0, s>>>(t.d_sys, t.d_grp, t.G);
+      grp_beta_final<<<gS, kBlock, 0, s>>>(t.d_sys);
+      grp_p_kernel<false><<<gQ, kBlock, 0, s>>>(t.d_sys, t.d_quad, t.Q);
+    }
   }
 }
 
@@ -1269,13 +1462,18 @@ int grow_table(hflmp_ctx *ctx, int **d, int **h, size_t *cap, size_t need) {
 int rebuild_tables(hflmp_server *sv, TableSet &t) {
   hflmp_ctx *ctx = sv->ctx;
   int U = 0, G = 0, Q = 0;
+  long long square64 = 0;
+  bool fits = true;
   for (int slot : sv->order) {
     Job &jb = sv->jobs[sv->slot_job[slot]];
+    fits = fits && jb.nunits <= kFoldUnits;
+    if (jb.d.mode == kModeFp64) square64 += (long long)jb.nunits * jb.nunits;
     jb.d.gsz = jb.d.mode == kModeFp64 ? kGroup64 : kQuad;
     U += jb.nunits;
     G += (jb.nunits + jb.d.gsz - 1) / jb.d.gsz;
     Q += (jb.nunits + kQuad - 1) / kQuad;
   }
+  t.fold = fits && square64 <= kFoldSquare64;
   if ((size_t)U > t.rec_cap) {
     if (t.d_rec) (void)hipFree(t.d_rec);
     t.d_rec = nullptr;

@@ -463,3 +463,48 @@ def test_serve_solo_alone_equals_mix(ctx):
     x_mix, i_mix = out[3]
     assert i_mix["iters"] == i_alone["iters"]
     assert np.array_equal(x_mix, x_alone)
+
+
+@pytest.mark.parametrize("precision", [64, 32])
+def test_serve_scalar_forms(ctx, precision):
+    """alpha, beta and the stopping test formed in the kernels that use them
+    (sets of systems of at most 1024 units of 256 rows) and in launches of
+    their own (beside a system of 1025): the same bits, at the edges of the
+    units, with the smallest last unit, at a cap and at a breakdown."""
+    def banded(n, seed):
+        import scipy.sparse as sp
+        rng = np.random.default_rng(seed)
+        w = [-rng.uniform(0.2, 1.0, n - d) for d in (1, 5) if d < n]
+        A = sp.diags(w + w, [d for d in (1, 5) if d < n] + [-d for d in (1, 5) if d < n], (n, n))
+        A = (A + sp.diags(1.2 * np.asarray(abs(A).sum(axis=1)).ravel() + 0.1)).tocsr()
+        A.sort_indices()
+        return (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data,
+                rng.uniform(-1, 1, n))
+    probes = [banded(n, n) for n in (2, 255, 256, 257, 1023, 1025, 4097)]
+    if precision == 64:
+        probes.append((np.array([0, 1, 2], np.int32), np.array([0, 1], np.int32),
+                       np.array([1.0, -1.0]), np.array([1.0, 1.0])))   # p.Ap = 0
+    large = [banded(n, 7) for n in (262144, 262145)]                    # 1024 and 1025 units
+
+    def solve(reqs, maxit=1000):
+        sv = hflmp.Server(ctx, 1024 * MB, max_active=16, chunk_iters=3, solo_min_nnz=1 << 30)
+        try:
+            ts = [sv.submit(*r, rtol=1e-8, maxit=maxit, precision=precision) for r in reqs]
+            while any(sv.poll(t)["state"] != 2 for t in ts):
+                sv.step()
+            return [sv.take(t) for t in ts]
+        finally:
+            sv.close()
+
+    for maxit in (1000, 4):
+        folded = solve(probes + large[:1], maxit)
+        apart = solve(probes + large, maxit)
+        for r, (x, i), (xa, ia) in zip(probes + large[:1], folded, apart):
+            assert (i["iters"], i["status"]) == (ia["iters"], ia["status"])
+            assert np.array_equal(x, xa)
+            if maxit == 1000 and i["status"] == 0:
+                res = r[3] - O.spmv(*r[:3], x)
+                assert np.linalg.norm(res) <= 2e-8 * np.linalg.norm(r[3])
+        assert all(i["status"] == 0 for _, i in folded[:7]) or maxit == 4
+        if precision == 64:
+            assert folded[7][1]["status"] == 3
