@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(kBlock)
   const T s = op.row_sum(tile, p, T(0), tr, prod);
   T part = 0;
   if (tr.has_row) {
-    __builtin_nontemporal_store(s, Ap + tr.row);
+    Ap[tr.row] = s;
     part = s * p[tr.row];
   }
   block_partial1(part, partials);

@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
     TileRow tr;
     const T s = op.row_sum(tile, p, T(0), tr, prod);
     if (tr.has_row) {
-      __builtin_nontemporal_store(s, Ap + tr.row);
+      Ap[tr.row] = s;
       acc += s * p[tr.row];
     }
   }
@@ -274,7 +274,7 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))
       if (has) {
         const T pv = __builtin_elementwise_fma(beta, pi, zi);
         pn[row] = pv;
-        __builtin_nontemporal_store(s, Ap + row);
+        Ap[row] = s;
         acc = __builtin_elementwise_fma(s, pv, acc);
       }
     }

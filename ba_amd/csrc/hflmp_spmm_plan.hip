@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(kPlanThreads, 4)
   plan_walk<T, CV, FULL, 4>(
       pv, k, rp, val, X, plan_lds, [](int, T *) {},
       [&](int i, const T *s, const T *) {
-        PlanCols<T, CV, FULL>::store(Y + (size_t)i * k, s, li, k);
+        PlanCols<T, CV, FULL>::template store<true>(Y + (size_t)i * k, s, li, k);
       });
 }
 

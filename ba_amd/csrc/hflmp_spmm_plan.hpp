@@ -288,12 +288,18 @@ struct PlanCols {
       __builtin_memcpy(x + p * kRun, &v, sizeof(v));
     });
   }
+  // STREAM: past the caches
+  template <bool STREAM>
   __device__ __forceinline__ static void store(T *dst, const T *x, int i, int k) {
     each([&](int p) {
       const int c = first(i, p);
       Piece v;
       __builtin_memcpy(&v, x + p * kRun, sizeof(v));
-      if (FULL || c < k) __builtin_nontemporal_store(v, reinterpret_cast<Piece *>(dst + c));
+      if (!FULL && c >= k) return;
+      if (STREAM)
+        __builtin_nontemporal_store(v, reinterpret_cast<Piece *>(dst + c));
+      else
+        *reinterpret_cast<Piece *>(dst + c) = v;
     });
   }
 };
