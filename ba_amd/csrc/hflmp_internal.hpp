@@ -260,6 +260,22 @@ template <typename T>
 __device__ __forceinline__ T ld_stream(const T *p) {
   return __builtin_nontemporal_load(p);
 }
+template <bool NT, typename T>
+__device__ __forceinline__ T ld_entry(const T *p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
+}
+
+// Bytes of a matrix's entries up to which products load them through the
+// caches: what the next product finds there depends on all of them fitting
+// the Infinity Cache (256 MB) with the vectors.  Larger matrices are loaded
+// past the caches, which they would only sweep.  Jacobi-CG on 3D Q1 in FP64
+// (SELL-64, offset form), ms a solve past and through the caches: 96^3, 195 MB,
+// 15.4 and 11.7; 104^3, 247 MB, 20.3 and 18.8; 108^3, 277 MB, 22.2 and 22.5;
+// 128^3, 459 MB, 36.8 and 38.6.
+constexpr size_t kCachedBytes = (size_t)256 << 20;
+inline bool entries_stream(long long entries, size_t entry_bytes) {
+  return (size_t)entries * entry_bytes > kCachedBytes;
+}
 
 // Buffer descriptor word 3 for raw (untyped) buffer access on gfx9-family
 // GPUs (gfx950 included).

@@ -107,6 +107,7 @@ struct CsrTileOp {
   using value_type = T;
   static constexpr int kLds = TileCap<T>::value;
   int nrow, R;
+  bool stream;  // entries past the caches (kCachedBytes)
   const int *rp;
   const IT *ci;
   const T *val;
@@ -116,7 +117,8 @@ struct CsrTileOp {
   }
   __device__ __forceinline__ T row_sum(long long unit, const T *x, T s, TileRow &tr,
                                        T *lds) const {
-    return tile_row_sum<T, false, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds);
+    return stream ? tile_row_sum<T, false, true, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds)
+                  : tile_row_sum<T, false, false, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds);
   }
 };
 
@@ -127,13 +129,9 @@ struct CsrTileOp {
 // cover the row's own entries, or with LOAD_ALL every entry position of the
 // slice (all allocated: 64 x smax entries), so that they need not wait for
 // len; the sum is the same either way.  NT: entries are loaded past the
-// caches (they are read once a launch).  U: chunk loads in flight per step.
+// caches (kCachedBytes).  U: chunk loads in flight per step.
 // GATHER_ALL: x is read for every entry loaded, padding included (its
 // column is 0; for an x that is cheap to read and has no limit to guard).
-template <typename V, bool NT>
-__device__ __forceinline__ V sell_ld(const V *p) {
-  return NT ? __builtin_nontemporal_load(p) : *p;
-}
 template <typename T, typename IT, bool SUB, bool NODIAG, bool LOAD_ALL, bool NT = true,
           int U = SellChunk<T>::U, bool GATHER_ALL = false>
 __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T *__restrict__ val,
@@ -157,8 +155,8 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
   for (int t = 0; t < TM; ++t) {
     if (t < nload) {
       const long long q = (long long)kSellRows * (full + t) + lane;
-      ct[t] = sell_ld<IT, NT>(col + q);
-      vt[t] = sell_ld<T, NT>(val + q);
+      ct[t] = ld_entry<NT>(col + q);
+      vt[t] = ld_entry<NT>(val + q);
     }
   }
   for (int j = 0; j < full; j += P * U) {
@@ -167,8 +165,8 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if ((LOAD_ALL || j + u * P < len) && j + u * P < full) {
-        cc[u] = sell_ld<IV, NT>(c + (j / P + u) * kWave);
-        vv[u] = sell_ld<TV, NT>(v + (j / P + u) * kWave);
+        cc[u] = ld_entry<NT>(c + (j / P + u) * kWave);
+        vv[u] = ld_entry<NT>(v + (j / P + u) * kWave);
       }
     }
     T xx[U][P];
@@ -218,7 +216,7 @@ __device__ __forceinline__ T sell_slice_sum(const IT *__restrict__ col, const T 
 // either's gathers, so that a wave keeps twice the bytes in flight.
 // smaxB = 0: no slice B (sB stays as given).  U: chunk loads in flight
 // per slice and step (the order of the sums does not depend on it).
-template <typename T, typename IT, int U = SellChunk<T>::U>
+template <typename T, typename IT, bool NT, int U = SellChunk<T>::U>
 __device__ __forceinline__ void sell_slice_sum2(const IT *__restrict__ colA,
                                                 const T *__restrict__ valA, int smaxA, int lenA,
                                                 const T *__restrict__ xA,
@@ -243,13 +241,13 @@ __device__ __forceinline__ void sell_slice_sum2(const IT *__restrict__ colA,
   for (int t = 0; t < TM; ++t) {
     if (t < nlA) {
       const long long q = (long long)kSellRows * (fullA + t) + lane;
-      ctA[t] = __builtin_nontemporal_load(colA + q);
-      vtA[t] = __builtin_nontemporal_load(valA + q);
+      ctA[t] = ld_entry<NT>(colA + q);
+      vtA[t] = ld_entry<NT>(valA + q);
     }
     if (t < nlB) {
       const long long q = (long long)kSellRows * (fullB + t) + lane;
-      ctB[t] = __builtin_nontemporal_load(colB + q);
-      vtB[t] = __builtin_nontemporal_load(valB + q);
+      ctB[t] = ld_entry<NT>(colB + q);
+      vtB[t] = ld_entry<NT>(valB + q);
     }
   }
   const int full = fullA > fullB ? fullA : fullB;
@@ -259,12 +257,12 @@ __device__ __forceinline__ void sell_slice_sum2(const IT *__restrict__ colA,
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (j + u * P < fullA) {
-        ccA[u] = __builtin_nontemporal_load(cA + (j / P + u) * kWave);
-        vvA[u] = __builtin_nontemporal_load(vA + (j / P + u) * kWave);
+        ccA[u] = ld_entry<NT>(cA + (j / P + u) * kWave);
+        vvA[u] = ld_entry<NT>(vA + (j / P + u) * kWave);
       }
       if (j + u * P < fullB) {
-        ccB[u] = __builtin_nontemporal_load(cB + (j / P + u) * kWave);
-        vvB[u] = __builtin_nontemporal_load(vB + (j / P + u) * kWave);
+        ccB[u] = ld_entry<NT>(cB + (j / P + u) * kWave);
+        vvB[u] = ld_entry<NT>(vB + (j / P + u) * kWave);
       }
     }
     T xxA[U][P], xxB[U][P];
@@ -309,6 +307,7 @@ struct SellOp {
   static constexpr int P = SellChunk<T>::P;
   static constexpr int U = SellChunk<T>::U;
   int nrow, nslice;
+  bool stream;  // entries past the caches (kCachedBytes)
   const long long *soff;
   const int *slen;
   const unsigned char *rlen;
@@ -338,8 +337,10 @@ struct SellOp {
     // int16 columns are offsets from the slice's first row
     const T *__restrict__ x = std::is_same<IT, int>::value ? x_in : x_in + sid * kSellRows;
     const int dcol = std::is_same<IT, int>::value ? row : lane;
-    return sell_slice_sum<T, IT, SUB, NODIAG, false>(col + base, val + base, smax, len, lane, x,
-                                                      dcol, s);
+    return stream ? sell_slice_sum<T, IT, SUB, NODIAG, false, true>(col + base, val + base, smax,
+                                                                    len, lane, x, dcol, s)
+                  : sell_slice_sum<T, IT, SUB, NODIAG, false, false>(col + base, val + base, smax,
+                                                                     len, lane, x, dcol, s);
   }
 };
 
@@ -389,7 +390,7 @@ __device__ __forceinline__ T sell_offset_sum(const T *__restrict__ val, ScalarPt
     const unsigned long long m = mask[j];
     ot[t] = off[j];
     mt[t] = full + t < K ? m : 0;
-    vt[t] = sell_ld<T, NT>(val + kSellRows * j + lane);
+    vt[t] = ld_entry<NT>(val + kSellRows * j + lane);
     xt[t] = xf(row + ot[t]);
   }
   auto add = [&](T a, T x, unsigned long long m, int o) {
@@ -406,7 +407,7 @@ __device__ __forceinline__ T sell_offset_sum(const T *__restrict__ val, ScalarPt
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
       const int c = c0 + u < nch ? c0 + u : nch - 1;
-      vv[u] = sell_ld<TV, NT>(v + c * kWave);
+      vv[u] = ld_entry<NT>(v + c * kWave);
 #pragma unroll
       for (int q = 0; q < P; ++q) {
         const unsigned long long m = mask[c * P + q];
@@ -438,6 +439,7 @@ struct SellOffOp {
   using value_type = T;
   static constexpr int kLds = 1;
   int nrow, ncol, nslice, max_off;
+  bool stream;  // entries past the caches (kCachedBytes)
   const long long *soff;
   const int *slen;
   const int *off;
@@ -465,10 +467,13 @@ struct SellOffOp {
     // below 2 GiB)
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T *>(x), 0, ncol * (int)sizeof(T), kRsrcWord3);
-    return sell_offset_sum<T, SUB, NODIAG, true>(
-        val + base, scalar_ptr(off) + base / kSellRows, scalar_ptr(mask) + base / kSellRows, K,
-        row, lane, [&](int c) { return buffer_load<T>(xr, (unsigned)c * (unsigned)sizeof(T)); },
-        s);
+    auto sum = [&](auto nt) {
+      return sell_offset_sum<T, SUB, NODIAG, decltype(nt)::value>(
+          val + base, scalar_ptr(off) + base / kSellRows, scalar_ptr(mask) + base / kSellRows, K,
+          row, lane, [&](int c) { return buffer_load<T>(xr, (unsigned)c * (unsigned)sizeof(T)); },
+          s);
+    };
+    return stream ? sum(std::true_type()) : sum(std::false_type());
   }
   // The row's sum over beta p + z in place of x (each rounded as one fused
   // multiply-add).
@@ -484,7 +489,7 @@ struct SellOffOp {
         const_cast<T *>(p), 0, ncol * (int)sizeof(T), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t zr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T *>(z), 0, ncol * (int)sizeof(T), kRsrcWord3);
-    return sell_offset_sum<T, false, false, true>(
+    return sell_offset_sum<T, false, false, false>(
         val + base, scalar_ptr(off) + base / kSellRows, scalar_ptr(mask) + base / kSellRows, K,
         sid * kSellRows + lane, lane,
         [&](int c) {
@@ -502,6 +507,7 @@ inline SellOffOp<T> sell_off_view(const hflmp_sell *m) {
   op.ncol = m->ncol;
   op.nslice = m->nslice;
   op.max_off = m->max_off;
+  op.stream = entries_stream(m->entries, sizeof(T));
   op.soff = m->soff;
   op.slen = m->slen;
   op.off = m->off;
@@ -524,6 +530,7 @@ inline SellOp<T, IT> sell_view(const hflmp_sell *m) {
   op.rlen = m->rlen;
   op.col = static_cast<const IT *>(m->col);
   op.val = static_cast<const T *>(m->val);
+  op.stream = entries_stream(m->entries, sizeof(T) + sizeof(IT));
   return op;
 }
 
@@ -533,6 +540,7 @@ inline CsrTileOp<T, int> csr_view(int nrow, int nnz, const int *rp, const int *c
   CsrTileOp<T, int> op;
   op.nrow = nrow;
   op.R = tile_rows(nrow, nnz, TileCap<T>::value);
+  op.stream = entries_stream(nnz, sizeof(T) + sizeof(int));
   op.rp = rp;
   op.ci = ci;
   op.val = val;

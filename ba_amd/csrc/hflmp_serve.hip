@@ -88,6 +88,7 @@ struct SysDesc {
   int nrow, nslice, nunits, unit0;
   int mode, col16;  // mixed: FP32 columns are int16 offsets from the slice start
   int col16_64;     // FP64 layout: the same (both as the device decided at admission)
+  int stream, stream32;  // FP64 and FP32 entries past the caches (kCachedBytes)
   int grp0, gsz;    // K2's groups of gsz units (kGroup64 or kQuad): the system's first
   int quad0;        // K3's groups of kQuad units: the system's first
   // FP64 SELL-64 (P = 2): the operator of FP64 systems and of the residuals
@@ -119,6 +120,7 @@ __host__ __device__ __forceinline__ SellOp<double, IT> op64(const SysDesc &d) {
   op.soff = d.soff;
   op.slen = d.slen;
   op.rlen = d.rlen;
+  op.stream = d.stream;
   op.col = static_cast<const IT *>(d.col);
   op.val = d.sval;
   return op;
@@ -132,6 +134,7 @@ __device__ __forceinline__ SellOp<float, IT> op32(const SysDesc &d) {
   op.soff = d.soff32;
   op.slen = d.slen32;
   op.rlen = d.rlen;
+  op.stream = d.stream32;
   op.col = static_cast<const IT *>(d.col32);
   op.val = d.sval32;
   return op;
@@ -577,7 +580,7 @@ __global__ void __launch_bounds__(kBlock)
 // results are dropped.
 template <typename T, typename IT>
 __global__ void __launch_bounds__(kBlock)
-    grp_spmv_kernel(const UnitRec *__restrict__ rec, int u0, int U) {
+    grp_spmv_kernel(const UnitRec *__restrict__ rec, int u0, int U, bool stream) {
   const long long u = xcd_tile(blockIdx.x, gridDim.x);
   if (u >= U) return;
   const UnitRec &r = rec[u0 + u];
@@ -595,9 +598,12 @@ __global__ void __launch_bounds__(kBlock)
   // int16 columns are offsets from the slice's first row
   const T *__restrict__ x = std::is_same<IT, int>::value ? p : p + srow;
   const int dcol = std::is_same<IT, int>::value ? row : lane;
-  const T s = sell_slice_sum<T, IT, false, false, true>(
-      static_cast<const IT *>(r.col) + sl.x, static_cast<const T *>(r.val) + sl.x, sl.y, len,
-      lane, x, dcol, T(0));
+  auto sum = [&](auto nt) {
+    return sell_slice_sum<T, IT, false, false, true, decltype(nt)::value>(
+        static_cast<const IT *>(r.col) + sl.x, static_cast<const T *>(r.val) + sl.x, sl.y, len,
+        lane, x, dcol, T(0));
+  };
+  const T s = stream ? sum(std::true_type()) : sum(std::false_type());
   if (!live) return;
   T part = 0;
   if (has_row) {
@@ -614,7 +620,7 @@ __global__ void __launch_bounds__(kBlock)
 // sums it (wave sums, then the waves in order).
 template <typename T, typename IT>
 __global__ void __launch_bounds__(kBlock)
-    grp_spmv_pair_kernel(const UnitRec *__restrict__ rec, int u0, int U) {
+    grp_spmv_pair_kernel(const UnitRec *__restrict__ rec, int u0, int U, bool stream) {
   const long long pr = xcd_tile(blockIdx.x, gridDim.x);
   if (pr >= (U + 1) / 2) return;
   const int ua = u0 + 2 * (int)pr;
@@ -636,10 +642,13 @@ __global__ void __launch_bounds__(kBlock)
   const T *__restrict__ xA = std::is_same<IT, int>::value ? pA : pA + srowA;
   const T *__restrict__ xB = std::is_same<IT, int>::value ? pB : pB + srowB;
   T sA = 0, sB = 0;
-  sell_slice_sum2<T, IT, 2>(static_cast<const IT *>(ra.col) + slA.x,
-                         static_cast<const T *>(ra.val) + slA.x, slA.y, lenA, xA,
-                         static_cast<const IT *>(rb.col) + slB.x,
-                         static_cast<const T *>(rb.val) + slB.x, slB.y, lenB, xB, lane, sA, sB);
+  auto sum2 = [&](auto nt) {
+    sell_slice_sum2<T, IT, decltype(nt)::value, 2>(
+        static_cast<const IT *>(ra.col) + slA.x, static_cast<const T *>(ra.val) + slA.x, slA.y,
+        lenA, xA, static_cast<const IT *>(rb.col) + slB.x,
+        static_cast<const T *>(rb.val) + slB.x, slB.y, lenB, xB, lane, sA, sB);
+  };
+  stream ? sum2(std::true_type()) : sum2(std::false_type());
   T partA = 0, partB = 0;
   if (liveA && hA) {
     static_cast<T *>(ra.Ap)[rowA] = sA;
@@ -1263,6 +1272,7 @@ void plan_job(Job &jb) {
 struct TableSet {
   long long version = -1;  // the version of the active set these tables hold
   int S = 0, U = 0;
+  bool stream = false;  // the products' entries past the caches (kCachedBytes)
   bool fold = false;  // K2 and K3 form the scalars (kFoldUnits)
   SysDesc *d_sys = nullptr, *h_sys = nullptr;  // [max_active]
   int *d_unit = nullptr, *h_unit = nullptr;    // [unit_cap]: FP64 systems' units first
@@ -1380,16 +1390,16 @@ void enqueue_chunk(const hflmp_server *sv, const TableSet &t, hipStream_t s) {
   for (int it = 0; it < sv->chunk; ++it) {
     if (ub[1] > ub[0])
       grp_spmv_kernel<double, short><<<grid(ub[1] - ub[0]), kBlock, 0, s>>>(t.d_rec, ub[0],
-                                                                              ub[1] - ub[0]);
+                                                                              ub[1] - ub[0], t.stream);
     if (ub[2] > ub[1])
       grp_spmv_kernel<double, int><<<grid(ub[2] - ub[1]), kBlock, 0, s>>>(t.d_rec, ub[1],
-                                                                            ub[2] - ub[1]);
+                                                                            ub[2] - ub[1], t.stream);
     if (ub[3] > ub[2])
       grp_spmv_pair_kernel<float, short><<<grid((ub[3] - ub[2] + 1) / 2), kBlock, 0, s>>>(
-          t.d_rec, ub[2], ub[3] - ub[2]);
+          t.d_rec, ub[2], ub[3] - ub[2], t.stream);
     if (ub[4] > ub[3])
       grp_spmv_pair_kernel<float, int><<<grid((ub[4] - ub[3] + 1) / 2), kBlock, 0, s>>>(
-          t.d_rec, ub[3], ub[4] - ub[3]);
+          t.d_rec, ub[3], ub[4] - ub[3], t.stream);
     if (t.fold) {
       grp_update_kernel<true><<<gG, kBlock, 0, s>>>(t.d_sys, t.d_grp, t.G);
       grp_p_kernel<true><<<gQ, kBlock, 0, s>>>(t.d_sys, t.d_quad, t.Q);
@@ -1463,16 +1473,20 @@ int rebuild_tables(hflmp_server *sv, TableSet &t) {
   hflmp_ctx *ctx = sv->ctx;
   int U = 0, G = 0, Q = 0;
   long long square64 = 0;
+  size_t entry_bytes = 0;
   bool fits = true;
   for (int slot : sv->order) {
     Job &jb = sv->jobs[sv->slot_job[slot]];
     fits = fits && jb.nunits <= kFoldUnits;
+    entry_bytes += jb.mode == kModeFp64 ? 10 * (size_t)jb.sp64.entries
+                                        : 6 * (size_t)jb.sp32.entries;
     if (jb.d.mode == kModeFp64) square64 += (long long)jb.nunits * jb.nunits;
     jb.d.gsz = jb.d.mode == kModeFp64 ? kGroup64 : kQuad;
     U += jb.nunits;
     G += (jb.nunits + jb.d.gsz - 1) / jb.d.gsz;
     Q += (jb.nunits + kQuad - 1) / kQuad;
   }
+  t.stream = entries_stream((long long)entry_bytes, 1);
   t.fold = fits && square64 <= kFoldSquare64;
   if ((size_t)U > t.rec_cap) {
     if (t.d_rec) (void)hipFree(t.d_rec);
@@ -1680,6 +1694,8 @@ void admit_describe(hflmp_server *sv, Job &jb, int slot) {
   d.nslice = jb.nslice;
   d.nunits = jb.nunits;
   d.mode = jb.mode;
+  d.stream = entries_stream(jb.sp64.entries, 10);
+  d.stream32 = entries_stream(jb.sp32.entries, 6);
   d.soff = static_cast<const long long *>(dp(jb.o_soff));
   d.slen = static_cast<const int *>(dp(jb.o_slen));
   d.rlen = static_cast<const unsigned char *>(dp(jb.o_rlen));

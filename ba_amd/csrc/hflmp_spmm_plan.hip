@@ -462,7 +462,11 @@ int plan_spmm(hflmp_ctx *ctx, const hflmp_spmm_plan *p, const int *rp, const T *
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              (int)lds));
   const int g = plan_grid(ctx, reinterpret_cast<const void *>(kern), p->nblk, lds);
-  kern<<<g, kPlanThreads, lds, ctx->stream>>>(plan_view(p), k, rp, val, X, Y);
+  // what the next product finds in the caches depends on X and Y too
+  const bool stream = entries_stream(
+      p->nnz + (long long)((size_t)(p->nrow + (long long)p->ncol) * k * sizeof(T) / (4 + sizeof(T))),
+      4 + sizeof(T));
+  kern<<<g, kPlanThreads, lds, ctx->stream>>>(plan_view(p, stream), k, rp, val, X, Y);
   HFLMP_LAUNCH_CHECK(ctx);
   return HFLMP_OK;
 }

@@ -91,11 +91,12 @@ struct PlanView {
   const int *__restrict__ ucol;
   const int *__restrict__ lidx;
   const int2 *__restrict__ rows;
+  bool stream;  // entries past the caches
 };
 
-inline PlanView plan_view(const hflmp_spmm_plan *p) {
+inline PlanView plan_view(const hflmp_spmm_plan *p, bool stream) {
   return PlanView{plan_geom(p->nrow, p->L, p->a, p->nl), p->nnz, p->R, p->nblk, p->umax,
-                  p->emax, p->uoff, p->ucol, p->lidx, p->rows};
+                  p->emax, p->uoff, p->ucol, p->lidx, p->rows, stream};
 }
 
 // LDS of the walk: the X rows of one block, then two buffers of the
@@ -221,12 +222,21 @@ __device__ __forceinline__ void plan_meta_load(PlanMetaRegs<T> &m, const PlanHdr
   // entries past the block's last read its first run's first entry
   const int j0 = __builtin_amdgcn_readlane(h.hreg, 0);
   const int jpad = j0 < pv.nnz ? j0 : pv.nnz - 1;
+  int j[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int e = t + q * kBlock;
-    const int j = e < h.ne ? e + base[q] : jpad;
-    m.li[q] = __builtin_nontemporal_load(pv.lidx + j);
-    m.v[q] = __builtin_nontemporal_load(val + j);
+  for (int q = 0; q < 4; ++q) j[q] = t + q * kBlock < h.ne ? t + q * kBlock + base[q] : jpad;
+  if (pv.stream) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      m.li[q] = __builtin_nontemporal_load(pv.lidx + j[q]);
+      m.v[q] = __builtin_nontemporal_load(val + j[q]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      m.li[q] = pv.lidx[j[q]];
+      m.v[q] = val[j[q]];
+    }
   }
 }
 

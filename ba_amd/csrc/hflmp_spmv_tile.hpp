@@ -68,9 +68,10 @@ __device__ __forceinline__ T lds_seq_sum(const T *__restrict__ prod, int lo, int
 
 // Returns s + sum_j val[j] * x[col[j]] over this thread's row of the tile.
 // SKIP_DIAG drops j with col[j] == row (y = (A - D) x).  IT = short reads
-// 16-bit offsets from the tile's first row.
+// 16-bit offsets from the tile's first row.  NT: entries are loaded past the
+// caches.
 // All threads of the workgroup must call this (it synchronises).
-template <typename T, bool SKIP_DIAG, typename IT = int>
+template <typename T, bool SKIP_DIAG, bool NT, typename IT = int>
 __device__ __forceinline__ T tile_row_sum(long long tile, int rows_per_tile, int nrow,
                                           const int *__restrict__ rp,
                                           const IT *__restrict__ ci,
@@ -103,8 +104,8 @@ __device__ __forceinline__ T tile_row_sum(long long tile, int rows_per_tile, int
     for (int u = 0; u < U; ++u) {
       const int k = t + u * kBlock;
       if (k < cnt_all) {
-        c[u] = ld_stream(ci + nz0 + k);
-        v[u] = ld_stream(val + nz0 + k);
+        c[u] = ld_entry<NT>(ci + nz0 + k);
+        v[u] = ld_entry<NT>(val + nz0 + k);
       }
     }
     int lo = 0, hi = 0;
@@ -145,8 +146,8 @@ __device__ __forceinline__ T tile_row_sum(long long tile, int rows_per_tile, int
       for (int u = 0; u < 4; ++u) {
         const int k = k0 + u * kBlock;
         if (k < cnt) {
-          c[u] = ld_stream(cb + k);
-          v[u] = ld_stream(vb + k);
+          c[u] = ld_entry<NT>(cb + k);
+          v[u] = ld_entry<NT>(vb + k);
         }
       }
 #pragma unroll
