@@ -612,7 +612,7 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
     gp = plan_grid(ctx, reinterpret_cast<const void *>(plan_kern), plan->nblk, lds);
     if (gp > g) gp = g / kXcds * kXcds;
   }
-  const bool stream = entries_stream(nnz, sizeof(T) + sizeof(int));
+  const int cached = entries_cached(nnz, 4 + sizeof(T), 4 * sizeof(T) * k * (size_t)nrow);
   const auto t0 = std::chrono::steady_clock::now();
   binit_state_kernel<T><<<1, kMaxRhs, 0, s>>>(st, k, maxit, atol, rtol, dtol);
   bcg_init_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, invd, B, X, R, P, part);
@@ -620,7 +620,7 @@ int batched_pcg(hflmp_ctx *ctx, int nrow, int nnz, int k, const int *rp, const i
   HFLMP_LAUNCH_CHECK(ctx);
   auto iteration = [&]() {
     if (plan) {
-      plan_kern<<<gp, kPlanThreads, lds, s>>>(plan_view(plan, stream), k, rp, val, P, AP, st, part);
+      plan_kern<<<gp, kPlanThreads, lds, s>>>(plan_view(plan, cached), k, rp, val, P, AP, st, part);
       bcg_alpha_final<T><<<k, kBlock, 0, s>>>(st, part, gp, k);
     } else {
       bcg_spmm_kernel<T><<<g, kBlock, 0, s>>>(nrow, k, rp, ci, val, P, AP, st, part);

@@ -568,7 +568,8 @@ int mpcg_jacobi(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
     CsrTileOp<float, short> op16;
     op16.nrow = nrow;
     op16.R = op32.R;
-    op16.stream = entries_stream(nnz, sizeof(float) + sizeof(short));
+    op16.cached =
+        entries_cached(nnz, sizeof(float) + sizeof(short), kCgVectors * sizeof(float) * nrow);
     op16.rp = rp;
     op16.ci = c16;
     op16.val = val32;

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -265,16 +266,41 @@ __device__ __forceinline__ T ld_entry(const T *p) {
   return NT ? __builtin_nontemporal_load(p) : *p;
 }
 
-// Bytes of a matrix's entries up to which products load them through the
-// caches: what the next product finds there depends on all of them fitting
-// the Infinity Cache (256 MB) with the vectors.  Larger matrices are loaded
-// past the caches, which they would only sweep.  Jacobi-CG on 3D Q1 in FP64
-// (SELL-64, offset form), ms a solve past and through the caches: 96^3, 195 MB,
-// 15.4 and 11.7; 104^3, 247 MB, 20.3 and 18.8; 108^3, 277 MB, 22.2 and 22.5;
-// 128^3, 459 MB, 36.8 and 38.6.
-constexpr size_t kCachedBytes = (size_t)256 << 20;
-inline bool entries_stream(long long entries, size_t entry_bytes) {
-  return (size_t)entries * entry_bytes > kCachedBytes;
+// How much of a matrix products load through the caches, for the next product
+// to find in the Infinity Cache (256 MB): `cached` of every kCachedParts
+// slices, tiles or blocks (interleaved, so that each XCD has its share), the
+// rest past the caches.  All of it where it about fits with the vectors that
+// are used between two products; else as much as leaves room for those and
+// for what streams through (216 MB in all), since a matrix that is too large
+// would sweep itself and them out.  Jacobi-CG on 3D Q1 in FP64 (SELL-64, offset
+// form), MB of matrix + vectors, ms a solve with none, part and all of the
+// matrix through the caches: 96^3, 197 + 44, 15.6 - 12.4; 100^3, 223 + 49, 17.7
+// 15.5 14.8; 104^3, 250 + 56, 20.1 17.2 18.8; 112^3, 312 + 69, 26.3 22.6 27.2;
+// 128^3, 464 + 103, 36.9 34.5 38.6.
+constexpr int kCachedParts = 64;
+inline int entries_cached(long long entries, size_t entry_bytes, size_t vector_bytes) {
+  constexpr size_t kAll = (size_t)264 << 20, kPart = (size_t)216 << 20;
+  const size_t bytes = (size_t)entries * entry_bytes;
+  if (bytes + vector_bytes <= kAll) return kCachedParts;
+  return vector_bytes < kPart && bytes > 0
+             ? (int)std::min<size_t>(kCachedParts, kCachedParts * (kPart - vector_bytes) / bytes)
+             : 0;
+}
+// Vectors that an iteration of the solvers uses between two products: x, r,
+// z, p, A p, D^-1.
+constexpr size_t kCgVectors = 6;
+
+// The same for a product by itself, which cannot know what comes before the
+// next one: all of a matrix that takes a third of the cache with x and y, else
+// none.  Of three 3D Q1 matrices in turn, us a product past and through the
+// caches: 64^3 (60 MB) 15.7 and 12.3, 96^3 (197 MB) 44.5 and 45.9, 128^3 in
+// FP32 (232 MB) 43.4 and 48.4.
+inline int entries_cached_once(long long entries, size_t entry_bytes, size_t vector_bytes) {
+  return (size_t)entries * entry_bytes + vector_bytes <= ((size_t)88 << 20) ? kCachedParts : 0;
+}
+// Whether part `i` is loaded past the caches.
+__device__ __forceinline__ bool past_caches(long long i, int cached) {
+  return (int)(i & (kCachedParts - 1)) >= cached;
 }
 
 // Buffer descriptor word 3 for raw (untyped) buffer access on gfx9-family

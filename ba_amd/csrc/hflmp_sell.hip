@@ -466,12 +466,14 @@ int sell_spmv(hflmp_ctx *ctx, const hflmp_sell *m, const T *x, T *y) {
   const unsigned grid = sell_grid(m->nrow);
   hipStream_t s = ctx->stream;
   if (m->off_form)
-    sell_spmv16_kernel<SellOffOp<T>, MODE><<<grid, kBlock, 0, s>>>(sell_off_view<T>(m), x, y);
+    sell_spmv16_kernel<SellOffOp<T>, MODE><<<grid, kBlock, 0, s>>>(
+        sell_off_view<T>(m, true), x, y);
   else if (m->col_bytes == 2)
-    sell_spmv16_kernel<SellOp<T, short>, MODE><<<grid, kBlock, 0, s>>>(sell_view<T, short>(m),
-                                                                        x, y);
+    sell_spmv16_kernel<SellOp<T, short>, MODE><<<grid, kBlock, 0, s>>>(
+        sell_view<T, short>(m, true), x, y);
   else
-    sell_spmv_kernel<SellOp<T, int>, MODE><<<grid, kBlock, 0, s>>>(sell_view<T, int>(m), x, y);
+    sell_spmv_kernel<SellOp<T, int>, MODE><<<grid, kBlock, 0, s>>>(
+        sell_view<T, int>(m, true), x, y);
   HFLMP_LAUNCH_CHECK(ctx);
   return HFLMP_OK;
 }

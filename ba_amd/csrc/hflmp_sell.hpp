@@ -107,7 +107,7 @@ struct CsrTileOp {
   using value_type = T;
   static constexpr int kLds = TileCap<T>::value;
   int nrow, R;
-  bool stream;  // entries past the caches (kCachedBytes)
+  int cached;  // entries_cached, by tiles
   const int *rp;
   const IT *ci;
   const T *val;
@@ -117,8 +117,9 @@ struct CsrTileOp {
   }
   __device__ __forceinline__ T row_sum(long long unit, const T *x, T s, TileRow &tr,
                                        T *lds) const {
-    return stream ? tile_row_sum<T, false, true, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds)
-                  : tile_row_sum<T, false, false, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds);
+    return past_caches(unit, cached)
+               ? tile_row_sum<T, false, true, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds)
+               : tile_row_sum<T, false, false, IT>(unit, R, nrow, rp, ci, val, x, s, tr, lds);
   }
 };
 
@@ -129,7 +130,7 @@ struct CsrTileOp {
 // cover the row's own entries, or with LOAD_ALL every entry position of the
 // slice (all allocated: 64 x smax entries), so that they need not wait for
 // len; the sum is the same either way.  NT: entries are loaded past the
-// caches (kCachedBytes).  U: chunk loads in flight per step.
+// caches.  U: chunk loads in flight per step.
 // GATHER_ALL: x is read for every entry loaded, padding included (its
 // column is 0; for an x that is cheap to read and has no limit to guard).
 template <typename T, typename IT, bool SUB, bool NODIAG, bool LOAD_ALL, bool NT = true,
@@ -307,7 +308,7 @@ struct SellOp {
   static constexpr int P = SellChunk<T>::P;
   static constexpr int U = SellChunk<T>::U;
   int nrow, nslice;
-  bool stream;  // entries past the caches (kCachedBytes)
+  int cached;  // entries_cached, by slices
   const long long *soff;
   const int *slen;
   const unsigned char *rlen;
@@ -337,10 +338,11 @@ struct SellOp {
     // int16 columns are offsets from the slice's first row
     const T *__restrict__ x = std::is_same<IT, int>::value ? x_in : x_in + sid * kSellRows;
     const int dcol = std::is_same<IT, int>::value ? row : lane;
-    return stream ? sell_slice_sum<T, IT, SUB, NODIAG, false, true>(col + base, val + base, smax,
-                                                                    len, lane, x, dcol, s)
-                  : sell_slice_sum<T, IT, SUB, NODIAG, false, false>(col + base, val + base, smax,
-                                                                     len, lane, x, dcol, s);
+    return past_caches(sid, cached)
+               ? sell_slice_sum<T, IT, SUB, NODIAG, false, true>(col + base, val + base, smax, len,
+                                                                 lane, x, dcol, s)
+               : sell_slice_sum<T, IT, SUB, NODIAG, false, false>(col + base, val + base, smax,
+                                                                  len, lane, x, dcol, s);
   }
 };
 
@@ -439,7 +441,7 @@ struct SellOffOp {
   using value_type = T;
   static constexpr int kLds = 1;
   int nrow, ncol, nslice, max_off;
-  bool stream;  // entries past the caches (kCachedBytes)
+  int cached;  // entries_cached, by slices
   const long long *soff;
   const int *slen;
   const int *off;
@@ -473,7 +475,7 @@ struct SellOffOp {
           row, lane, [&](int c) { return buffer_load<T>(xr, (unsigned)c * (unsigned)sizeof(T)); },
           s);
     };
-    return stream ? sum(std::true_type()) : sum(std::false_type());
+    return past_caches(sid, cached) ? sum(std::true_type()) : sum(std::false_type());
   }
   // The row's sum over beta p + z in place of x (each rounded as one fused
   // multiply-add).
@@ -500,14 +502,20 @@ struct SellOffOp {
   }
 };
 
+// once: for a product by itself, not an iteration's
+inline int sell_cached(const hflmp_sell *m, size_t entry_bytes, size_t vb, bool once) {
+  return once ? entries_cached_once(m->entries, entry_bytes, vb * ((size_t)m->nrow + m->ncol))
+              : entries_cached(m->entries, entry_bytes, kCgVectors * vb * m->nrow);
+}
+
 template <typename T>
-inline SellOffOp<T> sell_off_view(const hflmp_sell *m) {
+inline SellOffOp<T> sell_off_view(const hflmp_sell *m, bool once = false) {
   SellOffOp<T> op;
   op.nrow = m->nrow;
   op.ncol = m->ncol;
   op.nslice = m->nslice;
   op.max_off = m->max_off;
-  op.stream = entries_stream(m->entries, sizeof(T));
+  op.cached = sell_cached(m, sizeof(T), sizeof(T), once);
   op.soff = m->soff;
   op.slen = m->slen;
   op.off = m->off;
@@ -521,7 +529,7 @@ inline SellOffOp<T> sell_off_view(const hflmp_sell *m) {
 constexpr int kSellOffsets = 0x100;
 
 template <typename T, typename IT>
-inline SellOp<T, IT> sell_view(const hflmp_sell *m) {
+inline SellOp<T, IT> sell_view(const hflmp_sell *m, bool once = false) {
   SellOp<T, IT> op;
   op.nrow = m->nrow;
   op.nslice = m->nslice;
@@ -530,7 +538,7 @@ inline SellOp<T, IT> sell_view(const hflmp_sell *m) {
   op.rlen = m->rlen;
   op.col = static_cast<const IT *>(m->col);
   op.val = static_cast<const T *>(m->val);
-  op.stream = entries_stream(m->entries, sizeof(T) + sizeof(IT));
+  op.cached = sell_cached(m, sizeof(T) + sizeof(IT), sizeof(T), once);
   return op;
 }
 
@@ -540,7 +548,7 @@ inline CsrTileOp<T, int> csr_view(int nrow, int nnz, const int *rp, const int *c
   CsrTileOp<T, int> op;
   op.nrow = nrow;
   op.R = tile_rows(nrow, nnz, TileCap<T>::value);
-  op.stream = entries_stream(nnz, sizeof(T) + sizeof(int));
+  op.cached = entries_cached(nnz, sizeof(T) + sizeof(int), kCgVectors * sizeof(T) * nrow);
   op.rp = rp;
   op.ci = ci;
   op.val = val;

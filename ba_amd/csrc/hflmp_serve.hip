@@ -88,7 +88,7 @@ struct SysDesc {
   int nrow, nslice, nunits, unit0;
   int mode, col16;  // mixed: FP32 columns are int16 offsets from the slice start
   int col16_64;     // FP64 layout: the same (both as the device decided at admission)
-  int stream, stream32;  // FP64 and FP32 entries past the caches (kCachedBytes)
+  int cached, cached32;  // entries_cached of the FP64 and FP32 entries
   int grp0, gsz;    // K2's groups of gsz units (kGroup64 or kQuad): the system's first
   int quad0;        // K3's groups of kQuad units: the system's first
   // FP64 SELL-64 (P = 2): the operator of FP64 systems and of the residuals
@@ -120,7 +120,7 @@ __host__ __device__ __forceinline__ SellOp<double, IT> op64(const SysDesc &d) {
   op.soff = d.soff;
   op.slen = d.slen;
   op.rlen = d.rlen;
-  op.stream = d.stream;
+  op.cached = d.cached;
   op.col = static_cast<const IT *>(d.col);
   op.val = d.sval;
   return op;
@@ -134,7 +134,7 @@ __device__ __forceinline__ SellOp<float, IT> op32(const SysDesc &d) {
   op.soff = d.soff32;
   op.slen = d.slen32;
   op.rlen = d.rlen;
-  op.stream = d.stream32;
+  op.cached = d.cached32;
   op.col = static_cast<const IT *>(d.col32);
   op.val = d.sval32;
   return op;
@@ -578,9 +578,10 @@ __global__ void __launch_bounds__(kBlock)
 // p at the row and the slice's entries go out together; the sums are those
 // of SellOp::row_sum (same order, same predicates), and a stopped system's
 // results are dropped.
-template <typename T, typename IT>
+// NT: entries past the caches.
+template <typename T, typename IT, bool NT>
 __global__ void __launch_bounds__(kBlock)
-    grp_spmv_kernel(const UnitRec *__restrict__ rec, int u0, int U, bool stream) {
+    grp_spmv_kernel(const UnitRec *__restrict__ rec, int u0, int U) {
   const long long u = xcd_tile(blockIdx.x, gridDim.x);
   if (u >= U) return;
   const UnitRec &r = rec[u0 + u];
@@ -598,12 +599,9 @@ __global__ void __launch_bounds__(kBlock)
   // int16 columns are offsets from the slice's first row
   const T *__restrict__ x = std::is_same<IT, int>::value ? p : p + srow;
   const int dcol = std::is_same<IT, int>::value ? row : lane;
-  auto sum = [&](auto nt) {
-    return sell_slice_sum<T, IT, false, false, true, decltype(nt)::value>(
-        static_cast<const IT *>(r.col) + sl.x, static_cast<const T *>(r.val) + sl.x, sl.y, len,
-        lane, x, dcol, T(0));
-  };
-  const T s = stream ? sum(std::true_type()) : sum(std::false_type());
+  const T s = sell_slice_sum<T, IT, false, false, true, NT>(
+      static_cast<const IT *>(r.col) + sl.x, static_cast<const T *>(r.val) + sl.x, sl.y, len,
+      lane, x, dcol, T(0));
   if (!live) return;
   T part = 0;
   if (has_row) {
@@ -618,9 +616,9 @@ __global__ void __launch_bounds__(kBlock)
 // FP32 wave's loads are half the FP64 one's).  The units may belong to
 // different systems; each keeps its own partial, summed as unit_partial1
 // sums it (wave sums, then the waves in order).
-template <typename T, typename IT>
+template <typename T, typename IT, bool NT>
 __global__ void __launch_bounds__(kBlock)
-    grp_spmv_pair_kernel(const UnitRec *__restrict__ rec, int u0, int U, bool stream) {
+    grp_spmv_pair_kernel(const UnitRec *__restrict__ rec, int u0, int U) {
   const long long pr = xcd_tile(blockIdx.x, gridDim.x);
   if (pr >= (U + 1) / 2) return;
   const int ua = u0 + 2 * (int)pr;
@@ -642,13 +640,10 @@ __global__ void __launch_bounds__(kBlock)
   const T *__restrict__ xA = std::is_same<IT, int>::value ? pA : pA + srowA;
   const T *__restrict__ xB = std::is_same<IT, int>::value ? pB : pB + srowB;
   T sA = 0, sB = 0;
-  auto sum2 = [&](auto nt) {
-    sell_slice_sum2<T, IT, decltype(nt)::value, 2>(
-        static_cast<const IT *>(ra.col) + slA.x, static_cast<const T *>(ra.val) + slA.x, slA.y,
-        lenA, xA, static_cast<const IT *>(rb.col) + slB.x,
-        static_cast<const T *>(rb.val) + slB.x, slB.y, lenB, xB, lane, sA, sB);
-  };
-  stream ? sum2(std::true_type()) : sum2(std::false_type());
+  sell_slice_sum2<T, IT, NT, 2>(
+      static_cast<const IT *>(ra.col) + slA.x, static_cast<const T *>(ra.val) + slA.x, slA.y,
+      lenA, xA, static_cast<const IT *>(rb.col) + slB.x, static_cast<const T *>(rb.val) + slB.x,
+      slB.y, lenB, xB, lane, sA, sB);
   T partA = 0, partB = 0;
   if (liveA && hA) {
     static_cast<T *>(ra.Ap)[rowA] = sA;
@@ -1272,7 +1267,7 @@ void plan_job(Job &jb) {
 struct TableSet {
   long long version = -1;  // the version of the active set these tables hold
   int S = 0, U = 0;
-  bool stream = false;  // the products' entries past the caches (kCachedBytes)
+  bool stream = false;  // the set's entries past the caches: they do not all fit
   bool fold = false;  // K2 and K3 form the scalars (kFoldUnits)
   SysDesc *d_sys = nullptr, *h_sys = nullptr;  // [max_active]
   int *d_unit = nullptr, *h_unit = nullptr;    // [unit_cap]: FP64 systems' units first
@@ -1374,13 +1369,30 @@ void drop_graph(TableSet &t) {
   t.graph = nullptr;
 }
 
+// K1 of every form in the table.
+template <bool NT>
+void enqueue_products(const TableSet &t, hipStream_t s) {
+  auto grid = [](int n) { return (unsigned)(((n + kXcds - 1) / kXcds) * kXcds); };
+  const int *ub = t.ubeg;
+  const int n64s = ub[1] - ub[0], n64i = ub[2] - ub[1], n32s = ub[3] - ub[2], n32i = ub[4] - ub[3];
+  if (n64s > 0)
+    grp_spmv_kernel<double, short, NT><<<grid(n64s), kBlock, 0, s>>>(t.d_rec, ub[0], n64s);
+  if (n64i > 0)
+    grp_spmv_kernel<double, int, NT><<<grid(n64i), kBlock, 0, s>>>(t.d_rec, ub[1], n64i);
+  if (n32s > 0)
+    grp_spmv_pair_kernel<float, short, NT>
+        <<<grid((n32s + 1) / 2), kBlock, 0, s>>>(t.d_rec, ub[2], n32s);
+  if (n32i > 0)
+    grp_spmv_pair_kernel<float, int, NT>
+        <<<grid((n32i + 1) / 2), kBlock, 0, s>>>(t.d_rec, ub[3], n32i);
+}
+
 // The work of one chunk on the stream: starts of fresh FP64 systems, outer
 // steps of mixed systems, then `chunk` iterations.
 void enqueue_chunk(const hflmp_server *sv, const TableSet &t, hipStream_t s) {
   auto grid = [](int n) { return (unsigned)(((n + kXcds - 1) / kXcds) * kXcds); };
   const unsigned gU = grid(t.U), gG = grid(t.G), gQ = grid(t.Q);
   const unsigned gS = (unsigned)t.S;
-  const int *ub = t.ubeg;
   grp_init_kernel<<<gU, kBlock, 0, s>>>(t.d_sys, t.d_unit, t.U);
   grp_init_final<<<gS, kBlock, 0, s>>>(t.d_sys);
   grp_mix_correct_kernel<<<gU, kBlock, 0, s>>>(t.d_sys, t.d_unit, t.U);
@@ -1388,18 +1400,7 @@ void enqueue_chunk(const hflmp_server *sv, const TableSet &t, hipStream_t s) {
   grp_mix_residual_final<<<gS, kBlock, 0, s>>>(t.d_sys);
   grp_mix_prefresh_kernel<<<gU, kBlock, 0, s>>>(t.d_sys, t.d_unit, t.U);
   for (int it = 0; it < sv->chunk; ++it) {
-    if (ub[1] > ub[0])
-      grp_spmv_kernel<double, short><<<grid(ub[1] - ub[0]), kBlock, 0, s>>>(t.d_rec, ub[0],
-                                                                              ub[1] - ub[0], t.stream);
-    if (ub[2] > ub[1])
-      grp_spmv_kernel<double, int><<<grid(ub[2] - ub[1]), kBlock, 0, s>>>(t.d_rec, ub[1],
-                                                                            ub[2] - ub[1], t.stream);
-    if (ub[3] > ub[2])
-      grp_spmv_pair_kernel<float, short><<<grid((ub[3] - ub[2] + 1) / 2), kBlock, 0, s>>>(
-          t.d_rec, ub[2], ub[3] - ub[2], t.stream);
-    if (ub[4] > ub[3])
-      grp_spmv_pair_kernel<float, int><<<grid((ub[4] - ub[3] + 1) / 2), kBlock, 0, s>>>(
-          t.d_rec, ub[3], ub[4] - ub[3], t.stream);
+    t.stream ? enqueue_products<true>(t, s) : enqueue_products<false>(t, s);
     if (t.fold) {
       grp_update_kernel<true><<<gG, kBlock, 0, s>>>(t.d_sys, t.d_grp, t.G);
       grp_p_kernel<true><<<gQ, kBlock, 0, s>>>(t.d_sys, t.d_quad, t.Q);
@@ -1473,20 +1474,21 @@ int rebuild_tables(hflmp_server *sv, TableSet &t) {
   hflmp_ctx *ctx = sv->ctx;
   int U = 0, G = 0, Q = 0;
   long long square64 = 0;
-  size_t entry_bytes = 0;
+  size_t entry_bytes = 0, vector_bytes = 0;
   bool fits = true;
   for (int slot : sv->order) {
     Job &jb = sv->jobs[sv->slot_job[slot]];
     fits = fits && jb.nunits <= kFoldUnits;
     entry_bytes += jb.mode == kModeFp64 ? 10 * (size_t)jb.sp64.entries
                                         : 6 * (size_t)jb.sp32.entries;
+    vector_bytes += kCgVectors * (jb.mode == kModeFp64 ? 8 : 4) * (size_t)jb.nrow;
     if (jb.d.mode == kModeFp64) square64 += (long long)jb.nunits * jb.nunits;
     jb.d.gsz = jb.d.mode == kModeFp64 ? kGroup64 : kQuad;
     U += jb.nunits;
     G += (jb.nunits + jb.d.gsz - 1) / jb.d.gsz;
     Q += (jb.nunits + kQuad - 1) / kQuad;
   }
-  t.stream = entries_stream((long long)entry_bytes, 1);
+  t.stream = entries_cached((long long)entry_bytes, 1, vector_bytes) < kCachedParts;
   t.fold = fits && square64 <= kFoldSquare64;
   if ((size_t)U > t.rec_cap) {
     if (t.d_rec) (void)hipFree(t.d_rec);
@@ -1694,8 +1696,8 @@ void admit_describe(hflmp_server *sv, Job &jb, int slot) {
   d.nslice = jb.nslice;
   d.nunits = jb.nunits;
   d.mode = jb.mode;
-  d.stream = entries_stream(jb.sp64.entries, 10);
-  d.stream32 = entries_stream(jb.sp32.entries, 6);
+  d.cached = entries_cached(jb.sp64.entries, 10, kCgVectors * 8 * (size_t)jb.nrow);
+  d.cached32 = entries_cached(jb.sp32.entries, 6, kCgVectors * 4 * (size_t)jb.nrow);
   d.soff = static_cast<const long long *>(dp(jb.o_soff));
   d.slen = static_cast<const int *>(dp(jb.o_slen));
   d.rlen = static_cast<const unsigned char *>(dp(jb.o_rlen));

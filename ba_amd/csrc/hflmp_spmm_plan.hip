@@ -462,11 +462,10 @@ int plan_spmm(hflmp_ctx *ctx, const hflmp_spmm_plan *p, const int *rp, const T *
                                              hipFuncAttributeMaxDynamicSharedMemorySize,
                                              (int)lds));
   const int g = plan_grid(ctx, reinterpret_cast<const void *>(kern), p->nblk, lds);
-  // what the next product finds in the caches depends on X and Y too
-  const bool stream = entries_stream(
-      p->nnz + (long long)((size_t)(p->nrow + (long long)p->ncol) * k * sizeof(T) / (4 + sizeof(T))),
-      4 + sizeof(T));
-  kern<<<g, kPlanThreads, lds, ctx->stream>>>(plan_view(p, stream), k, rp, val, X, Y);
+  kern<<<g, kPlanThreads, lds, ctx->stream>>>(
+      plan_view(p, entries_cached_once(p->nnz, 4 + sizeof(T),
+                                       sizeof(T) * k * ((size_t)p->nrow + p->ncol))),
+      k, rp, val, X, Y);
   HFLMP_LAUNCH_CHECK(ctx);
   return HFLMP_OK;
 }

@@ -91,12 +91,13 @@ struct PlanView {
   const int *__restrict__ ucol;
   const int *__restrict__ lidx;
   const int2 *__restrict__ rows;
-  bool stream;  // entries past the caches
+  int cached;  // entries_cached, by blocks
 };
 
-inline PlanView plan_view(const hflmp_spmm_plan *p, bool stream) {
+inline PlanView plan_view(const hflmp_spmm_plan *p, int cached) {
   return PlanView{plan_geom(p->nrow, p->L, p->a, p->nl), p->nnz, p->R, p->nblk, p->umax,
-                  p->emax, p->uoff, p->ucol, p->lidx, p->rows, stream};
+                  p->emax, p->uoff, p->ucol, p->lidx, p->rows,
+                  cached};
 }
 
 // LDS of the walk: the X rows of one block, then two buffers of the
@@ -225,7 +226,7 @@ __device__ __forceinline__ void plan_meta_load(PlanMetaRegs<T> &m, const PlanHdr
   int j[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) j[q] = t + q * kBlock < h.ne ? t + q * kBlock + base[q] : jpad;
-  if (pv.stream) {
+  if (past_caches(h.b, pv.cached)) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       m.li[q] = __builtin_nontemporal_load(pv.lidx + j[q]);

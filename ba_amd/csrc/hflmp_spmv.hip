@@ -10,7 +10,7 @@ enum SpmvMode { kAssign = 0, kAdd = 1, kNoDiag = 2 };
 
 template <typename T, int MODE>
 __global__ void __launch_bounds__(kBlock)
-    csr_spmv_kernel(int nrow, int rows_per_tile, bool stream, const int *__restrict__ rp,
+    csr_spmv_kernel(int nrow, int rows_per_tile, int cached, const int *__restrict__ rp,
                     const int *__restrict__ ci, const T *__restrict__ val,
                     const T *__restrict__ x, T *__restrict__ y) {
   __shared__ T prod[TileCap<T>::value];
@@ -23,7 +23,8 @@ __global__ void __launch_bounds__(kBlock)
     if (threadIdx.x < rows_per_tile && r < nrow) s = y[r];
   }
   TileRow tr;
-  s = stream ? tile_row_sum<T, MODE == kNoDiag, true>(tile, rows_per_tile, nrow, rp, ci, val, x, s,
+  s = past_caches(tile, cached)
+          ? tile_row_sum<T, MODE == kNoDiag, true>(tile, rows_per_tile, nrow, rp, ci, val, x, s,
                                                       tr, prod)
              : tile_row_sum<T, MODE == kNoDiag, false>(tile, rows_per_tile, nrow, rp, ci, val, x,
                                                        s, tr, prod);
@@ -87,7 +88,8 @@ int spmv(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, const int *
   const long long ntiles = ((long long)nrow + R - 1) / R;
   const int grid = tile_grid(ntiles);
   csr_spmv_kernel<T, MODE><<<grid, kBlock, 0, ctx->stream>>>(
-      nrow, R, entries_stream(nnz, sizeof(T) + sizeof(int)), rp, ci, val, x, y);
+      nrow, R, entries_cached_once(nnz, sizeof(T) + sizeof(int), sizeof(T) * ((size_t)nrow + ncol)), rp,
+      ci, val, x, y);
   HFLMP_LAUNCH_CHECK(ctx);
   return HFLMP_OK;
 }

@@ -3,7 +3,7 @@
 //
 // One workgroup (256 threads) owns a tile of consecutive rows [r0, r1).
 // The tile's nonzeros are one contiguous range of col/val, so the whole
-// workgroup streams that range with coalesced non-temporal loads, gathers
+// workgroup streams that range with coalesced loads, gathers
 // x[col] through the cache (the banded FE stencil reuses every x entry
 // from L2), and stores the rounded products val*x in LDS.  Then thread t
 // adds the products of row r0+t from LDS in ascending storage order,
