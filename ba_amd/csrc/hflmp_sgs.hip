@@ -331,8 +331,15 @@ int build_packed(hflmp_ctx *ctx, const Blocks &blk, const int *h_rp, const int *
       rows[(size_t)l * W + t] = make_int4(i, e, d0, d1);
     }
   if (hipMalloc(&s.prow, sizeof(int4) * rows.size()) != hipSuccess ||
-      hipMalloc(&s.pent, sizeof(int2) * ent.size()) != hipSuccess)
-    return set_error(ctx, HFLMP_ENOMEM, "sgs_create: out of device memory");
+      hipMalloc(&s.pent, sizeof(int2) * ent.size()) != hipSuccess) {
+    // no room for the copy: the segments run
+    (void)hipGetLastError();
+    (void)hipFree(s.prow);
+    (void)hipFree(s.pent);
+    s.prow = nullptr;
+    s.pent = nullptr;
+    return HFLMP_OK;
+  }
   HFLMP_HIP_CHECK(ctx, hipMemcpy(s.prow, rows.data(), sizeof(int4) * rows.size(),
                                  hipMemcpyHostToDevice));
   HFLMP_HIP_CHECK(ctx, hipMemcpy(s.pent, ent.data(), sizeof(int2) * ent.size(),
