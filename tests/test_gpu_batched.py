@@ -168,3 +168,41 @@ def test_batched_pcg_plan_matches_csr_form(ctx):
     with pytest.raises(hflmp.HflmpError):
         hflmp.batched_pcg_jacobi(ctx, A, invd, dB, dX2, k, rtol=1e-8, maxit=5000, plan=P2)
     P.free(); P2.free(); A2.free(); A.free()
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 31, 32, 33, 63])
+def test_batched_pcg_column_counts(ctx, k):
+    """Rows side by side in the vector updates (64 // k of them, the last
+    group partial) and columns that stop at different iterations: each column
+    is the oracle's solve of it alone."""
+    rp, ci, v = hflmp.fe_system(1, 2, 13, hflmp.fe_kappa(2, 13, 1.0, k))
+    N = len(rp) - 1                                  # 196 rows
+    # zero on the boundary, whose rows are not symmetric (the oracle's CG does
+    # not converge otherwise either); every third column a single entry
+    B = np.stack([hflmp.fe_rhs(1, 2, 13, 100 + c) for c in range(k)], axis=1)
+    inner = np.flatnonzero(B[:, 0])
+    for c in range(0, k, 3):
+        B[:, c] = 0.0
+        B[inner[7 * c % len(inner)], c] = 1.0
+    if k > 1:
+        B[:, 1] = 0.0
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    invd = hflmp.invdiag(ctx, A)
+    for planned in (False, True):
+        dB, dX = ctx.upload(B.ravel()), ctx.zeros(N * k, np.float64)
+        P = hflmp.SpmmPlan(ctx, A, k) if planned else None
+        info = hflmp.batched_pcg_jacobi(ctx, A, invd, dB, dX, k, rtol=1e-10, maxit=2000, plan=P)
+        X = dX.download().reshape(N, k)
+        for c in range(k):
+            b = np.ascontiguousarray(B[:, c])
+            xo, io = O.cg(rp, ci, v, b, prec=O.PREC_JACOBI, rtol=1e-10, maxit=2000)
+            assert info["status"][c] == 0 and abs(info["iters"][c] - io["iters"]) <= 2
+            # both residuals are at most 1e-10 |b|; |A^-1| |b| <= cond |x|
+            res = b - O.spmv(rp, ci, v, np.ascontiguousarray(X[:, c]))
+            assert np.linalg.norm(res) <= 2e-10 * np.linalg.norm(b)
+            assert np.linalg.norm(X[:, c] - xo) <= 1e-7 * np.linalg.norm(xo)
+        assert k == 1 or info["iters"][1] == 0
+        for a in (dB, dX) + ((P,) if planned else ()):
+            a.free()
+    A.free()
+    invd.free()
