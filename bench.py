@@ -1229,8 +1229,9 @@ def main():
                               "traffic": tr16,
                               "hbm_GBps_measured_traffic": round(tr16 / t_16 / 1e9, 2)
                               if tr16 else None,
-                              "note": "compressed (int16 column offsets, 10 B per nonzero; the "
-                                      "layout HIP_CSR_lMatrix builds when every column fits); "
+                              "note": "compressed (the layout HIP_CSR_lMatrix builds: one "
+                                      "offset per slice and position where a slice's rows share "
+                                      "them, 8 B per nonzero, else int16 column offsets, 10 B); "
                                       "scored with the CSR bytes"}
 
     if not args.no_parity:
