@@ -239,39 +239,8 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // Row i's values: zero, then for each (cell, local index a) of the node in
-// ascending order and each local column b, val[(i, dof b)] += term.
-template <typename T>
-__device__ __forceinline__ void fe_row_values(int i, int nloc, const int *__restrict__ dofs,
-                                              const int *__restrict__ off,
-                                              const long long *__restrict__ inc,
-                                              const T *__restrict__ cell_mats,
-                                              const T *__restrict__ E,
-                                              const T *__restrict__ factor,
-                                              const int *__restrict__ row_ptr,
-                                              const int *__restrict__ col, T *val) {
-#pragma clang fp contract(off)
-  const int r0 = row_ptr[i], r1 = row_ptr[i + 1];
-  for (int p = r0; p < r1; ++p) val[p] = T(0);
-  for (int k = off[i]; k < off[i + 1]; ++k) {
-    const long long c = inc[k] / kMaxLoc;
-    const int a = (int)(inc[k] % kMaxLoc);
-    const int *cd = dofs + c * nloc;
-    const T f = factor ? factor[c] : T(1);
-    const T *Er = cell_mats ? cell_mats + (c * nloc + a) * nloc : E + a * nloc;
-    for (int b = 0; b < nloc; ++b) {
-      const int j = cd[b];
-      int lo = r0, hi = r1 - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (col[mid] < j) lo = mid + 1;
-        else hi = mid;
-      }
-      const T term = cell_mats ? Er[b] : f * Er[b];
-      val[lo] += term;
-    }
-  }
-}
-
+// ascending order and each local column b, val[(i, dof b)] += term.  One
+// thread a row.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     fe_values_kernel(int nnode, int nloc, const int *__restrict__ dofs,
@@ -279,18 +248,45 @@ __global__ void __launch_bounds__(kBlock)
                      const T *__restrict__ cell_mats, const T *__restrict__ E,
                      const T *__restrict__ factor, const int *__restrict__ row_ptr,
                      const int *__restrict__ col, T *__restrict__ val) {
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nnode; i += gridDim.x * kBlock)
-    fe_row_values<T>(i, nloc, dofs, off, inc, cell_mats, E, factor, row_ptr, col, val);
+#pragma clang fp contract(off)
+  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nnode; i += gridDim.x * kBlock) {
+    const int r0 = row_ptr[i], r1 = row_ptr[i + 1];
+    for (int p = r0; p < r1; ++p) val[p] = T(0);
+    for (int k = off[i]; k < off[i + 1]; ++k) {
+      const long long c = inc[k] / kMaxLoc;
+      const int a = (int)(inc[k] % kMaxLoc);
+      const int *cd = dofs + c * nloc;
+      const T f = factor ? factor[c] : T(1);
+      const T *Er = cell_mats ? cell_mats + (c * nloc + a) * nloc : E + a * nloc;
+      for (int b = 0; b < nloc; ++b) {
+        const int j = cd[b];
+        int lo = r0, hi = r1 - 1;
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (col[mid] < j) lo = mid + 1;
+          else hi = mid;
+        }
+        const T term = cell_mats ? Er[b] : f * Er[b];
+        val[lo] += term;
+      }
+    }
+  }
 }
 
 // The same with G >= nloc lanes a row, lane b on local column b, the row's
 // columns and sums in LDS: a cell's terms go to different columns (no cell
 // repeats a dof: the caller checks), so they are added side by side, and
-// cell after cell keeps each column's order.  Rows longer than kFeRow
-// entries go to one lane, as above.  With one thread a row every add was a
-// read and a write of memory behind a search through memory: 4.88 ms on
+// cell after cell keeps each column's order.  With one thread a row every add
+// was a read and a write of memory behind a search through memory: 4.88 ms on
 // 96^3 Q1 cells (24.1 M values), 0.22 ms with groups of 8.
-constexpr int kFeRow = 32;
+// LDS holds kFeRow entries of a row: as elements of more nodes have longer
+// rows, it follows the group (27 entries for 3D Q1, 49 for 2D Q3, 125 for 3D
+// Q2).  The group adds a longer row's terms in memory, a search and an add a
+// lane and cell.  32^3 3D Q2 cells (17.0 M values): 2.07 ms with one thread a
+// row, 3.81 with 32 entries in LDS and one lane for longer rows, 0.138 here;
+// 128^2 2D Q3 cells (3.7 M values) 0.20, 0.226, 0.027 ms.
+template <int G>
+constexpr int kFeRow = G <= 8 ? 32 : 4 * G;
 
 template <typename T, int G>
 __global__ void __launch_bounds__(kBlock)
@@ -298,12 +294,18 @@ __global__ void __launch_bounds__(kBlock)
                            const int *__restrict__ off, const long long *__restrict__ inc,
                            const T *__restrict__ cell_mats, const T *__restrict__ E,
                            const T *__restrict__ factor, const int *__restrict__ row_ptr,
-                           const int *__restrict__ col, T *__restrict__ val) {
+                           const int *__restrict__ col, T *val) {
 #pragma clang fp contract(off)
   constexpr int R = kBlock / G;  // rows of a workgroup
-  __shared__ T acc[R][kFeRow + 1];
-  __shared__ int cols[R][kFeRow + 1];
+  constexpr int W = kFeRow<G>;
+  __shared__ T acc[R][W + 1];
+  __shared__ int cols[R][W + 1];
   const int g = threadIdx.x / G, b = threadIdx.x % G;
+  // what the group's lanes have written is what they read next
+  auto in_order = []() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   // whole waves leave the loop together: a group's lanes are in one wave
   for (long long i0 = (long long)blockIdx.x * R; i0 < nnode; i0 += (long long)gridDim.x * R) {
     const long long il = i0 + g;
@@ -311,38 +313,56 @@ __global__ void __launch_bounds__(kBlock)
     const int r0 = row_ptr[i];
     const int n = il < nnode ? row_ptr[i + 1] - r0 : 0;
     const int k0 = off[i], k1 = il < nnode ? off[i + 1] : k0;
-    if (n > kFeRow) {
-      if (b == 0) fe_row_values<T>(i, nloc, dofs, off, inc, cell_mats, E, factor, row_ptr, col, val);
-      continue;
-    }
-    for (int p = b; p < n; p += G) {
-      cols[g][p] = col[r0 + p];
-      acc[g][p] = T(0);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    for (int k = k0; k < k1; ++k) {
-      if (b < nloc) {
-        const long long key = inc[k];
-        const long long c = key / kMaxLoc;
-        const int a = (int)(key % kMaxLoc);
-        const int j = dofs[c * nloc + b];
-        const T term = cell_mats ? cell_mats[(c * nloc + a) * nloc + b]
-                                 : (factor ? factor[c] : T(1)) * E[a * nloc + b];
-        // the last column not above j is j itself
-        int p = 0;
-#pragma unroll
-        for (int s = kFeRow / 2; s > 0; s >>= 1)
-          if (p + s < n && cols[g][p + s] <= j) p += s;
-        acc[g][p] += term;
+    // add(j, term) for each cell in turn, lane b's column and term
+    auto cells = [&](auto add) {
+      for (int k = k0; k < k1; ++k) {
+        if (b < nloc) {
+          const long long key = inc[k];
+          const long long c = key / kMaxLoc;
+          const int a = (int)(key % kMaxLoc);
+          const int j = dofs[c * nloc + b];
+          add(j, cell_mats ? cell_mats[(c * nloc + a) * nloc + b]
+                           : (factor ? factor[c] : T(1)) * E[a * nloc + b]);
+        }
+        in_order();
       }
-      // the next cell's adds see this one's
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+    };
+    if (n > W) {
+      for (int p = b; p < n; p += G) val[r0 + p] = T(0);
+      in_order();
+      cells([&](int j, T term) {
+        int lo = r0, hi = r0 + n - 1;
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (col[mid] < j) lo = mid + 1;
+          else hi = mid;
+        }
+        val[lo] += term;
+      });
+    } else {
+      for (int p = b; p < n; p += G) {
+        cols[g][p] = col[r0 + p];
+        acc[g][p] = T(0);
+      }
+      in_order();
+      auto sum = [&](auto top) {
+        cells([&](int j, T term) {
+          // the last column not above j is j itself
+          int p = 0;
+#pragma unroll
+          for (int s = decltype(top)::value; s > 0; s >>= 1)
+            if (p + s < n && cols[g][p + s] <= j) p += s;
+          acc[g][p] += term;
+        });
+      };
+      // a wave without longer rows searches in five steps
+      if (W > 32 && __any(n > 32))
+        sum(std::integral_constant<int, W / 2>());
+      else
+        sum(std::integral_constant<int, 16>());
+      for (int p = b; p < n; p += G) val[r0 + p] = acc[g][p];
+      in_order();
     }
-    for (int p = b; p < n; p += G) val[r0 + p] = acc[g][p];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
   }
 }
 

@@ -4,6 +4,8 @@ pattern and values bit-identical for the structured Q1/Q2 meshes (and,
 with the Dirichlet rows applied, equal to the generator's matrix), for
 random unstructured meshes with per-cell matrices, FP64 and FP32, and the
 refusals."""
+import time
+
 import numpy as np
 import pytest
 
@@ -107,3 +109,61 @@ def test_group_widths_and_row_lengths(ctx, dtype, nnode, ncell, nloc, repeat):
             assert np.array_equal(rp, ro) and np.array_equal(ci, co) and np.array_equal(v, vo)
     finally:
         mesh.free()
+
+
+def _best_seconds(ctx, f, n=7):
+    f()
+    best = np.inf
+    for _ in range(n):
+        ctx.sync()
+        t0 = time.perf_counter()
+        f()
+        ctx.sync()
+        best = min(best, time.perf_counter() - t0)
+    return best
+
+
+def _device_assemble(ctx, mesh, E):
+    """A call that assembles the mesh's values from E on the device alone."""
+    rp, ci = mesh.pattern()
+    val, dE = ctx.empty(mesh.nnz, np.float64), ctx.upload(E)
+    return (lambda: hflmp._call(ctx, "hflmp_fe_assemble_f64", mesh.h, None, dE.ptr, None,
+                                rp.ptr, ci.ptr, val.ptr)), (rp, ci, val, dE)
+
+
+@pytest.mark.parametrize("nnode,ncell,nloc", [
+    (33, 40, 4), (64, 40, 16), (65, 40, 16), (65, 40, 9),
+    (128, 40, 32), (129, 40, 32), (129, 40, 17), (400, 60, 32),
+])
+def test_rows_around_the_lds_row(ctx, nnode, ncell, nloc):
+    """Rows as long as a group's LDS row, one entry longer and much longer,
+    and one node in every cell."""
+    rng = np.random.default_rng(nnode * 100 + nloc)
+    dofs = np.stack([np.append(0, 1 + rng.choice(nnode - 1, nloc - 1, replace=False))
+                     for _ in range(ncell)]).astype(np.int32)
+    mats = rng.uniform(-1, 1, (ncell, nloc, nloc))
+    mesh = hflmp.FeMesh(ctx, nnode, dofs)
+    try:
+        rp, ci, v = _device_csr(ctx, mesh, cell_mats=mats)
+    finally:
+        mesh.free()
+    ro, co, vo = O.fe_assemble_cells(nnode, dofs, cell_mats=mats)
+    assert np.array_equal(rp, ro) and np.array_equal(ci, co) and np.array_equal(v, vo)
+
+
+def test_long_rows_keep_their_lanes(ctx):
+    """Rows of up to 125 entries (3D Q2) are no slower than by one thread a
+    row, the path of a mesh with a dof twice in a cell."""
+    rng = np.random.default_rng(1)
+    dofs = hflmp.fe_cell_dofs(2, 3, 20)
+    N, nloc = 41 ** 3, dofs.shape[1]
+    E = rng.uniform(-1, 1, (nloc, nloc))
+    t = []
+    for d in (dofs, np.concatenate([dofs, np.zeros((1, nloc), np.int32)])):
+        mesh = hflmp.FeMesh(ctx, N, d)
+        f, arrays = _device_assemble(ctx, mesh, E)
+        t.append(_best_seconds(ctx, f))
+        for a in arrays:
+            a.free()
+        mesh.free()
+    assert t[0] <= t[1], "%.0f us against %.0f" % (t[0] * 1e6, t[1] * 1e6)
