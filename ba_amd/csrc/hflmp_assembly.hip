@@ -165,30 +165,77 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// Ascending bitonic sort of one value a lane across the wave.
-__device__ __forceinline__ int wave_sort(int v) {
+// Ascending bitonic sort of V values a lane across the wave: value u of a
+// lane has index 64 u + lane.
+template <int V>
+__device__ __forceinline__ void wave_sort(int (&v)[V]) {
   const int lane = threadIdx.x & (kWave - 1);
 #pragma unroll
-  for (int k = 2; k <= kWave; k <<= 1)
+  for (int k = 2; k <= V * kWave; k <<= 1)
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const int w = __shfl_xor(v, j);
-      const bool low = ((lane & k) == 0) == ((lane & j) == 0);
-      v = low ? (w < v ? w : v) : (w > v ? w : v);
+    for (int j = k >> 1; j > 0; j >>= 1)
+#pragma unroll
+      for (int u = 0; u < V; ++u) {
+        if (j < kWave) {
+          const int w = __shfl_xor(v[u], j);
+          const bool up = ((u * kWave + lane) & k) == 0;
+          v[u] = up == ((lane & j) == 0) ? (w < v[u] ? w : v[u]) : (w > v[u] ? w : v[u]);
+        } else if ((u & (j / kWave)) == 0) {  // both values are this lane's
+          const int q = u | (j / kWave), x = v[u], y = v[q];
+          const bool up = ((u * kWave) & k) == 0;
+          v[u] = up == (x < y) ? x : y;
+          v[q] = up == (x < y) ? y : x;
+        }
+      }
+}
+
+// Distinct dofs of a row's m cells (incidences from lo) in ascending order,
+// at most 64 V candidates: their number; WRITE stores them at out.
+template <bool WRITE, int V>
+__device__ __forceinline__ int fe_row_sorted(int lo, int m, int nloc, int lk, int lb,
+                                             const int *__restrict__ dofs,
+                                             const long long *__restrict__ inc,
+                                             int kstep, int bstep, int *__restrict__ out) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int d[V];
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    d[u] = INT_MAX;
+    if (lk < m) d[u] = dofs[(inc[lo + lk] / kMaxLoc) * nloc + lb];
+    lk += kstep;
+    lb += bstep;
+    if (lb >= nloc) {
+      lb -= nloc;
+      ++lk;
     }
-  return v;
+  }
+  wave_sort(d);
+  int n = 0, last = 0;
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    int before = __shfl_up(d[u], 1);
+    if (lane == 0) before = last;
+    last = __builtin_amdgcn_readlane(d[u], kWave - 1);
+    const bool first = d[u] != INT_MAX && ((u == 0 && lane == 0) || d[u] != before);
+    const unsigned long long firsts = __ballot(first);
+    if (WRITE && first) out[n + __popcll(firsts & ((1ull << lane) - 1))] = d[u];
+    n += __popcll(firsts);
+  }
+  return n;
 }
 
 // Distinct dofs of row i's cells in ascending order: WRITE = false counts
 // them into len[i], WRITE = true stores them at col + row_ptr[i].
 // One wave a row.  Its candidates (every local dof of every cell, 64 for 3D
-// Q1) are loaded at once, one a lane, and sorted across the wave; a lane
-// whose dof differs from its lower neighbour's has a column.  On 96^3 Q1
-// cells (912,673 rows) the passes take 0.26 and 0.29 ms; one thread a row
+// Q1, up to 216 for 3D Q2) are loaded at once and sorted across the wave; a
+// candidate that differs from its lower neighbour is a column.  On 96^3 Q1
+// cells (912,673 rows) the passes take 0.26 and 0.28 ms; one thread a row
 // with a repeated search for the next smallest dof (27 x 64 loads, each lane
 // elsewhere) took 3.4 ms, and broadcasting the candidates in turn instead of
-// the sort 0.9 and 1.4 ms.  Rows of more candidates search for the next
-// smallest with the whole wave.
+// the sort 0.9 and 1.4 ms.  Rows of more than 512 candidates search for the
+// next smallest with the whole wave.  32^3 Q2 cells (274,625 rows, 17.0 M
+// entries): 0.20 ms a pass; with that search for all rows of more than 64
+// candidates 4.0 ms, with one thread a row 3.7.
 template <bool WRITE>
 __global__ void __launch_bounds__(kBlock)
     fe_pattern_kernel(int nnode, int nloc, const int *__restrict__ dofs,
@@ -197,24 +244,38 @@ __global__ void __launch_bounds__(kBlock)
                       int *__restrict__ col) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const int lk = lane / nloc, lb = lane - lk * nloc;  // candidate of this lane
+  // candidate of this lane, and the way to the one 64 on
+  const int lk = lane / nloc, lb = lane - lk * nloc;
+  const int kstep = kWave / nloc, bstep = kWave - kstep * nloc;
   const int nwave = gridDim.x * (kBlock / kWave);
+  // two passes over the wave's rows, so that the sort of 64, which most meshes
+  // need alone, keeps its lane masks in registers (one pass for all: 5% slower
+  // on 3D Q1 cells, 13 to 20% on 2D ones)
+  bool more = false;
   for (int i = blockIdx.x * (kBlock / kWave) + wid; i < nnode; i += nwave) {
     const int lo = off[i], m = off[i + 1] - lo;
+    if ((long long)m * nloc > kWave) {
+      more = true;
+      continue;
+    }
+    const int n = fe_row_sorted<WRITE, 1>(lo, m, nloc, lk, lb, dofs, inc, kstep, bstep,
+                                          WRITE ? col + row_ptr[i] : nullptr);
+    if (!WRITE && lane == 0) len[i] = n;
+  }
+  if (!more) return;
+  for (int i = blockIdx.x * (kBlock / kWave) + wid; i < nnode; i += nwave) {
+    const int lo = off[i], m = off[i + 1] - lo;
+    const long long cand = (long long)m * nloc;
+    if (cand <= kWave) continue;
     int *out = WRITE ? col + row_ptr[i] : nullptr;
     int n = 0;
-    if ((long long)m * nloc <= kWave) {
-      const int cand = m * nloc;
-      int d = INT_MAX;
-      if (lane < cand) d = dofs[(inc[lo + lk] / kMaxLoc) * nloc + lb];
-      d = wave_sort(d);
-      const int before = __shfl_up(d, 1);
-      const bool first = d != INT_MAX && (lane == 0 || d != before);
-      const unsigned long long firsts = __ballot(first);
-      n = __popcll(firsts);
-      if (WRITE && first) out[__popcll(firsts & ((1ull << lane) - 1))] = d;
+    if (cand <= 2 * kWave) {
+      n = fe_row_sorted<WRITE, 2>(lo, m, nloc, lk, lb, dofs, inc, kstep, bstep, out);
+    } else if (cand <= 4 * kWave) {
+      n = fe_row_sorted<WRITE, 4>(lo, m, nloc, lk, lb, dofs, inc, kstep, bstep, out);
+    } else if (cand <= 8 * kWave) {
+      n = fe_row_sorted<WRITE, 8>(lo, m, nloc, lk, lb, dofs, inc, kstep, bstep, out);
     } else {
-      const long long cand = (long long)m * nloc;
       int last = -1;
       for (;;) {
         int next = INT_MAX;
@@ -223,11 +284,7 @@ __global__ void __launch_bounds__(kBlock)
           const int d = dofs[(inc[lo + k] / kMaxLoc) * nloc + b];
           if (d > last && d < next) next = d;
         }
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-          const int w = __shfl_xor(next, o);
-          next = w < next ? w : next;
-        }
+        next = wave_min(next);
         if (next == INT_MAX) break;
         if (WRITE && lane == 0) out[n] = next;
         ++n;

@@ -167,3 +167,45 @@ def test_long_rows_keep_their_lanes(ctx):
             a.free()
         mesh.free()
     assert t[0] <= t[1], "%.0f us against %.0f" % (t[0] * 1e6, t[1] * 1e6)
+
+
+@pytest.mark.parametrize("nloc,ncells", [
+    (4, (16, 17, 32, 33, 64, 65, 128, 129)),      # 64, 128, 256 and 512 candidates
+    (27, (2, 3, 4, 5, 9, 10, 18, 19)),            # and not multiples of them
+    (32, (2, 3, 4, 5, 8, 9, 16, 17)),
+    (1, (1, 64, 65, 513)),
+])
+def test_candidates_of_a_row(ctx, nloc, ncells):
+    """One node in a given number of cells, for the counts at which the
+    pattern's rows are built in another way; few and many repeats."""
+    rng = np.random.default_rng(nloc)
+    for ncell in ncells:
+        for nnode in (nloc + 1, 40000):
+            dofs = np.stack([np.append(nnode - 1, rng.choice(nnode - 1, nloc - 1, replace=False))
+                             for _ in range(ncell)]).astype(np.int32)
+            mesh = hflmp.FeMesh(ctx, nnode, dofs)
+            try:
+                rp, ci = mesh.pattern()
+                rpd, cid = rp.download(), ci.download()[:mesh.nnz]
+                rp.free()
+                ci.free()
+            finally:
+                mesh.free()
+            ro, co, _ = O.fe_assemble_cells(nnode, dofs, E=np.ones((nloc, nloc)),
+                                            factor=np.ones(ncell))
+            assert np.array_equal(rpd, ro) and np.array_equal(cid, co), (ncell, nnode)
+
+
+def test_long_pattern_rows_keep_their_speed(ctx):
+    """The pattern of rows of more than 64 candidates (3D Q2: up to 216) takes
+    less than five times as long per entry as that of rows of 64 (3D Q1)."""
+    per_entry = []
+    for order, n in ((1, 40), (2, 20)):
+        mesh = hflmp.FeMesh(ctx, 41 ** 3, hflmp.fe_cell_dofs(order, 3, n))
+        rp, ci = mesh.pattern()
+        per_entry.append(_best_seconds(ctx, lambda: hflmp._call(
+            ctx, "hflmp_fe_mesh_pattern", mesh.h, rp.ptr, ci.ptr)) / mesh.nnz)
+        rp.free()
+        ci.free()
+        mesh.free()
+    assert per_entry[1] < 5 * per_entry[0], per_entry
