@@ -126,14 +126,19 @@ __global__ void __launch_bounds__(kBlock)
   if (base + kScanPer >= n && base < n) off[n] = (int)run;  // the last value's thread
 }
 
-// off[0..n] = exclusive scan of cnt, *total (device, optional) = the sum;
-// tile_sum holds ceil(n / kScanTile) values
-void scan_exclusive(hipStream_t s, int n, const int *cnt, int *off, long long *tile_sum,
-                    long long *total) {
+// tile_sum (ceil(n / kScanTile) values) = the tiles' exclusive offsets,
+// *total (device, optional) = the sum of cnt
+void scan_tile_offsets(hipStream_t s, int n, const int *cnt, long long *tile_sum,
+                       long long *total) {
   const int ntiles = (n + kScanTile - 1) / kScanTile;
   scan_tiles_kernel<<<ntiles, kBlock, 0, s>>>(n, cnt, tile_sum);
   scan_offsets_kernel<<<1, kFinalBlock, 0, s>>>(ntiles, tile_sum, total);
-  scan_write_kernel<<<ntiles, kBlock, 0, s>>>(n, cnt, tile_sum, off);
+}
+
+// off[0..n] = exclusive scan of cnt
+void scan_exclusive(hipStream_t s, int n, const int *cnt, int *off, long long *tile_sum) {
+  scan_tile_offsets(s, n, cnt, tile_sum, nullptr);
+  scan_write_kernel<<<(n + kScanTile - 1) / kScanTile, kBlock, 0, s>>>(n, cnt, tile_sum, off);
 }
 
 __global__ void __launch_bounds__(kBlock)
@@ -490,7 +495,7 @@ int hflmp_fe_mesh_create(hflmp_ctx *ctx, int nnode, int ncell, int nloc, const i
     return set_error(ctx, code, "fe_mesh_create: %s", msg);
   };
   // one allocation (each costs the host about as long as these kernels
-  // run): the mesh's arrays, then what only the build needs
+  // run); the counts of the build lie where the row lengths will
   const size_t ntile = ((size_t)nnode + kScanTile - 1) / kScanTile;
   size_t bytes = 0;
   auto take = [&](size_t b) {
@@ -503,8 +508,6 @@ int hflmp_fe_mesh_create(hflmp_ctx *ctx, int nnode, int ncell, int nloc, const i
   const size_t o_inc = take(sizeof(long long) * (size_t)n);
   const size_t o_len = take(sizeof(int) * (size_t)nnode);
   const size_t o_tile = take(sizeof(long long) * ntile);
-  const size_t o_cnt = take(sizeof(int) * (size_t)nnode);
-  const size_t o_scratch = take(sizeof(int) * ((size_t)nnode + 1));
   const size_t o_total = take(sizeof(long long));
   if (hipMalloc(reinterpret_cast<void **>(&m->block), bytes) != hipSuccess)
     return fail(HFLMP_ENOMEM, "out of device memory");
@@ -513,8 +516,7 @@ int hflmp_fe_mesh_create(hflmp_ctx *ctx, int nnode, int ncell, int nloc, const i
   m->inc = reinterpret_cast<long long *>(m->block + o_inc);
   m->row_len = reinterpret_cast<int *>(m->block + o_len);
   m->tile_sum = reinterpret_cast<long long *>(m->block + o_tile);
-  int *cnt = reinterpret_cast<int *>(m->block + o_cnt);
-  int *scratch_off = reinterpret_cast<int *>(m->block + o_scratch);
+  int *cnt = m->row_len;
   long long *total = reinterpret_cast<long long *>(m->block + o_total);
   hipStream_t s = ctx->stream;
   unsigned int *bad = ctx->red_counter + 32;
@@ -535,15 +537,15 @@ int hflmp_fe_mesh_create(hflmp_ctx *ctx, int nnode, int ncell, int nloc, const i
   std::memcpy(hbad, ctx->host_pinned, sizeof(hbad));
   m->repeated = hbad[1] != 0;
   if (hbad[0]) return fail(HFLMP_EINVAL, "a cell dof is outside [0, nnode)");
-  scan_exclusive(s, nnode, cnt, m->inc_off, m->tile_sum, nullptr);
+  scan_exclusive(s, nnode, cnt, m->inc_off, m->tile_sum);
   if ((rc = hflmp_fill_zero(ctx, cnt, sizeof(int) * (size_t)nnode)) != HFLMP_OK)
     return fail(rc, "fill");
   fe_incidence_kernel<<<grid_n(n), kBlock, 0, s>>>(n, nloc, m->dofs, m->inc_off, cnt, m->inc);
   fe_sort_kernel<<<grid_n(nnode), kBlock, 0, s>>>(nnode, m->inc_off, m->inc);
   fe_pattern_kernel<false><<<grid_n((long long)nnode * kWave), kBlock, 0, s>>>(
       nnode, nloc, m->dofs, m->inc_off, m->inc, m->row_len, nullptr, nullptr);
-  // total pattern entries (of the scan only the sum is needed)
-  scan_exclusive(s, nnode, m->row_len, scratch_off, m->tile_sum, total);
+  // total pattern entries
+  scan_tile_offsets(s, nnode, m->row_len, m->tile_sum, total);
   long long nnz = 0;
   const bool ok = hipGetLastError() == hipSuccess &&
                   hipMemcpyAsync(&nnz, total, sizeof(nnz), hipMemcpyDeviceToHost, s) ==
@@ -567,7 +569,7 @@ int hflmp_fe_mesh_pattern(hflmp_ctx *ctx, const hflmp_fe_mesh *m, int *row_ptr, 
   HFLMP_REQUIRE(ctx, m && row_ptr && (m->nnz == 0 || col), "fe_mesh_pattern: null pointer");
   HFLMP_REQUIRE(ctx, m->device == ctx->device, "fe_mesh_pattern: mesh on another device");
   hipStream_t s = ctx->stream;
-  scan_exclusive(s, m->nnode, m->row_len, row_ptr, m->tile_sum, nullptr);
+  scan_exclusive(s, m->nnode, m->row_len, row_ptr, m->tile_sum);
   fe_pattern_kernel<true><<<grid_n((long long)m->nnode * kWave), kBlock, 0, s>>>(
       m->nnode, m->nloc, m->dofs, m->inc_off, m->inc, nullptr, row_ptr, col);
   HFLMP_LAUNCH_CHECK(ctx);

@@ -4,6 +4,7 @@ pattern and values bit-identical for the structured Q1/Q2 meshes (and,
 with the Dirichlet rows applied, equal to the generator's matrix), for
 random unstructured meshes with per-cell matrices, FP64 and FP32, and the
 refusals."""
+import ctypes as C
 import time
 
 import numpy as np
@@ -209,3 +210,22 @@ def test_long_pattern_rows_keep_their_speed(ctx):
         ci.free()
         mesh.free()
     assert per_entry[1] < 5 * per_entry[0], per_entry
+
+
+def _free_bytes():
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_mesh_keeps_only_its_arrays(ctx):
+    """A mesh holds two integers a node (offsets and row lengths) beside the
+    cells' arrays; what only its build needs is not kept."""
+    nnode = 40_000_000
+    hflmp.FeMesh(ctx, 8, np.arange(8, dtype=np.int32).reshape(1, 8)).free()
+    before = _free_bytes()
+    mesh = hflmp.FeMesh(ctx, nnode, np.arange(8, dtype=np.int32).reshape(1, 8))
+    held = before - _free_bytes()
+    mesh.free()
+    assert 8 * nnode <= held < 9 * nnode, held
