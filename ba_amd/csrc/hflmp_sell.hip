@@ -6,9 +6,10 @@
 // products y = A x and y += A x are those of CPU_CSR_lMatrix::VectorMult /
 // VectorMultAdd (CPUsimple_csr_lmatrix.cc:76-111, lmatrix_csr_cpu.cc:
 // 1424-1450), bit for bit.
+#include <algorithm>
 #include <climits>
 #include <cstdio>
-#include <utility>
+#include <cstring>
 
 #include "hflmp_sell.hpp"
 
@@ -17,27 +18,40 @@ namespace {
 enum SellMode { kSellAssign = 0, kSellAdd = 1 };
 
 struct SellStats {
-  unsigned int long_rows;  // rows longer than 255 entries
+  int long_rows;           // not 0: a row has more than 255 entries
   unsigned int bad16;      // entries whose offset from the slice start needs more than 16 bits
-  unsigned int bad_off;    // slices that the offset form cannot hold
-  unsigned int bad16_off;  // bad16 as the offset count saw it (all of it if bad_off is 0)
+  int sample;              // above 0: the offset form would be far too large
+  int bad_off;             // not 0: that, or a slice that the offset form cannot hold
+  int bad16_off;           // bad16 as the offset count saw it (all of it if bad_off is 0)
   int max_off;             // the largest |offset|
+  long long entries;       // of the form with columns
+  long long kentries;      // of the offset form
 };
+
+// The offset form is taken where its bytes are below this part of the
+// columns' (offset_form_smaller).
+constexpr double kOffsetGain = 0.95;
+
+__host__ __device__ inline double offset_form_bytes(double entries, int vb) {
+  return entries * (vb + 12.0 / kSellRows);
+}
+__host__ __device__ inline double column_form_bytes(double entries, double rows, int vb,
+                                                    int col_bytes) {
+  return entries * (vb + col_bytes) + rows;
+}
 
 // Row lengths (a byte each) and, per slice, the longest row (m; where its
 // entries sit is sell_pos's business).
 // Threads walk rows in whole waves, so a wave is always one slice.
 __global__ void __launch_bounds__(kBlock)
     sell_lengths_kernel(int nrow, int nslice, const int *__restrict__ rp,
-                        unsigned char *__restrict__ rlen, int *__restrict__ slen,
-                        SellStats *stats) {
+                        unsigned char *__restrict__ rlen, int *__restrict__ slen) {
   const long long total = (long long)nslice * kSellRows;
   for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < total;
        i += (long long)gridDim.x * kBlock) {
     int len = 0;
     if (i < nrow) {
       len = rp[i + 1] - rp[i];
-      if (len > 255) atomicAdd(&stats->long_rows, 1u);
       rlen[i] = (unsigned char)(len > 255 ? 255 : len);
     }
     int m = len;
@@ -50,38 +64,115 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// soff[s] = sum over t < s of 64 slen[t]; soff[nslice] = entries.  One
-// workgroup: each thread scans a contiguous run of slices.
+// What the offset count leaves for a slice.
+struct SliceOffsets {
+  int len;   // distinct offsets; -1: the form cannot hold the slice
+  int most;  // the largest |offset|, or kFar if a column is beyond int16
+};
+constexpr int kFar = INT_MAX;
+
+__device__ __forceinline__ int slice_len(int v) { return v; }
+__device__ __forceinline__ int slice_len(SliceOffsets v) { return v.len > 0 ? v.len : 0; }
+
+// soff[s] = sum over t < s of 64 slen[t]; soff[nslice] = all, the entries.
+// S = int (the longest rows) starts *stats, S = SliceOffsets adds what the
+// slices' counts say together.  One workgroup, eight consecutive slices a
+// thread and step (33,000 slices: 14 us; with one run of slices a thread 56).
+template <typename S>
 __global__ void __launch_bounds__(kFinalBlock)
-    sell_scan_kernel(int nslice, const int *__restrict__ slen, long long *__restrict__ soff) {
-  __shared__ long long tot[kFinalBlock];
-  const int t = threadIdx.x;
-  const int per = (nslice + kFinalBlock - 1) / kFinalBlock;
-  const int lo = t * per < nslice ? t * per : nslice;
-  const int hi = lo + per < nslice ? lo + per : nslice;
-  long long s = 0;
-  for (int k = lo; k < hi; ++k) s += (long long)kSellRows * slen[k];
-  tot[t] = s;
-  __syncthreads();
-  // inclusive Hillis-Steele scan of the per-thread totals
-  for (int o = 1; o < kFinalBlock; o <<= 1) {
-    const long long add = t >= o ? tot[t - o] : 0;
+    sell_scan_kernel(int nslice, const S *__restrict__ slen, long long *__restrict__ soff,
+                     SellStats *stats) {
+  constexpr int U = 8, kWaves = kFinalBlock / kWave;
+  constexpr bool OFFS = std::is_same<S, SliceOffsets>::value;
+  __shared__ int tot[kWaves];  // (a step has at most 8192 x 255 entries a row)
+  int most = 0;
+  bool far = false, bad = false;
+  const int t = threadIdx.x, lane = t & (kWave - 1), wid = t / kWave;
+  long long run = 0;  // entries before the step's slices
+  S next[U];
+  auto load = [&](long long s0) {
+    const long long s = s0 + (long long)t * U;
+    if (s + U <= nslice) {
+      __builtin_memcpy(next, __builtin_assume_aligned(slen + s, 16), sizeof(next));
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) next[u] = s + u < nslice ? slen[s + u] : S{};
+    }
+  };
+  load(0);
+  for (long long s0 = 0; s0 < nslice; s0 += (long long)kFinalBlock * U) {
+    int m[U], sum = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      m[u] = slice_len(next[u]);
+      sum += m[u];
+      if constexpr (OFFS) {
+        bad = bad || next[u].len < 0;
+        far = far || next[u].most == kFar;
+        most = next[u].most > most ? next[u].most : most;
+      } else {
+        bad = bad || m[u] > 255;
+      }
+    }
+    load(s0 + (long long)kFinalBlock * U);
+    int incl = sum;  // over the wave's lanes up to this one
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int v = __shfl_up(incl, o);
+      if (lane >= o) incl += v;
+    }
+    if (lane == kWave - 1) tot[wid] = incl;
     __syncthreads();
-    tot[t] += add;
+    int before = incl - sum, all = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      if (w < wid) before += tot[w];
+      all += tot[w];
+    }
+    long long at[U];
+    at[0] = run + (long long)kSellRows * before;
+#pragma unroll
+    for (int u = 1; u < U; ++u) at[u] = at[u - 1] + (long long)kSellRows * m[u - 1];
+    const long long s = s0 + (long long)t * U;
+    if (s + U <= nslice) {
+      __builtin_memcpy(__builtin_assume_aligned(soff + s, 16), at, sizeof(at));
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + u < nslice) soff[s + u] = at[u];
+    }
+    run += (long long)kSellRows * all;
     __syncthreads();
   }
-  long long run = tot[t] - s;
-  for (int k = lo; k < hi; ++k) {
-    soff[k] = run;
-    run += (long long)kSellRows * slen[k];
+  const int any_bad = __syncthreads_or(bad);
+  if constexpr (OFFS) {
+    const int any_far = __syncthreads_or(far);
+    most = -wave_min(-most);
+    if (lane == 0) tot[wid] = most;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) most = tot[w] > most ? tot[w] : most;
+    if (t == 0) {
+      stats->bad_off = any_bad;
+      stats->bad16_off = any_far;
+      stats->max_off = most;
+      stats->kentries = run;
+    }
+  } else if (t == 0) {
+    *stats = SellStats{};
+    stats->long_rows = any_bad;
+    stats->entries = run;
   }
-  if (t == kFinalBlock - 1) soff[nslice] = tot[t];
+  if (t == 0) soff[nslice] = run;
 }
 
-// Counts entries whose column is not within int16 of its slice's first row.
+// Counts entries whose column is not within int16 of its slice's first row
+// (AFTER_OFFSETS: unless the offset count has seen every entry).
+template <bool AFTER_OFFSETS>
 __global__ void __launch_bounds__(kBlock)
     sell_band_kernel(int nrow, const int *__restrict__ rp, const int *__restrict__ ci,
                      SellStats *stats) {
+  if (AFTER_OFFSETS && !stats->bad_off) return;
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < nrow; i += gridDim.x * kBlock) {
     const int base = (i / kSellRows) * kSellRows;
     unsigned int bad = 0;
@@ -125,86 +216,194 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- offset form ------------------------------------------------------------
-// Walks slice s (one wave, lane = row) over the distinct column offsets of
-// its rows in ascending order: f(position, offset, whether this lane's row
-// has the entry, its CSR index).  Returns the number of offsets, or -1 where
-// a row's columns do not ascend strictly or the slice has more than 255.
-template <typename F>
-__device__ __forceinline__ int for_slice_offsets(int s, int nrow, const int *__restrict__ rp,
-                                                 const int *__restrict__ ci, F &&f) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int row = s * kSellRows + lane;
-  int k = 0, end = 0;
-  if (row < nrow) {
-    k = rp[row];
-    end = rp[row + 1];
+// A slice's entries are read from LDS where it has at most so many (28 a
+// row), where one wave has copied them: a lane on its row of the arrays
+// itself reads 64 lines at a time, of which little is left in the caches when
+// it comes to the next entry (3D Q1 128^3 in FP64: count 0.59 -> 0.09 ms, fill
+// 2.08 -> 0.33 ms; the fill of the form with columns 1.7 ms).
+constexpr int kStageEntries = 28 * kSellRows;
+
+// what the wave's lanes have written to LDS is what they read next
+__device__ __forceinline__ void wave_in_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename V>
+__device__ __forceinline__ void stage_entries(V *lds, const V *__restrict__ src, int n) {
+  constexpr int U = 8;
+  wave_in_order();  // (the slice before is done with)
+  for (int e0 = threadIdx.x & (kWave - 1); e0 < n; e0 += U * kWave) {
+    V v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + u * kWave < n) v[u] = src[e0 + u * kWave];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + u * kWave < n) lds[e0 + u * kWave] = v[u];
   }
+  wave_in_order();
+}
+
+// The rows of slice s: this lane's CSR range [k, end) and the slice's [first,
+// last).
+struct SliceRows {
+  int row, k, end, first, last;
+};
+__device__ __forceinline__ SliceRows slice_rows(int s, int nrow, const int *__restrict__ rp) {
+  SliceRows r;
+  r.row = s * kSellRows + (threadIdx.x & (kWave - 1));
+  const int i = r.row < nrow ? r.row : nrow;
+  r.k = rp[i];
+  r.end = rp[r.row < nrow ? r.row + 1 : nrow];
+  r.first = __builtin_amdgcn_readfirstlane(r.k);
+  r.last = __builtin_amdgcn_readlane(r.end, kWave - 1);
+  return r;
+}
+
+// Walks a slice (one wave, lane = row) over the distinct column offsets of
+// its rows in ascending order: f(position, offset, whether this lane's row
+// has the entry, its CSR index), with the columns from col(CSR index).
+// Returns the number of offsets, or -1 where a row's columns do not ascend
+// strictly or go_on(position) is false.
+template <typename Col, typename G, typename F>
+__device__ __forceinline__ int for_slice_offsets(const SliceRows &r, Col &&col, G &&go_on,
+                                                 F &&f) {
+  int k = r.k;
   // the row's current offset and the next one, loaded a step ahead
-  int off = k < end ? ci[k] - row : INT_MAX;
-  int next = k + 1 < end ? ci[k + 1] - row : INT_MAX;
+  int off = k < r.end ? col(k) - r.row : INT_MAX;
+  int next = k + 1 < r.end ? col(k + 1) - r.row : INT_MAX;
   for (int j = 0;; ++j) {
     const int m = wave_min(off);
     if (m == INT_MAX) return j;
-    if (j == 255) return -1;
+    if (!go_on(j)) return -1;
     const bool has = off == m;
     f(j, m, has, k);
     bool bad = false;
     if (has) {
       ++k;
       off = next;
-      next = k + 1 < end ? ci[k + 1] - row : INT_MAX;
+      next = k + 1 < r.end ? col(k + 1) - r.row : INT_MAX;
       bad = off <= m;
     }
     if (__any(bad)) return -1;
   }
 }
 
-// klen[s] = the slice's distinct offsets; counts slices the form cannot hold.
+// One slice's walk with the columns staged where they fit; lds: kStageEntries.
+template <typename G, typename F>
+__device__ __forceinline__ int count_offsets(int s, int nrow, const int *__restrict__ rp,
+                                             const int *__restrict__ ci, int *lds, G &&go_on,
+                                             F &&see) {
+  const SliceRows r = slice_rows(s, nrow, rp);
+  if (r.last - r.first > kStageEntries)
+    return for_slice_offsets(r, [&](int k) { return ci[k]; }, go_on, see);
+  stage_entries(lds, ci + r.first, r.last - r.first);
+  return for_slice_offsets(r, [&](int k) { return lds[k - r.first]; }, go_on, see);
+}
+
+// Positions of a slice up to which the offset form is the smaller one.
+__device__ __forceinline__ int offset_share(int m, int vb) {
+  return (int)(kOffsetGain * column_form_bytes((double)kSellRows * m, kSellRows, vb, 4) /
+               offset_form_bytes(kSellRows, vb));
+}
+
+// A look at kSampleSlices of the slices, evenly spaced, before all are
+// counted: where they take more than twice their share of positions, the
+// form is out of question (an unstructured matrix takes hundreds of positions
+// a slice, 0.29 ms for 512^2 2D Q1 nodes in random order; the look takes 0.01).
+constexpr int kSampleSlices = 64;
+
+__global__ void __launch_bounds__(kBlock)
+    sell_offsets_sample_kernel(int nrow, int nslice, int vb, const int *__restrict__ rp,
+                               const int *__restrict__ ci, const int *__restrict__ slen,
+                               SellStats *stats) {
+  __shared__ int cols[kSellSlicesPerBlock][kStageEntries];
+  __shared__ int over;
+  if (threadIdx.x == 0) over = 0;
+  __syncthreads();
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int i = blockIdx.x * kSellSlicesPerBlock + wid;
+  const int n = nslice < kSampleSlices ? nslice : kSampleSlices;
+  if (i < n) {
+    const int s = (int)((long long)i * nslice / n);
+    const int share = offset_share(slen[s], vb);
+    const int K = count_offsets(s, nrow, rp, ci, cols[wid],
+                                [&](int j) { return j < 3 * share && j < 255; },
+                                [](int, int, bool, int) {});
+    if ((threadIdx.x & (kWave - 1)) == 0) atomicAdd(&over, (K < 0 ? 3 * share : K) - 2 * share);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(&stats->sample, over);
+}
+
+// The distinct offsets of each slice.
 __global__ void __launch_bounds__(kBlock)
     sell_offsets_count_kernel(int nrow, int nslice, const int *__restrict__ rp,
-                              const int *__restrict__ ci, int *__restrict__ klen,
-                              SellStats *stats) {
+                              const int *__restrict__ ci, SliceOffsets *__restrict__ klen,
+                              const SellStats *__restrict__ stats) {
+  __shared__ int cols[kSellSlicesPerBlock][kStageEntries];
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int lane = threadIdx.x & (kWave - 1);
+  const bool sampled_out = stats->sample > 0;
   for (int s = blockIdx.x * kSellSlicesPerBlock + wid; s < nslice;
        s += gridDim.x * kSellSlicesPerBlock) {
-    const int lane = threadIdx.x & (kWave - 1);
-    bool far = false;  // a column beyond int16 of the slice's first row
-    int most = 0;
-    const int K = for_slice_offsets(s, nrow, rp, ci, [&](int, int o, bool has, int) {
-      far = far || (has && (o + lane < -32768 || o + lane > 32767));
-      const int a = o < 0 ? -o : o;
-      most = a > most ? a : most;
-    });
-    if (lane == 0 && most > stats->max_off) atomicMax(&stats->max_off, most);
-    if (__any(far) && lane == 0) atomicAdd(&stats->bad16_off, 1u);
-    if (lane == 0) {
-      klen[s] = K < 0 ? 0 : K;
-      if (K < 0) atomicAdd(&stats->bad_off, 1u);
+    SliceOffsets out{-1, 0};
+    if (!sampled_out) {
+      bool far = false;
+      out.len = count_offsets(
+          s, nrow, rp, ci, cols[wid], [](int j) { return j < 255; },
+          [&](int, int o, bool has, int) {
+            far = far || (has && (o + lane < -32768 || o + lane > 32767));
+            const int a = o < 0 ? -o : o;
+            out.most = a > out.most ? a : out.most;
+          });
+      if (__any(far)) out.most = kFar;
     }
+    if (lane == 0) klen[s] = out;
   }
 }
 
+// One wave a workgroup: the LDS of more would leave fewer in flight.
 template <typename T>
-__global__ void __launch_bounds__(kBlock)
+__global__ void __launch_bounds__(kWave)
     sell_offsets_fill_kernel(int nrow, int nslice, int P, const int *__restrict__ rp,
                              const int *__restrict__ ci, const T *__restrict__ val,
-                             const long long *__restrict__ koff, const int *__restrict__ klen,
+                             const long long *__restrict__ koff,
+                             const SliceOffsets *__restrict__ klen,
+                             long long *__restrict__ soff, int *__restrict__ slen,
                              int *__restrict__ off, unsigned long long *__restrict__ mask,
                              T *__restrict__ sval) {
-  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
-  const int lane = threadIdx.x & (kWave - 1);
-  for (int s = blockIdx.x * kSellSlicesPerBlock + wid; s < nslice;
-       s += gridDim.x * kSellSlicesPerBlock) {
+  __shared__ T vals[kStageEntries];
+  __shared__ int cols[kStageEntries];
+  const int lane = threadIdx.x;
+  for (int s = blockIdx.x; s < nslice; s += gridDim.x) {
     const long long base = koff[s];
-    const int K = klen[s];
-    for_slice_offsets(s, nrow, rp, ci, [&](int j, int o, bool has, int k) {
-      const unsigned long long m = __ballot(has);
-      if (lane == 0) {
-        off[base / kSellRows + j] = o;
-        mask[base / kSellRows + j] = m;
-      }
-      sval[sell_pos(base, K, P, lane, j)] = has ? val[k] : T(0);
-    });
+    const int K = slice_len(klen[s]);
+    const SliceRows r = slice_rows(s, nrow, rp);
+    if (lane == 0) {
+      soff[s] = base;
+      slen[s] = K;
+      if (s == nslice - 1) soff[nslice] = koff[nslice];
+    }
+    auto walk = [&](auto col, auto value) {
+      for_slice_offsets(r, col, [](int) { return true; }, [&](int j, int o, bool has, int k) {
+        const unsigned long long m = __ballot(has);
+        if (lane == 0) {
+          off[base / kSellRows + j] = o;
+          mask[base / kSellRows + j] = m;
+        }
+        sval[sell_pos(base, K, P, lane, j)] = has ? value(k) : T(0);
+      });
+    };
+    const int n = r.last - r.first;
+    if (n <= kStageEntries) {
+      stage_entries(cols, ci + r.first, n);
+      stage_entries(vals, val + r.first, n);
+      walk([&](int k) { return cols[k - r.first]; }, [&](int k) { return vals[k - r.first]; });
+    } else {
+      walk([&](int k) { return ci[k]; }, [&](int k) { return val[k]; });
+    }
   }
 }
 
@@ -271,14 +470,8 @@ void sell_free(hflmp_sell *m) {
   int cur = -1;
   (void)hipGetDevice(&cur);
   if (cur != m->device) (void)hipSetDevice(m->device);
-  (void)hipFree(m->soff);
-  (void)hipFree(m->slen);
-  (void)hipFree(m->rlen);
-  (void)hipFree(m->col);
-  (void)hipFree(m->off);
-  (void)hipFree(m->mask);
-  (void)hipFree(m->val);
-  (void)hipFree(m->check);
+  (void)hipFree(m->meta);
+  (void)hipFree(m->data);
   if (cur >= 0 && cur != m->device) (void)hipSetDevice(cur);
   delete m;
 }
@@ -303,125 +496,123 @@ int sell_create(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   m->chunk = SellChunk<T>::P;
   m->value_bytes = sizeof(T);
   m->col_bytes = 4;
-  SellStats *stats = nullptr;
-  long long *koff = nullptr;  // the offset form's slices
-  int *klen = nullptr;
+  // Three allocations (each costs the host several microseconds): what the
+  // layout keeps a slice and row, what only the build needs, and the entries.
+  char *build = nullptr;
   int rc = HFLMP_OK;
   auto fail = [&](int code, const char *msg) {
-    (void)hipFree(stats);
-    (void)hipFree(koff);
-    (void)hipFree(klen);
+    (void)hipFree(build);
     sell_free(m);
     return set_error(ctx, code, "sell_create: %s", msg);
   };
-  if (hipMalloc(&m->soff, sizeof(long long) * ((size_t)m->nslice + 1)) != hipSuccess ||
-      hipMalloc(&m->slen, sizeof(int) * (size_t)m->nslice) != hipSuccess ||
-      hipMalloc(&m->rlen, (size_t)nrow) != hipSuccess ||
-      hipMalloc(&m->check, sizeof(unsigned int)) != hipSuccess ||
-      hipMalloc(&stats, sizeof(SellStats)) != hipSuccess)
-    return fail(HFLMP_ENOMEM, "out of device memory");
-  if ((rc = hflmp_fill_zero(ctx, stats, sizeof(SellStats))) != HFLMP_OK) return fail(rc, "fill");
-  const long long lanes = (long long)m->nslice * kSellRows;
-  long long g = (lanes + kBlock - 1) / kBlock;
-  if (g > 65536) g = 65536;
-  sell_lengths_kernel<<<(unsigned)g, kBlock, 0, s>>>(nrow, m->nslice, rp, m->rlen, m->slen,
-                                                     stats);
-  sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, m->slen, m->soff);
+  size_t bytes = 0;
+  auto take = [&](size_t b) {
+    const size_t at = bytes;
+    bytes += (b + 255) & ~size_t(255);
+    return at;
+  };
+  auto alloc = [&](char **p) {
+    const size_t b = bytes;
+    bytes = 0;
+    return hipMalloc(reinterpret_cast<void **>(p), b) == hipSuccess;
+  };
+  const size_t soff_bytes = sizeof(long long) * ((size_t)m->nslice + 1);
+  const size_t slen_bytes = sizeof(int) * (size_t)m->nslice;
+  const size_t o_soff = take(soff_bytes), o_slen = take(slen_bytes), o_rlen = take((size_t)nrow);
+  const size_t o_check = take(sizeof(unsigned int));
+  if (!alloc(&m->meta)) return fail(HFLMP_ENOMEM, "out of device memory");
+  m->soff = reinterpret_cast<long long *>(m->meta + o_soff);
+  m->slen = reinterpret_cast<int *>(m->meta + o_slen);
+  m->rlen = reinterpret_cast<unsigned char *>(m->meta + o_rlen);
+  m->check = reinterpret_cast<unsigned int *>(m->meta + o_check);
   // x is read through 32-bit byte offsets in the offset form
   const bool try_off = (flags & (HFLMP_SELL_COL16 | kSellOffsets)) && nnz > 0 &&
                        (size_t)ncol * sizeof(T) < (1ull << 31) &&
                        (size_t)nrow * sizeof(T) < (1ull << 31);
+  const bool try16 = (flags & HFLMP_SELL_COL16) && nnz > 0;
+  const size_t o_stats = take(sizeof(SellStats));
+  const size_t o_koff = take(try_off ? soff_bytes : 0),
+               o_klen = take(try_off ? sizeof(SliceOffsets) * (size_t)m->nslice : 0);
+  if (!alloc(&build)) return fail(HFLMP_ENOMEM, "out of device memory");
+  SellStats *stats = reinterpret_cast<SellStats *>(build + o_stats);
+  long long *koff = reinterpret_cast<long long *>(build + o_koff);  // the offset form's slices
+  auto *klen = reinterpret_cast<SliceOffsets *>(build + o_klen);
+  const long long lanes = (long long)m->nslice * kSellRows;
+  long long g = (lanes + kBlock - 1) / kBlock;
+  if (g > 65536) g = 65536;
+  sell_lengths_kernel<<<(unsigned)g, kBlock, 0, s>>>(nrow, m->nslice, rp, m->rlen, m->slen);
+  sell_scan_kernel<int><<<1, kFinalBlock, 0, s>>>(m->nslice, m->slen, m->soff, stats);
   if (try_off) {
-    if (hipMalloc(&koff, sizeof(long long) * ((size_t)m->nslice + 1)) != hipSuccess ||
-        hipMalloc(&klen, sizeof(int) * (size_t)m->nslice) != hipSuccess)
-      return fail(HFLMP_ENOMEM, "out of device memory");
+    sell_offsets_sample_kernel<<<kSampleSlices / kSellSlicesPerBlock, kBlock, 0, s>>>(
+        nrow, m->nslice, (int)sizeof(T), rp, ci, m->slen, stats);
     sell_offsets_count_kernel<<<grid_for(lanes, 1), kBlock, 0, s>>>(nrow, m->nslice, rp, ci, klen,
                                                                     stats);
-    sell_scan_kernel<<<1, kFinalBlock, 0, s>>>(m->nslice, klen, koff);
+    sell_scan_kernel<SliceOffsets><<<1, kFinalBlock, 0, s>>>(m->nslice, klen, koff, stats);
+    if (try16) sell_band_kernel<true><<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
+  } else if (try16) {
+    sell_band_kernel<false><<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
   }
-  const bool try16 = (flags & HFLMP_SELL_COL16) && nnz > 0;
-  if (try16 && !try_off)
-    sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
   if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
   SellStats hs;
-  long long entries = 0, kentries = 0;
-  if (hipMemcpyAsync(&hs, stats, sizeof(hs), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipMemcpyAsync(&entries, m->soff + m->nslice, sizeof(entries), hipMemcpyDeviceToHost,
-                     s) != hipSuccess ||
-      (try_off && hipMemcpyAsync(&kentries, koff + m->nslice, sizeof(kentries),
-                                 hipMemcpyDeviceToHost, s) != hipSuccess) ||
+  if (hipMemcpyAsync(ctx->host_pinned, stats, sizeof(hs), hipMemcpyDeviceToHost, s) !=
+          hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail(HFLMP_EHIP, "HIP error while sizing");
-  if (try16 && try_off) {
-    hs.bad16 = hs.bad16_off;
-    if (hs.bad_off) {  // the count left slices early: look at every column
-      sell_band_kernel<<<grid_for(nrow, 1), kBlock, 0, s>>>(nrow, rp, ci, stats);
-      if (hipGetLastError() != hipSuccess ||
-          hipMemcpyAsync(&hs, stats, sizeof(hs), hipMemcpyDeviceToHost, s) != hipSuccess ||
-          hipStreamSynchronize(s) != hipSuccess)
-        return fail(HFLMP_EHIP, "HIP error while sizing");
-    }
-  }
+  std::memcpy(&hs, ctx->host_pinned, sizeof(hs));
   if (hs.long_rows)
     return fail(HFLMP_EFORMAT, "a row has more than 255 entries (use the CSR kernels)");
   // Padding is never loaded (a lane stops at its row's length), but it
   // costs memory and partly-used cache lines; refuse more than twice the
   // nonzeros of it.
-  if (!(flags & HFLMP_SELL_ANY_PADDING) && entries > 3LL * nnz + (long long)kSellRows * m->chunk)
+  if (!(flags & HFLMP_SELL_ANY_PADDING) &&
+      hs.entries > 3LL * nnz + (long long)kSellRows * m->chunk)
     return fail(HFLMP_EFORMAT, "row lengths vary too much within slices (use the CSR kernels)");
-  m->entries = entries;
-  if (try16 && hs.bad16 == 0) m->col_bytes = 2;
-  // The offset form where it is at least 5% smaller than the columns' (the
-  // product's time follows its bytes): value padding up to a quarter of the
-  // nonzeros in FP64, about half in FP32.  Structured Q1 meshes pad by 1 to
-  // 2%; a Q2 mesh, whose rows alternate between three patterns, by 56%, and
-  // keeps its columns.
-  const double off_bytes = (double)kentries * (sizeof(T) + 12.0 / kSellRows);
-  const double col_bytes = (double)entries * (sizeof(T) + m->col_bytes) + nrow;
-  if (try_off && hs.bad_off == 0 && off_bytes < 0.95 * col_bytes) {
-    m->off_form = 1;
-    m->max_off = hs.max_off;
-    m->entries = kentries;
-    std::swap(m->soff, koff);
-    std::swap(m->slen, klen);
-    const size_t np = (size_t)kentries / kSellRows;
-    if (hipMalloc(&m->off, np * sizeof(int)) != hipSuccess ||
-        hipMalloc(&m->mask, np * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc(&m->val, (size_t)kentries * sizeof(T)) != hipSuccess)
-      return fail(HFLMP_ENOMEM, "out of device memory");
-    sell_offsets_fill_kernel<T><<<grid_for(lanes, 1), kBlock, 0, s>>>(
-        nrow, m->nslice, m->chunk, rp, ci, val, m->soff, m->slen, m->off, m->mask,
+  if (try16 && (try_off && !hs.bad_off ? hs.bad16_off : hs.bad16) == 0) m->col_bytes = 2;
+  // The offset form where it is at least 5% smaller than the columns': the
+  // product's time follows its bytes, up to that line.  3D Q1 96^3 with a
+  // quarter of the entries dropped at random, FP64 (1.33 stored values an
+  // entry, 10.96 B against 12.43): 44.4 us, with columns 49.6; with 40%
+  // dropped, FP32 (1.64, 6.96 B against 8.16): 19.0 and 29.8 us.
+  m->off_form = try_off && hs.bad_off == 0 &&
+                offset_form_bytes((double)hs.kentries, sizeof(T)) <
+                    kOffsetGain * column_form_bytes((double)hs.entries, nrow, sizeof(T),
+                                                    m->col_bytes);
+  m->entries = m->off_form ? hs.kentries : hs.entries;
+  m->max_off = hs.max_off;
+  const size_t ne = m->entries > 0 ? (size_t)m->entries : 1;
+  const size_t np = m->off_form ? ne / kSellRows : 0;  // positions
+  const size_t o_val = take(ne * sizeof(T));
+  const size_t o_col = take(m->off_form ? 0 : ne * m->col_bytes);
+  const size_t o_mask = take(np * sizeof(unsigned long long)), o_off = take(np * sizeof(int));
+  if (!alloc(&m->data)) return fail(HFLMP_ENOMEM, "out of device memory");
+  m->val = m->data + o_val;
+  if (m->off_form) {
+    m->mask = reinterpret_cast<unsigned long long *>(m->data + o_mask);
+    m->off = reinterpret_cast<int *>(m->data + o_off);
+    const int grid = std::min(m->nslice, 1 << 20);
+    sell_offsets_fill_kernel<T><<<grid, kWave, 0, s>>>(
+        nrow, m->nslice, m->chunk, rp, ci, val, koff, klen, m->soff, m->slen, m->off, m->mask,
         static_cast<T *>(m->val));
-    if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
-    if (hipStreamSynchronize(s) != hipSuccess) return fail(HFLMP_EHIP, "HIP error in build");
-    (void)hipFree(stats);
-    (void)hipFree(koff);
-    (void)hipFree(klen);
-    *out = m;
-    return HFLMP_OK;
-  }
-  const size_t ne = entries > 0 ? (size_t)entries : 1;
-  if (hipMalloc(&m->col, ne * m->col_bytes) != hipSuccess ||
-      hipMalloc(&m->val, ne * sizeof(T)) != hipSuccess)
-    return fail(HFLMP_ENOMEM, "out of device memory");
-  if ((rc = hflmp_fill_zero(ctx, m->col, ne * m->col_bytes)) != HFLMP_OK) return fail(rc, "fill");
-  if ((rc = hflmp_fill_zero(ctx, m->val, ne * sizeof(T))) != HFLMP_OK) return fail(rc, "fill");
-  if (nnz > 0) {
-    if (m->col_bytes == 2)
-      sell_fill_kernel<T, short, true><<<grid_for(nrow, 1), kBlock, 0, s>>>(
-          nrow, m->chunk, rp, ci, val, m->soff, m->slen, static_cast<short *>(m->col),
-          static_cast<T *>(m->val), nullptr, nullptr);
-    else
-      sell_fill_kernel<T, int, true><<<grid_for(nrow, 1), kBlock, 0, s>>>(
-          nrow, m->chunk, rp, ci, val, m->soff, m->slen, static_cast<int *>(m->col),
-          static_cast<T *>(m->val), nullptr, nullptr);
+  } else {
+    m->col = m->data + o_col;
+    if ((rc = hflmp_fill_zero(ctx, m->col, ne * m->col_bytes)) != HFLMP_OK)
+      return fail(rc, "fill");
+    if ((rc = hflmp_fill_zero(ctx, m->val, ne * sizeof(T))) != HFLMP_OK) return fail(rc, "fill");
+    if (nnz > 0) {
+      if (m->col_bytes == 2)
+        sell_fill_kernel<T, short, true><<<grid_for(nrow, 1), kBlock, 0, s>>>(
+            nrow, m->chunk, rp, ci, val, m->soff, m->slen, static_cast<short *>(m->col),
+            static_cast<T *>(m->val), nullptr, nullptr);
+      else
+        sell_fill_kernel<T, int, true><<<grid_for(nrow, 1), kBlock, 0, s>>>(
+            nrow, m->chunk, rp, ci, val, m->soff, m->slen, static_cast<int *>(m->col),
+            static_cast<T *>(m->val), nullptr, nullptr);
+    }
   }
   if (hipGetLastError() != hipSuccess) return fail(HFLMP_EHIP, "launch failed");
-  // the stats buffer is freed only after the stream has used it
+  // the build's memory is freed only after the stream has used it
   if (hipStreamSynchronize(s) != hipSuccess) return fail(HFLMP_EHIP, "HIP error in build");
-  (void)hipFree(stats);
-  (void)hipFree(koff);
-  (void)hipFree(klen);
+  (void)hipFree(build);
   *out = m;
   return HFLMP_OK;
 }

@@ -48,6 +48,7 @@ struct hflmp_sell {
   int col_bytes;    // 4 (absolute int32) or 2 (int16 offset from the slice's first row)
   int value_bytes;  // 8 or 4
   long long entries;
+  char *meta, *data;    // the two allocations behind the arrays below
   long long *soff;      // nslice + 1 entry offsets
   int *slen;            // longest row of each slice (m): the first m - m mod P entries of a
                         // row sit in chunks of P, the rest in one-entry-per-lane blocks

@@ -4,8 +4,11 @@ slices cut short, every remainder of offsets to a block of loads, rows that
 miss entries, offsets that point outside x for other rows of the slice,
 infinities and NaN where only a missing entry would read them, y += A x and
 new values -- and the general form for rows it cannot hold."""
+import time
+
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from ba_amd import hflmp
 from oracle import oracle as O
@@ -183,3 +186,69 @@ def test_solvers_same_bits_as_columns(ctx):
         A.free()
         invd.free()
         db.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_uneven_slices(ctx, dtype):
+    """A few slices of about 200 offsets beside plain ones: it is all slices
+    together that decide."""
+    rng = np.random.default_rng(3)
+    ns, plain = 40, np.arange(-4, 5)
+    forms = set()
+    for wild in range(0, 12):
+        pick = set(rng.choice(ns, wild, replace=False).tolist())
+        rows = []
+        for i in range(ns * 64):  # wild: rows in threes share their offsets
+            first = i + (i % 64 // 3 * 11 if i // 64 in pick else 0)
+            rows.append(np.unique(np.clip(first + plain, 0, ns * 64 - 1)))
+        rp = np.concatenate([[0], np.cumsum([len(q) for q in rows])]).astype(np.int32)
+        ci = np.concatenate(rows).astype(np.int32)
+        v = rng.uniform(-1, 1, len(ci)).astype(dtype)
+        off = expected(rp, ci, ns * 64, v.itemsize)[1]
+        forms.add(off)
+        check(ctx, rp, ci, v, ns * 64, off, seed=wild)
+    assert forms == {True, False}
+
+
+@pytest.mark.parametrize("nrow", [64 * 8192 - 1, 64 * 8192, 64 * 8192 + 1, 64 * 24580])
+def test_many_slices(ctx, nrow):
+    """The offsets of the slices, around the slices that the scan takes a
+    step (8192)."""
+    lens = np.random.default_rng(nrow).integers(0, 4, nrow)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    j = np.arange(rp[-1]) - np.repeat(rp[:-1], lens)
+    ci = np.minimum(np.repeat(np.arange(nrow), lens), nrow - 4).astype(np.int32) + j.astype(np.int32)
+    v = np.random.default_rng(1).uniform(-1, 1, len(ci))
+    x = np.random.default_rng(2).uniform(-1, 1, nrow)
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    dx, dy = ctx.upload(x), ctx.zeros(nrow, np.float64)
+    ref = O.spmv(rp, ci, v, x)
+    for flags in (hflmp.SELL_ANY_PADDING, hflmp.SELL_ANY_PADDING | hflmp.SELL_COL16):
+        S = hflmp.SellMatrix(ctx, A, flags)
+        S.spmv(dx, dy)
+        S.free()
+        assert np.array_equal(dy.download(), ref)
+    for a in (dx, dy, A):
+        a.free()
+
+
+def test_unstructured_build_keeps_its_speed(ctx):
+    """Looking for shared offsets costs an unstructured matrix, which has none,
+    less than the rest of its build (int32 columns, which do not look)."""
+    rng = np.random.default_rng(0)
+    rp, ci, v = hflmp.fe_system(1, 2, 300)
+    n = len(rp) - 1
+    p = rng.permutation(n)
+    B = sp.csr_matrix((v, ci, rp), shape=(n, n))[p][:, p].tocsr()
+    B.sort_indices()
+    A = hflmp.CsrMatrix(ctx, B.indptr.astype(np.int32), B.indices.astype(np.int32), B.data)
+    best = {}
+    for flags in (0, hflmp.SELL_COL16) * 12:
+        ctx.sync()
+        t0 = time.perf_counter()
+        S = hflmp.SellMatrix(ctx, A, flags)
+        ctx.sync()
+        best[flags] = min(best.get(flags, np.inf), time.perf_counter() - t0)
+        S.free()
+    A.free()
+    assert best[hflmp.SELL_COL16] < 2 * best[0], best
