@@ -27,6 +27,7 @@
 // is where the sequential sweep's separate D pass leaves the value (no row
 // reads another row's scaled value before that row's backward step).
 #include <algorithm>
+#include <new>
 #include <vector>
 
 #include "hflmp_internal.hpp"
@@ -283,10 +284,19 @@ void sgs_free(hflmp_sgs *m) {
   delete m;
 }
 
+// Bytes that a sweep's copy may take on the host and the device: what the
+// pattern and FP64 values take four times over, or 16 MB where that is more, and at
+// most 1 GB.  (The copy of 2D Q1 96^2 takes 0.9 of the CSR arrays, of 3D Q1
+// 32^3 as well; eight slots a row with 16 entries each are 1.2 KB a row,
+// where a row may have few entries.)
+inline size_t pack_limit(size_t nnz, size_t n) {
+  return std::min<size_t>(std::max<size_t>(4 * (12 * nnz + 4 * n), 16 << 20), 1 << 30);
+}
+
 // The level-ordered copy (see sgs_packed_kernel) where it fits: levels of at
-// most kPackRows rows, at most kPackMaxE entries a row, and no more than
-// about eight slots a row (levels of very uneven width would waste the
-// rest).  h_rp, h_ci: the pattern on the host.
+// most kPackRows rows, at most kPackMaxE entries a row, no more than about
+// eight slots a row (levels of very uneven width would waste the rest), and
+// within pack_limit.  h_rp, h_ci: the pattern on the host.
 int build_packed(hflmp_ctx *ctx, const Blocks &blk, const int *h_rp, const int *h_ci, bool fwd,
                  const std::vector<int> &off, const std::vector<int> &perm, Sweep &s) {
   const int n = (int)perm.size(), nlev = s.levels;
@@ -320,8 +330,15 @@ int build_packed(hflmp_ctx *ctx, const Blocks &blk, const int *h_rp, const int *
   const int E = pack_width(most);
   const int D = kPackMaxE / E;
   const size_t lv = (size_t)nlev + 4 * (size_t)D;  // empty levels at the end
-  std::vector<int4> rows(lv * W, make_int4(-1, 0, 0, 0));
-  std::vector<int2> ent(lv * E * W, make_int2(0, 0));
+  if (lv * W * (sizeof(int4) + E * sizeof(int2)) > pack_limit(h_rp[n], n)) return HFLMP_OK;
+  std::vector<int4> rows;
+  std::vector<int2> ent;
+  try {
+    rows.assign(lv * W, make_int4(-1, 0, 0, 0));
+    ent.assign(lv * E * W, make_int2(0, 0));
+  } catch (const std::bad_alloc &) {
+    return HFLMP_OK;  // no room for the copy: the segments run
+  }
   for (int l = 0; l < nlev; ++l)
     for (int k = off[l]; k < off[l + 1]; ++k) {
       const int i = perm[k], t = k - off[l];
@@ -332,7 +349,6 @@ int build_packed(hflmp_ctx *ctx, const Blocks &blk, const int *h_rp, const int *
     }
   if (hipMalloc(&s.prow, sizeof(int4) * rows.size()) != hipSuccess ||
       hipMalloc(&s.pent, sizeof(int2) * ent.size()) != hipSuccess) {
-    // no room for the copy: the segments run
     (void)hipGetLastError();
     (void)hipFree(s.prow);
     (void)hipFree(s.pent);

@@ -402,8 +402,10 @@ int hflmp_mcsgs_destroy(hflmp_ctx *ctx, hflmp_mcsgs *m);
  * create() analyses the pattern on the host (h_row_ptr/h_col: HOST copies
  * of it, or both NULL to download the DEVICE arrays) and keeps the DEVICE
  * row_ptr, col and val pointers, which must outlive the object; new values
- * are used without a rebuild.  HFLMP_EFORMAT if a row has no diagonal
- * entry.  r and z may be the same array. */
+ * are used without a rebuild.  Sweeps of levels of at most 512 rows keep
+ * a copy of the pattern in level order: at most four times the bytes of the
+ * pattern with FP64 values, or 16 MB, for each of the two.  HFLMP_EFORMAT
+ * if a row has no diagonal entry.  r and z may be the same array. */
 typedef struct hflmp_sgs hflmp_sgs;
 typedef struct {
   int nrow, num_blocks;

@@ -6,8 +6,11 @@ counts, unsorted rows and FP32; then through the unchanged CG template
 (Init_SymmetricGaussSeidel / the block preconditioner) against the oracle's
 CG with the same preconditioner: iterations within 2, solution within
 1e-8."""
+import ctypes as C
+
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 from ba_amd import hflmp
 from oracle import oracle as O
@@ -162,3 +165,40 @@ def test_lmp_cg_sgs_vs_oracle(prec, nb):
     # SGS preconditions better than Jacobi on this system
     _, ij = O.cg(rp, ci, v, b, prec=O.PREC_JACOBI, rtol=1e-8, maxit=2000)
     assert io["iters"] < ij["iters"]
+
+
+def _free_bytes():
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_level_copy_is_bounded(ctx):
+    """Levels of 64 rows beside one of 512, rows of two entries beside one of
+    17: the level-ordered copy would be 30 times the matrix, so the sweeps run
+    without it, with the same bits."""
+    n = 100_000
+    rows = [[i] if i < 512 else [i - 64, i] for i in range(n)]
+    rows[5000] = list(range(4984, 5000)) + [5000]
+    rp = np.concatenate([[0], np.cumsum([len(q) for q in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    A = sp.csr_matrix((np.ones(len(ci)), ci, rp), shape=(n, n))
+    A = (A + A.T).tocsr()
+    A.sort_indices()
+    rp, ci = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+    rng = np.random.default_rng(4)
+    v = np.where(np.repeat(np.arange(n), np.diff(rp)) == ci, 4.0, rng.uniform(-1, 1, len(ci)))
+    r = rng.uniform(-1, 1, n)
+    _apply(ctx, rp[:601], ci[:rp[600]] % 600, v[:rp[600]], r[:600])  # (kernels loaded)
+    M = hflmp.CsrMatrix(ctx, rp, ci, v)
+    dr, dz = ctx.upload(r), ctx.empty(n, np.float64)
+    before = _free_bytes()
+    S = hflmp.Sgs(ctx, M, 1, host_pattern=(rp, ci))
+    held = before - _free_bytes()
+    S.apply(dr, dz)
+    S.destroy()
+    assert np.array_equal(dz.download(), O.sgs_apply(rp, ci, v, r))
+    for a in (dr, dz, M):
+        a.free()
+    assert held <= 2 * max(16 << 20, 4 * (12 * len(ci) + 4 * n)) + (8 << 20), held
