@@ -252,3 +252,123 @@ def test_unstructured_build_keeps_its_speed(ctx):
         S.free()
     A.free()
     assert best[hflmp.SELL_COL16] < 2 * best[0], best
+
+
+def _solve(ctx, A, flags, invd, b, short=0, **kw):
+    """x and info of Jacobi-CG over the layout; short: bytes left out of the
+    workspace."""
+    S = hflmp.SellMatrix(ctx, A, flags)
+    need = ctx.L.hflmp_pcg_workspace_bytes(S.nrow, S.nnz, S.dtype.itemsize)
+    work, db, dx = ctx.empty(need - short, np.uint8), ctx.upload(b), ctx.zeros(A.nrow, b.dtype)
+    try:
+        info = hflmp.pcg_jacobi_sell(ctx, S, invd, db, dx, work=work, **kw)
+        return dx.download(), info["iters"], info["status"], info["res_final"]
+    finally:
+        for a in (work, db, dx, S):
+            a.free()
+
+
+def _assert_same(got, want):
+    assert got[1:] == want[1:] and np.array_equal(got[0], want[0])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("dim,n", [(2, 120), (3, 24)])
+def test_two_launch_stops(ctx, dtype, dim, n):
+    """More rows than one workgroup takes, so the offset form runs two launches
+    an iteration: stopped at odd and even iterations by maxit (the host polls
+    every 16) and by dtol, converged, started at the solution, and in a
+    workspace without the second p, it leaves what three launches over int32
+    columns leave."""
+    rp, ci, v = hflmp.fe_system(1, dim, n, hflmp.fe_kappa(dim, n, 1.0, 2))
+    assert len(rp) - 1 > 8192 and expected(rp, ci, len(rp) - 1, np.dtype(dtype).itemsize)[1]
+    A = hflmp.CsrMatrix(ctx, rp, ci, v.astype(dtype))
+    invd = hflmp.invdiag(ctx, A)
+    b = (hflmp.fe_rhs(1, dim, n, 3) != 0).astype(dtype)  # whose residual grows at first
+    rtol = 1e-8 if dtype == np.float64 else 1e-4
+    runs = [(1, dict(maxit=m, rtol=0.0, dtol=1e30)) for m in (1, 2, 3, 15, 16, 17, 32, 33)]
+    runs += [(2, dict(dtol=t, rtol=rtol)) for t in ((2.0, 3.0, 4.5) if dim == 2 else (1.5, 1.9))]
+    runs += [(0, dict(rtol=rtol, dtol=1e30)), (0, dict(rtol=rtol, atol=1e6))]
+    iters = set()
+    for status, kw in runs:
+        want = _solve(ctx, A, 0, invd, b, **kw)
+        assert want[2] == status
+        iters.add(want[1])
+        _assert_same(_solve(ctx, A, hflmp.SELL_COL16, invd, b, **kw), want)
+        _assert_same(_solve(ctx, A, hflmp.SELL_COL16, invd, b, short=256, **kw), want)
+    assert 0 in iters and {k % 2 for k in iters} == {0, 1}
+    A.free()
+    invd.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("block,rhs,iters", [
+    ([[1]], [1], 0),                                                    # every other row -1
+    ([[1, -1, -1], [-1, 1, 0], [-1, 0, 2]], [0, 2, 0], 1),
+    ([[1, 0, -1], [0, 1, 0], [-1, 0, 1]], [2, -2, 0], 2),
+    ([[-1, 1, 0, -1], [1, 1, -2, 1], [0, -2, 2, 0], [-1, 1, 0, 1]], [-1, 0, 2, -1], 3)])
+def test_two_launch_breakdown(ctx, dtype, block, rhs, iters):
+    """p.Ap = 0 at the first and at later iterations: blocks of small whole
+    numbers whose steps are dyadic, so that every sum is exact in any order
+    (rows hold zeros at their block's other offsets)."""
+    block, m = np.array(block, dtype), len(block)
+    n = 9000 // m * m
+    offs = np.arange(1 - m, m) if m > 1 else np.arange(-1, 2)
+    i = np.repeat(np.arange(n), len(offs))
+    j = i + np.tile(offs, n)
+    same = (j // m == i // m) & (j < n)
+    v = np.where(same, block[i % m, j % m], 0).astype(dtype)
+    if m == 1:
+        v *= 1 - 2 * (i % 2)
+    keep = (j >= 0) & (j < n)
+    ci, v = j[keep].astype(np.int32), v[keep]
+    rp = np.concatenate([[0], np.cumsum(np.bincount(i[keep], minlength=n))]).astype(np.int32)
+    assert expected(rp, ci, n, v.itemsize)[1]
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    invd = hflmp.invdiag(ctx, A)
+    b = np.tile(np.array(rhs, dtype), n // m)
+    want = _solve(ctx, A, 0, invd, b, dtol=1e30)
+    assert want[1:3] == (iters, 3)
+    _assert_same(_solve(ctx, A, hflmp.SELL_COL16, invd, b, dtol=1e30), want)
+    A.free()
+    invd.free()
+
+
+@pytest.mark.parametrize("dim,n", [(2, 120), (3, 24)])
+def test_refined_solve_two_launches(ctx, dim, n):
+    """The refined solve over FP32 in the offset form (two launches) and over
+    int32 columns (three): the same x, corrections and inner iterations, with
+    the search direction kept from inner solves of odd and even length."""
+    rp, ci, v = hflmp.fe_system(1, dim, n, hflmp.fe_kappa(dim, n, 1.0, 2))
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    A32 = A.astype_f32()
+    invd = hflmp.invdiag(ctx, A32)
+    db = ctx.upload(hflmp.fe_rhs(1, dim, n, 3))
+    S64 = hflmp.SellMatrix(ctx, A, 0)
+    forms = [hflmp.SellMatrix(ctx, A32, f) for f in (0, hflmp.SELL_COL16)]
+    assert expected(rp, ci, A.nrow, 4)[1]
+    need = ctx.L.hflmp_mpcg_sell_workspace_bytes(A.nrow)
+    first = set()
+    for flags in (0, hflmp.MP_RELIABLE):
+        for kw in (dict(inner_rtol=0.3), dict(inner_rtol=0.1), dict(inner_rtol=1e-2),
+                   dict(inner_rtol=1e-6, inner_maxit=7), dict(inner_rtol=1e-6, inner_maxit=8)):
+            got = []
+            for S32, short in ((forms[0], 0), (forms[1], 0), (forms[1], 256)):
+                dx, work = ctx.zeros(A.nrow, np.float64), ctx.empty(need - short, np.uint8)
+                one = hflmp.mpcg_jacobi_sell(ctx, S64, S32, invd, db, dx, rtol=1e-9, max_outer=1,
+                                             flags=flags, work=work, **kw)
+                first.add(one["inner_iters"] % 2)
+                dx.free()
+                dx = ctx.zeros(A.nrow, np.float64)
+                info = hflmp.mpcg_jacobi_sell(ctx, S64, S32, invd, db, dx, rtol=1e-9,
+                                              max_outer=200, flags=flags, work=work, **kw)
+                got.append((dx.download(), info["outer_iters"], info["inner_iters"],
+                            info["status"], info["res_final"]))
+                dx.free()
+                work.free()
+            assert got[0][1] > 1
+            _assert_same(got[1], got[0])
+            _assert_same(got[2], got[0])
+    assert first == {0, 1}
+    for a in (S64, db, invd, A32.val, A, *forms):
+        a.free()
