@@ -311,7 +311,9 @@ int create_plan(hflmp_ctx *ctx, int nrow, int ncol, int nnz, const int *rp, cons
   // candidates: runs of consecutive rows, then patches of lines of L rows
   std::vector<PlanGeom> cand;
   for (int r : {64, 32, 16, 8, 4}) cand.push_back(plan_geom(nrow, nrow, r, 1));
-  // (patches of a multiple of 4 rows: the four waves take equal shares)
+  // (patches of a multiple of 4 rows: a wave computes four at a time.  A block
+  // of fewer than 16 rows leaves computing waves idle; its staging, which all
+  // blocks share out alike, then decides.)
   if (L > 0)
     for (int nl = 2; nl <= kPlanMaxRuns; ++nl)
       for (int a = 2; a <= 16 && a <= L && a * nl <= 64; ++a)

@@ -399,6 +399,16 @@ __device__ __forceinline__ void plan_strip(T *s, const unsigned char *xl, int po
 // with a row a wave and its entries read from LDS by all lanes, 463 with
 // broadcasts, 412 with the roles apart, 303 with four rows (16 vectors: 449
 // with broadcasts, 390, 155; FP32, 64 vectors: 345, 298, 200).
+// Blocks of fewer than 16 rows give only R / 4 waves a turn, and are still
+// faster than a row a wave: 3D Q1 48^3 (blocks of 8 rows in FP64), us, a row a
+// wave and now: 64 vectors 136 and 100, 16 vectors 135 and 49; blocks of 4
+// rows of 75 entries, the most work for one wave, 64 vectors 56 and 57, 16
+// vectors 55 and 27.
+// The code is long (28 to 37 KB for four columns a lane) and entries of up to
+// 88 MB are loaded through the caches, so repeated products gain more than one
+// after other work; one call between two waits of the host, the caches swept
+// in between: 2D Q1 64^2, 64 vectors, FP64 27.2 -> 20.9 us (repeated 18.3 -> 11.4),
+// 400^2 83.8 -> 75.6 (64.7 -> 42.6).
 //
 // pre(i, u) leaves CV values for row i before its sums (what the epilogue
 // needs, loaded early); epi(i, s, u) gets row i's sums of the lane's columns
