@@ -295,7 +295,7 @@ constexpr size_t kCgVectors = 6;
 // none.  Of three 3D Q1 matrices in turn, us a product past and through the
 // caches: 64^3 (60 MB) 15.7 and 12.3, 96^3 (197 MB) 44.5 and 45.9, 128^3 in
 // FP32 (232 MB) 43.4 and 48.4.  (A product right after a kernel that has
-// written 1 GB waits for the cache to write that back: 64^3 18.7 past and 27.9
+// written 1 GB waits for the cache to write that back: 64^3 19.0 past and 27.9
 // through the caches, after one that has read 1 GB 18.7 and 16.3.)
 inline int entries_cached_once(long long entries, size_t entry_bytes, size_t vector_bytes) {
   return (size_t)entries * entry_bytes + vector_bytes <= ((size_t)88 << 20) ? kCachedParts : 0;

@@ -27,7 +27,6 @@
 // is where the sequential sweep's separate D pass leaves the value (no row
 // reads another row's scaled value before that row's backward step).
 #include <algorithm>
-#include <new>
 #include <vector>
 
 #include "hflmp_internal.hpp"
@@ -235,6 +234,41 @@ __global__ void __launch_bounds__(kPackRows)
   }
 }
 
+// The level-ordered copy: a thread a slot (lv levels of W, those past the
+// last one empty), slot l W + t from row t of level l: the entries that the
+// sweep subtracts, in storage order, and the first and last diagonal positions.
+template <bool FWD>
+__global__ void __launch_bounds__(kBlock)
+    sgs_pack_kernel(Blocks blk, const int *__restrict__ rp, const int *__restrict__ ci,
+                    const int *__restrict__ perm, const int *__restrict__ loff, int nlev,
+                    long long lv, int W, int E, int4 *__restrict__ rows, int2 *__restrict__ ent) {
+  for (long long k = (long long)blockIdx.x * kBlock + threadIdx.x; k < lv * W;
+       k += (long long)gridDim.x * kBlock) {
+    const long long l = k / W;
+    const int t = (int)(k - l * W);
+    int2 *mine = ent + l * E * W + t;
+    int4 d = make_int4(-1, 0, 0, 0);
+    if (l < nlev && t < loff[l + 1] - loff[l]) {
+      const int i = perm[loff[l] + t];
+      int lo, hi;
+      blk.range(i, lo, hi);
+      d = make_int4(i, 0, -1, -1);
+      for (int j = rp[i]; j < rp[i + 1]; ++j) {
+        const int c = ci[j];
+        if (c == i) {
+          if (d.z < 0) d.z = j;
+          d.w = j;
+          if (FWD) break;
+        } else if (FWD ? (c >= lo && c < i) : (c > i && c < hi)) {
+          mine[(long long)d.y++ * W] = make_int2(j, c);
+        }
+      }
+    }
+    for (int e = d.y; e < E; ++e) mine[(long long)e * W] = make_int2(0, 0);
+    rows[k] = d;
+  }
+}
+
 // A sweep's launches: a single level (rows k0..k1) or a run of small levels.
 struct Segment {
   bool small;
@@ -244,7 +278,7 @@ struct Segment {
 struct Sweep {
   int levels = 0;
   int *perm = nullptr;  // rows sorted by level (DEVICE)
-  int *loff = nullptr;  // level offsets into perm, levels + 1 (DEVICE)
+  int *loff = nullptr;  // level offsets into perm, levels + 1 (behind perm)
   std::vector<Segment> seg;
   // level-ordered copy of the pattern (packW = 0: none, the segments run)
   int packW = 0, packE = 0;
@@ -268,9 +302,7 @@ namespace {
 
 void sweep_free(Sweep &s) {
   (void)hipFree(s.perm);
-  (void)hipFree(s.loff);
   (void)hipFree(s.prow);
-  (void)hipFree(s.pent);
   s.perm = s.loff = nullptr;
   s.prow = nullptr;
   s.pent = nullptr;
@@ -284,99 +316,98 @@ void sgs_free(hflmp_sgs *m) {
   delete m;
 }
 
-// Bytes that a sweep's copy may take on the host and the device: what the
-// pattern and FP64 values take four times over, or 16 MB where that is more, and at
-// most 1 GB.  (The copy of 2D Q1 96^2 takes 0.9 of the CSR arrays, of 3D Q1
+// Bytes that a sweep's copy may take: what the pattern and FP64 values take
+// four times over, or 16 MB where that is more, and at most 1 GB.  (The copy of 2D Q1 96^2 takes 0.9 of the CSR arrays, of 3D Q1
 // 32^3 as well; eight slots a row with 16 entries each are 1.2 KB a row,
 // where a row may have few entries.)
 inline size_t pack_limit(size_t nnz, size_t n) {
   return std::min<size_t>(std::max<size_t>(4 * (12 * nnz + 4 * n), 16 << 20), 1 << 30);
 }
 
+// The pattern on the device, for the build: the caller's arrays where it was
+// downloaded from them, else a copy of the host's on first use (the caller's
+// device arrays need not hold it yet).
+struct DevicePattern {
+  int nrow, nnz;
+  const int *rp, *ci;      // the caller's, or null
+  const int *h_rp, *h_ci;
+  int *copy = nullptr;
+  ~DevicePattern() { (void)hipFree(copy); }
+  int get(hflmp_ctx *ctx) {
+    if (rp) return HFLMP_OK;
+    if (hipMalloc(&copy, sizeof(int) * ((size_t)nrow + 1 + nnz)) != hipSuccess) {
+      (void)hipGetLastError();
+      return HFLMP_ENOMEM;
+    }
+    HFLMP_HIP_CHECK(ctx, hipMemcpy(copy, h_rp, sizeof(int) * ((size_t)nrow + 1),
+                                   hipMemcpyHostToDevice));
+    HFLMP_HIP_CHECK(ctx, hipMemcpy(copy + nrow + 1, h_ci, sizeof(int) * (size_t)nnz,
+                                   hipMemcpyHostToDevice));
+    rp = copy;
+    ci = copy + nrow + 1;
+    return HFLMP_OK;
+  }
+};
+
 // The level-ordered copy (see sgs_packed_kernel) where it fits: levels of at
-// most kPackRows rows, at most kPackMaxE entries a row, no more than about
-// eight slots a row (levels of very uneven width would waste the rest), and
-// within pack_limit.  h_rp, h_ci: the pattern on the host.
-int build_packed(hflmp_ctx *ctx, const Blocks &blk, const int *h_rp, const int *h_ci, bool fwd,
-                 const std::vector<int> &off, const std::vector<int> &perm, Sweep &s) {
-  const int n = (int)perm.size(), nlev = s.levels;
-  int widest = 0, most = 0;
+// most kPackRows rows, at most kPackMaxE entries a row (most), no more than
+// about eight slots a row (levels of very uneven width would waste the rest),
+// and within pack_limit.  off: the level offsets; perm and loff are on the
+// device already.  Without room for it the segments run.
+template <bool FWD>
+int build_packed(hflmp_ctx *ctx, const Blocks &blk, DevicePattern &pat,
+                 const std::vector<int> &off, int most, Sweep &s) {
+  const int n = blk.nrow, nlev = s.levels;
+  int widest = 0;
   for (int l = 0; l < nlev; ++l) widest = std::max(widest, off[l + 1] - off[l]);
   const int W = (widest + kWave - 1) / kWave * kWave;
-  if (W > kPackRows || (long long)nlev * W > 8LL * n + 65536) return HFLMP_OK;
-  // the entries of row i that the sweep subtracts, in storage order, and the
-  // first and last diagonal positions
-  auto row_entries = [&](int i, int &d0, int &d1, auto &&f) {
-    int lo, hi;
-    blk.range(i, lo, hi);
-    d0 = d1 = -1;
-    for (int j = h_rp[i]; j < h_rp[i + 1]; ++j) {
-      const int c = h_ci[j];
-      if (c == i) {
-        if (d0 < 0) d0 = j;
-        d1 = j;
-        if (fwd) break;
-      } else if (fwd ? (c >= lo && c < i) : (c > i && c < hi)) {
-        f(j, c);
-      }
-    }
-  };
-  for (int i = 0; i < n; ++i) {
-    int d0, d1, cnt = 0;
-    row_entries(i, d0, d1, [&](int, int) { ++cnt; });
-    most = std::max(most, cnt);
-  }
-  if (most > kPackMaxE) return HFLMP_OK;
+  if (W > kPackRows || (long long)nlev * W > 8LL * n + 65536 || most > kPackMaxE) return HFLMP_OK;
   const int E = pack_width(most);
   const int D = kPackMaxE / E;
   const size_t lv = (size_t)nlev + 4 * (size_t)D;  // empty levels at the end
-  if (lv * W * (sizeof(int4) + E * sizeof(int2)) > pack_limit(h_rp[n], n)) return HFLMP_OK;
-  std::vector<int4> rows;
-  std::vector<int2> ent;
-  try {
-    rows.assign(lv * W, make_int4(-1, 0, 0, 0));
-    ent.assign(lv * E * W, make_int2(0, 0));
-  } catch (const std::bad_alloc &) {
-    return HFLMP_OK;  // no room for the copy: the segments run
-  }
-  for (int l = 0; l < nlev; ++l)
-    for (int k = off[l]; k < off[l + 1]; ++k) {
-      const int i = perm[k], t = k - off[l];
-      int d0, d1, e = 0;
-      row_entries(i, d0, d1,
-                  [&](int j, int c) { ent[((size_t)l * E + e++) * W + t] = make_int2(j, c); });
-      rows[(size_t)l * W + t] = make_int4(i, e, d0, d1);
-    }
-  if (hipMalloc(&s.prow, sizeof(int4) * rows.size()) != hipSuccess ||
-      hipMalloc(&s.pent, sizeof(int2) * ent.size()) != hipSuccess) {
+  const size_t row_bytes = lv * W * sizeof(int4), ent_bytes = lv * W * E * sizeof(int2);
+  if (row_bytes + ent_bytes > pack_limit(pat.nnz, n)) return HFLMP_OK;
+  const int rc = pat.get(ctx);
+  if (rc) return rc == HFLMP_ENOMEM ? HFLMP_OK : rc;
+  char *copy = nullptr;
+  if (hipMalloc(reinterpret_cast<void **>(&copy), row_bytes + ent_bytes) != hipSuccess) {
     (void)hipGetLastError();
-    (void)hipFree(s.prow);
-    (void)hipFree(s.pent);
-    s.prow = nullptr;
-    s.pent = nullptr;
     return HFLMP_OK;
   }
-  HFLMP_HIP_CHECK(ctx, hipMemcpy(s.prow, rows.data(), sizeof(int4) * rows.size(),
-                                 hipMemcpyHostToDevice));
-  HFLMP_HIP_CHECK(ctx, hipMemcpy(s.pent, ent.data(), sizeof(int2) * ent.size(),
-                                 hipMemcpyHostToDevice));
+  s.prow = reinterpret_cast<int4 *>(copy);
+  s.pent = reinterpret_cast<int2 *>(copy + row_bytes);
+  sgs_pack_kernel<FWD><<<grid_for((long long)(lv * W), 1), kBlock, 0, ctx->stream>>>(
+      blk, pat.rp, pat.ci, s.perm, s.loff, nlev, (long long)lv, W, E, s.prow, s.pent);
+  HFLMP_LAUNCH_CHECK(ctx);
+  HFLMP_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+  (void)hipFree(s.perm);
+  s.perm = s.loff = nullptr;
   s.packW = W;
   s.packE = E;
   return HFLMP_OK;
 }
 
-// Counting sort of the rows by level, the launch segments, and the upload.
+// Counting sort of the rows by level, its upload, and the copy or the launch
+// segments.  most: entries that a row takes part with.
+template <bool FWD>
 int build_sweep(hflmp_ctx *ctx, const std::vector<int> &level, int nlev, const Blocks &blk,
-                const int *h_rp, const int *h_ci, bool fwd, Sweep &s) {
+                DevicePattern &pat, int most, Sweep &s) {
   const int n = (int)level.size();
-  std::vector<int> off((size_t)nlev + 1, 0), perm(n);
+  // perm, then off
+  std::vector<int> host((size_t)n + nlev + 1), off((size_t)nlev + 1, 0);
   for (int i = 0; i < n; ++i) ++off[level[i] + 1];
   for (int l = 0; l < nlev; ++l) off[l + 1] += off[l];
+  std::copy(off.begin(), off.end(), host.begin() + n);
   std::vector<int> fill(off.begin(), off.end() - 1);
-  for (int i = 0; i < n; ++i) perm[fill[level[i]]++] = i;  // ascending rows within a level
+  for (int i = 0; i < n; ++i) host[fill[level[i]]++] = i;  // ascending rows within a level
   s.levels = nlev;
   s.seg.clear();
-  const int rc = build_packed(ctx, blk, h_rp, h_ci, fwd, off, perm, s);
+  if (hipMalloc(&s.perm, sizeof(int) * host.size()) != hipSuccess)
+    return set_error(ctx, HFLMP_ENOMEM, "sgs_create: out of device memory");
+  s.loff = s.perm + n;
+  HFLMP_HIP_CHECK(ctx, hipMemcpy(s.perm, host.data(), sizeof(int) * host.size(),
+                                 hipMemcpyHostToDevice));
+  const int rc = build_packed<FWD>(ctx, blk, pat, off, most, s);
   if (rc || s.packW) return rc;
   for (int l = 0; l < nlev;) {
     if (off[l + 1] - off[l] > kSmallLevel) {
@@ -389,13 +420,6 @@ int build_sweep(hflmp_ctx *ctx, const std::vector<int> &level, int nlev, const B
     s.seg.push_back({true, l, e});
     l = e;
   }
-  if (hipMalloc(&s.perm, sizeof(int) * (size_t)(n > 0 ? n : 1)) != hipSuccess ||
-      hipMalloc(&s.loff, sizeof(int) * ((size_t)nlev + 1)) != hipSuccess)
-    return set_error(ctx, HFLMP_ENOMEM, "sgs_create: out of device memory");
-  HFLMP_HIP_CHECK(ctx, hipMemcpy(s.perm, perm.data(), sizeof(int) * (size_t)n,
-                                 hipMemcpyHostToDevice));
-  HFLMP_HIP_CHECK(ctx, hipMemcpy(s.loff, off.data(), sizeof(int) * ((size_t)nlev + 1),
-                                 hipMemcpyHostToDevice));
   return HFLMP_OK;
 }
 
@@ -432,16 +456,19 @@ int sgs_create(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
   Blocks blk{nrow, num_blocks, nrow / num_blocks};
   // forward levels (rows ascending): entries up to the first diagonal one
   std::vector<int> lev(nrow);
-  int nf = 0;
+  int nf = 0, most_f = 0, most_b = 0;  // levels, and the entries of a row
   for (int i = 0; i < nrow; ++i) {
     int lo, hi;
     blk.range(i, lo, hi);
-    int l = 0;
+    int l = 0, cnt = 0;
     bool diag = false;
     for (int j = h_rp[i]; j < h_rp[i + 1]; ++j) {
       const int c = h_ci[j];
       if (c >= lo && c < hi) {
-        if (c < i) l = std::max(l, lev[c] + 1);
+        if (c < i) {
+          l = std::max(l, lev[c] + 1);
+          ++cnt;
+        }
         if (c == i) {
           diag = true;
           break;
@@ -452,6 +479,7 @@ int sgs_create(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
       return set_error(ctx, HFLMP_EFORMAT, "sgs_create: row %d has no diagonal entry", i);
     lev[i] = l;
     nf = std::max(nf, l + 1);
+    most_f = std::max(most_f, cnt);
   }
   auto *m = new hflmp_sgs();
   m->device = ctx->device;
@@ -462,7 +490,8 @@ int sgs_create(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
   m->rp = rp;
   m->ci = ci;
   m->val = val;
-  int rc = build_sweep(ctx, lev, nf, blk, h_rp, h_ci, true, m->fwd);
+  DevicePattern pat{nrow, nnz, hrp.empty() ? nullptr : rp, hrp.empty() ? nullptr : ci, h_rp, h_ci};
+  int rc = build_sweep<true>(ctx, lev, nf, blk, pat, most_f, m->fwd);
   if (rc) {
     sgs_free(m);
     return rc;
@@ -472,15 +501,19 @@ int sgs_create(hflmp_ctx *ctx, int nrow, int nnz, const int *rp, const int *ci,
   for (int i = nrow - 1; i >= 0; --i) {
     int lo, hi;
     blk.range(i, lo, hi);
-    int l = 0;
+    int l = 0, cnt = 0;
     for (int j = h_rp[i]; j < h_rp[i + 1]; ++j) {
       const int c = h_ci[j];
-      if (c > i && c < hi) l = std::max(l, lev[c] + 1);
+      if (c > i && c < hi) {
+        l = std::max(l, lev[c] + 1);
+        ++cnt;
+      }
     }
+    most_b = std::max(most_b, cnt);
     lev[i] = l;  // rows above i already hold their backward levels
     nbk = std::max(nbk, l + 1);
   }
-  rc = build_sweep(ctx, lev, nbk, blk, h_rp, h_ci, false, m->bwd);
+  rc = build_sweep<false>(ctx, lev, nbk, blk, pat, most_b, m->bwd);
   if (rc) {
     sgs_free(m);
     return rc;

@@ -7,6 +7,7 @@ counts, unsorted rows and FP32; then through the unchanged CG template
 CG with the same preconditioner: iterations within 2, solution within
 1e-8."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -202,3 +203,49 @@ def test_level_copy_is_bounded(ctx):
     for a in (dr, dz, M):
         a.free()
     assert held <= 2 * max(16 << 20, 4 * (12 * len(ci) + 4 * n)) + (8 << 20), held
+
+
+def test_level_copy_costs_little_to_make(ctx):
+    """Making the sweeps' level-ordered copies takes less than half as long as
+    the rest of the analysis: the same mesh with one row of 17 lower and one
+    of 17 upper entries has none."""
+    rp, ci, v = hflmp.fe_system(1, 2, 200)
+    n = len(rp) - 1
+    far = 30 + 2 * np.arange(17)  # (through COO: stored zeros stay)
+    B = sp.coo_matrix((np.append(v, np.ones(34)),
+                       (np.concatenate([np.repeat(np.arange(n), np.diff(rp)), np.full(17, n - 1),
+                                        np.zeros(17, int)]),
+                        np.concatenate([ci, n - 1 - far, far]))), shape=(n, n)).tocsr()
+    B.sort_indices()
+    best = []
+    for q in ((rp, ci, v), (B.indptr.astype(np.int32), B.indices.astype(np.int32), B.data)):
+        M = hflmp.CsrMatrix(ctx, *q)
+        t = []
+        for _ in range(9):
+            ctx.sync()
+            t0 = time.perf_counter()
+            S = hflmp.Sgs(ctx, M, 1, host_pattern=q[:2])
+            t.append(time.perf_counter() - t0)
+            S.destroy()
+        M.free()
+        best.append(min(t))
+    assert best[0] < 1.5 * best[1], best
+
+
+def test_host_pattern_alone_at_creation(ctx):
+    """With the pattern given on the host, the device arrays need not hold it
+    before the first apply."""
+    rp, ci, v = hflmp.fe_system(1, 2, 40)
+    r = np.random.default_rng(1).uniform(-1, 1, len(rp) - 1)
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    A.rp.copy_from_host(np.zeros_like(rp))
+    A.ci.copy_from_host(np.zeros_like(ci))
+    S = hflmp.Sgs(ctx, A, 1, host_pattern=(rp, ci))
+    A.rp.copy_from_host(rp)
+    A.ci.copy_from_host(ci)
+    dr, dz = ctx.upload(r), ctx.empty(len(r), np.float64)
+    S.apply(dr, dz)
+    assert np.array_equal(dz.download(), O.sgs_apply(rp, ci, v, r))
+    S.destroy()
+    for a in (dr, dz, A):
+        a.free()
