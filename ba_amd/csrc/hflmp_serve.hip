@@ -282,11 +282,11 @@ __device__ __forceinline__ bool quad_of(const SysDesc *__restrict__ sys,
 }
 
 // Where K2 leaves a unit's partials of r.r and r.z (element stride * unit).
-// K2 may still read K1's partials of p.Ap elsewhere in the system, so they
-// lie beside those: of the four floats a unit of a mixed system K1 takes one
-// and K2 the last two; of the two doubles of an FP64 system K1 takes one and
-// r.r the other, and r.z goes into Ap, at the unit's first row, which K2
-// itself has read for the last time.
+// FOLD: K2 may still read K1's partials of p.Ap elsewhere in the system, so
+// they lie beside those: of the four floats a unit of a mixed system K1 takes
+// one and K2 the last two; of the two doubles of an FP64 system K1 takes one
+// and r.r the other, and r.z goes into Ap, at the unit's first row, which K2
+// itself has read for the last time.  Else they replace K1's, side by side.
 template <typename T>
 struct UpdatePartials {
   T *rr;
@@ -294,8 +294,10 @@ struct UpdatePartials {
   T *rz;
   int rz_stride;
 };
+template <bool FOLD>
 __device__ __forceinline__ UpdatePartials<double> update_partials64(const SysDesc &d) {
-  return {d.part + d.nunits, 1, d.Ap, kBlock};
+  if (FOLD) return {d.part + d.nunits, 1, d.Ap, kBlock};
+  return {d.part, 2, d.part + 1, 2};
 }
 __device__ __forceinline__ UpdatePartials<float> update_partials32(const SysDesc &d) {
   float *base = part32(d) + 2 * (size_t)d.nunits;
@@ -842,7 +844,7 @@ __global__ void __launch_bounds__(kBlock)
     if (FOLD ? !fold_alpha(st, live, d.part, d.nunits, first, alpha) : !live) return;
     if (!FOLD) alpha = st->alpha;
     quad_update(i0, iend, alpha, d.p, d.Ap, d.x, d.r, d.z, pv, av, xv, rv, dv, rr, rz);
-    quad_partial2(rr, rz, update_partials64(d), g * k, jend);
+    quad_partial2(rr, rz, update_partials64<FOLD>(d), g * k, jend);
   } else {
     float pv[kQuad], av[kQuad], xv[kQuad], rv[kQuad], dv[kQuad], rr[kQuad], rz[kQuad];
     quad_load5(i0, iend, d.p32, d.Ap32, d.c32, d.r32, d.invd32, pv, av, xv, rv, dv);
@@ -864,7 +866,7 @@ __global__ void __launch_bounds__(kBlock) grp_beta_final(const SysDesc *__restri
     CgState<double> *st = &d.st->s64;
     if (st->status != kIterate) return;
     double rr, rz;
-    update_totals<8>(update_partials64(d), d.nunits, rr, rz);
+    update_totals<8>(update_partials64<false>(d), d.nunits, rr, rz);
     if (threadIdx.x == 0) {
       const int iter = st->iter + 1;
       const double res = sqrt(rr);
@@ -943,7 +945,7 @@ __global__ void __launch_bounds__(kBlock)
     CgState<double> *st = &d.st->s64;
     if (FOLD) {
       if (st->go == kGoStopped ||
-          fold_beta(st, update_partials64(d), d.nunits, first, beta) != kIterate)
+          fold_beta(st, update_partials64<true>(d), d.nunits, first, beta) != kIterate)
         return;
     } else {
       if (st->status != kIterate) return;
