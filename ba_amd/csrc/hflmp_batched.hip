@@ -236,22 +236,37 @@ struct BState {
 
 // per-column partial sums of one or two quantities, stored [q][column][block]
 // so that each column's partials are contiguous for its finalize workgroup.
-// Lane l holds column l, or with `sub` rows side by side column l mod k.
+// Lane l holds column l, or with `sub` rows side by side column l mod k; those
+// are added in pairs first, 32, 16, ... rows apart.  (One lane a column adding
+// all of them from LDS: 256 dependent adds for one column, 34 us an iteration
+// against 19 on 4,225 rows.)
 template <typename T, int NQ>
 __device__ __forceinline__ void block_col_partials(const T (&a)[NQ], int k, T *__restrict__ part,
                                                    int sub = 1) {
   __shared__ T lds[NQ][kWavesPerBlock][kWave];
   const int lane = threadIdx.x & (kWave - 1), wid = threadIdx.x / kWave;
+  T v[NQ];
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) lds[q][wid][lane] = a[q];
+  for (int q = 0; q < NQ; ++q) v[q] = a[q];
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    if (o >= sub) continue;  // (uniform)
+    const bool has = lane + o * k < sub * k;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const T w = __shfl_down(v[q], o * k);
+      if (has) v[q] += w;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) lds[q][wid][lane] = v[q];
   __syncthreads();
   if (wid == 0 && lane < k) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       T s = 0;
 #pragma unroll
-      for (int w = 0; w < kWavesPerBlock; ++w)
-        for (int j = 0; j < sub; ++j) s += lds[q][w][lane + j * k];
+      for (int w = 0; w < kWavesPerBlock; ++w) s += lds[q][w][lane];
       part[((size_t)q * k + lane) * gridDim.x + blockIdx.x] = s;
     }
   }

@@ -206,3 +206,22 @@ def test_batched_pcg_column_counts(ctx, k):
             a.free()
     A.free()
     invd.free()
+
+
+def test_few_columns_are_not_slower(ctx):
+    """An iteration on one column, its rows side by side in the waves, takes no
+    longer than on 64."""
+    rp, ci, v = hflmp.fe_system(1, 2, 64)
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    invd = hflmp.invdiag(ctx, A)
+    best = {1: np.inf, 64: np.inf}
+    for k in (1, 64) * 6:
+        B = ctx.upload(np.random.default_rng(k).uniform(-1, 1, A.nrow * k))
+        X = ctx.zeros(A.nrow * k, np.float64)
+        info = hflmp.batched_pcg_jacobi(ctx, A, invd, B, X, k, maxit=64, rtol=0.0)
+        best[k] = min(best[k], info["seconds"])
+        B.free()
+        X.free()
+    A.free()
+    invd.free()
+    assert best[1] < best[64], best
