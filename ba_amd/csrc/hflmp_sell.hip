@@ -407,27 +407,38 @@ __global__ void __launch_bounds__(kWave)
   }
 }
 
-// New values for the same pattern (thread per row); rows whose length
-// changed are skipped and counted.
+// New values for the same pattern; rows whose length changed are skipped and
+// counted.  A wave a slice, its values by way of LDS as in the fill (3D Q1
+// 64^3 in FP64: 52 us a call; a thread a row 142, the form with columns 125).
 template <typename T>
-__global__ void __launch_bounds__(kBlock)
-    sell_offsets_values_kernel(int nrow, int P, const int *__restrict__ rp,
+__global__ void __launch_bounds__(kWave)
+    sell_offsets_values_kernel(int nrow, int nslice, int P, const int *__restrict__ rp,
                                const T *__restrict__ val, const long long *__restrict__ koff,
                                const int *__restrict__ klen,
                                const unsigned long long *__restrict__ mask,
                                T *__restrict__ sval, const unsigned char *__restrict__ rlen,
                                unsigned int *changed) {
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < nrow; i += gridDim.x * kBlock) {
-    const int s = i / kSellRows, lane = i % kSellRows;
+  __shared__ T vals[kStageEntries];
+  const int lane = threadIdx.x;
+  for (int s = blockIdx.x; s < nslice; s += gridDim.x) {
     const long long base = koff[s];
     const int K = klen[s];
-    int k = rp[i];
-    if (rp[i + 1] - k != (int)rlen[i]) {
-      atomicAdd(changed, 1u);
-      continue;
+    const SliceRows r = slice_rows(s, nrow, rp);
+    const bool same = r.row < nrow && r.end - r.k == (int)rlen[r.row];
+    if (r.row < nrow && !same) atomicAdd(changed, 1u);
+    auto put = [&](auto value) {
+      int k = r.k;
+      for (int j = 0; j < K; ++j)
+        if (same && ((mask[base / kSellRows + j] >> lane) & 1))
+          sval[sell_pos(base, K, P, lane, j)] = value(k++);
+    };
+    const int n = r.last - r.first;
+    if (n <= kStageEntries && __all(r.k >= r.first && r.end <= r.last)) {
+      stage_entries(vals, val + r.first, n);
+      put([&](int k) { return vals[k - r.first]; });
+    } else {
+      put([&](int k) { return val[k]; });
     }
-    for (int j = 0; j < K; ++j)
-      if ((mask[base / kSellRows + j] >> lane) & 1) sval[sell_pos(base, K, P, lane, j)] = val[k++];
   }
 }
 
@@ -628,9 +639,9 @@ int sell_set_values(hflmp_ctx *ctx, hflmp_sell *m, const int *rp, const T *val) 
   int rc = hflmp_fill_zero(ctx, m->check, sizeof(unsigned int));
   if (rc) return rc;
   if (m->off_form)
-    sell_offsets_values_kernel<T><<<grid_for(m->nrow, 1), kBlock, 0, s>>>(
-        m->nrow, m->chunk, rp, val, m->soff, m->slen, m->mask, static_cast<T *>(m->val), m->rlen,
-        m->check);
+    sell_offsets_values_kernel<T><<<std::min(m->nslice, 1 << 20), kWave, 0, s>>>(
+        m->nrow, m->nslice, m->chunk, rp, val, m->soff, m->slen, m->mask,
+        static_cast<T *>(m->val), m->rlen, m->check);
   else
     sell_fill_kernel<T, int, false><<<grid_for(m->nrow, 1), kBlock, 0, s>>>(
       m->nrow, m->chunk, rp, nullptr, val, m->soff, m->slen, nullptr, static_cast<T *>(m->val),

@@ -372,3 +372,21 @@ def test_refined_solve_two_launches(ctx, dim, n):
     assert first == {0, 1}
     for a in (S64, db, invd, A32.val, A, *forms):
         a.free()
+
+
+def test_new_values_keep_their_speed(ctx):
+    """Refreshing the offset form's values takes no longer than refreshing
+    the form with int32 columns."""
+    rp, ci, v = hflmp.fe_system(1, 3, 64)
+    A = hflmp.CsrMatrix(ctx, rp, ci, v)
+    S = {f: hflmp.SellMatrix(ctx, A, f) for f in (0, hflmp.SELL_COL16)}
+    best = {f: np.inf for f in S}
+    for f in tuple(S) * 12:
+        ctx.sync()
+        t0 = time.perf_counter()
+        S[f].set_values(A)
+        ctx.sync()
+        best[f] = min(best[f], time.perf_counter() - t0)
+    for a in (*S.values(), A):
+        a.free()
+    assert best[hflmp.SELL_COL16] < best[0], best
