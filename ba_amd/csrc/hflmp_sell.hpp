@@ -35,8 +35,8 @@
 // ascending column order (the form is chosen only for such rows), so
 // ascending offsets are its storage order and the sums the same.
 // Measured (128^3 Q1, int16 columns before): FP64 SpMV 105.6 -> 91.6 us
-// (509 MB, 5.6 TB/s), the CG's 107.5 -> 98.5 us; FP32, the mixed solver's,
-// 57.6 -> 41.6 us.
+// (471 MB of arrays; 544 MB of traffic, 5.9 TB/s), the CG's 107.5 -> 98.5 us;
+// FP32, the mixed solver's, 57.6 -> 41.6 us.
 #pragma once
 
 #include "hflmp_spmv_tile.hpp"

@@ -11,9 +11,10 @@ val per nonzero, int32 row_ptr, x read once, y written once).
 
 Reported beside it, each measured in the same run:
   * the SpMV of the CSR-array row-tile kernel and of the compressed SELL-64
-    layout with int16 column offsets (the layout HIP_CSR_lMatrix builds
-    when every column fits; scored with the same CSR bytes, reported
-    separately as a compressed format);
+    layout that HIP_CSR_lMatrix builds (one column offset per slice and
+    position where a slice's rows share them, as here, else int16 columns
+    where they fit; scored with the same CSR bytes, reported separately as
+    a compressed format);
   * parity of both layouts against the oracle (bit-exact);
   * Jacobi-CG to 1e-8 on the same system (CSR and SELL operators);
   * mixed precision: log-normal diffusivity 128^3, FP32-inner / FP64-refined
@@ -218,8 +219,16 @@ def cg_record(info, N, nnz, vb=8):
             "res_final_rel": info["res_final"] / info["res_init"]}
 
 
+def sell_name(S):
+    """The form of a SELL-64 matrix, for the report."""
+    i = S.info()
+    if i["device_bytes"] < i["entries"] * (i["value_bytes"] + i["col_bytes"]):
+        return "SELL-64, offset form (no stored columns)"
+    return "SELL-64, int%d columns" % (8 * i["col_bytes"])
+
+
 def bench_cg(hflmp, ctx, A, S, Sw, b):
-    """Jacobi-CG to 1e-8 through SELL-64 with int16 columns (S, the layout
+    """Jacobi-CG to 1e-8 through compressed SELL-64 (S, the layout
     HIP_CSR_lMatrix builds), SELL-64 with int32 columns (Sw) and the CSR
     tiles (second solve of each timed)."""
     N, nnz = A.nrow, A.nnz
@@ -240,8 +249,7 @@ def bench_cg(hflmp, ctx, A, S, Sw, b):
                 xs = dx.download()
             dx.free()
         res[name] = cg_record(info, N, nnz)
-    res["sell"]["layout"] = "SELL-64, int16 columns" if S.info()["col_bytes"] == 2 \
-        else "SELL-64, int32 columns"
+    res["sell"]["layout"] = sell_name(S)
     db.free(); invd.free()
     return res, xs
 
@@ -266,6 +274,7 @@ def bench_c1(hflmp, n=256, seed=20241201):
         gi = hflmp.pcg_jacobi_sell(ctx, S, invd, db, dx, maxit=20000, rtol=1e-8)
         xg = dx.download()
         dx.free()
+    operator = sell_name(S)
     S.free(); invd.free(); db.free(); A.free()
     ctx.close()
     cpu, _ = cpu_cg(rp, ci, v, b, 1e-8, xg, gi["iters"])
@@ -275,7 +284,7 @@ def bench_c1(hflmp, n=256, seed=20241201):
     return {"workload": "2D Q1 Poisson %d^2 cells (%d DoFs, %d nonzeros), FP64, Jacobi-CG "
                         "to 1e-8, RHS seed %d" % (n, N, len(ci), seed),
             "gpu": {"iters": gi["iters"], "seconds_to_tol": round(gi["seconds"], 5),
-                    "operator": "SELL-64, int16 columns"},
+                    "operator": operator},
             "cpu_reference_path": cpu,
             "cpu_single_thread": {"seconds_to_tol": round(t1, 4), "iters": i1["iters"],
                                   "what": "CPUsimple platform: every operation on one thread"},
@@ -475,9 +484,9 @@ def bench_assembly(hflmp, n, kappa_seed=KAPPA_SEED):
 
 def bench_mixed(hflmp, n):
     """C3: log-normal diffusivity (sigma = 1), 128^3 Q1, relative residual
-    1e-10: plain FP64 CG vs FP32-inner / FP64-refined CG, both through the
-    SELL-64 operators with int16 columns; FP64 CG with int32 columns is
-    timed beside them."""
+    1e-10: plain FP64 CG vs FP32-inner / FP64-refined CG, both through
+    compressed SELL-64 operators; FP64 CG with int32 columns is timed beside
+    them."""
     from oracle import oracle as O
     kap = hflmp.fe_kappa(3, n, 1.0, KAPPA_SEED)
     rp, ci, v = hflmp.fe_system(1, 3, n, kap)
@@ -493,12 +502,10 @@ def bench_mixed(hflmp, n):
     db = ctx.upload(b)
     out = {"workload": "3D Q1 log-normal diffusivity (sigma 1) %d^3, Jacobi, rtol 1e-10" % n,
            "seeds": {"kappa": KAPPA_SEED, "rhs": RHS_SEED},
-           "timing": "FP64 (int16 and int32 columns), reliable and restart solves in turn, "
+           "timing": "FP64 (compressed and int32 columns), reliable and restart solves in turn, "
                      "3 rounds after a warm-up round, fastest round of each",
-           "fp64_operator": "SELL-64, %s columns" % ("int16" if S64.info()["col_bytes"] == 2
-                                                      else "int32"),
-           "fp32_operator": "SELL-64, %s columns" % ("int16" if S32.info()["col_bytes"] == 2
-                                                      else "int32")}
+           "fp64_operator": sell_name(S64),
+           "fp32_operator": sell_name(S32)}
     # The three solves are timed in turn, three rounds after a warm-up
     # round, and each keeps its fastest round: run-to-run drift of the
     # device then touches all three alike.
@@ -940,7 +947,7 @@ def run_server_stream(hflmp, ctx, feed_specs, arrivals, cfg, rtol, precision, ke
 
 def run_singles(hflmp, ctx, specs, rtol):
     """One at a time, device-resident FP64 Jacobi-CG per request: upload,
-    SELL-64 build (int16 columns where they fit), Jacobi, solve, download.
+    compressed SELL-64 build, Jacobi, solve, download.
     The requests come from the same generator as the server's (RequestFeed,
     8 host threads working ahead of the solves), so both runs share the
     host with the generation.  Returns the requests too (for parity)."""
@@ -1307,7 +1314,7 @@ def main():
         out["cpu_baseline_naive"] = naive
         if "cg" in out:
             # CG time to 1e-8 at 128^3 along the reference's CPU path, and
-            # the GPU's int16 SELL-64 solve against it
+            # the GPU's compressed SELL-64 solve against it
             g = out["cg"]["sell"]
             ccg, _ = cpu_cg(rp, ci, v, b, 1e-8, x_cg, g["iters"])
             ccg["speedup_gpu_sell_int16_vs_cpu"] = round(ccg["seconds_to_tol"] /
