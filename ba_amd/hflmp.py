@@ -675,7 +675,8 @@ EFORMAT = -6
 
 class SellMatrix:
     """SELL-64 device layout of a device CSR matrix (hflmp_sell_*), built on
-    the device; flags SELL_COL16 asks for int16 slice-offset columns."""
+    the device; flags SELL_COL16 allows compressed columns (one offset per
+    slice and position, or int16 slice offsets)."""
 
     def __init__(self, ctx, A, flags=0):
         self.ctx = ctx

@@ -456,8 +456,11 @@ int hflmp_pcg_jacobi_f32(hflmp_ctx *ctx, int nrow, int nnz, const int *row_ptr,
                          void *work, size_t work_bytes, hflmp_solve_info *info);
 /* The same solve with the operator in SELL-64 layout.  The products are
  * identical; the dot products group their per-workgroup partials over 256
- * rows instead of one CSR tile, so iterates agree to rounding.  Workspace
- * as hflmp_pcg_workspace_bytes(nrow, nnz, value_bytes). */
+ * rows instead of one CSR tile, so iterates agree to rounding.  Systems of a
+ * few thousand rows run all iterations in one workgroup, and small ones
+ * without stored columns two kernels an iteration, with the same results.
+ * Workspace as hflmp_pcg_workspace_bytes(nrow, nnz, value_bytes); one vector
+ * less is accepted and runs three kernels. */
 int hflmp_pcg_jacobi_sell_f64(hflmp_ctx *ctx, const hflmp_sell *A,
                               const double *invdiag, const double *b, double *x,
                               int maxit, double atol, double rtol, double dtol,
@@ -804,8 +807,8 @@ int hflmp_mpcg_jacobi(hflmp_ctx *ctx, int nrow, int nnz, const int *row_ptr,
                       double inner_rtol, int flags, void *work, size_t work_bytes,
                       hflmp_mp_info *info);
 /* The same refinement with both operators in SELL-64 layout: A64 (FP64
- * values) for the residual and A32 (FP32 values, int16 columns where they
- * fit) for the inner solve; flags: HFLMP_MP_RELIABLE.  Workspace:
+ * values) for the residual and A32 (FP32 values, compressed columns where
+ * they fit) for the inner solve; flags: HFLMP_MP_RELIABLE.  Workspace:
  * hflmp_mpcg_sell_workspace_bytes. */
 size_t hflmp_mpcg_sell_workspace_bytes(int nrow);
 int hflmp_mpcg_jacobi_sell(hflmp_ctx *ctx, const hflmp_sell *A64,
