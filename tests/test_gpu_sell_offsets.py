@@ -233,8 +233,9 @@ def test_many_slices(ctx, nrow):
 
 
 def test_unstructured_build_keeps_its_speed(ctx):
-    """Looking for shared offsets costs an unstructured matrix, which has none,
-    less than the rest of its build (int32 columns, which do not look)."""
+    """Looking for shared offsets, which an unstructured matrix does not have,
+    does not make its build 2.3 times that with int32 columns, which does not
+    look (1.6 measured; 2.9 to 3.6 with all slices walked)."""
     rng = np.random.default_rng(0)
     rp, ci, v = hflmp.fe_system(1, 2, 300)
     n = len(rp) - 1
@@ -251,7 +252,7 @@ def test_unstructured_build_keeps_its_speed(ctx):
         best[flags] = min(best.get(flags, np.inf), time.perf_counter() - t0)
         S.free()
     A.free()
-    assert best[hflmp.SELL_COL16] < 2 * best[0], best
+    assert best[hflmp.SELL_COL16] < 2.3 * best[0], best
 
 
 def _solve(ctx, A, flags, invd, b, short=0, **kw):
